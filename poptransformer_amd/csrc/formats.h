@@ -78,6 +78,11 @@ struct FmtF16 : F16Product {
     return bitcast<f16x8>(raw[j]);
   }
   static __device__ __forceinline__ float finish(float acc, Scale) { return acc; }
+  // of gemm_block_kernel: features of a stage; a lane's bytes of an operand, where those of half m of 64 features lie, and the operand
+  static constexpr int kStage = 32;
+  typedef f16x8 Piece;
+  static constexpr int piece_at(int m) { return m * 1024; }
+  static __device__ __forceinline__ f16x8 operand(Piece p) { return p; }
 };
 
 
@@ -146,6 +151,28 @@ struct FmtF8 : F16Product {
   static __device__ __forceinline__ float finish(float acc, Scale s) { return acc * s.mul; }
 };
 
+// F143 weights for gemm_block_kernel.  Moved to fp16 bits 13..7 with their sign in bit 15 the seven magnitude bits are the
+// fp16 number decode(byte) * 2^-7, subnormals among them, which the matrix unit takes at their value: three instructions for two
+// weights (the 2^7 joins the exponent of the sum) where f143_pair, whose result is the number itself, has five.
+struct FmtF143Block : FmtF8<0> {
+  static __device__ __forceinline__ Scale load_scale(const void* scale, const int32_t* x_scale, int, int) {
+    const int e = reinterpret_cast<const int32_t*>(scale)[0] + (x_scale ? x_scale[0] : 0);
+    return Scale{ldexpf(1.0f, e + 7)};
+  }
+  static constexpr int kStage = 64;                          // (a vector holds 64 features of a channel)
+  typedef u32x2 Piece;
+  static constexpr int piece_at(int m) { return m * 8; }
+  static __device__ __forceinline__ uint32_t pair(uint32_t bytes, uint32_t select) {
+    typedef short i16x2 __attribute__((ext_vector_type(2)));
+    const i16x2 t = bitcast<i16x2>(__builtin_amdgcn_perm(0, bytes, select)) >> (short)1;      // sign in bits 15 and 14
+    return bitcast<uint32_t>(t) & 0xBF80BF80u;
+  }
+  static __device__ __forceinline__ f16x8 operand(Piece p) {
+    const u32x4 r = {pair(p[0], 0x010C000Cu), pair(p[0], 0x030C020Cu), pair(p[1], 0x010C000Cu), pair(p[1], 0x030C020Cu)};
+    return bitcast<f16x8>(r);
+  }
+};
+
 
 // bf16 weights and activations: the tiles of FmtF16 with bf16 elements (an operand travels through the core as the
 // sixteen bytes it is), and the fp32 epilogue.
@@ -156,7 +183,16 @@ struct FmtBF16 {
   static __device__ __forceinline__ Scale load_scale(const void*, const int32_t*, int, int) { return Scale{}; }
   static __device__ __forceinline__ f16x8 a_operand(const u32x4 (&raw)[4], int j, Scale) { return bitcast<f16x8>(raw[j]); }
   static __device__ __forceinline__ float finish(float acc, Scale) { return acc; }
+  static constexpr int kStage = 32;
+  typedef f16x8 Piece;
+  static constexpr int piece_at(int m) { return m * 1024; }
+  static __device__ __forceinline__ f16x8 operand(Piece p) { return p; }
   static __device__ __forceinline__ f32x4 mma(f16x8 a, f16x8 b, f32x4 c) {
     return __builtin_amdgcn_mfma_f32_16x16x32_bf16(bitcast<bf16x8>(a), bitcast<bf16x8>(b), c, 0, 0, 0);
   }
 };
+
+// the formats of gemm_block_kernel
+template <> struct BlockFormat<FmtF16> { static constexpr bool ok = true; typedef FmtF16 type; };
+template <> struct BlockFormat<FmtBF16> { static constexpr bool ok = true; typedef FmtBF16 type; };
+template <> struct BlockFormat<FmtF8<0>> { static constexpr bool ok = true; typedef FmtF143Block type; };

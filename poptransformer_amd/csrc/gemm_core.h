@@ -227,6 +227,33 @@ __device__ __forceinline__ void wide_put_pair4(const GemmMat& mat, int m, int n,
   }
 }
 
+// eight of them, n a multiple of eight
+__device__ __forceinline__ void wide_put8(const GemmMat& mat, int m, int n, f32x4 v0, f32x4 v1) {
+  const WideOut& w = mat.wide;
+  if (n + 8 <= w.n_main && (w.ld & 7) == 0 && !w.out_f32 && !w.mul) {
+    bf16x8 b;
+#pragma unroll
+    for (int r = 0; r < 8; ++r) b[r] = (bf16)wide_value(w, n + r, r < 4 ? v0[r & 3] : v1[r & 3]);
+    *reinterpret_cast<bf16x8*>(reinterpret_cast<bf16*>(mat.Y) + (size_t)m * w.ld + n) = b;
+    return;
+  }
+  wide_put4(mat, m, n, v0);
+  wide_put4(mat, m, n + 4, v1);
+}
+
+__device__ __forceinline__ void wide_put_pair8(const GemmMat& mat, int m, int n, f32x4 g0, f32x4 g1, f32x4 u0, f32x4 u1) {
+  const WideOut& w = mat.wide;
+  if (n + 8 <= w.n_main && (w.ld & 7) == 0 && !w.out_f32 && !w.mul) {
+    bf16x8 b;
+#pragma unroll
+    for (int r = 0; r < 8; ++r) b[r] = (bf16)wide_pair_value(w, n + r, r < 4 ? g0[r & 3] : g1[r & 3], r < 4 ? u0[r & 3] : u1[r & 3]);
+    *reinterpret_cast<bf16x8*>(reinterpret_cast<bf16*>(mat.Y) + (size_t)m * w.ld + n) = b;
+    return;
+  }
+  wide_put_pair4(mat, m, n, g0, u0);
+  wide_put_pair4(mat, m, n + 4, g1, u1);
+}
+
 // the rows from m0 on
 static inline void wide_skip_rows(GemmMat& mat, int m0) {
   WideOut& w = mat.wide;
@@ -1277,18 +1304,50 @@ __global__ __launch_bounds__(NWV * 64) void gemm_tile_kernel(GemmArgs a) {
 }
 
 // Second half of a K split: adds the slices' fp32 sums of one matrix and applies what the one-kernel form
-// applies to its sum (the format's scale, bias, activation, epilogue).
-template <class Fmt>
+// applies to its sum (the format's scale, bias, activation, epilogue).  V: channels of a thread (four where they divide: 16 bytes
+// of every slice).
+template <class Fmt, int V>
 __global__ __launch_bounds__(256) void splitk_finish_kernel(GemmArgs a) {
   const GemmMat& mat = a.mat[0];
   const int N = mat.N;
   const size_t total = (size_t)a.M * N;
-  const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
+  const size_t i = ((size_t)blockIdx.x * 256 + threadIdx.x) * V;
   if (i >= total) return;
   const int m = (int)(i / N), n = (int)(i % N);
-  float t = 0.f;
-  for (int sl = 0; sl < a.ksplit; ++sl) t += a.part[(size_t)sl * total + i];
-  gemm_put<Fmt>(a, mat, m, n, N, Fmt::finish(t, Fmt::load_scale(mat.scale, a.x_scale, n, N)));
+  if constexpr (V == 4) {
+    f32x4 t = {0.f, 0.f, 0.f, 0.f};
+    for (int sl = 0; sl < a.ksplit; ++sl) {
+      const f32x4 v = *reinterpret_cast<const f32x4*>(a.part + (size_t)sl * total + i);
+#pragma unroll
+      for (int r = 0; r < 4; ++r) t[r] += v[r];
+    }
+    if constexpr (Fmt::kWide) {
+      wide_put4(mat, m, n, t);
+    } else {
+      f16x4 y;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        f16 y0 = (f16)Fmt::finish(t[r], Fmt::load_scale(mat.scale, a.x_scale, n + r, N));
+        if (mat.bias) y0 = y0 + mat.bias[n + r];
+        y[r] = apply_epilogue(a.epi, apply_act(mat.act, y0), m, n + r, N);
+      }
+      *reinterpret_cast<f16x4*>(mat.Y + i) = y;
+    }
+  } else {
+    float t = 0.f;
+    for (int sl = 0; sl < a.ksplit; ++sl) t += a.part[(size_t)sl * total + i];
+    gemm_put<Fmt>(a, mat, m, n, N, Fmt::finish(t, Fmt::load_scale(mat.scale, a.x_scale, n, N)));
+  }
+}
+
+template <class Fmt>
+static void launch_splitk_finish(const GemmArgs& a, hipStream_t s) {
+  const size_t total = (size_t)a.M * a.mat[0].N;
+  // (four channels of a row at once where no four cross its end and Y's vectors are whole)
+  if (a.mat[0].N % 4 == 0 && (Fmt::kWide || pta_aligned(a.mat[0].Y, 8)))
+    hipLaunchKernelGGL((splitk_finish_kernel<Fmt, 4>), dim3((unsigned)((total / 4 + 255) / 256)), dim3(256), 0, s, a);
+  else
+    hipLaunchKernelGGL((splitk_finish_kernel<Fmt, 1>), dim3((unsigned)((total + 255) / 256)), dim3(256), 0, s, a);
 }
 
 template <class Fmt, int MT, int KQ, bool PAIR, int NWV = TILE_WAVES>
@@ -1308,10 +1367,7 @@ static int launch_gemm_tile(const GemmArgs& a, int total_nb, hipStream_t s, cons
   const int per_wg = PAIR ? WPG : 2 * WPG;
   const int nsl = a.ksplit > 1 ? a.ksplit : 1;
   hipLaunchKernelGGL((gemm_tile_kernel<Fmt, MT, KQ, PAIR, NWV>), dim3(total_nb / per_wg, nsl), dim3(NWV * 64), smem, s, a);
-  if (nsl > 1) {
-    const size_t total = (size_t)a.M * a.mat[0].N;
-    hipLaunchKernelGGL(splitk_finish_kernel<Fmt>, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, s, a);
-  }
+  if (nsl > 1) launch_splitk_finish<Fmt>(a, s);
   return PTA_OK;
 }
 
@@ -1556,7 +1612,7 @@ static int reserve_gemm_rows(size_t* smem, const char* name) {
   return PTA_OK;
 }
 
-// Tiles of listed rows (at most RG * 128 each, up to max_tiles of them) of a matrix, or of a gate / up pair; wide formats.
+// As launch_gemm_block_listed, where the rows lie further apart than its 32-bit offsets reach.
 template <class Fmt, int RG, bool PAIR>
 static int launch_gemm_listed(const GemmArgs& a, int total_nb, int max_tiles, const ListedRows& rows, hipStream_t s, const char* name) {
   size_t smem;
@@ -1579,21 +1635,18 @@ static int launch_gemm_rows(const GemmArgs& a, int total_nb, hipStream_t s, cons
   const int nsl = a.ksplit > 1 ? a.ksplit : 1;
   const int per = (groups * row_blocks + 7) / 8;
   hipLaunchKernelGGL((gemm_rows_kernel<Fmt, RG, PAIR>), dim3(per * 8, nsl), dim3(ROWS_WAVES * 64), smem, s, a, groups, row_blocks, AllRows{});
-  if (nsl > 1) {
-    const size_t total = (size_t)a.M * a.mat[0].N;
-    hipLaunchKernelGGL((splitk_finish_kernel<Fmt>), dim3((unsigned)((total + 255) / 256)), dim3(256), 0, s, a);
-  }
+  if (nsl > 1) launch_splitk_finish<Fmt>(a, s);
   return PTA_OK;
 }
 
 // The sums of a wave's tile (RG row groups x NST channel blocks; lane l holds channels st * 16 + (l / 16) * 4 + r of
-// row l % 16 of each row group) go out: unit cw of the workgroup, first block blk0 of matrix mi, rows from row0.
+// row l % 16 of each row group) go out: unit cw of the workgroup, first block blk0 of matrix mi, rows from row0 of M,
+// to the rows of Y that `order` lists (null: the same).
 template <class Fmt, int NST, int RG, bool PAIR>
 __device__ __forceinline__ void panel_store(const GemmArgs& a, f32x4 (&acc)[RG][NST], unsigned char* smem, int cw, int mi, int blk0,
-                                            int row0, int nsl, typename Fmt::Scale s0, typename Fmt::Scale s1) {
+                                            int row0, int nsl, typename Fmt::Scale s0, typename Fmt::Scale s1, int M, const int32_t* order = nullptr) {
   constexpr int SW = NST * 16 + 4;                // floats per row of a wave's epilogue strip
   const int lane = threadIdx.x & 63;
-  const int M = a.M;
   // Lane l holds channels st * 16 + (l / 16) * 4 + r of row l % 16 of each row group.  Row group by row group the
   // sums pass through a strip of LDS of the wave's own (the row buffers are free after the last barrier) and come
   // back with eight consecutive channels of one row per lane: one 16-byte store per lane, whole 128-byte stretches
@@ -1626,6 +1679,10 @@ __device__ __forceinline__ void panel_store(const GemmArgs& a, f32x4 (&acc)[RG][
         const f32x4 g0 = *reinterpret_cast<const f32x4*>(strip + rr * SW + c0), g1 = *reinterpret_cast<const f32x4*>(strip + rr * SW + c0 + 4);
         const f32x4 u0 = *reinterpret_cast<const f32x4*>(strip + rr * SW + NST / 2 * 16 + c0), u1 = *reinterpret_cast<const f32x4*>(strip + rr * SW + NST / 2 * 16 + c0 + 4);
         if (m >= M) continue;
+        if constexpr (Fmt::kWide) {
+          wide_put_pair8(mat, order ? order[m] : m, n, g0, g1, u0, u1);
+          continue;
+        }
         f16x8 y;
 #pragma unroll
         for (int j = 0; j < 8; ++j)
@@ -1658,6 +1715,10 @@ __device__ __forceinline__ void panel_store(const GemmArgs& a, f32x4 (&acc)[RG][
             for (int j = 0; j < 8; ++j)
               if (n + j < N) p[j] = j < 4 ? v0[j & 3] : v1[j & 3];
           }
+          continue;
+        }
+        if constexpr (Fmt::kWide) {
+          wide_put8(mat, order ? order[m] : m, n, v0, v1);
           continue;
         }
         f16x8 y;
@@ -1899,7 +1960,307 @@ __global__ __launch_bounds__(PANEL_WAVES * 64) __attribute__((amdgpu_waves_per_e
 
   const typename Fmt::Scale s0 = Fmt::load_scale(a.mat[PAIR ? 0 : mi].scale, a.x_scale, 0, 1);   // no format's finish uses the per-channel part
   const typename Fmt::Scale s1 = Fmt::load_scale(a.mat[PAIR ? 1 : mi].scale, a.x_scale, 0, 1);
-  panel_store<Fmt, NST, RG, PAIR>(a, acc, smem, cw, mi, blk0, row0, nsl, s0, s1);
+  panel_store<Fmt, NST, RG, PAIR>(a, acc, smem, cw, mi, blk0, row0, nsl, s0, s1, M);
+}
+
+// ------------------------------------------------------------------------------------------
+// Variant for hundreds of rows of formats with more than one vector per tile (16-bit and FP8 weights): both operands
+// through LDS.  A workgroup of 8 waves (2 row halves x 4 channel quarters) owns 32 * RG rows and 256 channels (a
+// pair: 128 gate and 128 up channels); loads that write LDS directly bring stages of Fmt::kStage features of both.
+// At 256 x 256 a 64-feature step is 64 KiB for 8.4 MFLOP, a quarter of the bytes per product that gemm_rows_kernel's
+// workgroups (256 x 128, weights through registers) take.
+// What bounds it: the matrix unit at the clock that the power leaves (1.7 GHz in long launches), and the loads.  A step of 64
+// features takes 1.1 us without them on zeros, 1.27 on random numbers, 1.5 from the caches and 1.6 to 1.75 with weights
+// from HBM (1.2 PFLOP/s; 128 rows: 0.85 to 0.95).  FP8: two stages of 64 features 1.75, three 1.6; 16-bit: two of 64 or five of 32 alike.
+// One load per block of MFMAs: a compute unit holds a wave that asks for more at once.
+// Channels need not divide: blocks past a matrix's last one lie past its descriptor and read as zeros.
+// ------------------------------------------------------------------------------------------
+constexpr int BLOCK_WAVES = 8;
+constexpr int BLOCK_CB = 16;                 // channel blocks of a workgroup
+constexpr double BLOCK_STEP_256 = 1.6, BLOCK_STEP_128 = 0.92;      // us of a step of 64 features (measured, all compute units at work)
+
+// v, of which the compiler no longer knows where it is from
+__device__ __forceinline__ u32x4 as_computed(u32x4 v) {
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    uint32_t e = v[i];
+    asm volatile("" : "+v"(e));
+    v[i] = e;
+  }
+  return v;
+}
+
+// a pointer that is the same in every lane, in scalar registers
+__device__ __forceinline__ const unsigned char* uniform_pointer(const unsigned char* p) {
+  const uint64_t v = reinterpret_cast<uint64_t>(p);
+  const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)v), hi = __builtin_amdgcn_readfirstlane((uint32_t)(v >> 32));
+  return reinterpret_cast<const unsigned char*>((uint64_t)hi << 32 | lo);
+}
+
+template <class Fmt>
+constexpr int block_stage_bytes(int rg) { return rg * 32 * Fmt::kStage * 2 + BLOCK_CB * Fmt::kVec * 8 * Fmt::kStage; }
+template <class Fmt>
+constexpr int block_stages(int rg) { return 160 * 1024 / block_stage_bytes<Fmt>(rg) < 5 ? 160 * 1024 / block_stage_bytes<Fmt>(rg) : 5; }
+
+template <class Fmt, int RG, bool PAIR, class Rows = AllRows>
+__global__ __launch_bounds__(BLOCK_WAVES * 64) __attribute__((amdgpu_waves_per_eu(2, 2))) void gemm_block_kernel(GemmArgs a, int group0, int groups, int row_blocks, Rows rows) {
+  constexpr int KV = Fmt::kVec, NST = 4;
+  constexpr int SF = Fmt::kStage;                 // features of a stage: 32 or 64
+  constexpr int WVEC = KV * 8 * SF;               // bytes of a channel block's features of a stage
+  constexpr int ROWS = RG * 32;
+  constexpr int XB = ROWS * SF * 2;               // bytes of a stage's rows
+  constexpr int STAGE = XB + BLOCK_CB * WVEC;
+  constexpr int NS = block_stages<Fmt>(RG);
+  constexpr int PPR = SF / 8;                     // 16-byte pieces of a row
+  constexpr int RPL = 64 / PPR;                   // rows of a load
+  constexpr int XL = ROWS / RPL / BLOCK_WAVES;    // row loads per wave and stage
+  constexpr int WL = WVEC / 1024;                 // loads per channel block; a wave brings two blocks
+  constexpr int LOADS = XL + 2 * WL;
+  constexpr int WAIT = (NS - 2) * LOADS;          // loads that may be on their way when a stage must have landed
+  static_assert((SF == 32 || SF == 64) && WVEC % 1024 == 0 && XL >= 1 && NS >= 2 && WAIT < 16, "stages");
+  extern __shared__ __align__(16) unsigned char smem[];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int wr = wave >> 2, wc = wave & 3;
+  const int K = a.K;
+  // workgroup id -> tile as in gemm_panel_kernel: contiguous stretches of the tile list per die, the row block fastest
+  int per = (int)gridDim.x / 8;
+  if constexpr (Rows::kListed) {                  // (the launch has room for the most tiles there can be)
+    row_blocks = *rows.n_tiles;
+    per = (groups * row_blocks + 7) / 8;
+    if ((int)blockIdx.x / 8 >= per) return;
+  }
+  const int tile = ((int)blockIdx.x % 8) * per + (int)blockIdx.x / 8;
+  if (tile >= groups * row_blocks) return;
+  const int row_block = tile % row_blocks;
+  int group = group0 + tile / row_blocks;
+  int M = a.M;
+  const int32_t* order = nullptr;
+  size_t weight_at = 0;
+  if constexpr (Rows::kListed) {
+    const int32_t* t = rows.tiles + row_block * 4;
+    weight_at = (size_t)t[0] * rows.weight_bytes;
+    order = rows.order + t[1];
+    M = t[2];
+  }
+  const int row0 = Rows::kListed ? 0 : row_block * ROWS;
+  int mi = 0;
+  if constexpr (!PAIR) {
+#pragma unroll
+    for (int i = 0; i < 3; ++i) {
+      const int g = i < a.count ? (a.mat[i].N + 255) / 256 : 0;
+      if (mi == i && i + 1 < a.count && group >= g) { group -= g; mi = i + 1; }
+    }
+  }
+  const int blk0 = group * (PAIR ? BLOCK_CB / 2 : BLOCK_CB);      // first block within its matrix
+  // the slice's features in steps of 64
+  const int nsl = a.ksplit > 1 ? a.ksplit : 1;
+  const int all = (K + 63) / 64, per_slice = ((a.KT + nsl - 1) / nsl) * 2;
+  const int first = (int)blockIdx.y * per_slice;
+  const int last = first + per_slice < all ? first + per_slice : all;
+  const int steps = last > first ? last - first : 0;
+
+  // this wave brings blocks 2 wave and 2 wave + 1 of the workgroup's sixteen (of a pair: eight gate, then eight up blocks)
+  const GemmMat& wm = a.mat[PAIR ? wave >> 2 : mi];
+  const int wb = blk0 + 2 * (PAIR ? wave & 3 : wave);
+  const uint32_t blk_bytes = (uint32_t)a.KT * (KV * 1024);
+  int there = (wm.N + 15) / 16 - wb;
+  there = __builtin_amdgcn_readfirstlane(there < 0 ? 0 : there < 2 ? there : 2);
+  const unsigned char* wp = uniform_pointer(reinterpret_cast<const unsigned char*>(wm.tiled) + weight_at + (size_t)(there ? wb : 0) * blk_bytes);
+  const __amdgpu_buffer_rsrc_t wres = __builtin_amdgcn_make_buffer_rsrc(const_cast<unsigned char*>(wp), 0, (int)(there * blk_bytes), 0x00020000);
+  const f16* X = a.mat[mi].X ? a.mat[mi].X : a.X;
+  const int rows_here = M - row0 < ROWS ? M - row0 : ROWS;
+  const __amdgpu_buffer_rsrc_t xres = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<f16*>(X + (size_t)row0 * K), 0, Rows::kListed ? 0x7fffffff : (int)((size_t)rows_here * K * 2), 0x00020000);
+
+  // A row's 16-byte pieces are exchanged: piece c of row r at c ^ swap(r), so that the sixteen rows of an operand read
+  // cover 256 bytes of banks once, and every eight of them 128.
+  auto swap = [](int r) { return SF == 64 ? ((r >> 1) & 7) ^ ((r & 1) << 2) : ((r >> 2) & 3) ^ (r & 2); };
+  const int lane_row = lane / PPR;
+  const int piece = (lane % PPR) ^ swap(RPL == 8 ? (wave & 1) * 8 + lane_row : lane_row);      // (the same in all loads of a lane)
+  const int x0 = (wave * RPL + lane_row) * (K * 2) + piece * 16;  // byte offset of its first row (past the last row: past the descriptor)
+  int listed[XL];
+  if constexpr (Rows::kListed) {
+#pragma unroll
+    for (int j = 0; j < XL; ++j) {
+      const int r = (j * BLOCK_WAVES + wave) * RPL + lane_row;
+      listed[j] = r < M ? order[r] / rows.x_div * (K * 2) + piece * 16 : -1;
+    }
+  }
+  // load q of stage s (of the K axis) into LDS at byte `at`; past the slice's end: zeros, from nowhere
+  const int end = last * (64 / SF);
+  auto bring = [&](int s, int at, int q) {
+    const bool in = s < end;
+    if (q < XL) {
+      const int off = Rows::kListed ? listed[q] : x0 + q * (BLOCK_WAVES * RPL * 2) * K;
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(xres, (__attribute__((address_space(3))) void*)(smem + at + (q * BLOCK_WAVES + wave) * 1024), 16,
+                                               in && s * SF + piece * 8 < K ? off : -1, s * (SF * 2), 0, 0);
+    } else {
+      const int b = (q - XL) / WL, v = (q - XL) % WL;
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(wres, (__attribute__((address_space(3))) void*)(smem + at + XB + (2 * wave + b) * WVEC + v * 1024), 16,
+                                               in ? (int)(b * blk_bytes) + lane * 16 : -1, s * WVEC + v * 1024, 0, 0);
+    }
+  };
+
+  f32x4 acc[RG][NST];
+#pragma unroll
+  for (int rg = 0; rg < RG; ++rg)
+#pragma unroll
+    for (int st = 0; st < NST; ++st) acc[rg][st] = f32x4{0.f, 0.f, 0.f, 0.f};
+
+  // operands of 32 features: half m of the stage at byte `at` (stages of 32 features are their half)
+  typedef typename Fmt::Piece Piece;              // a lane's bytes of a weight operand
+  const int a_at = XB + (PAIR ? wc * 2 : wc * 4) * WVEC + lane * 16;
+  auto a_piece = [&](int at, int m, int st) {
+    const int blk = PAIR ? st % 2 + (st / 2) * (BLOCK_CB / 2) : st;
+    return *reinterpret_cast<const Piece*>(smem + at + a_at + blk * WVEC + (SF == 64 ? Fmt::piece_at(m) : 0));
+  };
+  const int b_row = (wr * (RG * 16) + (lane & 15)) * (SF * 2);
+  const int b0 = b_row + ((lane >> 4) ^ swap(lane & 15)) * 16, b1 = SF == 64 ? b_row + ((4 + (lane >> 4)) ^ swap(lane & 15)) * 16 : b0;
+  auto b_operand = [&](int at, int m, int rg) { return *reinterpret_cast<const f16x8*>(smem + at + (m ? b1 : b0) + rg * (SF * 32)); };
+
+  // One pipeline over all steps: a step is two halves of 32 features, a half four blocks of RG MFMAs with one weight operand
+  // each.  The row operands of the next half are requested while this one's are multiplied (two sets of registers), the
+  // weight operand four blocks ahead.  The barrier stands where everything of a stage has been requested: behind it
+  // the stage takes what is NS stages on.  (The last half requests operands of one that does not exist and
+  // drops them: a condition here would stand between the MFMAs.)
+  f16x8 xf[2][RG];
+  Piece ahead[NST];
+#pragma unroll
+  for (int n = 0; n < NS; ++n)
+#pragma unroll
+    for (int q = 0; q < LOADS; ++q) bring(first * (64 / SF) + n, n * STAGE, q);
+  __builtin_amdgcn_s_waitcnt(0x0f70);             // vmcnt(0)
+  __syncthreads();
+#pragma unroll
+  for (int rg = 0; rg < RG; ++rg) xf[0][rg] = b_operand(0, 0, rg);
+#pragma unroll
+  for (int st = 0; st < NST; ++st) ahead[st] = a_piece(0, 0, st);
+  // (the compiler would otherwise make one load of these and of the same ones at the end of a step, at the step's begin)
+#pragma unroll
+  for (int rg = 0; rg < RG; ++rg) xf[0][rg] = bitcast<f16x8>(as_computed(bitcast<u32x4>(xf[0][rg])));
+  int at = 0, stage = first * (64 / SF) + NS;     // the stage whose operands are multiplied; the one to be asked for next
+  for (int i = 0; i < steps; ++i) {
+#pragma unroll
+    for (int m = 0; m < 2; ++m) {
+      const bool turn = SF == 32 || m == 1;       // this half's stage has been requested as a whole
+      const int nx = turn ? (at + STAGE == NS * STAGE ? 0 : at + STAGE) : at;
+      if (turn) {
+        __builtin_amdgcn_s_waitcnt(0x0070 | WAIT);      // the next stage has landed, and this wave's requests from this one
+        __builtin_amdgcn_s_barrier();
+        __builtin_amdgcn_sched_barrier(0);
+      }
+#pragma unroll
+      for (int st = 0; st < NST; ++st) {
+        if (turn) {
+#pragma unroll
+          for (int q = st * LOADS / NST; q < (st + 1) * LOADS / NST; ++q) bring(stage, at, q);
+        }
+        const f16x8 av = Fmt::operand(ahead[st]);
+        ahead[st] = a_piece(nx, 1 - m, st);
+#pragma unroll
+        for (int r = 0; r < RG / 4; ++r) xf[1 - m][st * (RG / 4) + r] = b_operand(nx, 1 - m, st * (RG / 4) + r);
+#pragma unroll
+        for (int rg = 0; rg < RG; ++rg) acc[rg][st] = Fmt::mma(av, xf[m][rg], acc[rg][st]);
+        __builtin_amdgcn_sched_barrier(0);        // (the requests stay where they are)
+      }
+      if (turn) ++stage;
+      at = nx;
+    }
+  }
+  __builtin_amdgcn_s_waitcnt(0x0070);
+  __syncthreads();                                // (what follows reuses the stages)
+  const typename Fmt::Scale s0 = Fmt::load_scale(a.mat[PAIR ? 0 : mi].scale, a.x_scale, 0, 1);   // no format's finish uses the per-channel part
+  const typename Fmt::Scale s1 = Fmt::load_scale(a.mat[PAIR ? 1 : mi].scale, a.x_scale, 0, 1);
+  panel_store<Fmt, NST, RG, PAIR>(a, acc, smem, wave, mi, blk0 + wc * (PAIR ? 2 : 4), row0 + wr * (RG * 16), nsl, s0, s1, M, order);
+}
+
+template <class Fmt, int RG, bool PAIR, class Rows>
+static int reserve_gemm_block(const char* name) {
+  static bool ready = false;
+  constexpr int smem = block_stages<Fmt>(RG) * block_stage_bytes<Fmt>(RG);
+  static_assert(smem <= 160 * 1024 && smem >= BLOCK_WAVES * 16 * 68 * 4, "LDS");
+  if (!ready) {
+    PTA_REQUIRE(hipFuncSetAttribute((const void*)gemm_block_kernel<Fmt, RG, PAIR, Rows>, hipFuncAttributeMaxDynamicSharedMemorySize, smem) == hipSuccess,
+                "%s: cannot reserve %d bytes of LDS", name, smem);
+    ready = true;
+  }
+  return PTA_OK;
+}
+
+// channel groups of the launch
+static inline int block_groups(const GemmArgs& a, bool pair) {
+  int g = 0;
+  for (int i = 0; i < (pair ? 1 : a.count); ++i) g += pair ? (a.mat[i].N + 127) / 128 : (a.mat[i].N + 255) / 256;
+  return g;
+}
+
+// channel groups [group0, group1) of the launch
+template <class Fmt, int RG, bool PAIR>
+static int launch_gemm_block(const GemmArgs& a, int group0, int group1, hipStream_t s, const char* name) {
+  const int rc = reserve_gemm_block<Fmt, RG, PAIR, AllRows>(name);
+  if (rc) return rc;
+  const int groups = group1 - group0, row_blocks = (a.M + RG * 32 - 1) / (RG * 32);
+  const int nsl = a.ksplit > 1 ? a.ksplit : 1;
+  const int per = (groups * row_blocks + 7) / 8;
+  hipLaunchKernelGGL((gemm_block_kernel<Fmt, RG, PAIR>), dim3(per * 8, nsl), dim3(BLOCK_WAVES * 64), block_stages<Fmt>(RG) * block_stage_bytes<Fmt>(RG), s, a,
+                     group0, groups, row_blocks, AllRows{});
+  if (nsl > 1) launch_splitk_finish<Fmt>(a, s);
+  return PTA_OK;
+}
+
+// Tiles of listed rows (at most RG * 32 each, up to max_tiles of them) of a matrix, or of a gate / up pair; wide formats.  x_rows:
+// rows of X.  (2048 rows, 6 of 32 experts of 4096 x 1376 each: pairs 579 -> 334 us, downs 373 -> 241, against gemm_rows_kernel)
+template <class Fmt, int RG, bool PAIR>
+static int launch_gemm_block_listed(const GemmArgs& a, size_t x_rows, int max_tiles, const ListedRows& rows, hipStream_t s, const char* name) {
+  if (x_rows * a.K * 2 > 0x7fffffffu) return launch_gemm_listed<Fmt, RG / 4, PAIR>(a, (a.mat[0].N + 15) / 16, max_tiles, rows, s, name);
+  const int rc = reserve_gemm_block<Fmt, RG, PAIR, ListedRows>(name);
+  if (rc) return rc;
+  const int groups = block_groups(a, PAIR);
+  hipLaunchKernelGGL((gemm_block_kernel<Fmt, RG, PAIR, ListedRows>), dim3((groups * max_tiles + 7) / 8 * 8), dim3(BLOCK_WAVES * 64),
+                     block_stages<Fmt>(RG) * block_stage_bytes<Fmt>(RG), s, a, 0, groups, max_tiles, rows);
+  return PTA_OK;
+}
+
+// How a launch is cut: the cheapest of 256 or 128 rows per workgroup, K in slices of workgroups (one matrix, a
+// workspace at hand), or the channel groups of the whole rounds with 256 rows and the rest with 128 - twice the workgroups, each half as long.
+template <class Fmt, bool PAIR>
+static int dispatch_gemm_block(const GemmArgs& a, hipStream_t s, const char* name) {
+  const int cus = device_compute_units(), groups = block_groups(a, PAIR);
+  const int blocks8 = (a.M + 255) / 256, blocks4 = (a.M + 127) / 128;
+  const double steps = (a.K + 63) / 64;
+  auto cost = [&](bool tall, int tiles, int nsl) {
+    const double finish = nsl > 1 ? 5.0 + (double)a.M * a.mat[0].N * (4.0 * nsl + 6.0) / 4.5e6 : 0.0;
+    return ((tiles * nsl + cus - 1) / cus) * ((tall ? BLOCK_STEP_256 : BLOCK_STEP_128) * steps / nsl + (tall ? 9.0 : 6.0)) + finish;
+  };
+  double best = cost(true, groups * blocks8, 1);
+  int how = 0, slices = 1;                        // 0: 256 rows, 1: 128 rows, 2: both
+  const double low = cost(false, groups * blocks4, 1);
+  if (low < best) { best = low; how = 1; }
+  const int whole = (groups * blocks8 / cus) * cus / blocks8;
+  if (whole > 0 && whole < groups) {
+    const double both = cost(true, whole * blocks8, 1) + cost(false, (groups - whole) * blocks4, 1) + 4.0;
+    if (both < best) { best = both; how = 2; }
+  }
+  if (!PAIR && a.count == 1 && a.part)
+    for (int nsl = 2; nsl <= GEMM_MAX_KSPLIT; ++nsl) {
+      if (a.KT < nsl * 4 || a.part_bytes < (size_t)nsl * a.M * a.mat[0].N * sizeof(float)) break;
+      for (int low_rows = 0; low_rows < 2; ++low_rows) {
+        const double c = cost(!low_rows, groups * (low_rows ? blocks4 : blocks8), nsl);
+        if (c < best) { best = c; how = low_rows; slices = nsl; }
+      }
+    }
+  GemmArgs b = a;
+  b.ksplit = slices;
+  int rc;
+  if (how == 2) {
+    rc = launch_gemm_block<Fmt, 8, PAIR>(b, 0, whole, s, name);
+    if (!rc) rc = launch_gemm_block<Fmt, 4, PAIR>(b, whole, groups, s, name);
+  } else {
+    rc = how == 0 ? launch_gemm_block<Fmt, 8, PAIR>(b, 0, groups, s, name) : launch_gemm_block<Fmt, 4, PAIR>(b, 0, groups, s, name);
+  }
+  if (rc) return rc;
+  PTA_CHECK_LAUNCH(name);
+  return PTA_OK;
 }
 
 // whether every matrix of the launch is a whole number of wave tiles of `nst` channel blocks and all share one input
@@ -1932,10 +2293,7 @@ static int launch_gemm_panel(const GemmArgs& a, int unit0, int unit1, hipStream_
   const int nsl = a.ksplit > 1 ? a.ksplit : 1;
   const int per = (groups * row_blocks + 7) / 8;
   hipLaunchKernelGGL((gemm_panel_kernel<Fmt, NST, RG, KH, PAIR>), dim3(per * 8, nsl), dim3(PANEL_WAVES * 64), smem, s, a, groups, row_blocks, unit0, unit1);
-  if (nsl > 1) {
-    const size_t total = (size_t)a.M * a.mat[0].N;
-    hipLaunchKernelGGL((splitk_finish_kernel<Fmt>), dim3((unsigned)((total + 255) / 256)), dim3(256), 0, s, a);
-  }
+  if (nsl > 1) launch_splitk_finish<Fmt>(a, s);
   return PTA_OK;
 }
 
@@ -1988,7 +2346,9 @@ static void launch_gemv(const GemmArgs& a, int total_nb, hipStream_t s) {
 template <class Fmt, bool PAIR>
 static int dispatch_gemv(const GemmArgs& a, int total_nb, hipStream_t s, const char* name);
 
-// More than 64 rows.  Beyond 128 rows gemm_panel_kernel, up to 128 (fp16 weights: any number) gemm_rows_kernel, where
+template <class Fmt> struct BlockFormat { static constexpr bool ok = false; };
+
+// More than 64 rows.  Beyond 128 rows gemm_block_kernel or (INT4) gemm_panel_kernel, up to 128 gemm_rows_kernel, where
 // the channel blocks divide into their workgroup tiles; a single matrix with few channels also splits K when a workspace is at hand.  Otherwise
 // the rows go through the smaller paths in turn, 64 at a time.
 template <class Fmt, bool PAIR>
@@ -1999,9 +2359,16 @@ static int dispatch_many_rows(const GemmArgs& a, int total_nb, hipStream_t s, co
   const bool tiles = a.epi.norm == PTA_NORM_NONE && tile_fits(a, per_wg, Fmt::kWide ? 0 : 2, PAIR);
   // More than 128 rows (measured on whole prompt passes of the 7B shape, gemm_rows_kernel against this: 6.5 against
   // 7.2 ms at 128 rows, 7.7 against 7.3 at 192, 8.1 against 7.5 at 256): 128-row panels through LDS, the weights
-  // straight into registers.  Formats of up to two vectors per tile only - with four (fp16) two tiles of four
-  // streams do not fit the registers.
-  if constexpr (Fmt::kVec <= 2) {
+  // straight into registers.
+  // Formats with a form of gemm_block_kernel: all launches of more than 128 rows.  Measured against the kernels they had before (us):
+  // FP8, 1000 rows: 4096 x 2 x 13696 pair 500 -> 198, 13696 x 4096 311 -> 110, 4096 x 4608 145 -> 60 (gemm_panel_kernel, whose two
+  // vectors per tile spill); bf16, 2048 rows: 4096 x 4096 102 -> 70, 11008 x 4096 261 -> 190; fp16 4096 x 2 x 11008 pair, 2048
+  // rows 564 -> 326, 512 rows 176 -> 103, 160 rows 83 -> 60 (gemm_rows_kernel).  At 65 to 128 rows the pair and 11008 features
+  // lose (0.75 to 0.9) what small matrices win (1.3): those stay.
+  if constexpr (BlockFormat<Fmt>::ok) {
+    if (a.M > 128 && a.epi.norm == PTA_NORM_NONE) return dispatch_gemm_block<typename BlockFormat<Fmt>::type, PAIR>(a, s, name);
+  }
+  if constexpr (Fmt::kVec <= 2 && !BlockFormat<Fmt>::ok) {
     if (a.M > 128 && panel_fits(a, 4, PAIR)) {
       const int units = PAIR ? total_nb / 2 : total_nb / 4;
       const int row_blocks = (a.M + 127) / 128;
@@ -2035,14 +2402,16 @@ static int dispatch_many_rows(const GemmArgs& a, int total_nb, hipStream_t s, co
     // fragments in registers, weights through LDS: 256 rows per workgroup where that still fills the machine,
     // else 128; few workgroups and one matrix: K in slices as well
     const int groups = total_nb / per_wg;
-    const bool two = a.M > 128 && (long)groups * ((a.M + 255) / 256) * 2 >= (long)cus;
+    const bool two = !BlockFormat<Fmt>::ok && a.M > 128 && (long)groups * ((a.M + 255) / 256) * 2 >= (long)cus;
     const int wgs = groups * (two ? (a.M + 255) / 256 : (a.M + 127) / 128);
     GemmArgs b = a;
     int nsl = wgs > 0 ? cus / wgs : 1;
     nsl = nsl > GEMM_MAX_KSPLIT ? GEMM_MAX_KSPLIT : nsl;
     while (nsl > 1 && a.KT < nsl * 8) --nsl;
     if (!PAIR && a.count == 1 && a.part && nsl > 1 && a.part_bytes >= (size_t)nsl * a.M * a.mat[0].N * sizeof(float)) b.ksplit = nsl;
-    const int rc = two ? launch_gemm_rows<Fmt, 2, PAIR>(b, total_nb, s, name) : launch_gemm_rows<Fmt, 1, PAIR>(b, total_nb, s, name);
+    int rc;
+    if constexpr (BlockFormat<Fmt>::ok) rc = launch_gemm_rows<Fmt, 1, PAIR>(b, total_nb, s, name);
+    else rc = two ? launch_gemm_rows<Fmt, 2, PAIR>(b, total_nb, s, name) : launch_gemm_rows<Fmt, 1, PAIR>(b, total_nb, s, name);
     if (rc) return rc;
     PTA_CHECK_LAUNCH(name);
     return PTA_OK;

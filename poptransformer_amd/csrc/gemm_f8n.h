@@ -576,7 +576,7 @@ __global__ __launch_bounds__(PANEL_WAVES * 64) __attribute__((amdgpu_waves_per_e
   }
   if (!active) return;
   const Fmt::Scale s0 = Fmt::load_scale(m0.scale, a.x_scale, 0, 1), s1 = Fmt::load_scale(m1.scale, a.x_scale, 0, 1);
-  panel_store<Fmt, NST, RG, PAIR>(a, acc, smem, cw, mi, blk0, row0, nsl, s0, s1);
+  panel_store<Fmt, NST, RG, PAIR>(a, acc, smem, cw, mi, blk0, row0, nsl, s0, s1, M);
 }
 
 // LDS of gemm_f8n_panel_kernel: two stages of both operands and their flags; the parts' meeting; the epilogue strips
@@ -606,10 +606,7 @@ static int launch_gemm_f8n_panel(const GemmArgs& a, int unit0, int unit1, hipStr
   const int nsl = a.ksplit > 1 ? a.ksplit : 1;
   const int per = (groups * row_blocks + 7) / 8;
   hipLaunchKernelGGL((gemm_f8n_panel_kernel<NST, RG, KH, PAIR>), dim3(per * 8, nsl), dim3(PANEL_WAVES * 64), smem, s, a, groups, row_blocks, unit0, unit1);
-  if (nsl > 1) {
-    const size_t total = (size_t)a.M * a.mat[0].N;
-    hipLaunchKernelGGL((splitk_finish_kernel<FmtF8<0>>), dim3((unsigned)((total + 255) / 256)), dim3(256), 0, s, a);
-  }
+  if (nsl > 1) launch_splitk_finish<FmtF8<0>>(a, s);
   return PTA_OK;
 }
 

@@ -300,8 +300,9 @@ static int launch_listed(const EA& a, hipStream_t s, const char* name) {
   }
   make_epilogue(nullptr, &g.epi, name);
   const ListedRows rows{a.lists, a.lists + at.tiles, a.lists + at.order, pta_bf16_tiled_bytes(a.routed.N, a.routed.K), PAIR ? a.choices : 1};
-  return a.tile_rows == 256 ? launch_gemm_listed<FmtBF16, 2, PAIR>(g, a.routed.N / 16, at.max_tiles, rows, s, name)
-                            : launch_gemm_listed<FmtBF16, 1, PAIR>(g, a.routed.N / 16, at.max_tiles, rows, s, name);
+  const size_t x_rows = (size_t)a.rows * (PAIR ? 1 : a.choices);
+  return a.tile_rows == 256 ? launch_gemm_block_listed<FmtBF16, 8, PAIR>(g, x_rows, at.max_tiles, rows, s, name)
+                            : launch_gemm_block_listed<FmtBF16, 4, PAIR>(g, x_rows, at.max_tiles, rows, s, name);
 }
 
 extern "C" int pta_experts(const EA* args, pta_stream_t stream) {
