@@ -270,7 +270,7 @@ struct GemmArgs {
   int M, K, KT;
   GemmEpilogue epi;
   // PAIR mode (SwiGLU): mat[0] is the gate weight, mat[1] the up weight, output in mat[0].Y.
-  // K split across workgroups (gemm_tile_kernel, one matrix): slice blockIdx.y of `ksplit` writes its fp32
+  // K split across workgroups (gemm_own_kernel and the kernels for more rows, one matrix): slice blockIdx.y of `ksplit` writes its fp32
   // sums to part[slice][M][N]; splitk_finish_kernel adds the slices and applies the epilogue.
   float* part;
   size_t part_bytes;
@@ -590,7 +590,7 @@ __global__ __launch_bounds__(NW * 64) void gemv_lds_kernel(GemmArgs a) {
 }
 
 // ------------------------------------------------------------------------------------------
-// Variant for 4 < M <= 64 when all matrices of the launch share X: one workgroup of 16 waves per
+// Variant for 4 < M <= 16 when all matrices of the launch share X: one workgroup of 16 waves per
 // compute unit's worth of work.  A workgroup owns NB 16-channel blocks (blocks g, g + G, ... of
 // the launch's G workgroups); wave w takes the feature tiles w, w + 16, ... of ALL of them, so the
 // activation fragments of a tile (the B operands: 4 KiB per 16 rows, against 1 KiB of INT4
@@ -1098,7 +1098,7 @@ static int launch_gemv_stream(const GemmArgs& a, int total_nb, int cus, hipStrea
 }
 
 // ------------------------------------------------------------------------------------------
-// Variant for 16 < M <= 64: the activation rows of a feature tile are staged in LDS once per
+// Variant for 16 < M <= 64 and launches of more workgroups than compute units (and pairs of up to 32 rows): the activation rows of a feature tile are staged in LDS once per
 // workgroup and shared by its waves, so that the B operands (4 KiB per 16 rows and tile, against
 // 1 KiB of INT4 weights) come from LDS and not from the L2.
 // A workgroup of 8 waves owns 2 * (8 / KQ) weight streams of 16 channels (consecutive channel blocks
@@ -1126,11 +1126,7 @@ __global__ __launch_bounds__(NWV * 64) void gemm_tile_kernel(GemmArgs a) {
   const int kq = wave / WPG, wg_ = wave % WPG;  // K group, wave within the group
   const int tig = wg_ * 64 + lane;              // thread index within the group
   const int K = a.K, M = a.M;
-  // feature tiles of this workgroup: all of them, or slice blockIdx.y of a K split
-  const int nsl = a.ksplit > 1 ? a.ksplit : 1;
-  const int per_slice = (a.KT + nsl - 1) / nsl;
-  const int kt_first = (int)blockIdx.y * per_slice;
-  const int KT = kt_first + per_slice < a.KT ? kt_first + per_slice : a.KT;     // end of the slice
+  const int KT = a.KT;
 
   // the two weight streams of this wave
   int mi = 0;
@@ -1148,7 +1144,7 @@ __global__ __launch_bounds__(NWV * 64) void gemm_tile_kernel(GemmArgs a) {
     const GemmMat& m = a.mat[PAIR ? st : mi];
     nb[st] = PAIR ? first_blk + wg_ : first_blk - m.nb_begin + 2 * wg_ + st;
     sc[st] = Fmt::load_scale(m.scale, a.x_scale, nb[st] * 16 + (lane & 15), m.N);
-    wp[st] = reinterpret_cast<const u32x4*>(m.tiled) + (size_t)nb[st] * a.KT * (64 * KV) + lane;
+    wp[st] = reinterpret_cast<const u32x4*>(m.tiled) + (size_t)nb[st] * KT * (64 * KV) + lane;
   }
   const f16* X = a.mat[mi].X ? a.mat[mi].X : a.X;
 
@@ -1184,39 +1180,28 @@ __global__ __launch_bounds__(NWV * 64) void gemm_tile_kernel(GemmArgs a) {
   };
 
   f16* xbuf = xs + (size_t)kq * 2 * XBUF;
-  const int steps = (KT - kt_first + KQ - 1) / KQ;
+  const int steps = (KT + KQ - 1) / KQ;
   u32x4 w_cur[2][KV], w_nxt[2][KV], xv[VPT];
-  fetch_w(kt_first + kq, w_cur);
-  fetch_x(kt_first + kq, xv);
+  fetch_w(kq, w_cur);
+  fetch_x(kq, xv);
   store_x(xbuf, xv);
   __syncthreads();
   for (int i = 0; i < steps; ++i) {
-    const int kt = kt_first + kq + i * KQ, ktn = kt + KQ;
+    const int kt = kq + i * KQ, ktn = kt + KQ;
     const bool more = i + 1 < steps;
     if (more) { fetch_w(ktn, w_nxt); fetch_x(ktn, xv); }
     const f16* cur = xbuf + (i & 1) * XBUF + (lane & 15) * TILE_XSTRIDE + (lane >> 4) * 8;
     if (kt < KT) {
 #pragma unroll
       for (int m = 0; m < 4; ++m) {
-        if constexpr (MT <= 4) {
-          f16x8 xb[MT];
+        f16x8 xb[MT];
 #pragma unroll
-          for (int mt = 0; mt < MT; ++mt) xb[mt] = *reinterpret_cast<const f16x8*>(cur + mt * 16 * TILE_XSTRIDE + m * 32);
+        for (int mt = 0; mt < MT; ++mt) xb[mt] = *reinterpret_cast<const f16x8*>(cur + mt * 16 * TILE_XSTRIDE + m * 32);
 #pragma unroll
-          for (int st = 0; st < 2; ++st) {
-            const f16x8 av = Fmt::a_operand(w_cur[st], m, sc[st]);
+        for (int st = 0; st < 2; ++st) {
+          const f16x8 av = Fmt::a_operand(w_cur[st], m, sc[st]);
 #pragma unroll
-            for (int mt = 0; mt < MT; ++mt) acc[st][mt] = Fmt::mma(av, xb[mt], acc[st][mt]);
-          }
-        } else {
-          // many row groups: both weight fragments decoded once, then one activation fragment at a time feeds both
-          const f16x8 av0 = Fmt::a_operand(w_cur[0], m, sc[0]), av1 = Fmt::a_operand(w_cur[1], m, sc[1]);
-#pragma unroll
-          for (int mt = 0; mt < MT; ++mt) {
-            const f16x8 xb = *reinterpret_cast<const f16x8*>(cur + mt * 16 * TILE_XSTRIDE + m * 32);
-            acc[0][mt] = Fmt::mma(av0, xb, acc[0][mt]);
-            acc[1][mt] = Fmt::mma(av1, xb, acc[1][mt]);
-          }
+          for (int mt = 0; mt < MT; ++mt) acc[st][mt] = Fmt::mma(av, xb[mt], acc[st][mt]);
         }
       }
     }
@@ -1230,34 +1215,6 @@ __global__ __launch_bounds__(NWV * 64) void gemm_tile_kernel(GemmArgs a) {
     __syncthreads();
   }
 
-  if constexpr (KQ == 1) {
-    // one K group: every wave holds finished sums.  Lane l has channels (l / 16) * 4 + r, r = 0..3, of row l % 16 of
-    // each row group, for both of its streams.
-    const GemmMat& mat = a.mat[PAIR ? 0 : mi];
-    const int N = mat.N;
-#pragma unroll
-    for (int mt = 0; mt < MT; ++mt) {
-      const int m = mt * 16 + (lane & 15);
-      if (m >= M) continue;
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        if (PAIR) {
-          const int n = nb[0] * 16 + (lane >> 4) * 4 + r;
-          if (n >= N) continue;
-          gemm_put_pair<Fmt>(a, m, n, N, Fmt::finish(acc[0][mt][r], sc[0]), Fmt::finish(acc[1][mt][r], sc[1]));
-        } else {
-#pragma unroll
-          for (int st = 0; st < 2; ++st) {
-            const int n = nb[st] * 16 + (lane >> 4) * 4 + r;
-            if (n >= N) continue;
-            if (nsl > 1) { a.part[((size_t)blockIdx.y * M + m) * N + n] = acc[st][mt][r]; continue; }
-            gemm_put<Fmt>(a, mat, m, n, N, Fmt::finish(acc[st][mt][r], sc[st]));
-          }
-        }
-      }
-    }
-    return;
-  }
   // partial sums of the K groups meet in LDS (the staging area is free after the last barrier)
 #pragma unroll
   for (int st = 0; st < 2; ++st)
@@ -1288,10 +1245,6 @@ __global__ __launch_bounds__(NWV * 64) void gemm_tile_kernel(GemmArgs a) {
 #pragma unroll
       for (int q = 0; q < KQ; ++q) t += red[((((q * WPG + wslot) * 2 + (PAIR ? g : st)) * MT + mt) * 4 + r) * 64 + ln];
       sum[g] = t;
-    }
-    if (!PAIR && nsl > 1) {                // a slice of a K split: the raw fp32 sum; the finishing kernel does the rest
-      a.part[((size_t)blockIdx.y * M + m) * N + n] = sum[0];
-      continue;
     }
 #pragma unroll
     for (int g = 0; g < (PAIR ? 2 : 1); ++g) sum[g] = Fmt::finish(sum[g], sc[0]);   // no format's finish uses the per-channel part
@@ -1355,7 +1308,7 @@ static int launch_gemm_tile(const GemmArgs& a, int total_nb, hipStream_t s, cons
   static bool ready = false;
   constexpr int WPG = NWV / KQ;
   const size_t stage = (size_t)KQ * 2 * MT * 16 * TILE_XSTRIDE * 2;
-  const size_t redb = KQ == 1 ? 0 : (size_t)NWV * 2 * MT * 256 * 4;      // one K group: no meeting in LDS
+  const size_t redb = (size_t)NWV * 2 * MT * 256 * 4;
   const size_t smem = stage > redb ? stage : redb;
   static_assert((size_t)KQ * 2 * MT * 16 * TILE_XSTRIDE * 2 <= 160 * 1024, "staging beyond the LDS of a compute unit");
   if (!ready) {
@@ -1365,8 +1318,313 @@ static int launch_gemm_tile(const GemmArgs& a, int total_nb, hipStream_t s, cons
     ready = true;
   }
   const int per_wg = PAIR ? WPG : 2 * WPG;
+  hipLaunchKernelGGL((gemm_tile_kernel<Fmt, MT, KQ, PAIR, NWV>), dim3(total_nb / per_wg), dim3(NWV * 64), smem, s, a);
+  return PTA_OK;
+}
+
+// a pointer that is the same in every lane, in scalar registers
+__device__ __forceinline__ const unsigned char* uniform_pointer(const unsigned char* p) {
+  const uint64_t v = reinterpret_cast<uint64_t>(p);
+  const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)v), hi = __builtin_amdgcn_readfirstlane((uint32_t)(v >> 32));
+  return reinterpret_cast<const unsigned char*>((uint64_t)hi << 32 | lo);
+}
+
+// ------------------------------------------------------------------------------------------
+// Variant for more than 8 rows and few workgroups: each wave multiplies feature tiles of its own.
+// A workgroup of 8 waves owns NB blocks of 16 channels (of one matrix; for a SwiGLU pair of both) and MT * 16 rows (all of up to
+// 64, else a row block); its wave w takes
+// the feature tiles w, w + 8, ... of its slice of K.  A wave's rows travel global -> registers -> LDS -> registers: the loads take
+// 256 bytes of 4 rows each (in the matrix unit's operand order, 64 bytes of 16 rows, the same bytes take twice as long), the LDS
+// area belongs to the wave alone and turns them into operands, so that nothing in the loop waits for another wave, and the rows
+// and weights of the next tile are in flight (16 KiB and NB KiB a wave at 64 rows) while one is multiplied.  The waves' sums meet
+// in LDS at the end.
+// What bounds it is the rows: every workgroup reads all of them, and a compute unit gets 112 GB/s out of its L2 when all read
+// (4.6 us for 64 rows of 4096 features).  Parts of a launch of 64 rows, 4096 x 11008 INT4 (15.5 us before the end's arguments were
+// read ahead, 14.2 with it): 3 us an empty one, 4.1 the rows, 2 the weights, 1 products and decoding, 2 to 3 the end.
+// Before (gemm_tile_kernel, whose waves wait for one another at every step): 21.8 us.  16 requests in flight a wave are enough;
+// twice as many at 32 rows were slower by 0.6 us.
+// ------------------------------------------------------------------------------------------
+constexpr int OWN_WAVES = 8;
+// weight streams of a workgroup that the registers hold (F152's decoding takes more of them), and channel blocks
+template <class Fmt> struct OwnStreams { static constexpr int cap = Fmt::kVec == 4 ? 3 : 4; };
+template <class Fmt, bool PAIR> constexpr int own_cap(int mt) { return (OwnStreams<Fmt>::cap + (Fmt::kVec == 1 && mt <= 2 ? 1 : 0)) / (PAIR ? 2 : 1); }
+constexpr int own_ahead(int mt) { return mt <= 1 ? 2 : 1; }
+
+// v, read from memory at this point and kept in scalar registers
+template <class T>
+__device__ __forceinline__ void in_register(T& v) { asm volatile("" : "+s"(v)); }
+
+template <class Fmt, int MT, int NB, bool PAIR>
+__global__ __launch_bounds__(OWN_WAVES * 64) __attribute__((amdgpu_waves_per_eu(2, 2))) void gemm_own_kernel(GemmArgs a, int groups) {
+  constexpr int NACC = PAIR ? 2 : 1, NS = NB * NACC;       // weight streams
+  constexpr int KV = Fmt::kVec;
+  extern __shared__ __align__(16) unsigned char smem[];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int K = a.K;
+  // Grid: 8 groups of channels, the row blocks, the slices' groups by eights.  A group's row blocks are multiples of eight apart: on one
+  // XCD, whose L2 has its weights for all.  (One flat index, divided here, cost 1.5 us a launch.)
+  const int row_block = blockIdx.y, eights = (groups + 7) / 8;
+  int slice = 0, group = blockIdx.z;
+  while (group >= eights) group -= eights, ++slice;
+  group = group * 8 + blockIdx.x;
+  if (group >= groups) return;
+  const int row0 = row_block * (MT * 16), M = a.M - row0 < MT * 16 ? a.M - row0 : MT * 16;
+  int mi = 0;
+  if (!PAIR) {
+#pragma unroll
+    for (int i = 0; i < 3; ++i) {
+      const int here = ((a.mat[i].N + 15) / 16 + NB - 1) / NB;
+      if (i + 1 < a.count && mi == i && group >= here) { group -= here; mi = i + 1; }
+    }
+  }
+  const GemmMat& mat = a.mat[mi];
+  const int N = mat.N, blocks = (N + 15) / 16;
   const int nsl = a.ksplit > 1 ? a.ksplit : 1;
-  hipLaunchKernelGGL((gemm_tile_kernel<Fmt, MT, KQ, PAIR, NWV>), dim3(total_nb / per_wg, nsl), dim3(NWV * 64), smem, s, a);
+  const int per_slice = (a.KT + nsl - 1) / nsl;
+  const int kt_first = slice * per_slice;
+  const int kt_end = kt_first + per_slice < a.KT ? kt_first + per_slice : a.KT;
+
+  typename Fmt::Scale sc[NS];
+  __amdgpu_buffer_rsrc_t wr[NS];
+  const int block_bytes = a.KT * KV * 1024;
+#pragma unroll
+  for (int st = 0; st < NS; ++st) {
+    const GemmMat& m = PAIR ? a.mat[st & 1] : mat;
+    int nb = group * NB + st / NACC;
+    nb = nb < blocks ? nb : blocks - 1;                    // (blocks past the last one: multiplied, never stored)
+    sc[st] = Fmt::load_scale(m.scale, a.x_scale, nb * 16 + (lane & 15), m.N);
+    const unsigned char* from = uniform_pointer(reinterpret_cast<const unsigned char*>(m.tiled) + (size_t)nb * block_bytes);
+    wr[st] = __builtin_amdgcn_make_buffer_rsrc(const_cast<unsigned char*>(from), 0, block_bytes, 0x00020000);
+  }
+  // rows past the last one lie past the buffer's end and read as zeros
+  const unsigned char* X = uniform_pointer(reinterpret_cast<const unsigned char*>((mat.X ? mat.X : a.X) + (size_t)row0 * K));
+  const int row_bytes = K * 2, x_bytes = M * row_bytes;
+  const __amdgpu_buffer_rsrc_t xr = __builtin_amdgcn_make_buffer_rsrc(const_cast<unsigned char*>(X), 0, x_bytes, 0x00020000);
+  const int tiles = (kt_end - kt_first - wave + OWN_WAVES - 1) / OWN_WAVES;
+  auto tile = [&](int i) { return i < tiles ? kt_first + wave + OWN_WAVES * i : kt_end; };
+  // 16 rows of a tile lie in LDS with 256 bytes a row, the 16-byte vector c of row r at place c ^ r: the reads, one vector of 16
+  // rows, meet in no bank.  Lane l of load j fills place l % 16 of row j * 4 + l / 16.
+  constexpr int AHEAD = own_ahead(MT), RING = AHEAD * MT;   // tiles, and row groups of tiles, that the area holds
+  unsigned char* const area = smem + wave * (RING * 4096);
+  int xlane[4], xfeature[4];
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    const int r = j * 4 + (lane >> 4), c = (lane & 15) ^ r;
+    xlane[j] = r * row_bytes + c * 16;
+    xfeature[j] = c * 8;
+  }
+  // requests for tiles and features past the last one lie past the buffers' ends: they read as zeros from nowhere, and the loop
+  // has no branch round them
+  auto x_at = [&](int kt, int (&at)[4]) {
+    const int left = kt < kt_end ? K - kt * 128 : 0;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) at[j] = xfeature[j] < left ? xlane[j] : x_bytes;
+  };
+  int x_tile, x_lane[4];                                   // the tile whose rows are requested
+  auto next_x = [&](int kt) { x_tile = kt; x_at(kt, x_lane); };
+  auto fetch_x = [&](int mt, int place) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(xr, (__attribute__((address_space(3))) void*)(area + place * 4096 + j * 1024), 16,
+                                               x_lane[j] + mt * 16 * row_bytes, x_tile * 256, 0, 0);
+  };
+  auto fetch_w = [&](int kt, u32x4 (&to)[NS][KV]) {
+    const int at = kt < kt_end ? lane * 16 : block_bytes;
+#pragma unroll
+    for (int st = 0; st < NS; ++st)
+#pragma unroll
+      for (int v = 0; v < KV; ++v) to[st][v] = __builtin_amdgcn_raw_buffer_load_b128(wr[st], at, (kt * KV + v) * 1024, 2);
+  };
+
+  f32x4 acc[NS][MT];
+#pragma unroll
+  for (int st = 0; st < NS; ++st)
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt) acc[st][mt] = f32x4{0.f, 0.f, 0.f, 0.f};
+  // Requests are made in the order x(0), w(0), x(1), w(1), ...: this many follow those of a row group when it is waited for
+  constexpr int BEHIND = 4 * (RING - 1) + AHEAD * NS * KV;
+  constexpr int WAIT = 0x0f70 | (BEHIND & 15) | (BEHIND >> 4) << 14;
+  static_assert(BEHIND < 64, "the counter of requests");
+  u32x4 w[2][NS][KV];
+  f16x8 xb[2][4];
+  auto read_x = [&](int place, f16x8 (&to)[4]) {
+    __builtin_amdgcn_s_waitcnt(WAIT);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) to[j] = *reinterpret_cast<const f16x8*>(area + place * 4096 + (lane & 15) * 256 + (((j * 4 + (lane >> 4)) ^ (lane & 15)) * 16));
+  };
+  // tile i: TURN is i modulo what makes the places in the area and the buffers of w and xb come round again
+  auto step = [&](int i, auto turn) {
+    constexpr int TURN = decltype(turn)::value;
+    f16x8 av[NS][4];
+#pragma unroll
+    for (int st = 0; st < NS; ++st)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) av[st][j] = Fmt::a_operand(w[TURN & 1][st], j, sc[st]);
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt) {
+      constexpr int Q0 = TURN * MT;
+      const int q = Q0 + mt, place = (q + 1) % RING;        // the next row group: read while this one is multiplied, then requested anew
+      if (mt == MT - 1) {
+        __builtin_amdgcn_sched_barrier(0);
+        fetch_w(tile(i + 2), w[TURN & 1]);
+        next_x(tile(i + 1 + AHEAD));
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      read_x(place, xb[(q + 1) & 1]);
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+#pragma unroll
+        for (int st = 0; st < NS; ++st) acc[st][mt] = Fmt::mma(av[st][j], xb[q & 1][j], acc[st][mt]);
+      __builtin_amdgcn_s_waitcnt(0xc07f);                  // lgkmcnt(0): the operands are out of LDS, their place is free
+      __builtin_amdgcn_sched_barrier(0);
+      fetch_x((mt + 1) % MT, place);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  };
+  if (AHEAD == 1) fetch_w(tile(0), w[0]);
+#pragma unroll
+  for (int t = 0; t < AHEAD; ++t) {
+    next_x(tile(t));
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt) fetch_x(mt, t * MT + mt);
+    __builtin_amdgcn_sched_barrier(0);
+    fetch_w(tile(AHEAD == 1 ? 1 : t), w[AHEAD == 1 ? 1 : t]);
+    __builtin_amdgcn_sched_barrier(0);
+  }
+  next_x(tile(AHEAD));
+  read_x(0, xb[0]);
+  __builtin_amdgcn_s_waitcnt(0xc07f);
+  __builtin_amdgcn_sched_barrier(0);
+  fetch_x(0, 0);
+  __builtin_amdgcn_sched_barrier(0);
+  // What the end needs of the arguments is read while the first rows are on their way: each line of them is a round trip to memory
+  // of its own otherwise, one after another behind the products.
+  GemmMat out = mat;
+  GemmEpilogue epi = a.epi;
+  in_register(out.Y);
+  if constexpr (Fmt::kWide) {
+    WideOut& o = out.wide;
+    in_register(o.ld); in_register(o.n_main); in_register(o.out_f32); in_register(o.tail); in_register(o.tail_count);
+    in_register(o.tail_bias); in_register(o.cap); in_register(o.clamped); in_register(o.limit); in_register(o.slope);
+    in_register(o.bias); in_register(o.bias2); in_register(o.act); in_register(o.mul); in_register(o.mul_f32); in_register(o.accumulate);
+  } else {
+    in_register(out.bias); in_register(out.act);
+    in_register(epi.bias); in_register(epi.residual); in_register(epi.act); in_register(epi.mul); in_register(epi.post_scale);
+    in_register(epi.out_fp8_scale); in_register(epi.out_fp8_format);
+  }
+  // (in pairs, with no way out between the two: where paths meet, the compiler waits for what is in flight on either)
+  int i = 0;
+  for (; i + 1 < tiles; i += 2) {
+    step(i, std::integral_constant<int, 0>{});
+    step(i + 1, std::integral_constant<int, 1>{});
+  }
+  if (i < tiles) step(i, std::integral_constant<int, 0>{});
+  __builtin_amdgcn_s_waitcnt(0x0f70);                      // vmcnt(0): nothing is on its way into LDS any more
+
+  __syncthreads();
+  f32x4* red = reinterpret_cast<f32x4*>(smem);             // [OWN_WAVES][NS][MT][64]
+#pragma unroll
+  for (int st = 0; st < NS; ++st)
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt) red[((wave * NS + st) * MT + mt) * 64 + lane] = acc[st][mt];
+  __syncthreads();
+  constexpr int OUTS = NB * MT * 64, ITEMS = (OUTS + OWN_WAVES * 64 - 1) / (OWN_WAVES * 64);      // four channels of a row each
+  f32x4 sums[ITEMS][NACC];
+#pragma unroll
+  for (int it = 0; it < ITEMS; ++it) {
+    const int o = it * (OWN_WAVES * 64) + threadIdx.x, b = o / (MT * 64), at = o % (MT * 64);
+    if (OUTS % (OWN_WAVES * 64) == 0 || o < OUTS) {
+#pragma unroll
+      for (int g = 0; g < NACC; ++g) {
+        f32x4 t = red[(b * NACC + g) * MT * 64 + at];
+#pragma unroll
+        for (int v = 1; v < OWN_WAVES; ++v) {
+          const f32x4 p = red[(v * NS + b * NACC + g) * MT * 64 + at];
+#pragma unroll
+          for (int r = 0; r < 4; ++r) t[r] += p[r];
+        }
+        sums[it][g] = t;
+      }
+    }
+  }
+  const bool vectors = (N & 3) == 0 && ((reinterpret_cast<uintptr_t>(out.Y) | reinterpret_cast<uintptr_t>(epi.residual)) & 7) == 0;
+  const bool direct = !out.bias && out.act == PTA_ACT_NONE && !epi.bias && epi.act == PTA_ACT_NONE && !epi.mul &&
+                      epi.post_scale == 0.0f && !epi.out_fp8_scale;
+#pragma unroll
+  for (int it = 0; it < ITEMS; ++it) {
+    const int o = it * (OWN_WAVES * 64) + threadIdx.x, b = o / (MT * 64), at = o % (MT * 64);
+    const int m = row0 + (at >> 6) * 16 + (at & 15), n = (group * NB + b) * 16 + ((at >> 4) & 3) * 4;
+    if (o >= OUTS || m >= a.M || n >= N) continue;
+    const f32x4 (&t)[NACC] = sums[it];
+    if (!PAIR && nsl > 1) {                // a slice of a K split: the raw fp32 sums; the finishing kernel does the rest
+      float* p = a.part + ((size_t)slice * a.M + m) * N + n;
+      if ((N & 3) == 0) {
+        *reinterpret_cast<f32x4*>(p) = t[0];
+      } else {
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+          if (n + r < N) p[r] = t[0][r];
+      }
+      continue;
+    }
+    if constexpr (Fmt::kWide) {
+      if constexpr (PAIR) wide_put_pair4(out, m, n, t[0], t[NACC - 1]);
+      else wide_put4(out, m, n, t[0]);
+    } else {
+      f16* y = out.Y + (size_t)m * N + n;
+      f16x4 v;
+      if (!PAIR && direct) {               // nothing but the residual stream to add
+        const f16* from = epi.residual + (size_t)m * N + n;
+        f16x4 res = {0, 0, 0, 0};
+        if (epi.residual && vectors) res = *reinterpret_cast<const f16x4*>(from);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          if (epi.residual && !vectors && n + r < N) res[r] = from[r];
+          v[r] = (f16)Fmt::finish(t[0][r], sc[0]);                   // no format's finish uses the per-channel part
+          if (epi.residual) v[r] = v[r] + res[r];
+          if (!vectors && n + r < N) y[r] = v[r];
+        }
+        if (vectors) *reinterpret_cast<f16x4*>(y) = v;
+        continue;
+      }
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        if (n + r >= N) continue;
+        if constexpr (PAIR) {
+          v[r] = swiglu_out(epi, (f16)Fmt::finish(t[0][r], sc[0]), (f16)Fmt::finish(t[NACC - 1][r], sc[1]));
+        } else {
+          f16 y0 = (f16)Fmt::finish(t[0][r], sc[0]);
+          if (out.bias) y0 = y0 + out.bias[n + r];
+          v[r] = apply_epilogue(epi, apply_act(out.act, y0), m, n + r, N);
+        }
+        if (!vectors) y[r] = v[r];
+      }
+      if (vectors) *reinterpret_cast<f16x4*>(y) = v;
+    }
+  }
+}
+
+static inline int own_groups(const GemmArgs& a, int nb, bool pair) {
+  int groups = 0;
+  for (int i = 0; i < (pair ? 1 : a.count); ++i) groups += ((a.mat[i].N + 15) / 16 + nb - 1) / nb;
+  return groups;
+}
+
+template <class Fmt, int MT, int NB, bool PAIR>
+static int launch_gemm_own(const GemmArgs& a, hipStream_t s, const char* name) {
+  static bool ready = false;
+  constexpr int NS = NB * (PAIR ? 2 : 1), STAGE = 4 * own_ahead(MT);
+  const size_t smem = (size_t)OWN_WAVES * MT * 1024 * (NS > STAGE ? NS : STAGE);
+  if (!ready) {
+    PTA_REQUIRE(hipFuncSetAttribute((const void*)gemm_own_kernel<Fmt, MT, NB, PAIR>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                    (int)smem) == hipSuccess, "%s: cannot reserve %zu bytes of LDS", name, smem);
+    ready = true;
+  }
+  const int nsl = a.ksplit > 1 ? a.ksplit : 1;
+  const int groups = own_groups(a, NB, PAIR), row_blocks = (a.M + MT * 16 - 1) / (MT * 16);
+  hipLaunchKernelGGL((gemm_own_kernel<Fmt, MT, NB, PAIR>), dim3(8, row_blocks, (groups + 7) / 8 * nsl), dim3(OWN_WAVES * 64), smem, s, a, groups);
   if (nsl > 1) launch_splitk_finish<Fmt>(a, s);
   return PTA_OK;
 }
@@ -1990,13 +2248,6 @@ __device__ __forceinline__ u32x4 as_computed(u32x4 v) {
   return v;
 }
 
-// a pointer that is the same in every lane, in scalar registers
-__device__ __forceinline__ const unsigned char* uniform_pointer(const unsigned char* p) {
-  const uint64_t v = reinterpret_cast<uint64_t>(p);
-  const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)v), hi = __builtin_amdgcn_readfirstlane((uint32_t)(v >> 32));
-  return reinterpret_cast<const unsigned char*>((uint64_t)hi << 32 | lo);
-}
-
 template <class Fmt>
 constexpr int block_stage_bytes(int rg) { return rg * 32 * Fmt::kStage * 2 + BLOCK_CB * Fmt::kVec * 8 * Fmt::kStage; }
 template <class Fmt>
@@ -2297,6 +2548,58 @@ static int launch_gemm_panel(const GemmArgs& a, int unit0, int unit1, hipStream_
   return PTA_OK;
 }
 
+template <class Fmt, int MT, bool PAIR>
+static int launch_gemm_own_for(const GemmArgs& a, int nb, hipStream_t s, const char* name) {
+  constexpr int CAP = own_cap<Fmt, PAIR>(MT);
+  if (CAP >= 5 && nb == 5) return launch_gemm_own<Fmt, MT, CAP >= 5 ? 5 : 1, PAIR>(a, s, name);
+  if (CAP >= 4 && nb == 4) return launch_gemm_own<Fmt, MT, CAP >= 4 ? 4 : 1, PAIR>(a, s, name);
+  if (CAP >= 3 && nb == 3) return launch_gemm_own<Fmt, MT, CAP >= 3 ? 3 : 1, PAIR>(a, s, name);
+  if (CAP >= 2 && nb == 2) return launch_gemm_own<Fmt, MT, CAP >= 2 ? 2 : 1, PAIR>(a, s, name);
+  return launch_gemm_own<Fmt, MT, 1, PAIR>(a, s, name);
+}
+
+struct OwnPlan { int mt, nb, slices, rounds; double us; };
+
+// The row groups and channel blocks of a workgroup and the slices of K that come out shortest.  The constants (us a tile of a wave: its
+// own, of a row group, of a channel block - its products, and its weights, which the row blocks share; of the second launch of a
+// split) are fitted to measured launches: they order the choices.  64 rows, INT4, 11008 x 4096, blocks x slices: 1 x 1 23.5, 2 x 2
+// 19.2, 4 x 4 20.5 us; 4096 x 11008: 1 block 29.3, 2 21.9, 3 14.5, 4 16.4; 4096 x 4096: 1 x 1 11.1, 1 x 2 16.3, 2 x 2 11.9, 4 x 4 13.4.
+template <class Fmt, bool PAIR>
+static OwnPlan plan_gemm_own(const GemmArgs& a) {
+  constexpr double PRODUCTS = Fmt::kVec == 1 ? 0.48 : Fmt::kVec == 2 ? 0.6 : 0.7, WEIGHTS = Fmt::kVec == 1 ? 0.0 : Fmt::kVec == 2 ? 0.36 : 0.9;
+  const int cus = device_compute_units();
+  const int row_blocks = (a.M + 63) / 64;
+  const bool split = !PAIR && a.count == 1 && a.part && a.M > 16;
+  OwnPlan best{((a.M + 15) / 16 + row_blocks - 1) / row_blocks, 1, 1, 0, 0.0};
+  for (int nb = 1; nb <= own_cap<Fmt, PAIR>(best.mt); ++nb) {
+    const int groups = own_groups(a, nb, PAIR) * row_blocks;
+    for (int sl = 1; sl <= (split ? GEMM_MAX_KSPLIT : 1); ++sl) {
+      if (sl > 1 && (a.KT < sl * OWN_WAVES || a.part_bytes < (size_t)sl * a.M * a.mat[0].N * sizeof(float))) break;
+      const int rounds = (groups * sl + cus - 1) / cus, tiles = ((a.KT + sl - 1) / sl + OWN_WAVES - 1) / OWN_WAVES;
+      double us = 3.2 + rounds * tiles * (0.5 + 0.29 * best.mt + (PRODUCTS + WEIGHTS / row_blocks) * nb * (PAIR ? 2 : 1));
+      if (sl > 1) {
+        const double size = (double)a.M * a.mat[0].N / 262144;
+        us += 2.7 * sl - 0.9 + (size > 1 ? 0.5 * sl * (size - 1) : 0.0);
+      }
+      if (best.rounds == 0 || us < best.us) best.nb = nb, best.slices = sl, best.rounds = rounds, best.us = us;
+    }
+  }
+  return best;
+}
+
+template <class Fmt, bool PAIR>
+static int launch_gemm_own_plan(const GemmArgs& a, const OwnPlan& p, hipStream_t s, const char* name) {
+  GemmArgs b = a;
+  b.ksplit = p.slices;
+  const int rc = p.mt <= 1   ? launch_gemm_own_for<Fmt, 1, PAIR>(b, p.nb, s, name)
+                 : p.mt == 2 ? launch_gemm_own_for<Fmt, 2, PAIR>(b, p.nb, s, name)
+                 : p.mt == 3 ? launch_gemm_own_for<Fmt, 3, PAIR>(b, p.nb, s, name)
+                             : launch_gemm_own_for<Fmt, 4, PAIR>(b, p.nb, s, name);
+  if (rc) return rc;
+  PTA_CHECK_LAUNCH(name);
+  return PTA_OK;
+}
+
 // whether the launch fits gemm_tile_kernel with `per_wg` channel blocks per workgroup: every matrix
 // a whole number of workgroups, enough feature tiles for the K groups
 static inline bool tile_fits(const GemmArgs& a, int per_wg, int kq, bool pair) {
@@ -2331,9 +2634,7 @@ template <class Fmt, int MT, bool PAIR>
 static void launch_gemv(const GemmArgs& a, int total_nb, hipStream_t s) {
   // Waves per block: enough to split K finely when there are few channel blocks, fewer when
   // the grid alone already fills the machine.  The LDS reduction buffer caps the wide cases.
-  if constexpr (MT == 4 && PAIR) {
-    hipLaunchKernelGGL((gemv_mfma_kernel<Fmt, MT, 4, PAIR>), dim3(total_nb), dim3(4 * 64), 0, s, a);
-  } else if constexpr (MT == 4 || PAIR) {
+  if constexpr (PAIR) {
     hipLaunchKernelGGL((gemv_mfma_kernel<Fmt, MT, 8, PAIR>), dim3(total_nb), dim3(8 * 64), 0, s, a);
   } else {
     if (a.KT >= 16 && total_nb <= 1024)
@@ -2353,6 +2654,17 @@ template <class Fmt> struct BlockFormat { static constexpr bool ok = false; };
 // the rows go through the smaller paths in turn, 64 at a time.
 template <class Fmt, bool PAIR>
 static int dispatch_many_rows(const GemmArgs& a, int total_nb, hipStream_t s, const char* name) {
+  // One round of gemm_own_kernel's workgroups: it (us, against the kernels below; a launch of theirs takes 15 and more however small).
+  // INT4: 4096 x 4096, 72 rows 11.4 against 23.1, 256 rows 18.3 against 37.5; 768 x 3072, 205 rows 8.8 against 24.7; 11008 x 4096,
+  // 256 rows 36 against 49.  fp16: 768 x 3072, 205 rows 9.8 against 15.5; 2048 x 2048, 256 rows 11.2 against 19.4; F143 4096 x 4096,
+  // 256 rows 20.6 against 29.6.  More rounds: to 128 rows two (4096 x 11008, 128 rows, INT4 29.8 against 40.9, F143 35.8 against 44.3,
+  // fp16 44 against 47), of INT4 weights three (their pair of 11008 channels 41.5 against 48.0), and small launches (768 x 3072,
+  // 512 rows, INT4 16.0 against 25.1); beyond, these lose: 4096 x 11008, 160 rows, INT4 42.8 against 39.8, fp16 60 against 44.
+  if (a.epi.norm == PTA_NORM_NONE) {
+    const OwnPlan plan = plan_gemm_own<Fmt, PAIR>(a);
+    if (plan.rounds == 1 || (a.M <= 128 && plan.rounds <= (Fmt::kVec == 1 ? 3 : 2)) || plan.us <= (Fmt::kVec == 1 ? 22.0 : 11.0))
+      return launch_gemm_own_plan<Fmt, PAIR>(a, plan, s, name);
+  }
   const int cus = device_compute_units();
   const int per_wg = PAIR ? 4 : 8;
   // (few features: the wide formats only, whose other path would take 64 rows per launch)
@@ -2452,30 +2764,41 @@ static int dispatch_gemv(const GemmArgs& a, int total_nb, hipStream_t s, const c
     if (a.KT >= 16 && total_nb <= 1024 && !PAIR) launch_gemv_lds<Fmt, 16, PAIR>(a, total_nb, s);
     else launch_gemv_lds<Fmt, 8, PAIR>(a, total_nb, s);
   } else {
-    bool shared_x = true;
-    for (int i = 0; i < a.count; ++i) shared_x = shared_x && a.mat[i].X == nullptr;
-    const int per_cu = (total_nb + device_compute_units() - 1) / device_compute_units();
-    if (a.M > 16 && a.epi.norm == PTA_NORM_NONE) {
-      // the staged kernel where its workgroups fill the machine: 2 streams x 4 K groups (4 channel blocks,
-      // or 2 SwiGLU pairs, per workgroup); for M <= 32 also 8 K groups (half as many blocks per workgroup)
-      const int cus = device_compute_units();
-      const int wgs4 = total_nb / (PAIR ? 2 : 4), wgs8 = total_nb / (PAIR ? 1 : 2);
+    const int cus = device_compute_units();
+    const int per_cu = (total_nb + cus - 1) / cus;
+    const int mt = (a.M + 15) / 16;
+    if (a.epi.norm == PTA_NORM_NONE && a.M > 8) {
+      // gemm_own_kernel or gemm_tile_kernel (16 rows: gemv_wide_kernel, gemv_stream_kernel).  Both sides in us, INT4 unless named.
+      // One round of gemm_own_kernel's workgroups: it.  64 rows, 4096 x 11008: 14.5 against 21.8, 4096 x 4096 11.1 against 15.2,
+      // 2048 x 2048 7.1 against 11.8; 32 rows 11.1 against 14.3, 8.0 against 11.2, 5.6 against 9.4; F143, 64 rows, 4096 x 4096
+      // 11.9 against 16.2; bf16 14.5 against 18.2; with odd channel counts, which gemm_tile_kernel cannot take, 1000 channels at
+      // 64 rows 9.6 against 19.5.
+      // Several rounds: each begins with nothing on its way.  Weights of one vector a tile lose a little (32000 channels, 64 rows
+      // 32.4 against 31.4), those of two win beyond 32 rows (F143 41.8 against 51.6), so does a pair of either (11008 channels, 64
+      // rows 29.2 against 39.7; F143 40.8 against 46.9), fp16 ones lose (72.5 against 68.3).  Pairs of up to 32 rows: 22.4 against
+      // 21.6.  9 to 16 rows, one round: 9.3 against 11.7 (4096 x 11008, 16 rows), K of 13696 13.5 against 17.8, pair of 2048 x 5632
+      // 7.4 against 10.0; fp16 only where every compute unit has one block or none (11008 x 4096 22.5 against 26.4; 4096 x 4608 14.7
+      // against 13.3).
+      const int wgs4 = total_nb / (PAIR ? 2 : 4);
+      const OwnPlan plan = plan_gemm_own<Fmt, PAIR>(a);
+      const bool one_round = plan.rounds == 1;
+      bool own, tile = false;
+      if (a.M <= 16) {
+        own = !a.prefer_stream && a.KT >= 16 && one_round && (Fmt::kVec <= 2 || (!PAIR && total_nb <= cus));
+      } else {
+        tile = tile_fits(a, PAIR ? 2 : 4, 4, PAIR) && 2 * wgs4 >= cus;
+        if (tile && PAIR) own = mt > 2 && Fmt::kVec <= 2;
+        else if (tile) own = one_round || (mt > 2 && Fmt::kVec == 2);
+        else own = a.KT >= 8 || mt > 2;
+      }
+      if (own) return launch_gemm_own_plan<Fmt, PAIR>(a, plan, s, name);
       int rc = 1;
-      // one matrix, too few channel blocks to fill the machine, scratch at hand: split K too
-      int nsl = wgs4 > 0 ? cus / wgs4 : 1;
-      nsl = nsl > GEMM_MAX_KSPLIT ? GEMM_MAX_KSPLIT : nsl;
-      while (nsl > 1 && a.KT < nsl * 8) --nsl;
-      if (!PAIR && a.count == 1 && a.part && nsl > 1 && tile_fits(a, 4, 4, false) &&
-          a.part_bytes >= (size_t)nsl * a.M * a.mat[0].N * sizeof(float)) {
-        GemmArgs b = a;
-        b.ksplit = nsl;
-        rc = a.M <= 32 ? launch_gemm_tile<Fmt, 2, 4, PAIR>(b, total_nb, s, name) : launch_gemm_tile<Fmt, 4, 4, PAIR>(b, total_nb, s, name);
-      } else if (tile_fits(a, PAIR ? 2 : 4, 4, PAIR) && 2 * wgs4 >= cus) {
+      if (tile) {
         // What bounds these launches is the bytes through the busiest compute unit: a workgroup reads all rows of X
         // beside its weights.  More workgroups than compute units (20480 channels: 320 of 64 channels): workgroups
         // of 16 waves and 128 channels where their rounds come out shorter - 160 of 768 KiB against two rounds of
         // 640 at 64 rows.  Measured, 4096 x 20480: 26.0 against 40.7 us at 64 rows, 24.7 against 38.2 at 48, 18.8
-        // against 20.8 at 32; in a single round they lose (4096 x 11008 at 64 rows: 24.9 against 21.5 us).
+        // against 20.8 at 32.
         bool wide = false;
         if constexpr (!PAIR && Fmt::kVec <= 2) {
           // (beyond 32 rows with INT4 weights only: with two vectors per tile the 16 waves' registers do not hold it)
@@ -2489,34 +2812,31 @@ static int dispatch_gemv(const GemmArgs& a, int total_nb, hipStream_t s, const c
             else if constexpr (Fmt::kVec == 1) rc = launch_gemm_tile<Fmt, 4, 4, false, 16>(a, total_nb, s, name);
           }
         }
-        if (!wide)
-        rc = a.M <= 32 ? launch_gemm_tile<Fmt, 2, 4, PAIR>(a, total_nb, s, name) : launch_gemm_tile<Fmt, 4, 4, PAIR>(a, total_nb, s, name);
-      } else if (a.M <= 32 && tile_fits(a, PAIR ? 1 : 2, 8, PAIR) && 2 * wgs8 >= cus) {
-        rc = launch_gemm_tile<Fmt, 2, 8, PAIR>(a, total_nb, s, name);
+        if (!wide && a.M <= 32) rc = launch_gemm_tile<Fmt, 2, 4, PAIR>(a, total_nb, s, name);
+        else if constexpr (PAIR ? Fmt::kVec > 2 : Fmt::kVec != 2) {
+          if (!wide) rc = launch_gemm_tile<Fmt, 4, 4, PAIR>(a, total_nb, s, name);
+        }
       }
       if (rc < 0) return rc;
       if (rc == 0) { PTA_CHECK_LAUNCH(name); return PTA_OK; }
     }
-    if (shared_x && a.KT >= 8) {
+    if (all_shared_x && a.M <= 16 && a.KT >= 8) {
       int rc;
       bool streamed = false;
       if constexpr (Fmt::kVec * (PAIR ? 2 : 1) <= 4) {
         // gemv_stream_kernel where gemv_wide_kernel's rounds of workgroups come out longer than an even share of the
         // blocks (856 blocks: 286 workgroups of 3 = two rounds = 6 block times, against 4), or on request
-        if (stream_fits(a) && total_nb >= device_compute_units() && (a.prefer_stream || wide_block_times<Fmt, PAIR>(total_nb, per_cu) > per_cu)) {
-          rc = launch_gemv_stream<Fmt, PAIR>(a, total_nb, device_compute_units(), s, name);
+        if (stream_fits(a) && total_nb >= cus && (a.prefer_stream || wide_block_times<Fmt, PAIR>(total_nb, per_cu) > per_cu)) {
+          rc = launch_gemv_stream<Fmt, PAIR>(a, total_nb, cus, s, name);
           streamed = true;
         }
       }
       if (streamed) {}
-      else if (a.M <= 16 && a.epi.norm != PTA_NORM_NONE) rc = launch_gemv_wide_for<Fmt, 1, PAIR, true>(a, total_nb, per_cu, s, name);
-      else if (a.M <= 16) rc = launch_gemv_wide_for<Fmt, 1, PAIR>(a, total_nb, per_cu, s, name);
-      else if (a.M <= 32) rc = launch_gemv_wide_for<Fmt, 2, PAIR>(a, total_nb, per_cu, s, name);
-      else rc = launch_gemv_wide_for<Fmt, 4, PAIR>(a, total_nb, per_cu, s, name);
+      else if (a.epi.norm != PTA_NORM_NONE) rc = launch_gemv_wide_for<Fmt, 1, PAIR, true>(a, total_nb, per_cu, s, name);
+      else rc = launch_gemv_wide_for<Fmt, 1, PAIR>(a, total_nb, per_cu, s, name);
       if (rc) return rc;
     } else if (a.M <= 16) launch_gemv<Fmt, 1, PAIR>(a, total_nb, s);
-    else if (a.M <= 32) launch_gemv<Fmt, 2, PAIR>(a, total_nb, s);
-    else launch_gemv<Fmt, 4, PAIR>(a, total_nb, s);
+    else launch_gemv<Fmt, 2, PAIR>(a, total_nb, s);        // (17 to 32 rows of fewer than 8 feature tiles)
   }
   PTA_CHECK_LAUNCH(name);
   return PTA_OK;

@@ -6,7 +6,9 @@ import torch
 pytestmark = pytest.mark.gpu
 
 SHAPES = [  # rows, features, channels: one past and one short of a tile of 128 / 256 rows, 64 features, 16 / 256 channels
-    (129, 8, 16), (255, 72, 250), (256, 64, 256), (257, 136, 264), (384, 200, 520), (1000, 1000, 48), (513, 4096, 272)]
+    (129, 8, 16), (255, 72, 250), (256, 64, 256), (257, 136, 264), (384, 200, 520), (1000, 1000, 48), (513, 4096, 272),
+    # more workgroups than gemm_own_kernel takes
+    (129, 2056, 8200), (255, 4104, 4100), (513, 2056, 2056), (1000, 1032, 1040)]
 
 
 def close(got, ref, magnitude, K, bits):
@@ -85,7 +87,7 @@ def test_inputs_of_their_own():
 
 
 @pytest.mark.parametrize("kind", ["f16", "f8"])
-@pytest.mark.parametrize("M, Kd, N", [(129, 72, 40), (256, 128, 128), (515, 1032, 136), (2048, 256, 5632)])
+@pytest.mark.parametrize("M, Kd, N", [(129, 72, 40), (256, 128, 128), (515, 1032, 136), (2048, 256, 5632), (135, 2056, 4104)])
 def test_pair(kind, M, Kd, N):
     from poptransformer_amd import kernels as K
     x, w = operands(M, Kd, 2 * N, 7)
@@ -104,7 +106,7 @@ def test_pair(kind, M, Kd, N):
     assert ((out.double() - ref).abs() <= bound).all()
 
 
-@pytest.mark.parametrize("M, Kd, main, tail", [(129, 72, 248, 5), (257, 1000, 512, 32), (1100, 264, 64, 0), (300, 2048, 264, 0)])
+@pytest.mark.parametrize("M, Kd, main, tail", [(129, 72, 248, 5), (257, 1000, 512, 32), (1100, 264, 64, 0), (300, 2048, 264, 0), (257, 2056, 4088, 5)])
 @pytest.mark.parametrize("slices", [False, True])
 def test_wide_results_with_tail(M, Kd, main, tail, slices):
     from poptransformer_amd import hybrid_kernels as HK

@@ -1,0 +1,128 @@
+"""Products of 9 rows and more (gemm_own_kernel) at the edges of its tiles and of its row blocks, against float64."""
+import pytest
+import torch
+from tests.test_gpu_many_rows import close, f8_weight, operands
+
+pytestmark = pytest.mark.gpu
+
+# rows at the ends of a row group; features one past, short of and on a tile of 128, with 1, 2 and an odd number of tiles for a wave and
+# with waves that have none; channels short of a block, of four and of a workgroup's blocks, and odd ones
+SHAPES = [(9, 2056, 40), (16, 4096, 4112), (17, 8, 16), (31, 1000, 250), (32, 1160, 264), (33, 136, 1000), (48, 2048, 272), (47, 3080, 11),
+          (49, 520, 4100), (64, 4096, 2064), (63, 2176, 8200), (64, 24, 20),
+          # row blocks of 48 and 64 rows, the last one with one row and full; groups of channels that are no multiple of eight
+          (65, 1160, 264), (128, 4096, 4112), (129, 136, 1000), (205, 768, 2304), (256, 2056, 520), (1024, 768, 768)]
+
+
+def weight_of(kind, w):
+    """(weight, its numbers)"""
+    from poptransformer_amd import kernels as K
+    if kind == "f16":
+        return K.F16Weight(w.half()), w.half().double()
+    if kind == "f8":
+        return f8_weight(w)
+    if kind == "f152":
+        scale = torch.tensor([-1], dtype=torch.int32, device="cuda")
+        codes = K.half_to_fp8(w.half(), scale, "F152")
+        return K.F8Weight(codes, scale, "F152"), K.fp8_to_half(codes, scale, "F152").double()
+    g = torch.Generator(device="cuda").manual_seed(w.shape[0])
+    packed = torch.randint(-128, 128, (w.shape[0], w.shape[1] // 2), generator=g, device="cuda", dtype=torch.int8)
+    scale = (torch.rand(w.shape[0], generator=g, device="cuda") * 0.01 + 0.002).half()
+    return K.W4Weight(packed, scale), K.int4_to_half(packed, scale).double().T.contiguous()
+
+
+@pytest.mark.parametrize("kind", ["int4", "f16", "f8", "f152"])
+@pytest.mark.parametrize("M, Kd, N", SHAPES)
+@pytest.mark.parametrize("slices", [False, True])
+def test_half_results(kind, M, Kd, N, slices):
+    from poptransformer_amd import kernels as K
+    x, w = operands(M, Kd, N, 3)
+    x = x.half()
+    tw, plain = weight_of(kind, w)
+    out = torch.full((M, N), float("nan"), dtype=torch.float16, device="cuda")
+    K.linear(x, [tw], [out], workspace=K.linear_workspace(M, N, "cuda") if slices else None)
+    close(out, x.double() @ plain.T, x.double().abs() @ plain.abs().T, Kd, 11)
+
+
+@pytest.mark.parametrize("M, N, offset", [(20, 264, 0), (33, 250, 0), (64, 264, 1), (150, 250, 1)])
+def test_residual_in_place_and_results_off_their_alignment(M, N, offset):
+    from poptransformer_amd import kernels as K
+    Kd = 1160
+    x, w = operands(M, Kd, N, 5)
+    x = x.half()
+    tw, plain = weight_of("int4", w)
+    store = torch.randn(M * N + 1, generator=torch.Generator(device="cuda").manual_seed(1), device="cuda").half()
+    out = store[offset:offset + M * N].view(M, N)
+    before = out.clone()
+    K.linear(x, [tw], [out], residual=out)
+    ref, mag = x.double() @ plain.T, x.double().abs() @ plain.abs().T
+    # the sum is rounded, then its sum with the residual
+    bound = 2.0 ** -11 * (ref.abs() + (ref + before.double()).abs()) * 1.001 + (Kd + 2) * 2.0 ** -24 * mag + 2.0 ** -23
+    assert ((out.double() - ref - before.double()).abs() <= bound).all()
+
+
+@pytest.mark.parametrize("kind", ["int4", "f16", "f8"])
+@pytest.mark.parametrize("M", [12, 40, 130])
+def test_several_matrices_with_inputs_and_biases_of_their_own(kind, M):
+    from poptransformer_amd import kernels as K
+    Kd, sizes = 2056, (40, 256, 270, 16)
+    xs, tws, plains, biases, outs = [], [], [], [], []
+    for i, n in enumerate(sizes):
+        x, w = operands(M, Kd, n, 10 + i)
+        tw, plain = weight_of(kind, w)
+        xs.append(x.half()), tws.append(tw), plains.append(plain)
+        biases.append(torch.randn(n, device="cuda").half())
+        outs.append(torch.empty((M, n), dtype=torch.float16, device="cuda"))
+    K.linear(None, tws, outs, biases=biases, xs=xs)
+    for x, out, plain, b in zip(xs, outs, plains, biases):
+        ref, mag = x.double() @ plain.T, x.double().abs() @ plain.abs().T
+        bound = 2.0 ** -11 * (ref.abs() + (ref + b.double()).abs()) * 1.001 + (Kd + 2) * 2.0 ** -24 * mag + 2.0 ** -23
+        assert ((out.double() - ref - b.double()).abs() <= bound).all()
+
+
+@pytest.mark.parametrize("kind", ["int4", "f16", "f8"])
+@pytest.mark.parametrize("M, Kd, N", [(16, 2048, 40), (24, 1032, 44), (48, 128, 100), (64, 2048, 4128), (100, 1032, 44), (129, 264, 520)])
+def test_pair(kind, M, Kd, N):
+    from poptransformer_amd import kernels as K
+    x, w = operands(M, Kd, 2 * N, 7)
+    # (the FP8 weights hold +-120, INT4 ones sums of up to 2048 * 5 * 0.1: gate and up stay far below 2^8, their product below 65504)
+    x = (x if kind == "f16" else x * 0.02).half()
+    (g, gp), (u, up) = weight_of(kind, w[:N].contiguous()), weight_of(kind, w[N:].contiguous())
+    out = torch.empty((M, N), dtype=torch.float16, device="cuda")
+    K.linear(x, [g, u], [out, out], swiglu=True)
+    gate, upv = x.double() @ gp.T, x.double() @ up.T
+    ref = torch.nn.functional.silu(gate) * upv
+    # roundings of gate (whose error silu at most multiplies by 1.1), up, swish and the product, each 2^-11, and those of the sums
+    mag_g, mag_u = x.double().abs() @ gp.abs().T, x.double().abs() @ up.abs().T
+    dg, du = 2.0 ** -11 * gate.abs() + (Kd + 2) * 2.0 ** -24 * mag_g, 2.0 ** -11 * upv.abs() + (Kd + 2) * 2.0 ** -24 * mag_u
+    bound = 1.1 * dg * (upv.abs() + du) + du * torch.nn.functional.silu(gate).abs() + 2.5 * 2.0 ** -11 * ref.abs() + 2.0 ** -20 * (1 + upv.abs())
+    assert ((out.double() - ref).abs() <= bound).all()
+
+
+@pytest.mark.parametrize("M, Kd, main, tail", [(12, 2056, 248, 5), (20, 1000, 512, 32), (64, 264, 64, 0), (40, 2048, 264, 3), (200, 520, 250, 3)])
+@pytest.mark.parametrize("slices", [False, True])
+def test_wide_results_with_tail(M, Kd, main, tail, slices):
+    from poptransformer_amd import hybrid_kernels as HK
+    x, w = operands(M, Kd, main + tail, 11)
+    x, w = x.to(torch.bfloat16), w.to(torch.bfloat16)
+    W = HK.WideWeight(w, torch.bfloat16, tail=tail)
+    out = torch.full((M, main), float("nan"), device="cuda")
+    t = torch.full((M * max(tail, 1),), float("nan"), device="cuda")
+    HK.linear(x, W, out, M, ld=main, tail=t if tail else None, workspace=HK.linear_workspace(M, main + tail, "cuda") if slices else None)
+    ref, mag = x.double() @ w.double().T, x.double().abs() @ w.double().abs().T
+    close(out, ref[:, :main], mag[:, :main], Kd, 24)
+    if tail:
+        close(t[:M * tail].view(M, tail), ref[:, main:], mag[:, main:], Kd, 24)
+
+
+@pytest.mark.parametrize("kind", ["int4", "f16"])
+def test_rows_past_the_last_and_features_past_the_end_are_not_read(kind):
+    """NaN around the rows of X must not reach a result: the last row group's missing rows, and the features past K of the last tile."""
+    from poptransformer_amd import kernels as K
+    M, Kd, N = 35, 1032, 20
+    store = torch.full((M + 64, Kd), float("nan"), dtype=torch.float16, device="cuda")
+    x, w = operands(M, Kd, N, 17)
+    store[:M] = x.half()
+    tw, plain = weight_of(kind, w)
+    out = torch.empty((M, N), dtype=torch.float16, device="cuda")
+    K.linear(store[:M], [tw], [out])
+    close(out, x.half().double() @ plain.T, x.half().double().abs() @ plain.abs().T, Kd, 11)
