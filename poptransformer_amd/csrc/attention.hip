@@ -242,6 +242,7 @@ struct AttnArgs {
   float* part;        // [B*Hq, nsplit, D + 2]: running max, denominator, numerator
   f16* out;           // [B, Hq*D]
   int B, Hq, Hkv, max_len, nsplit;
+  float per_head, per_group;         // 1 / Hq, 1 / (query heads of a KV head): of prompt_attention_mfma_kernel
   int rows;           // consecutive positions per sequence (1 in the decode step): row r of a sequence sits at step + r
   int kv_scale;       // FP8 rings (KV8 kernels): rows hold F143 bytes of value * 2^-kv_scale
   int use_scale;
@@ -487,16 +488,25 @@ static int attn_splits(int B, int Hq, int max_len) {
 // ------------------------------------------------------------------------------------------
 // Attention of many rows at once (the prompt passes) on the matrix unit, head size D = 64 or 128, fp16 or F143 cache.
 // One workgroup of four waves per (sequence, query head, 64 or 128 rows of the pass); wave w owns one or two
-// groups of 16 rows.  The cache rows go through LDS 32 at a time, K as it lies, V transposed; per step a wave computes,
-// for each of its row groups,
-//   S^T = K Q^T     (two 16 x 16 tiles, D / 32 MFMAs each: lane l then holds the scores of query row l % 16 for
-//                    cache rows (l / 16) * 4 + 0..3 of each tile - which IS the layout of an A operand whose
+// groups of 16 rows.  The cache rows go through LDS 64 at a time, as they lie and without passing through registers (an F143
+// cache: decoded on the way), two stages in turn with one barrier a step; per step a wave computes, for each of its row groups,
+//   S^T = K Q^T     (four 16 x 16 tiles, D / 32 MFMAs each: lane l then holds the scores of query row l % 16 for
+//                    cache rows (l / 16) * 4 + 0..3 of each tile - two of which ARE the layout of a B operand whose
 //                    k index runs over those eight cache rows),
 //   the roundings of the reference on the scores (fp16 MatMul output, fp16 multiply by 1/sqrt(D)), the online
 //   softmax in fp32 per query row (partners: lanes l ^ 16, l ^ 32), probabilities rounded to fp16 (the
 //   reference's softmax output is fp16),
-//   O += P V        (D / 16 tiles of 16 x 16 over the head size, B operands from the transposed V rows);
-// every K and V operand read from LDS serves all row groups of the wave.
+//   O^T += V^T P^T  (D / 16 tiles of 16 x 16 over the head size, A operands by transposing LDS reads: four cache rows of a feature a
+//                    lane; a lane's accumulators all belong to its own query row, so the correction is its own number);
+// every K and V operand read from LDS serves all row groups of the wave.  A lane sums the probabilities it holds; the four lanes of
+// a query row add theirs at the end.
+// What bounds it is a workgroup's chain of steps, the longest over all the positions: the last rows' workgroups are launched first, and a
+// step is kept short - 64 rows to a barrier, no transposition by 2-byte stores, no exchange between lanes but that of the maximum.
+// The heads of an XCD are its own (its L2 then holds their K and V): grid x is the head modulo eight.
+// Before (32 rows a step, V transposed by 2-byte stores, two barriers): us for one sequence of 32 heads of 128, 300 rows 17.4 -> 12.1,
+// 1000 59.2 -> 33.9, 2048 169 -> 107, 4000 593 -> 244; 64 rows behind 900 43.1 -> 24.1; F143, 1000 rows 63.9 -> 44.3; 8 x 12 heads of 64,
+// 1000 rows 84.9 -> 59.  17 rows 5.5 -> 6.2: a step of 64 where 32 would do (skipping its second half by a branch cost the long ones
+// a tenth).
 // Row r of the pass sits at position step + r and attends to cache rows [0, min(step + r + 1, max_len)), as in
 // attn_partial_kernel.  Outputs differ from that kernel in the last bits (another summation order, fp16
 // probabilities); both are held to 1e-2 against the oracle.
@@ -509,33 +519,54 @@ constexpr int PA_VSTRIDE = 32 + 8;       // halves per staged row of V^T
 // down the features, 8 * PA_VSTRIDE halves apart) over the banks; pairs of dwords stay together for the 8-byte reads.
 __device__ __forceinline__ int pa_vt_at(int d, int p) { return d * PA_VSTRIDE + ((((p >> 1) ^ ((d >> 4) << 1))) << 1) + (p & 1); }
 
+constexpr int PA_KEYS = 64;              // cache rows of a step
+
+// 16-byte piece c of staged row p lies at place c ^ pa_key(p): neither the operand reads (a piece of sixteen rows) nor the transposing
+// ones (two pieces of sixteen rows) meet in a bank.
+template <int D>
+__device__ __forceinline__ int pa_key(int p) { return D == 128 ? p & 15 : (p >> 1) & 7; }
+
+// the larger of this lane's value and that of lane ^ 16, of lane ^ 32
+__device__ __forceinline__ float max_over_quarters(float v) {
+  const auto h = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  v = fmaxf(__uint_as_float(h[0]), __uint_as_float(h[1]));
+  const auto w = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  return fmaxf(__uint_as_float(w[0]), __uint_as_float(w[1]));
+}
+
 // PA_RG: row groups of 16 per wave (a workgroup takes 4 * PA_RG * 16 rows of the pass).  Two where that still gives every
 // compute unit two workgroups or more (a wave's dependent chains - MFMA, maximum, exponentials, MFMA - need company
 // on their SIMD), else one.
 // KV8: the rings hold F143 bytes of value * 2^-kv_scale (as in attn_partial_kernel): a thread loads eight bytes where
-// it loads eight halves of an fp16 ring, decodes them on their way into LDS, and the power of two goes to the fp32
+// LDS receives eight halves of an fp16 ring, decodes them on their way there, and the power of two goes to the fp32
 // scores before they are rounded and to the result.
 template <int D, int PA_RG, bool KV8 = false>
 __global__ __launch_bounds__(PA_THREADS) void prompt_attention_mfma_kernel(AttnArgs a) {
   static_assert(D == 64 || D == 128, "head size");
-  constexpr int PA_KSTRIDE = D + 8;        // halves per staged K row
-  constexpr int NV = D / 64;               // 16-byte vectors of K (and of V) per thread and step: 32 rows of D / 8
-  const float kv_mul = KV8 ? ldexpf(1.0f, a.kv_scale) : 1.0f;
+  constexpr int VPR = D / 8, ROW = D * 2;                  // 16-byte pieces, and bytes, of a row
+  constexpr int STAGE = PA_KEYS * ROW;                     // bytes of a step's K, and of its V
+  constexpr int NV = PA_KEYS * VPR / PA_THREADS;           // pieces of K (and of V) per thread and step
   constexpr int PA_ROWS = 4 * PA_RG * 16;
-  __shared__ __align__(16) f16 ks[32 * PA_KSTRIDE];
-  __shared__ __align__(16) f16 vt[D * PA_VSTRIDE];
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int h = blockIdx.y, b = blockIdx.z;
-  const int kvh = h / (a.Hq / a.Hkv);
+  typedef short s16x4 __attribute__((ext_vector_type(4)));
+  __shared__ __align__(16) unsigned char smem[2 * 2 * STAGE];          // [stage][K, V][PA_KEYS][D]
+  const float kv_mul = KV8 ? ldexpf(1.0f, a.kv_scale) : 1.0f;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int head = (int)blockIdx.z * 8 + (int)blockIdx.x;
+  if (head >= a.B * a.Hq) return;
+  // (quotients of numbers below 2^20 by the reciprocals: an integer division takes 0.3 us of a kernel's start)
+  const int b = __builtin_amdgcn_readfirstlane((int)(((float)head + 0.5f) * a.per_head)), h = head - b * a.Hq;
+  const int kvh = __builtin_amdgcn_readfirstlane((int)(((float)h + 0.5f) * a.per_group));
+  const int row_block = (int)(gridDim.y - 1 - blockIdx.y);
   const int step0 = *a.step;
-  const int r0 = (int)blockIdx.x * PA_ROWS + wave * (PA_RG * 16);          // first row of this wave within the pass
+  const int r0 = row_block * PA_ROWS + wave * (PA_RG * 16);            // first row of this wave within the pass
   auto valid_of = [&](int row) { const int v = step0 + row + 1; return row < a.rows ? (v < a.max_len ? v : a.max_len) : 0; };
   f16x8 qf[PA_RG][D / 32];
-  int my_valid[PA_RG];
+  int my_valid[PA_RG], all_valid[PA_RG];                   // cache rows that this lane's query row attends to, that every row of the group does
 #pragma unroll
   for (int g = 0; g < PA_RG; ++g) {
     const int qrow = r0 + g * 16 + (lane & 15);
     my_valid[g] = valid_of(qrow);
+    all_valid[g] = r0 + g * 16 + 15 < a.rows ? valid_of(r0 + g * 16) : 0;
 #pragma unroll
     for (int m = 0; m < D / 32; ++m) {
       qf[g][m] = f16x8{};
@@ -544,14 +575,11 @@ __global__ __launch_bounds__(PA_THREADS) void prompt_attention_mfma_kernel(AttnA
   }
   const int last_of_wave = r0 + PA_RG * 16 - 1 < a.rows ? r0 + PA_RG * 16 - 1 : a.rows - 1;
   const int wave_valid = r0 < a.rows ? valid_of(last_of_wave) : 0;
-  const int last_of_wg = (int)blockIdx.x * PA_ROWS + PA_ROWS - 1 < a.rows ? (int)blockIdx.x * PA_ROWS + PA_ROWS - 1 : a.rows - 1;
+  const int last_of_wg = row_block * PA_ROWS + PA_ROWS - 1 < a.rows ? row_block * PA_ROWS + PA_ROWS - 1 : a.rows - 1;
   const int wg_valid = valid_of(last_of_wg);
-  const f16* kbase = a.kring + ((size_t)b * a.Hkv + kvh) * a.max_len * D;
-  const f16* vbase = a.vring + ((size_t)b * a.Hkv + kvh) * a.max_len * D;
-  const uint8_t* kbase8 = reinterpret_cast<const uint8_t*>(a.kring) + ((size_t)b * a.Hkv + kvh) * a.max_len * D;
-  const uint8_t* vbase8 = reinterpret_cast<const uint8_t*>(a.vring) + ((size_t)b * a.Hkv + kvh) * a.max_len * D;
+  const size_t ring = ((size_t)b * a.Hkv + kvh) * a.max_len * D;       // elements before this head's rows
 
-  float run_m[PA_RG], run_l[PA_RG];
+  float run_m[PA_RG], run_l[PA_RG];                        // of the lane's query row; the sum of the probabilities this lane holds
   f32x4 o[PA_RG][D / 16];
 #pragma unroll
   for (int g = 0; g < PA_RG; ++g) {
@@ -560,122 +588,134 @@ __global__ __launch_bounds__(PA_THREADS) void prompt_attention_mfma_kernel(AttnA
     for (int jd = 0; jd < D / 16; ++jd) o[g][jd] = f32x4{0.f, 0.f, 0.f, 0.f};
   }
 
-  // cache rows p .. p + 31: 32 * D / 8 vectors of 16 bytes each of K and V, NV per thread; they are requested one step
-  // ahead, so that their way from memory runs beside the step's arithmetic
-  f16x8 kv[NV], vv[NV];
+  // cache rows p .. p + 63, requested one step ahead.  fp16: straight into the stage, rows past the last valid one past the
+  // descriptor's end: zeros.  KV8: into registers.
+  const __amdgpu_buffer_rsrc_t kr = __builtin_amdgcn_make_buffer_rsrc(const_cast<f16*>(a.kring + (KV8 ? 0 : ring)), 0, KV8 ? 0 : wg_valid * ROW, 0x00020000);
+  const __amdgpu_buffer_rsrc_t vr = __builtin_amdgcn_make_buffer_rsrc(const_cast<f16*>(a.vring + (KV8 ? 0 : ring)), 0, KV8 ? 0 : wg_valid * ROW, 0x00020000);
   u32x2 kq[NV], vq[NV];       // KV8: the bytes as stored
-  auto request = [&](int p) {
+  auto request = [&](int p, unsigned char* stage) {
 #pragma unroll
     for (int i = 0; i < NV; ++i) {
-      const int c = (int)threadIdx.x + i * PA_THREADS;
-      const int row = c / (D / 8), col = (c % (D / 8)) * 8;
-      kv[i] = f16x8{}; vv[i] = f16x8{};
-      kq[i] = u32x2{0, 0}; vq[i] = u32x2{0, 0};      // (the byte 0 is the value 0)
-      if (p + row < wg_valid) {
-        if constexpr (KV8) {
-          kq[i] = *reinterpret_cast<const u32x2*>(kbase8 + (size_t)(p + row) * D + col);
-          vq[i] = *reinterpret_cast<const u32x2*>(vbase8 + (size_t)(p + row) * D + col);
-        } else {
-          kv[i] = *reinterpret_cast<const f16x8*>(kbase + (size_t)(p + row) * D + col);
-          vv[i] = *reinterpret_cast<const f16x8*>(vbase + (size_t)(p + row) * D + col);
+      if constexpr (KV8) {
+        const int c = (int)threadIdx.x + i * PA_THREADS, row = c / VPR, col = (c % VPR) * 8;
+        kq[i] = u32x2{0, 0}; vq[i] = u32x2{0, 0};          // (the byte 0 is the value 0)
+        if (p + row < wg_valid) {
+          kq[i] = *reinterpret_cast<const u32x2*>(reinterpret_cast<const uint8_t*>(a.kring) + ring + (size_t)(p + row) * D + col);
+          vq[i] = *reinterpret_cast<const u32x2*>(reinterpret_cast<const uint8_t*>(a.vring) + ring + (size_t)(p + row) * D + col);
         }
+      } else {
+        const int q = i * (PA_THREADS / 64) + wave;        // 64 places of 16 bytes: LDS receives them lane after lane
+        const int row = (q * 64 + lane) / VPR, piece = (lane % VPR) ^ pa_key<D>(row);
+        const int from = (p + row) * ROW + piece * 16;
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(kr, (__attribute__((address_space(3))) void*)(stage + q * 1024), 16, from, 0, 0, 0);
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(vr, (__attribute__((address_space(3))) void*)(stage + STAGE + q * 1024), 16, from, 0, 0, 0);
       }
     }
   };
-  request(0);
-  for (int p0 = 0; p0 < wg_valid; p0 += 32) {
-    __syncthreads();
+  auto decode = [&](unsigned char* stage) {
 #pragma unroll
     for (int i = 0; i < NV; ++i) {
-      const int c = (int)threadIdx.x + i * PA_THREADS;
-      const int row = c / (D / 8), col = (c % (D / 8)) * 8;
-      if constexpr (KV8) {
-        kv[i] = f143_decode8(kq[i][0], kq[i][1]);
-        vv[i] = f143_decode8(vq[i][0], vq[i][1]);
-      }
-      *reinterpret_cast<f16x8*>(ks + row * PA_KSTRIDE + col) = kv[i];
-#pragma unroll
-      for (int e = 0; e < 8; ++e) vt[pa_vt_at(col + e, row)] = vv[i][e];
+      const int c = (int)threadIdx.x + i * PA_THREADS, row = c / VPR, at = row * ROW + ((c % VPR) ^ pa_key<D>(row)) * 16;
+      *reinterpret_cast<f16x8*>(stage + at) = f143_decode8(kq[i][0], kq[i][1]);
+      *reinterpret_cast<f16x8*>(stage + STAGE + at) = f143_decode8(vq[i][0], vq[i][1]);
     }
-    if (p0 + 32 < wg_valid) request(p0 + 32);
-    __syncthreads();
+  };
+  // K operands: row l % 16 of a tile, features (l / 16) * 8 + 0..7 of each 32
+  const int k_row = (lane & 15) * ROW, k_key = pa_key<D>(lane & 15);
+  // V operands: sixteen lanes read four rows of sixteen features, four features a lane, and receive one feature of the four rows each
+  const int v_at = ((lane >> 4) * 4 + ((lane & 15) >> 2)), v_row = v_at * ROW + (lane & 1) * 8, v_key = pa_key<D>(v_at), v_piece = (lane & 3) >> 1;
+
+  request(0, smem);
+  int turn = 0;
+  for (int p0 = 0; p0 < wg_valid; p0 += PA_KEYS, turn ^= 1) {
+    unsigned char* const stage = smem + turn * (2 * STAGE);
+    if constexpr (KV8) decode(stage);
+    else __builtin_amdgcn_s_waitcnt(0x0f70);               // vmcnt(0): this wave's share of the step's rows has landed
+    __syncthreads();                                       // (and every wave is done with the other stage)
+    if (p0 + PA_KEYS < wg_valid) request(p0 + PA_KEYS, smem + (turn ^ 1) * (2 * STAGE));
     if (p0 >= wave_valid) continue;
-    f32x4 sc[PA_RG][2];
+    f32x4 sc[PA_RG][4];
 #pragma unroll
-    for (int hh = 0; hh < 2; ++hh) {
+    for (int hh = 0; hh < 4; ++hh) {
 #pragma unroll
       for (int g = 0; g < PA_RG; ++g) sc[g][hh] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int m = 0; m < D / 32; ++m) {
-        const f16x8 kf = *reinterpret_cast<const f16x8*>(ks + (hh * 16 + (lane & 15)) * PA_KSTRIDE + m * 32 + (lane >> 4) * 8);
+        const f16x8 kf = *reinterpret_cast<const f16x8*>(stage + hh * 16 * ROW + k_row + (((m * 4 + (lane >> 4)) ^ k_key) * 16));
 #pragma unroll
         for (int g = 0; g < PA_RG; ++g) sc[g][hh] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kf, qf[g][m], sc[g][hh], 0, 0, 0);
       }
     }
-    f16x8 pa[PA_RG];
-    float cr[PA_RG][4];
+    f16x8 pa[PA_RG][2];
 #pragma unroll
     for (int g = 0; g < PA_RG; ++g) {
-      float x[8];
+      float x[16];
 #pragma unroll
-      for (int hh = 0; hh < 2; ++hh)
+      for (int e = 0; e < 16; ++e) {
+        f16 s16 = (f16)(KV8 ? sc[g][e >> 2][e & 3] * kv_mul : sc[g][e >> 2][e & 3]);      // fp16 output of the q.K^T MatMul
+        if (a.use_scale) s16 = s16 * a.scale;       // fp16 multiply by fp16(1/sqrt(D))
+        x[e] = (float)s16;
+      }
+      if (p0 + PA_KEYS > all_valid[g]) {
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          f16 s16 = (f16)(KV8 ? sc[g][hh][r] * kv_mul : sc[g][hh][r]);      // fp16 output of the q.K^T MatMul
-          if (a.use_scale) s16 = s16 * a.scale;       // fp16 multiply by fp16(1/sqrt(D))
-          const int pos = p0 + hh * 16 + (lane >> 4) * 4 + r;
-          x[hh * 4 + r] = pos < my_valid[g] ? (float)s16 : -INFINITY;
-        }
+        for (int e = 0; e < 16; ++e)
+          if (p0 + (e >> 2) * 16 + (lane >> 4) * 4 + (e & 3) >= my_valid[g]) x[e] = -INFINITY;
+      }
       float mx = x[0];
 #pragma unroll
-      for (int e = 1; e < 8; ++e) mx = fmaxf(mx, x[e]);
-      mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
-      mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
-      const float new_m = fmaxf(run_m[g], mx);
-      const float corr = run_m[g] == -INFINITY ? 0.f : __expf(run_m[g] - new_m);
+      for (int e = 1; e < 16; ++e) mx = fmaxf(mx, x[e]);
+      const float new_m = fmaxf(run_m[g], max_over_quarters(mx));
+      const float base = new_m == -INFINITY ? 0.f : new_m; // (nothing valid yet: the exponentials of -inf are zeros)
+      if (__any(new_m > run_m[g])) {
+        const float corr = __expf(run_m[g] - base);
+        run_l[g] *= corr;
+#pragma unroll
+        for (int jd = 0; jd < D / 16; ++jd)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) o[g][jd][r] *= corr;
+        run_m[g] = new_m;
+      }
       float psum = 0.f;
 #pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        const float pe = x[e] == -INFINITY ? 0.f : __expf(x[e] - new_m);
+      for (int e = 0; e < 16; ++e) {
+        const float pe = __expf(x[e] - base);
         psum += pe;
-        pa[g][e] = (f16)pe;
+        pa[g][e >> 3][e & 7] = (f16)pe;
       }
-      psum += __shfl_xor(psum, 16, 64);
-      psum += __shfl_xor(psum, 32, 64);
-      run_l[g] = run_l[g] * corr + psum;
-      run_m[g] = new_m;
-      // the accumulators' rows are query rows (lane / 16) * 4 + r: their correction factors sit in lanes of that index
-#pragma unroll
-      for (int r = 0; r < 4; ++r) cr[g][r] = __shfl(corr, (lane >> 4) * 4 + r, 64);
+      run_l[g] += psum;
     }
 #pragma unroll
     for (int jd = 0; jd < D / 16; ++jd) {
-      // cache rows (lane / 16) * 4 + 0..3 and 16 + the same of feature jd * 16 + lane % 16
-      const int d = jd * 16 + (lane & 15);
-      const f16x4 v0 = *reinterpret_cast<const f16x4*>(vt + pa_vt_at(d, (lane >> 4) * 4));
-      const f16x4 v1 = *reinterpret_cast<const f16x4*>(vt + pa_vt_at(d, 16 + (lane >> 4) * 4));
-      const f16x8 vb = {v0[0], v0[1], v0[2], v0[3], v1[0], v1[1], v1[2], v1[3]};
 #pragma unroll
-      for (int g = 0; g < PA_RG; ++g) {
+      for (int kg = 0; kg < 2; ++kg) {
+        // cache rows (lane / 16) * 4 + 0..3 and 16 + the same of these 32, of feature jd * 16 + lane % 16
+        unsigned char* const from = stage + STAGE + kg * 32 * ROW + v_row + (((jd * 2 + v_piece) ^ v_key) * 16);
+        const f16x4 v0 = bitcast<f16x4>(__builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4*)(from)));
+        const f16x4 v1 = bitcast<f16x4>(__builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4*)(from + 16 * ROW)));
+        const f16x8 vb = {v0[0], v0[1], v0[2], v0[3], v1[0], v1[1], v1[2], v1[3]};
 #pragma unroll
-        for (int r = 0; r < 4; ++r) o[g][jd][r] *= cr[g][r];
-        o[g][jd] = __builtin_amdgcn_mfma_f32_16x16x32_f16(pa[g], vb, o[g][jd], 0, 0, 0);
+        for (int g = 0; g < PA_RG; ++g) o[g][jd] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vb, pa[g][kg], o[g][jd], 0, 0, 0);
       }
     }
   }
+  const bool vectors = (reinterpret_cast<uintptr_t>(a.out) & 7) == 0;
 #pragma unroll
   for (int g = 0; g < PA_RG; ++g) {
-    float lr[4];
+    float l = run_l[g];
+    l += __shfl_xor(l, 16, 64);
+    l += __shfl_xor(l, 32, 64);
+    const int row = r0 + g * 16 + (lane & 15);
+    if (row >= a.rows) continue;
+    f16* out = a.out + (((size_t)b * a.rows + row) * a.Hq + h) * D + (lane >> 4) * 4;
 #pragma unroll
-    for (int r = 0; r < 4; ++r) lr[r] = __shfl(run_l[g], (lane >> 4) * 4 + r, 64);
+    for (int jd = 0; jd < D / 16; ++jd) {
+      f16x4 y;
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int row = r0 + g * 16 + (lane >> 4) * 4 + r;
-      if (row >= a.rows) continue;
-#pragma unroll
-      for (int jd = 0; jd < D / 16; ++jd)
-        a.out[(((size_t)b * a.rows + row) * a.Hq + h) * D + jd * 16 + (lane & 15)] =
-            attn_result(a, (f16)((KV8 ? o[g][jd][r] * kv_mul : o[g][jd][r]) / lr[r]));
+      for (int r = 0; r < 4; ++r) {
+        y[r] = attn_result(a, (f16)((KV8 ? o[g][jd][r] * kv_mul : o[g][jd][r]) / l));
+        if (!vectors) out[jd * 16 + r] = y[r];
+      }
+      if (vectors) *reinterpret_cast<f16x4*>(out + jd * 16) = y;
     }
   }
 }
@@ -1013,11 +1053,13 @@ static int attention_rows(const char* name, const pta_half* q, const void* kv_ri
   if (rows >= 16) {        // many rows: on the matrix unit, no splits, no workspace
     int dev = 0, cus = 256;
     if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0) cus = 256;
-    const bool two = (long)((rows + 127) / 128) * Hq * B >= 2L * cus;
-    const dim3 grid(two ? (rows + 127) / 128 : (rows + 63) / 64, Hq, B);
+    const bool two = !(kv8 && D == 128) && (long)((rows + 127) / 128) * Hq * B >= 2L * cus;
+    PTA_REQUIRE((long)B * Hq < (1L << 20), "%s: %d sequences of %d heads", name, B, Hq);
+    a.per_head = 1.0f / (float)Hq; a.per_group = (float)Hkv / (float)Hq;
+    const dim3 grid(8, two ? (rows + 127) / 128 : (rows + 63) / 64, (B * Hq + 7) / 8);
     auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, grid, dim3(PA_THREADS), 0, (hipStream_t)stream, a); };
     if (D == 128) {
-      if (kv8) { if (two) go(prompt_attention_mfma_kernel<128, 2, true>); else go(prompt_attention_mfma_kernel<128, 1, true>); }
+      if (kv8) go(prompt_attention_mfma_kernel<128, 1, true>);           // (two groups: more registers than two waves a SIMD have)
       else { if (two) go(prompt_attention_mfma_kernel<128, 2, false>); else go(prompt_attention_mfma_kernel<128, 1, false>); }
     } else {
       if (kv8) { if (two) go(prompt_attention_mfma_kernel<64, 2, true>); else go(prompt_attention_mfma_kernel<64, 1, true>); }

@@ -1,0 +1,48 @@
+"""prompt_attention_mfma_kernel at the ends of its row groups, workgroups and steps of 64 cache rows, against float64."""
+import math
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+CASES = [  # sequences, rows, query heads, KV heads, ring, step
+    (1, 16, 1, 1, 16, 0), (1, 17, 8, 8, 64, 0), (2, 63, 5, 5, 128, 0), (1, 64, 9, 3, 130, 65), (3, 65, 12, 4, 200, 63), (1, 129, 16, 2, 192, 40),
+    (2, 128, 7, 7, 100, 20), (1, 300, 32, 32, 512, 1)]
+
+
+@pytest.mark.parametrize("kv8", [False, True])
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("B, rows, Hq, Hkv, ring, step", [c for c in CASES if c[1] <= c[4]])
+@pytest.mark.parametrize("offset", [0, 1])
+def test_against_float64(B, rows, Hq, Hkv, ring, step, D, kv8, offset):
+    from poptransformer_amd import kernels as K
+    g = torch.Generator(device="cuda").manual_seed(rows)
+    randn = lambda *s: torch.randn(s, generator=g, device="cuda")
+    q = randn(B, rows, Hq, D).half()
+    # rows of the ring past the last valid one hold NaN (F143 has none: its largest value)
+    n = min(step + rows, ring)
+    if kv8:
+        codes = K.half_to_fp8(randn(2 * B * Hkv * ring, D).half(), torch.tensor([0], dtype=torch.int32, device="cuda"), "F143").view(2, B, Hkv, ring, D)
+        codes[:, :, :, n:] = 0x7F
+        kv = K.fp8_to_half(codes.view(-1, D), torch.tensor([0], dtype=torch.int32, device="cuda"), "F143").view(codes.shape)
+    else:
+        kv = codes = randn(2, B, Hkv, ring, D).half()
+        codes[:, :, :, n:] = float("nan")
+    store = torch.full((B * rows * Hq * D + 1,), float("nan"), dtype=torch.float16, device="cuda")
+    out = store[offset:offset + B * rows * Hq * D].view(B, rows, Hq, D)
+    K.prompt_attention(q, codes, torch.tensor(step, dtype=torch.int32, device="cuda"), K.decode_attention_workspace(B * rows, Hq, D, ring, "cuda"), out,
+                       B, rows, Hq, Hkv, D, ring, True, kv_scale=0 if kv8 else None)
+    k, v = (t[:, :, :n].double().repeat_interleave(Hq // Hkv, dim=1) for t in kv)
+    scale = torch.tensor(1 / math.sqrt(D), dtype=torch.float16, device="cuda")
+    s = ((q.double().transpose(1, 2).contiguous().float() @ k.transpose(2, 3).contiguous().float()).half() * scale).double()
+    valid = torch.clamp(torch.arange(rows, device="cuda") + step + 1, max=ring)
+    seen = torch.arange(n, device="cuda")[None, :] < valid[:, None]
+    p = torch.softmax(s.masked_fill(~seen, -math.inf), dim=-1)
+    ref, mag = p @ v, p @ v.abs()
+    # the probabilities' rounding (2^-11, below 2^-14 steps of 2^-25 on numbers whose largest is 1), the result's, fp32 sums; a score whose sum
+    # rounds to the other fp16 neighbour, and then its product with the scale, moves its probability by 2 * 2^-10 of the score
+    top = s.masked_fill(~seen, 0).abs().amax(-1, keepdim=True)
+    bound = (2.0 ** -11 * 2 + 4 * 2.0 ** -10 * top + n * 2.0 ** -20) * mag + n * 2.0 ** -25 * v.abs().amax() + 2.0 ** -24
+    got = out.double().transpose(1, 2)
+    assert torch.isfinite(got).all()
+    assert ((got - ref).abs() <= bound).all(), ((got - ref).abs() / bound).max().item()
