@@ -277,23 +277,50 @@ struct GemmArgs {
   int ksplit;          // 0 or 1: no split
   int prefer_stream;   // host side: up to 16 rows go to gemv_stream_kernel wherever it fits
 };
+// v, read from memory at this point and kept in scalar registers
+template <class T>
+__device__ __forceinline__ void in_register(T& v) { asm volatile("" : "+s"(v)); }
+
+// What the end of a kernel needs of its arguments, read at this point: while the first loads are on their way, that is.  Read where it
+// is used, each line of the arguments is a round trip to memory of its own, one after another behind the products.
+template <class Fmt, bool PAIR>
+__device__ __forceinline__ void read_end(GemmMat& mat, GemmEpilogue& epi) {
+  in_register(mat.Y);
+  if constexpr (Fmt::kWide) {
+    WideOut& o = mat.wide;
+    in_register(o.ld); in_register(o.n_main); in_register(o.out_f32);
+    in_register(o.bias); in_register(o.mul); in_register(o.mul_f32); in_register(o.accumulate);
+    if constexpr (PAIR) {
+      in_register(o.clamped); in_register(o.limit); in_register(o.slope); in_register(o.bias2);
+    } else {
+      in_register(o.tail); in_register(o.tail_count); in_register(o.tail_bias); in_register(o.cap); in_register(o.act);
+    }
+  } else {
+    if constexpr (!PAIR) {
+      in_register(mat.bias); in_register(mat.act); in_register(epi.bias); in_register(epi.residual); in_register(epi.act);
+      in_register(epi.mul); in_register(epi.post_scale);
+    }
+    in_register(epi.out_fp8_scale); in_register(epi.out_fp8_format);
+  }
+}
+
 // One finished fp32 sum of a matrix, or of a gate / up pair, on its way out.
 template <class Fmt>
-__device__ __forceinline__ void gemm_put(const GemmArgs& a, const GemmMat& mat, int m, int n, int N, float sum) {
+__device__ __forceinline__ void gemm_put(const GemmEpilogue& epi, const GemmMat& mat, int m, int n, int N, float sum) {
   if constexpr (Fmt::kWide) {
     wide_put(mat, m, n, sum);
   } else {
     f16 y0 = (f16)sum;
     if (mat.bias) y0 = y0 + mat.bias[n];
     y0 = apply_act(mat.act, y0);
-    mat.Y[(size_t)m * N + n] = apply_epilogue(a.epi, y0, m, n, N);
+    mat.Y[(size_t)m * N + n] = apply_epilogue(epi, y0, m, n, N);
   }
 }
 
 template <class Fmt>
-__device__ __forceinline__ void gemm_put_pair(const GemmArgs& a, int m, int n, int N, float gate, float up) {
-  if constexpr (Fmt::kWide) wide_put_pair(a.mat[0], m, n, gate, up);
-  else a.mat[0].Y[(size_t)m * N + n] = swiglu_out(a.epi, (f16)gate, (f16)up);
+__device__ __forceinline__ void gemm_put_pair(const GemmEpilogue& epi, const GemmMat& mat, int m, int n, int N, float gate, float up) {
+  if constexpr (Fmt::kWide) wide_put_pair(mat, m, n, gate, up);
+  else mat.Y[(size_t)m * N + n] = swiglu_out(epi, (f16)gate, (f16)up);
 }
 
 static inline int device_compute_units();
@@ -397,9 +424,9 @@ __global__ __launch_bounds__(NW * 64) void gemv_mfma_kernel(GemmArgs a) {
       sum[g] = Fmt::finish(t, sc[g]);
     }
     if (PAIR) {
-      gemm_put_pair<Fmt>(a, m, n, N, sum[0], sum[1]);
+      gemm_put_pair<Fmt>(a.epi, a.mat[0], m, n, N, sum[0], sum[1]);
     } else {
-      gemm_put<Fmt>(a, a.mat[mi], m, n, N, sum[0]);
+      gemm_put<Fmt>(a.epi, a.mat[mi], m, n, N, sum[0]);
     }
   }
 }
@@ -446,6 +473,13 @@ __global__ __launch_bounds__(NW * 64) void gemv_lds_kernel(GemmArgs a) {
     for (int g = 0; g < NACC; ++g)
 #pragma unroll
       for (int v = 0; v < KV; ++v) wcur[g][v] = __builtin_nontemporal_load(wp[g] + ((size_t)kt * KV + v) * 64);
+  }
+  // (bf16, 1 row, 2048 x 2048: 4.4 against 4.6 us; the fp16 epilogue's few arguments gain nothing)
+  GemmMat wide;
+  GemmEpilogue none{};
+  if constexpr (Fmt::kWide) {
+    wide = a.mat[PAIR ? 0 : mi];
+    read_end<Fmt, PAIR>(wide, none);
   }
   // stage X (zero beyond K), normalising its rows on the way when a norm is fused
   {
@@ -582,9 +616,9 @@ __global__ __launch_bounds__(NW * 64) void gemv_lds_kernel(GemmArgs a) {
       sum[g] = Fmt::finish(t, sc[g]);
     }
     if (PAIR) {
-      gemm_put_pair<Fmt>(a, m, n, N, sum[0], sum[1]);
+      gemm_put_pair<Fmt>(a.epi, Fmt::kWide ? wide : a.mat[0], m, n, N, sum[0], sum[1]);
     } else {
-      gemm_put<Fmt>(a, a.mat[mi], m, n, N, sum[0]);
+      gemm_put<Fmt>(a.epi, Fmt::kWide ? wide : a.mat[mi], m, n, N, sum[0]);
     }
   }
 }
@@ -599,13 +633,12 @@ __global__ __launch_bounds__(NW * 64) void gemv_lds_kernel(GemmArgs a) {
 // ------------------------------------------------------------------------------------------
 constexpr int WIDE_WAVES = 16;
 
-template <class Fmt, int MT, int NB, bool PAIR, bool NORM = false>
+template <class Fmt, int NB, bool PAIR, bool NORM = false>
 __global__ __launch_bounds__(WIDE_WAVES * 64) void gemv_wide_kernel(GemmArgs a, int total_nb) {
-  static_assert(!NORM || MT == 1, "the fused norm covers up to 16 rows");
   constexpr int NACC = PAIR ? 2 : 1;
   constexpr int KV = Fmt::kVec;
   extern __shared__ __align__(16) unsigned char smem[];
-  float* red = reinterpret_cast<float*>(smem);          // [WIDE_WAVES][NB][NACC][MT][256]
+  float* red = reinterpret_cast<float*>(smem);          // [WIDE_WAVES][NB][NACC][256]
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int G = gridDim.x;
   const int K = a.K, KT = a.KT;
@@ -633,23 +666,17 @@ __global__ __launch_bounds__(WIDE_WAVES * 64) void gemv_wide_kernel(GemmArgs a, 
       wp[b][g] = reinterpret_cast<const u32x4*>(m.tiled) + (size_t)nb[b] * KT * (64 * KV) + lane;
     }
   }
-  const f16* xrow[MT];
-#pragma unroll
-  for (int mt = 0; mt < MT; ++mt) {
-    int mrow = mt * 16 + (lane & 15);
-    mrow = mrow < a.M ? mrow : a.M - 1;                 // padding rows compute values that are never stored
-    xrow[mt] = a.X + (size_t)mrow * K + (lane >> 4) * 8;
-  }
+  int row = lane & 15;
+  row = row < a.M ? row : a.M - 1;                      // padding rows compute values that are never stored
+  const f16* xrow = a.X + (size_t)row * K + (lane >> 4) * 8;
 
-  f32x4 acc[NB][NACC][MT];
+  f32x4 acc[NB][NACC];
 #pragma unroll
   for (int b = 0; b < NB; ++b)
 #pragma unroll
-    for (int g = 0; g < NACC; ++g)
-#pragma unroll
-      for (int mt = 0; mt < MT; ++mt) acc[b][g][mt] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int g = 0; g < NACC; ++g) acc[b][g] = f32x4{0.f, 0.f, 0.f, 0.f};
 
-  // Fused norm (MT == 1): a first pass over this wave's activation fragments gives the row sums (lane l
+  // Fused norm: a first pass over this wave's activation fragments gives the row sums (lane l
   // holds row l % 16, features (l / 16) * 8 + 0..7 of every 32), they meet over the lane groups and, in
   // LDS, over the waves; the product pass then normalises every fragment it loads, with the numerics of
   // pta_rmsnorm / pta_layer_norm_ce (rows > 1 variant).
@@ -661,7 +688,7 @@ __global__ __launch_bounds__(WIDE_WAVES * 64) void gemv_wide_kernel(GemmArgs a, 
       for (int j = 0; j < 4; ++j) {
         const int k = kt * 128 + j * 32;
         if (k + (lane >> 4) * 8 < K) {
-          const f16x8 v = *reinterpret_cast<const f16x8*>(xrow[0] + k);
+          const f16x8 v = *reinterpret_cast<const f16x8*>(xrow + k);
 #pragma unroll
           for (int e = 0; e < 8; ++e) { const float f = (float)v[e]; s1 += f; s2 = __builtin_fmaf(f, f, s2); }
         }
@@ -686,197 +713,147 @@ __global__ __launch_bounds__(WIDE_WAVES * 64) void gemv_wide_kernel(GemmArgs a, 
       n_r = (f16)(1.0f / sqrtf(var));
     }
   };
-  if constexpr (MT == 1) {
-    // UN feature tiles per step, all of their loads requested before the first product (a tile
-    // beyond KT repeats the last one with zero activations)
-    constexpr int UN = NB * NACC * KV <= 4 ? 2 : 1;
-    u32x4 w[UN][NB][NACC][KV];
-    f16x8 xb[UN][4];
-    auto load_w = [&](int kt0) {
+  // UN feature tiles per step, all of their loads requested before the first product (a tile
+  // beyond KT repeats the last one with zero activations)
+  constexpr int UN = NB * NACC * KV <= 4 ? 2 : 1;
+  u32x4 w[UN][NB][NACC][KV];
+  f16x8 xb[UN][4];
+  auto load_w = [&](int kt0) {
 #pragma unroll
-      for (int u = 0; u < UN; ++u) {
-        const int kt_ = kt0 + u * WIDE_WAVES;
-        const int kt = kt_ < KT ? kt_ : KT - 1;
-#pragma unroll
-        for (int b = 0; b < NB; ++b)
-#pragma unroll
-          for (int g = 0; g < NACC; ++g)
-#pragma unroll
-            for (int v = 0; v < KV; ++v)
-              w[u][b][g][v] = __builtin_nontemporal_load(wp[b][g] + ((size_t)kt * KV + v) * 64);
-      }
-    };
-    auto load_x = [&](int kt0) {
-#pragma unroll
-      for (int u = 0; u < UN; ++u) {
-        const int kt_ = kt0 + u * WIDE_WAVES;
-        const bool there = kt_ < KT;
-        const int kt = there ? kt_ : KT - 1;
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          const int k = kt * 128 + j * 32;
-          const f16x8 z = {0, 0, 0, 0, 0, 0, 0, 0};
-          const bool in = there && k + (lane >> 4) * 8 < K;
-          xb[u][j] = in ? *reinterpret_cast<const f16x8*>(xrow[0] + k) : z;
-          if (NORM && in) {
-            const f16x8 gm = *reinterpret_cast<const f16x8*>(a.epi.norm_weight + k + (lane >> 4) * 8);
-            if (a.epi.norm == PTA_NORM_RMS) {
-#pragma unroll
-              for (int e = 0; e < 8; ++e) xb[u][j][e] = (xb[u][j][e] * n_r) * gm[e];
-            } else {
-              const f16x8 bt = *reinterpret_cast<const f16x8*>(a.epi.norm_bias + k + (lane >> 4) * 8);
-#pragma unroll
-              for (int e = 0; e < 8; ++e) xb[u][j][e] = ((xb[u][j][e] - n_mean) * n_r) * gm[e] + bt[e];
-            }
-          }
-        }
-      }
-    };
-    auto products = [&]() {
-#pragma unroll
-      for (int u = 0; u < UN; ++u)
-#pragma unroll
-        for (int j = 0; j < 4; ++j)
-#pragma unroll
-          for (int b = 0; b < NB; ++b)
-#pragma unroll
-            for (int g = 0; g < NACC; ++g)
-              acc[b][g][0] = Fmt::mma(Fmt::a_operand(w[u][b][g], j, sc[b][g]), xb[u][j],
-                                                                    acc[b][g][0]);
-    };
-    int kt0 = wave;
-    if constexpr (NORM) {
-      // Fused norm: the first weight tiles are requested before the pass over the activations that gives the
-      // row statistics (lane l holds row l % 16, features (l / 16) * 8 + 0..7 of every 32; the sums meet over
-      // the lane groups and, in LDS, over the waves), so that pass runs while they are on their way.  The
-      // product pass then normalises every fragment it loads, with the numerics of pta_rmsnorm /
-      // pta_layer_norm_ce (rows > 1 variant).
-      if (kt0 < KT) load_w(kt0);
-      norm_statistics();
-      if (kt0 < KT) {
-        load_x(kt0);
-        products();
-        kt0 += WIDE_WAVES * UN;
-      }
-    }
-    for (; kt0 < KT; kt0 += WIDE_WAVES * UN) {
-      load_w(kt0);
-      load_x(kt0);
-      products();
-    }
-  } else {
-    // several row groups: the activation fragments of one 32-feature slice at a time (16 bytes per
-    // lane and row group), each used for all blocks before the next slice is read
-    for (int kt = wave; kt < KT; kt += WIDE_WAVES) {
-      u32x4 w[NB][NACC][KV];
+    for (int u = 0; u < UN; ++u) {
+      const int kt_ = kt0 + u * WIDE_WAVES;
+      const int kt = kt_ < KT ? kt_ : KT - 1;
 #pragma unroll
       for (int b = 0; b < NB; ++b)
 #pragma unroll
         for (int g = 0; g < NACC; ++g)
 #pragma unroll
-          for (int v = 0; v < KV; ++v) w[b][g][v] = __builtin_nontemporal_load(wp[b][g] + ((size_t)kt * KV + v) * 64);
+          for (int v = 0; v < KV; ++v)
+            w[u][b][g][v] = __builtin_nontemporal_load(wp[b][g] + ((size_t)kt * KV + v) * 64);
+    }
+  };
+  auto load_x = [&](int kt0) {
+#pragma unroll
+    for (int u = 0; u < UN; ++u) {
+      const int kt_ = kt0 + u * WIDE_WAVES;
+      const bool there = kt_ < KT;
+      const int kt = there ? kt_ : KT - 1;
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
         const int k = kt * 128 + j * 32;
         const f16x8 z = {0, 0, 0, 0, 0, 0, 0, 0};
-        f16x8 xb[MT];
+        const bool in = there && k + (lane >> 4) * 8 < K;
+        xb[u][j] = in ? *reinterpret_cast<const f16x8*>(xrow + k) : z;
+        if (NORM && in) {
+          const f16x8 gm = *reinterpret_cast<const f16x8*>(a.epi.norm_weight + k + (lane >> 4) * 8);
+          if (a.epi.norm == PTA_NORM_RMS) {
 #pragma unroll
-        for (int mt = 0; mt < MT; ++mt)
-          xb[mt] = k + (lane >> 4) * 8 < K ? *reinterpret_cast<const f16x8*>(xrow[mt] + k) : z;
+            for (int e = 0; e < 8; ++e) xb[u][j][e] = (xb[u][j][e] * n_r) * gm[e];
+          } else {
+            const f16x8 bt = *reinterpret_cast<const f16x8*>(a.epi.norm_bias + k + (lane >> 4) * 8);
+#pragma unroll
+            for (int e = 0; e < 8; ++e) xb[u][j][e] = ((xb[u][j][e] - n_mean) * n_r) * gm[e] + bt[e];
+          }
+        }
+      }
+    }
+  };
+  auto products = [&]() {
+#pragma unroll
+    for (int u = 0; u < UN; ++u)
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
 #pragma unroll
         for (int b = 0; b < NB; ++b)
 #pragma unroll
-          for (int g = 0; g < NACC; ++g) {
-            const f16x8 av = Fmt::a_operand(w[b][g], j, sc[b][g]);
-#pragma unroll
-            for (int mt = 0; mt < MT; ++mt)
-              acc[b][g][mt] = Fmt::mma(av, xb[mt], acc[b][g][mt]);
-          }
-      }
+          for (int g = 0; g < NACC; ++g)
+            acc[b][g] = Fmt::mma(Fmt::a_operand(w[u][b][g], j, sc[b][g]), xb[u][j],
+                                                                  acc[b][g]);
+  };
+  int kt0 = wave;
+  if constexpr (NORM) {
+    // Fused norm: the first weight tiles are requested before the pass over the activations that gives the
+    // row statistics (lane l holds row l % 16, features (l / 16) * 8 + 0..7 of every 32; the sums meet over
+    // the lane groups and, in LDS, over the waves), so that pass runs while they are on their way.  The
+    // product pass then normalises every fragment it loads, with the numerics of pta_rmsnorm /
+    // pta_layer_norm_ce (rows > 1 variant).
+    if (kt0 < KT) load_w(kt0);
+    norm_statistics();
+    if (kt0 < KT) {
+      load_x(kt0);
+      products();
+      kt0 += WIDE_WAVES * UN;
     }
   }
+  for (; kt0 < KT; kt0 += WIDE_WAVES * UN) {
+    load_w(kt0);
+    load_x(kt0);
+    products();
+  }
 
-  // The accumulator of lane l holds channels (l/16)*4 + r, r = 0..3, for activation row l%16 of its group.
+  // The accumulator of lane l holds channels (l/16)*4 + r, r = 0..3, for activation row l%16.
 #pragma unroll
   for (int b = 0; b < NB; ++b)
 #pragma unroll
     for (int g = 0; g < NACC; ++g)
 #pragma unroll
-      for (int mt = 0; mt < MT; ++mt)
-#pragma unroll
-        for (int r = 0; r < 4; ++r)
-          red[((((wave * NB + b) * NACC + g) * MT + mt) * 4 + r) * 64 + lane] = acc[b][g][mt][r];
+      for (int r = 0; r < 4; ++r) red[(((wave * NB + b) * NACC + g) * 4 + r) * 64 + lane] = acc[b][g][r];
   __syncthreads();
-  // The 256 outputs (16 rows x 16 channels) of (block b, row group mt) are finished by the quarter
-  // (b * MT + mt) % 4 of the workgroup, thread t of it taking row (t / 16) % 16, channel t % 16.
+  // The 256 outputs (16 rows x 16 channels) of block b are finished by quarter b of the workgroup, thread t of it taking row
+  // (t / 16) % 16, channel t % 16.
   const int quarter = threadIdx.x >> 8;
 #pragma unroll
   for (int b = 0; b < NB; ++b) {
+    if (b != quarter) continue;
+    const int nn = threadIdx.x & 15, m = (threadIdx.x >> 4) & 15;
+    const GemmMat& mat = a.mat[PAIR ? 0 : mi[b]];
+    const int N = mat.N, n = nb[b] * 16 + nn;
+    if ((int)blockIdx.x + b * G >= total_nb || m >= a.M || n >= N) continue;
+    const int r = nn & 3, ln = (nn >> 2) * 16 + m;
+    float sum[NACC];
 #pragma unroll
-    for (int mt = 0; mt < MT; ++mt) {
-      if (((b * MT + mt) & 3) != quarter) continue;
-      const int nn = threadIdx.x & 15, m = mt * 16 + ((threadIdx.x >> 4) & 15);
-      const GemmMat& mat = a.mat[PAIR ? 0 : mi[b]];
-      const int N = mat.N, n = nb[b] * 16 + nn;
-      if ((int)blockIdx.x + b * G >= total_nb || m >= a.M || n >= N) continue;
-      const int r = nn & 3, ln = (nn >> 2) * 16 + (m & 15);
-      float sum[NACC];
+    for (int g = 0; g < NACC; ++g) {
+      float t = 0.f;
 #pragma unroll
-      for (int g = 0; g < NACC; ++g) {
-        float t = 0.f;
-#pragma unroll
-        for (int w = 0; w < WIDE_WAVES; ++w) t += red[((((w * NB + b) * NACC + g) * MT + mt) * 4 + r) * 64 + ln];
-        sum[g] = Fmt::finish(t, sc[b][g]);      // no format's finish uses the per-channel part of the scale
-      }
-      if (PAIR) {
-        gemm_put_pair<Fmt>(a, m, n, N, sum[0], sum[1]);
-      } else {
-        gemm_put<Fmt>(a, mat, m, n, N, sum[0]);
-      }
+      for (int w = 0; w < WIDE_WAVES; ++w) t += red[(((w * NB + b) * NACC + g) * 4 + r) * 64 + ln];
+      sum[g] = Fmt::finish(t, sc[b][g]);      // no format's finish uses the per-channel part of the scale
     }
+    if (PAIR) gemm_put_pair<Fmt>(a.epi, mat, m, n, N, sum[0], sum[NACC - 1]);
+    else gemm_put<Fmt>(a.epi, mat, m, n, N, sum[0]);
   }
 }
 
-template <class Fmt, int MT, int NB, bool PAIR, bool NORM = false>
+template <class Fmt, int NB, bool PAIR, bool NORM>
 static int launch_gemv_wide(const GemmArgs& a, int total_nb, hipStream_t s, const char* name) {
   static bool ready = false;
-  const size_t smem = (size_t)WIDE_WAVES * NB * (PAIR ? 2 : 1) * MT * 256 * sizeof(float);
-  static_assert(WIDE_WAVES * NB * (PAIR ? 2 : 1) * MT * 1024 <= 128 * 1024, "reduction buffer beyond 128 KiB of LDS");
+  const size_t smem = (size_t)WIDE_WAVES * NB * (PAIR ? 2 : 1) * 256 * sizeof(float);
   if (!ready) {
-    PTA_REQUIRE(hipFuncSetAttribute((const void*)gemv_wide_kernel<Fmt, MT, NB, PAIR, NORM>,
+    PTA_REQUIRE(hipFuncSetAttribute((const void*)gemv_wide_kernel<Fmt, NB, PAIR, NORM>,
                                     hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem) == hipSuccess,
                 "%s: cannot reserve %zu bytes of LDS", name, smem);
     ready = true;
   }
-  hipLaunchKernelGGL((gemv_wide_kernel<Fmt, MT, NB, PAIR, NORM>), dim3((total_nb + NB - 1) / NB), dim3(WIDE_WAVES * 64), smem, s,
+  hipLaunchKernelGGL((gemv_wide_kernel<Fmt, NB, PAIR, NORM>), dim3((total_nb + NB - 1) / NB), dim3(WIDE_WAVES * 64), smem, s,
                      a, total_nb);
   return PTA_OK;
 }
 
-// blocks per workgroup: the launch's share per compute unit, capped by what the registers of a wave
-// (weight tiles in flight) and the LDS reduction buffer (8 KiB-groups of partial sums) hold
-// the longest chain of channel blocks a compute unit multiplies under launch_gemv_wide_for (M <= 16)
+// blocks per workgroup: the launch's share per compute unit, capped by what the registers of a wave (weight tiles in flight) hold
 template <class Fmt, bool PAIR>
-static int wide_block_times(int total_nb, int per_cu);
+constexpr int wide_cap() { return Fmt::kVec * (PAIR ? 2 : 1) <= 4 ? 3 : 2; }
 
-template <class Fmt, int MT, bool PAIR, bool NORM = false>
+template <class Fmt, bool PAIR, bool NORM>
 static int launch_gemv_wide_for(const GemmArgs& a, int total_nb, int per_cu, hipStream_t s, const char* name) {
-  constexpr int NACC = PAIR ? 2 : 1;
-  constexpr int cap_regs = Fmt::kVec * NACC <= 4 ? 3 : 2;
-  constexpr int cap_lds = 8 / (NACC * MT) >= 1 ? 8 / (NACC * MT) : 1;
-  constexpr int cap = cap_regs < cap_lds ? cap_regs : cap_lds;
-  if (per_cu <= 1 || cap == 1) return launch_gemv_wide<Fmt, MT, 1, PAIR, NORM>(a, total_nb, s, name);
-  if (per_cu == 2 || cap == 2) return launch_gemv_wide<Fmt, MT, cap >= 2 ? 2 : 1, PAIR, NORM>(a, total_nb, s, name);
-  return launch_gemv_wide<Fmt, MT, cap >= 3 ? 3 : 1, PAIR, NORM>(a, total_nb, s, name);
+  constexpr int cap = wide_cap<Fmt, PAIR>();
+  if (per_cu <= 1) return launch_gemv_wide<Fmt, 1, PAIR, NORM>(a, total_nb, s, name);
+  if (per_cu == 2 || cap == 2) return launch_gemv_wide<Fmt, 2, PAIR, NORM>(a, total_nb, s, name);
+  return launch_gemv_wide<Fmt, cap, PAIR, NORM>(a, total_nb, s, name);
 }
 
+// the longest chain of channel blocks a compute unit multiplies under launch_gemv_wide_for
 template <class Fmt, bool PAIR>
 static int wide_block_times(int total_nb, int per_cu) {
-  constexpr int NACC = PAIR ? 2 : 1;
-  constexpr int cap_regs = Fmt::kVec * NACC <= 4 ? 3 : 2;
-  constexpr int cap_lds = 8 / NACC;
-  constexpr int cap = cap_regs < cap_lds ? cap_regs : cap_lds;
-  const int nb = per_cu < cap ? per_cu : cap;
+  const int nb = per_cu < wide_cap<Fmt, PAIR>() ? per_cu : wide_cap<Fmt, PAIR>();
   const int cus = device_compute_units();
   const int wgs = (total_nb + nb - 1) / nb;
   return (wgs + cus - 1) / cus * nb;
@@ -1039,9 +1016,9 @@ void gemv_stream_kernel(GemmArgs a, int total_nb) {
           sum[g] = Fmt::finish(t, sc[g]);        // no format's finish uses the per-channel part of the scale
         }
         if (PAIR) {
-          gemm_put_pair<Fmt>(a, m, n, N, sum[0], sum[1]);
+          gemm_put_pair<Fmt>(a.epi, a.mat[0], m, n, N, sum[0], sum[1]);
         } else if constexpr (Fmt::kWide) {
-          gemm_put<Fmt>(a, mat, m, n, N, sum[0]);
+          gemm_put<Fmt>(a.epi, mat, m, n, N, sum[0]);
         } else {
           // as apply_epilogue, with the operands that came with the weights
           f16 y0 = (f16)sum[0];
@@ -1249,9 +1226,9 @@ __global__ __launch_bounds__(NWV * 64) void gemm_tile_kernel(GemmArgs a) {
 #pragma unroll
     for (int g = 0; g < (PAIR ? 2 : 1); ++g) sum[g] = Fmt::finish(sum[g], sc[0]);   // no format's finish uses the per-channel part
     if (PAIR) {
-      gemm_put_pair<Fmt>(a, m, n, N, sum[0], sum[1]);
+      gemm_put_pair<Fmt>(a.epi, a.mat[0], m, n, N, sum[0], sum[1]);
     } else {
-      gemm_put<Fmt>(a, mat, m, n, N, sum[0]);
+      gemm_put<Fmt>(a.epi, mat, m, n, N, sum[0]);
     }
   }
 }
@@ -1289,7 +1266,7 @@ __global__ __launch_bounds__(256) void splitk_finish_kernel(GemmArgs a) {
   } else {
     float t = 0.f;
     for (int sl = 0; sl < a.ksplit; ++sl) t += a.part[(size_t)sl * total + i];
-    gemm_put<Fmt>(a, mat, m, n, N, Fmt::finish(t, Fmt::load_scale(mat.scale, a.x_scale, n, N)));
+    gemm_put<Fmt>(a.epi, mat, m, n, N, Fmt::finish(t, Fmt::load_scale(mat.scale, a.x_scale, n, N)));
   }
 }
 
@@ -1349,10 +1326,9 @@ constexpr int OWN_WAVES = 8;
 template <class Fmt> struct OwnStreams { static constexpr int cap = Fmt::kVec == 4 ? 3 : 4; };
 template <class Fmt, bool PAIR> constexpr int own_cap(int mt) { return (OwnStreams<Fmt>::cap + (Fmt::kVec == 1 && mt <= 2 ? 1 : 0)) / (PAIR ? 2 : 1); }
 constexpr int own_ahead(int mt) { return mt <= 1 ? 2 : 1; }
-
-// v, read from memory at this point and kept in scalar registers
-template <class T>
-__device__ __forceinline__ void in_register(T& v) { asm volatile("" : "+s"(v)); }
+// tiles of weights in flight or in use: a tile of 16 rows takes less time than its weights' way from memory (13696 x 4096, 8 rows: F143
+// 17.4 -> 14.9 us, INT4 12.3 -> 10.9; at 32 rows no gain)
+constexpr int own_depth(int mt, int vectors) { return mt == 1 && vectors <= 4 ? 4 : 2; }
 
 template <class Fmt, int MT, int NB, bool PAIR>
 __global__ __launch_bounds__(OWN_WAVES * 64) __attribute__((amdgpu_waves_per_eu(2, 2))) void gemm_own_kernel(GemmArgs a, int groups) {
@@ -1441,37 +1417,41 @@ __global__ __launch_bounds__(OWN_WAVES * 64) __attribute__((amdgpu_waves_per_eu(
   for (int st = 0; st < NS; ++st)
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt) acc[st][mt] = f32x4{0.f, 0.f, 0.f, 0.f};
-  // Requests are made in the order x(0), w(0), x(1), w(1), ...: this many follow those of a row group when it is waited for
+  // Requests are made in the order x(0), w(n), x(1), w(n + 1), ...: this many follow those of a row group when it is waited for
   constexpr int BEHIND = 4 * (RING - 1) + AHEAD * NS * KV;
-  constexpr int WAIT = 0x0f70 | (BEHIND & 15) | (BEHIND >> 4) << 14;
   static_assert(BEHIND < 64, "the counter of requests");
-  u32x4 w[2][NS][KV];
+  constexpr int DEPTH = own_depth(MT, NS * KV);
+  u32x4 w[DEPTH][NS][KV];
   f16x8 xb[2][4];
-  auto read_x = [&](int place, f16x8 (&to)[4]) {
-    __builtin_amdgcn_s_waitcnt(WAIT);
+  auto read_x = [&](int place, f16x8 (&to)[4], auto behind) {
+    constexpr int N = decltype(behind)::value;
+    __builtin_amdgcn_s_waitcnt(0x0f70 | (N & 15) | (N >> 4) << 14);
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int j = 0; j < 4; ++j) to[j] = *reinterpret_cast<const f16x8*>(area + place * 4096 + (lane & 15) * 256 + (((j * 4 + (lane >> 4)) ^ (lane & 15)) * 16));
   };
-  // tile i: TURN is i modulo what makes the places in the area and the buffers of w and xb come round again
-  auto step = [&](int i, auto turn) {
-    constexpr int TURN = decltype(turn)::value;
+  // tile i: TURN is i modulo what makes the places in the area and the buffers of w and xb come round again; LAST: how many of the
+  // last tiles, which request no more weights, came before it (-1: it is none of them)
+  auto step = [&](int i, auto turn, auto last) {
+    constexpr int TURN = decltype(turn)::value, LAST = decltype(last)::value;
+    constexpr int SHORT = LAST > AHEAD ? AHEAD : LAST < 0 ? 0 : LAST, SHORT_NEXT = LAST + 1 > AHEAD ? AHEAD : LAST + 1;
     f16x8 av[NS][4];
 #pragma unroll
     for (int st = 0; st < NS; ++st)
 #pragma unroll
-      for (int j = 0; j < 4; ++j) av[st][j] = Fmt::a_operand(w[TURN & 1][st], j, sc[st]);
+      for (int j = 0; j < 4; ++j) av[st][j] = Fmt::a_operand(w[TURN][st], j, sc[st]);
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt) {
       constexpr int Q0 = TURN * MT;
       const int q = Q0 + mt, place = (q + 1) % RING;        // the next row group: read while this one is multiplied, then requested anew
       if (mt == MT - 1) {
         __builtin_amdgcn_sched_barrier(0);
-        fetch_w(tile(i + 2), w[TURN & 1]);
+        if constexpr (LAST < 0) fetch_w(tile(i + DEPTH), w[TURN]);
         next_x(tile(i + 1 + AHEAD));
         __builtin_amdgcn_sched_barrier(0);
       }
-      read_x(place, xb[(q + 1) & 1]);
+      if (mt == MT - 1) read_x(place, xb[(q + 1) & 1], std::integral_constant<int, BEHIND - SHORT_NEXT * NS * KV>{});
+      else read_x(place, xb[(q + 1) & 1], std::integral_constant<int, BEHIND - SHORT * NS * KV>{});
 #pragma unroll
       for (int j = 0; j < 4; ++j)
 #pragma unroll
@@ -1482,7 +1462,9 @@ __global__ __launch_bounds__(OWN_WAVES * 64) __attribute__((amdgpu_waves_per_eu(
       __builtin_amdgcn_sched_barrier(0);
     }
   };
-  if (AHEAD == 1) fetch_w(tile(0), w[0]);
+#pragma unroll
+  for (int t = 0; t < DEPTH - AHEAD; ++t) fetch_w(tile(t), w[t]);
+  __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
   for (int t = 0; t < AHEAD; ++t) {
     next_x(tile(t));
@@ -1490,11 +1472,11 @@ __global__ __launch_bounds__(OWN_WAVES * 64) __attribute__((amdgpu_waves_per_eu(
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt) fetch_x(mt, t * MT + mt);
     __builtin_amdgcn_sched_barrier(0);
-    fetch_w(tile(AHEAD == 1 ? 1 : t), w[AHEAD == 1 ? 1 : t]);
+    fetch_w(tile(DEPTH - AHEAD + t), w[DEPTH - AHEAD + t]);
     __builtin_amdgcn_sched_barrier(0);
   }
   next_x(tile(AHEAD));
-  read_x(0, xb[0]);
+  read_x(0, xb[0], std::integral_constant<int, BEHIND>{});
   __builtin_amdgcn_s_waitcnt(0xc07f);
   __builtin_amdgcn_sched_barrier(0);
   fetch_x(0, 0);
@@ -1503,24 +1485,27 @@ __global__ __launch_bounds__(OWN_WAVES * 64) __attribute__((amdgpu_waves_per_eu(
   // of its own otherwise, one after another behind the products.
   GemmMat out = mat;
   GemmEpilogue epi = a.epi;
-  in_register(out.Y);
-  if constexpr (Fmt::kWide) {
-    WideOut& o = out.wide;
-    in_register(o.ld); in_register(o.n_main); in_register(o.out_f32); in_register(o.tail); in_register(o.tail_count);
-    in_register(o.tail_bias); in_register(o.cap); in_register(o.clamped); in_register(o.limit); in_register(o.slope);
-    in_register(o.bias); in_register(o.bias2); in_register(o.act); in_register(o.mul); in_register(o.mul_f32); in_register(o.accumulate);
-  } else {
-    in_register(out.bias); in_register(out.act);
-    in_register(epi.bias); in_register(epi.residual); in_register(epi.act); in_register(epi.mul); in_register(epi.post_scale);
-    in_register(epi.out_fp8_scale); in_register(epi.out_fp8_format);
-  }
-  // (in pairs, with no way out between the two: where paths meet, the compiler waits for what is in flight on either)
+  read_end<Fmt, PAIR>(out, epi);
+  // (in pairs or fours, with no way out between them: where paths meet, the compiler waits for what is in flight on either)
+  using std::integral_constant;
   int i = 0;
-  for (; i + 1 < tiles; i += 2) {
-    step(i, std::integral_constant<int, 0>{});
-    step(i + 1, std::integral_constant<int, 1>{});
+  for (; i + DEPTH - 1 < tiles; i += DEPTH) {
+    step(i, integral_constant<int, 0>{}, integral_constant<int, -1>{});
+    step(i + 1, integral_constant<int, 1>{}, integral_constant<int, -1>{});
+    if constexpr (DEPTH == 4) {
+      step(i + 2, integral_constant<int, 2>{}, integral_constant<int, -1>{});
+      step(i + 3, integral_constant<int, 3>{}, integral_constant<int, -1>{});
+    }
   }
-  if (i < tiles) step(i, std::integral_constant<int, 0>{});
+  if (i < tiles) {
+    step(i, integral_constant<int, 0>{}, integral_constant<int, 0>{});
+    if constexpr (DEPTH == 4) {
+      if (i + 1 < tiles) {
+        step(i + 1, integral_constant<int, 1>{}, integral_constant<int, 1>{});
+        if (i + 2 < tiles) step(i + 2, integral_constant<int, 2>{}, integral_constant<int, 2>{});
+      }
+    }
+  }
   __builtin_amdgcn_s_waitcnt(0x0f70);                      // vmcnt(0): nothing is on its way into LDS any more
 
   __syncthreads();
@@ -1827,7 +1812,7 @@ __global__ __launch_bounds__(ROWS_WAVES * 64) __attribute__((amdgpu_waves_per_eu
       for (int r = 0; r < 4; ++r) {
         const int n = (first_blk + st) * 16 + (lane >> 4) * 4 + r;
         if (m >= M || n >= mat.N) continue;
-        gemm_put_pair<Fmt>(a, m, n, mat.N, Fmt::finish(g4[r], sg), Fmt::finish(u4[r], su));
+        gemm_put_pair<Fmt>(a.epi, a.mat[0], m, n, mat.N, Fmt::finish(g4[r], sg), Fmt::finish(u4[r], su));
       }
     }
   } else {
@@ -1850,7 +1835,7 @@ __global__ __launch_bounds__(ROWS_WAVES * 64) __attribute__((amdgpu_waves_per_eu
         const int n = stream_blk(st) * 16 + (lane >> 4) * 4 + r;
         if (m >= M || n >= N) continue;
         if (nsl > 1) { a.part[((size_t)blockIdx.y * M + m) * N + n] = v4[r]; continue; }
-        gemm_put<Fmt>(a, mat, m, n, N, Fmt::finish(v4[r], s1));
+        gemm_put<Fmt>(a.epi, mat, m, n, N, Fmt::finish(v4[r], s1));
       }
     }
   }
@@ -2767,7 +2752,7 @@ static int dispatch_gemv(const GemmArgs& a, int total_nb, hipStream_t s, const c
     const int cus = device_compute_units();
     const int per_cu = (total_nb + cus - 1) / cus;
     const int mt = (a.M + 15) / 16;
-    if (a.epi.norm == PTA_NORM_NONE && a.M > 8) {
+    if (a.epi.norm == PTA_NORM_NONE && a.M > 4) {
       // gemm_own_kernel or gemm_tile_kernel (16 rows: gemv_wide_kernel, gemv_stream_kernel).  Both sides in us, INT4 unless named.
       // One round of gemm_own_kernel's workgroups: it.  64 rows, 4096 x 11008: 14.5 against 21.8, 4096 x 4096 11.1 against 15.2,
       // 2048 x 2048 7.1 against 11.8; 32 rows 11.1 against 14.3, 8.0 against 11.2, 5.6 against 9.4; F143, 64 rows, 4096 x 4096
@@ -2778,13 +2763,17 @@ static int dispatch_gemv(const GemmArgs& a, int total_nb, hipStream_t s, const c
       // rows 29.2 against 39.7; F143 40.8 against 46.9), fp16 ones lose (72.5 against 68.3).  Pairs of up to 32 rows: 22.4 against
       // 21.6.  9 to 16 rows, one round: 9.3 against 11.7 (4096 x 11008, 16 rows), K of 13696 13.5 against 17.8, pair of 2048 x 5632
       // 7.4 against 10.0; fp16 only where every compute unit has one block or none (11008 x 4096 22.5 against 26.4; 4096 x 4608 14.7
-      // against 13.3).
+      // against 13.3).  5 to 8 rows: long K (13696 x 4096, 8 rows, INT4 10.9 against 13.5, F143 14.9 against 17.7, fp16 24.9 against 26.2;
+      // 5632 x 2048, F143 7.7 against 8.3, but 5 rows 6.6 against 6.3 with INT4), INT4 pairs (2048 x 5632, 8.0 against 9.1) and many
+      // channels (4096 x 20480, 13.2 against 15.9); 4096 x 4096 is even or lost (F143 7.5 against 7.1).
       const int wgs4 = total_nb / (PAIR ? 2 : 4);
       const OwnPlan plan = plan_gemm_own<Fmt, PAIR>(a);
       const bool one_round = plan.rounds == 1;
       bool own, tile = false;
       if (a.M <= 16) {
         own = !a.prefer_stream && a.KT >= 16 && one_round && (Fmt::kVec <= 2 || (!PAIR && total_nb <= cus));
+        if (a.M <= 8)
+          own = own && ((a.KT >= 40 && a.M >= 7) || (a.KT >= 64 && Fmt::kVec <= 2) || (Fmt::kVec == 1 && (PAIR || total_nb > 4 * cus)));
       } else {
         tile = tile_fits(a, PAIR ? 2 : 4, 4, PAIR) && 2 * wgs4 >= cus;
         if (tile && PAIR) own = mt > 2 && Fmt::kVec <= 2;
@@ -2832,8 +2821,8 @@ static int dispatch_gemv(const GemmArgs& a, int total_nb, hipStream_t s, const c
         }
       }
       if (streamed) {}
-      else if (a.epi.norm != PTA_NORM_NONE) rc = launch_gemv_wide_for<Fmt, 1, PAIR, true>(a, total_nb, per_cu, s, name);
-      else rc = launch_gemv_wide_for<Fmt, 1, PAIR>(a, total_nb, per_cu, s, name);
+      else if (a.epi.norm != PTA_NORM_NONE) rc = launch_gemv_wide_for<Fmt, PAIR, true>(a, total_nb, per_cu, s, name);
+      else rc = launch_gemv_wide_for<Fmt, PAIR, false>(a, total_nb, per_cu, s, name);
       if (rc) return rc;
     } else if (a.M <= 16) launch_gemv<Fmt, 1, PAIR>(a, total_nb, s);
     else launch_gemv<Fmt, 2, PAIR>(a, total_nb, s);        // (17 to 32 rows of fewer than 8 feature tiles)

@@ -40,7 +40,7 @@ __global__ __launch_bounds__(NORM_THREADS) void norm_kernel(const f16* __restric
   __shared__ float sh[NORM_THREADS / 64];
   const size_t base = (size_t)blockIdx.x * cols;
   const int nvec = cols >> 3;
-  f16x8 v[NORM_MAX_VEC], gv[NORM_MAX_VEC], bv[NORM_MAX_VEC], pv[MIX ? NORM_MAX_VEC : 1];
+  f16x8 v[NORM_MAX_VEC], gv[NORM_MAX_VEC], bv[NORM_MAX_VEC], pv[MIX ? NORM_MAX_VEC : 1], wv[MIX ? NORM_MAX_VEC : 1][3];
   float s = 0.f, sq = 0.f;
   // (the weights are requested with the row: one round trip to memory before the sums instead of one on either side)
 #pragma unroll
@@ -50,7 +50,12 @@ __global__ __launch_bounds__(NORM_THREADS) void norm_kernel(const f16* __restric
       v[i] = *reinterpret_cast<const f16x8*>(x + base + (size_t)c * 8);
       gv[i] = *reinterpret_cast<const f16x8*>(gamma + (size_t)c * 8);
       if (MODE != 0) bv[i] = *reinterpret_cast<const f16x8*>(beta + (size_t)c * 8);
-      if (MIX) pv[i] = *reinterpret_cast<const f16x8*>(mix.prev + base + (size_t)c * 8);
+      if (MIX) {
+        pv[i] = *reinterpret_cast<const f16x8*>(mix.prev + base + (size_t)c * 8);
+#pragma unroll
+        for (int j = 0; j < 3; ++j)
+          if (mix.w[j]) wv[i][j] = *reinterpret_cast<const f16x8*>(mix.w[j] + (size_t)c * 8);
+      }
     }
   }
 #pragma unroll
@@ -110,10 +115,9 @@ __global__ __launch_bounds__(NORM_THREADS) void norm_kernel(const f16* __restric
 #pragma unroll
         for (int j = 0; j < 3; ++j) {
           if (!mix.w[j]) continue;
-          const f16x8 wv = *reinterpret_cast<const f16x8*>(mix.w[j] + (size_t)c * 8);
           f16x8 m;
 #pragma unroll
-          for (int e = 0; e < 8; ++e) m[e] = o[e] * wv[e] + (one - wv[e]) * pv[i][e];
+          for (int e = 0; e < 8; ++e) m[e] = o[e] * wv[i][j][e] + (one - wv[i][j][e]) * pv[i][e];
           *reinterpret_cast<f16x8*>(mix.out[j] + base + (size_t)c * 8) = m;
         }
         *reinterpret_cast<f16x8*>(mix.prev + base + (size_t)c * 8) = o;
