@@ -242,7 +242,8 @@ struct AttnArgs {
   float* part;        // [B*Hq, nsplit, D + 2]: running max, denominator, numerator
   f16* out;           // [B, Hq*D]
   int B, Hq, Hkv, max_len, nsplit;
-  float per_head, per_group;         // 1 / Hq, 1 / (query heads of a KV head): of prompt_attention_mfma_kernel
+  float per_head, per_group;         // 1 / Hq, 1 / (query heads of a KV head), and
+  int head0;                         // the first of the launch's B * Hq heads: of prompt_attention_mfma_kernel
   int rows;           // consecutive positions per sequence (1 in the decode step): row r of a sequence sits at step + r
   int kv_scale;       // FP8 rings (KV8 kernels): rows hold F143 bytes of value * 2^-kv_scale
   int use_scale;
@@ -551,11 +552,12 @@ __global__ __launch_bounds__(PA_THREADS) void prompt_attention_mfma_kernel(AttnA
   __shared__ __align__(16) unsigned char smem[2 * 2 * STAGE];          // [stage][K, V][PA_KEYS][D]
   const float kv_mul = KV8 ? ldexpf(1.0f, a.kv_scale) : 1.0f;
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int head = (int)blockIdx.z * 8 + (int)blockIdx.x;
+  const int head = a.head0 + (int)blockIdx.z * 8 + (int)blockIdx.x;
   if (head >= a.B * a.Hq) return;
   // (quotients of numbers below 2^20 by the reciprocals: an integer division takes 0.3 us of a kernel's start)
-  const int b = __builtin_amdgcn_readfirstlane((int)(((float)head + 0.5f) * a.per_head)), h = head - b * a.Hq;
-  const int kvh = __builtin_amdgcn_readfirstlane((int)(((float)h + 0.5f) * a.per_group));
+  const bool small = head < (1 << 20);
+  const int b = small ? __builtin_amdgcn_readfirstlane((int)(((float)head + 0.5f) * a.per_head)) : head / a.Hq, h = head - b * a.Hq;
+  const int kvh = small ? __builtin_amdgcn_readfirstlane((int)(((float)h + 0.5f) * a.per_group)) : h / (a.Hq / a.Hkv);
   const int row_block = (int)(gridDim.y - 1 - blockIdx.y);
   const int step0 = *a.step;
   const int r0 = row_block * PA_ROWS + wave * (PA_RG * 16);            // first row of this wave within the pass
@@ -1054,10 +1056,14 @@ static int attention_rows(const char* name, const pta_half* q, const void* kv_ri
     int dev = 0, cus = 256;
     if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0) cus = 256;
     const bool two = !(kv8 && D == 128) && (long)((rows + 127) / 128) * Hq * B >= 2L * cus;
-    PTA_REQUIRE((long)B * Hq < (1L << 20), "%s: %d sequences of %d heads", name, B, Hq);
     a.per_head = 1.0f / (float)Hq; a.per_group = (float)Hkv / (float)Hq;
-    const dim3 grid(8, two ? (rows + 127) / 128 : (rows + 63) / 64, (B * Hq + 7) / 8);
-    auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, grid, dim3(PA_THREADS), 0, (hipStream_t)stream, a); };
+    auto go = [&](auto kernel) {
+      for (; a.head0 < B * Hq; a.head0 += 8 * 65535) {                // (as many heads as a grid's z holds)
+        const int eights = (B * Hq - a.head0 + 7) / 8;
+        const dim3 grid(8, two ? (rows + 127) / 128 : (rows + 63) / 64, eights < 65535 ? eights : 65535);
+        hipLaunchKernelGGL(kernel, grid, dim3(PA_THREADS), 0, (hipStream_t)stream, a);
+      }
+    };
     if (D == 128) {
       if (kv8) go(prompt_attention_mfma_kernel<128, 1, true>);           // (two groups: more registers than two waves a SIMD have)
       else { if (two) go(prompt_attention_mfma_kernel<128, 2, false>); else go(prompt_attention_mfma_kernel<128, 1, false>); }
