@@ -488,9 +488,8 @@ static int attn_splits(int B, int Hq, int max_len) {
 
 // ------------------------------------------------------------------------------------------
 // Attention of many rows at once (the prompt passes) on the matrix unit, head size D = 64 or 128, fp16 or F143 cache.
-// One workgroup of four waves per (sequence, query head, 64 or 128 rows of the pass); wave w owns one or two
-// groups of 16 rows.  The cache rows go through LDS 64 at a time, as they lie and without passing through registers (an F143
-// cache: decoded on the way), two stages in turn with one barrier a step; per step a wave computes, for each of its row groups,
+// One workgroup of four waves per (sequence, query head, 64 rows of the pass); wave w owns 16 of them.  The cache rows go through LDS 64 at a time, as they lie and without passing through registers (an F143
+// cache: decoded on the way), two stages in turn with one barrier a step; per step a wave computes
 //   S^T = K Q^T     (four 16 x 16 tiles, D / 32 MFMAs each: lane l then holds the scores of query row l % 16 for
 //                    cache rows (l / 16) * 4 + 0..3 of each tile - two of which ARE the layout of a B operand whose
 //                    k index runs over those eight cache rows),
@@ -498,15 +497,15 @@ static int attn_splits(int B, int Hq, int max_len) {
 //   softmax in fp32 per query row (partners: lanes l ^ 16, l ^ 32), probabilities rounded to fp16 (the
 //   reference's softmax output is fp16),
 //   O^T += V^T P^T  (D / 16 tiles of 16 x 16 over the head size, A operands by transposing LDS reads: four cache rows of a feature a
-//                    lane; a lane's accumulators all belong to its own query row, so the correction is its own number);
-// every K and V operand read from LDS serves all row groups of the wave.  A lane sums the probabilities it holds; the four lanes of
+//                    lane; a lane's accumulators all belong to its own query row, so the correction is its own number).
+// A lane sums the probabilities it holds; the four lanes of
 // a query row add theirs at the end.
 // What bounds it is a workgroup's chain of steps, the longest over all the positions: the last rows' workgroups are launched first, and a
 // step is kept short - 64 rows to a barrier, no transposition by 2-byte stores, no exchange between lanes but that of the maximum.
 // The heads of an XCD are its own (its L2 then holds their K and V): grid x is the head modulo eight.
 // Before (32 rows a step, V transposed by 2-byte stores, two barriers): us for one sequence of 32 heads of 128, 300 rows 17.4 -> 12.1,
-// 1000 59.2 -> 33.9, 2048 169 -> 107, 4000 593 -> 244; 64 rows behind 900 43.1 -> 24.1; F143, 1000 rows 63.9 -> 44.3; 8 x 12 heads of 64,
-// 1000 rows 84.9 -> 59.  17 rows 5.5 -> 6.2: a step of 64 where 32 would do (skipping its second half by a branch cost the long ones
+// 1000 59.2 -> 33.9, 2048 169 -> 87, 4000 593 -> 250; 64 rows behind 900 43.1 -> 24.1; F143, 1000 rows 63.9 -> 44.3; 8 x 12 heads of 64,
+// 1000 rows 84.9 -> 45.  17 rows 5.5 -> 6.2: a step of 64 where 32 would do (skipping its second half by a branch cost the long ones
 // a tenth).
 // Row r of the pass sits at position step + r and attends to cache rows [0, min(step + r + 1, max_len)), as in
 // attn_partial_kernel.  Outputs differ from that kernel in the last bits (another summation order, fp16
@@ -521,6 +520,7 @@ constexpr int PA_VSTRIDE = 32 + 8;       // halves per staged row of V^T
 __device__ __forceinline__ int pa_vt_at(int d, int p) { return d * PA_VSTRIDE + ((((p >> 1) ^ ((d >> 4) << 1))) << 1) + (p & 1); }
 
 constexpr int PA_KEYS = 64;              // cache rows of a step
+constexpr int PA_ROWS = 64;              // rows of the pass of a workgroup: 16 a wave
 
 // 16-byte piece c of staged row p lies at place c ^ pa_key(p): neither the operand reads (a piece of sixteen rows) nor the transposing
 // ones (two pieces of sixteen rows) meet in a bank.
@@ -535,19 +535,17 @@ __device__ __forceinline__ float max_over_quarters(float v) {
   return fmaxf(__uint_as_float(w[0]), __uint_as_float(w[1]));
 }
 
-// PA_RG: row groups of 16 per wave (a workgroup takes 4 * PA_RG * 16 rows of the pass).  Two where that still gives every
-// compute unit two workgroups or more (a wave's dependent chains - MFMA, maximum, exponentials, MFMA - need company
-// on their SIMD), else one.
+// (Two row groups a wave, each operand read serving both, were measured: 2048 rows of 32 heads of 128 103 against 87 us, 8 x 12 heads of
+// 64, 1000 rows 56 against 45, 4000 rows 246 against 250 - a wave's chain of MFMA, maximum, exponentials, MFMA wants company, not length.)
 // KV8: the rings hold F143 bytes of value * 2^-kv_scale (as in attn_partial_kernel): a thread loads eight bytes where
 // LDS receives eight halves of an fp16 ring, decodes them on their way there, and the power of two goes to the fp32
 // scores before they are rounded and to the result.
-template <int D, int PA_RG, bool KV8 = false>
+template <int D, bool KV8>
 __global__ __launch_bounds__(PA_THREADS) void prompt_attention_mfma_kernel(AttnArgs a) {
   static_assert(D == 64 || D == 128, "head size");
   constexpr int VPR = D / 8, ROW = D * 2;                  // 16-byte pieces, and bytes, of a row
   constexpr int STAGE = PA_KEYS * ROW;                     // bytes of a step's K, and of its V
   constexpr int NV = PA_KEYS * VPR / PA_THREADS;           // pieces of K (and of V) per thread and step
-  constexpr int PA_ROWS = 4 * PA_RG * 16;
   typedef short s16x4 __attribute__((ext_vector_type(4)));
   __shared__ __align__(16) unsigned char smem[2 * 2 * STAGE];          // [stage][K, V][PA_KEYS][D]
   const float kv_mul = KV8 ? ldexpf(1.0f, a.kv_scale) : 1.0f;
@@ -560,35 +558,27 @@ __global__ __launch_bounds__(PA_THREADS) void prompt_attention_mfma_kernel(AttnA
   const int kvh = small ? __builtin_amdgcn_readfirstlane((int)(((float)h + 0.5f) * a.per_group)) : h / (a.Hq / a.Hkv);
   const int row_block = (int)(gridDim.y - 1 - blockIdx.y);
   const int step0 = *a.step;
-  const int r0 = row_block * PA_ROWS + wave * (PA_RG * 16);            // first row of this wave within the pass
+  const int r0 = row_block * PA_ROWS + wave * 16;            // first row of this wave within the pass
   auto valid_of = [&](int row) { const int v = step0 + row + 1; return row < a.rows ? (v < a.max_len ? v : a.max_len) : 0; };
-  f16x8 qf[PA_RG][D / 32];
-  int my_valid[PA_RG], all_valid[PA_RG];                   // cache rows that this lane's query row attends to, that every row of the group does
+  const int qrow = r0 + (lane & 15);
+  // cache rows that this lane's query row attends to, that every row of the wave does
+  const int my_valid = valid_of(qrow), all_valid = r0 + 15 < a.rows ? valid_of(r0) : 0;
+  f16x8 qf[D / 32];
 #pragma unroll
-  for (int g = 0; g < PA_RG; ++g) {
-    const int qrow = r0 + g * 16 + (lane & 15);
-    my_valid[g] = valid_of(qrow);
-    all_valid[g] = r0 + g * 16 + 15 < a.rows ? valid_of(r0 + g * 16) : 0;
-#pragma unroll
-    for (int m = 0; m < D / 32; ++m) {
-      qf[g][m] = f16x8{};
-      if (qrow < a.rows) qf[g][m] = *reinterpret_cast<const f16x8*>(a.q + (((size_t)b * a.rows + qrow) * a.Hq + h) * D + m * 32 + (lane >> 4) * 8);
-    }
+  for (int m = 0; m < D / 32; ++m) {
+    qf[m] = f16x8{};
+    if (qrow < a.rows) qf[m] = *reinterpret_cast<const f16x8*>(a.q + (((size_t)b * a.rows + qrow) * a.Hq + h) * D + m * 32 + (lane >> 4) * 8);
   }
-  const int last_of_wave = r0 + PA_RG * 16 - 1 < a.rows ? r0 + PA_RG * 16 - 1 : a.rows - 1;
+  const int last_of_wave = r0 + 15 < a.rows ? r0 + 15 : a.rows - 1;
   const int wave_valid = r0 < a.rows ? valid_of(last_of_wave) : 0;
   const int last_of_wg = row_block * PA_ROWS + PA_ROWS - 1 < a.rows ? row_block * PA_ROWS + PA_ROWS - 1 : a.rows - 1;
   const int wg_valid = valid_of(last_of_wg);
   const size_t ring = ((size_t)b * a.Hkv + kvh) * a.max_len * D;       // elements before this head's rows
 
-  float run_m[PA_RG], run_l[PA_RG];                        // of the lane's query row; the sum of the probabilities this lane holds
-  f32x4 o[PA_RG][D / 16];
+  float run_m = -INFINITY, run_l = 0.f;                    // of the lane's query row; the sum of the probabilities this lane holds
+  f32x4 o[D / 16];
 #pragma unroll
-  for (int g = 0; g < PA_RG; ++g) {
-    run_m[g] = -INFINITY; run_l[g] = 0.f;
-#pragma unroll
-    for (int jd = 0; jd < D / 16; ++jd) o[g][jd] = f32x4{0.f, 0.f, 0.f, 0.f};
-  }
+  for (int jd = 0; jd < D / 16; ++jd) o[jd] = f32x4{0.f, 0.f, 0.f, 0.f};
 
   // cache rows p .. p + 63, requested one step ahead.  fp16: straight into the stage, rows past the last valid one past the
   // descriptor's end: zeros.  KV8: into registers.
@@ -636,56 +626,51 @@ __global__ __launch_bounds__(PA_THREADS) void prompt_attention_mfma_kernel(AttnA
     __syncthreads();                                       // (and every wave is done with the other stage)
     if (p0 + PA_KEYS < wg_valid) request(p0 + PA_KEYS, smem + (turn ^ 1) * (2 * STAGE));
     if (p0 >= wave_valid) continue;
-    f32x4 sc[PA_RG][4];
+    f32x4 sc[4];
 #pragma unroll
     for (int hh = 0; hh < 4; ++hh) {
-#pragma unroll
-      for (int g = 0; g < PA_RG; ++g) sc[g][hh] = f32x4{0.f, 0.f, 0.f, 0.f};
+      sc[hh] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int m = 0; m < D / 32; ++m) {
         const f16x8 kf = *reinterpret_cast<const f16x8*>(stage + hh * 16 * ROW + k_row + (((m * 4 + (lane >> 4)) ^ k_key) * 16));
-#pragma unroll
-        for (int g = 0; g < PA_RG; ++g) sc[g][hh] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kf, qf[g][m], sc[g][hh], 0, 0, 0);
+        sc[hh] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kf, qf[m], sc[hh], 0, 0, 0);
       }
     }
-    f16x8 pa[PA_RG][2];
+    float x[16];
 #pragma unroll
-    for (int g = 0; g < PA_RG; ++g) {
-      float x[16];
-#pragma unroll
-      for (int e = 0; e < 16; ++e) {
-        f16 s16 = (f16)(KV8 ? sc[g][e >> 2][e & 3] * kv_mul : sc[g][e >> 2][e & 3]);      // fp16 output of the q.K^T MatMul
-        if (a.use_scale) s16 = s16 * a.scale;       // fp16 multiply by fp16(1/sqrt(D))
-        x[e] = (float)s16;
-      }
-      if (p0 + PA_KEYS > all_valid[g]) {
-#pragma unroll
-        for (int e = 0; e < 16; ++e)
-          if (p0 + (e >> 2) * 16 + (lane >> 4) * 4 + (e & 3) >= my_valid[g]) x[e] = -INFINITY;
-      }
-      float mx = x[0];
-#pragma unroll
-      for (int e = 1; e < 16; ++e) mx = fmaxf(mx, x[e]);
-      const float new_m = fmaxf(run_m[g], max_over_quarters(mx));
-      const float base = new_m == -INFINITY ? 0.f : new_m; // (nothing valid yet: the exponentials of -inf are zeros)
-      if (__any(new_m > run_m[g])) {
-        const float corr = __expf(run_m[g] - base);
-        run_l[g] *= corr;
-#pragma unroll
-        for (int jd = 0; jd < D / 16; ++jd)
-#pragma unroll
-          for (int r = 0; r < 4; ++r) o[g][jd][r] *= corr;
-        run_m[g] = new_m;
-      }
-      float psum = 0.f;
-#pragma unroll
-      for (int e = 0; e < 16; ++e) {
-        const float pe = __expf(x[e] - base);
-        psum += pe;
-        pa[g][e >> 3][e & 7] = (f16)pe;
-      }
-      run_l[g] += psum;
+    for (int e = 0; e < 16; ++e) {
+      f16 s16 = (f16)(KV8 ? sc[e >> 2][e & 3] * kv_mul : sc[e >> 2][e & 3]);      // fp16 output of the q.K^T MatMul
+      if (a.use_scale) s16 = s16 * a.scale;       // fp16 multiply by fp16(1/sqrt(D))
+      x[e] = (float)s16;
     }
+    if (p0 + PA_KEYS > all_valid) {
+#pragma unroll
+      for (int e = 0; e < 16; ++e)
+        if (p0 + (e >> 2) * 16 + (lane >> 4) * 4 + (e & 3) >= my_valid) x[e] = -INFINITY;
+    }
+    float mx = x[0];
+#pragma unroll
+    for (int e = 1; e < 16; ++e) mx = fmaxf(mx, x[e]);
+    const float new_m = fmaxf(run_m, max_over_quarters(mx));
+    const float base = new_m == -INFINITY ? 0.f : new_m;   // (nothing valid yet: the exponentials of -inf are zeros)
+    if (__any(new_m > run_m)) {
+      const float corr = __expf(run_m - base);
+      run_l *= corr;
+#pragma unroll
+      for (int jd = 0; jd < D / 16; ++jd)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) o[jd][r] *= corr;
+      run_m = new_m;
+    }
+    f16x8 pa[2];
+    float psum = 0.f;
+#pragma unroll
+    for (int e = 0; e < 16; ++e) {
+      const float pe = __expf(x[e] - base);
+      psum += pe;
+      pa[e >> 3][e & 7] = (f16)pe;
+    }
+    run_l += psum;
 #pragma unroll
     for (int jd = 0; jd < D / 16; ++jd) {
 #pragma unroll
@@ -695,30 +680,24 @@ __global__ __launch_bounds__(PA_THREADS) void prompt_attention_mfma_kernel(AttnA
         const f16x4 v0 = bitcast<f16x4>(__builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4*)(from)));
         const f16x4 v1 = bitcast<f16x4>(__builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4*)(from + 16 * ROW)));
         const f16x8 vb = {v0[0], v0[1], v0[2], v0[3], v1[0], v1[1], v1[2], v1[3]};
-#pragma unroll
-        for (int g = 0; g < PA_RG; ++g) o[g][jd] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vb, pa[g][kg], o[g][jd], 0, 0, 0);
+        o[jd] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vb, pa[kg], o[jd], 0, 0, 0);
       }
     }
   }
+  run_l += __shfl_xor(run_l, 16, 64);
+  run_l += __shfl_xor(run_l, 32, 64);
+  if (qrow >= a.rows) return;
   const bool vectors = (reinterpret_cast<uintptr_t>(a.out) & 7) == 0;
+  f16* out = a.out + (((size_t)b * a.rows + qrow) * a.Hq + h) * D + (lane >> 4) * 4;
 #pragma unroll
-  for (int g = 0; g < PA_RG; ++g) {
-    float l = run_l[g];
-    l += __shfl_xor(l, 16, 64);
-    l += __shfl_xor(l, 32, 64);
-    const int row = r0 + g * 16 + (lane & 15);
-    if (row >= a.rows) continue;
-    f16* out = a.out + (((size_t)b * a.rows + row) * a.Hq + h) * D + (lane >> 4) * 4;
+  for (int jd = 0; jd < D / 16; ++jd) {
+    f16x4 y;
 #pragma unroll
-    for (int jd = 0; jd < D / 16; ++jd) {
-      f16x4 y;
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        y[r] = attn_result(a, (f16)((KV8 ? o[g][jd][r] * kv_mul : o[g][jd][r]) / l));
-        if (!vectors) out[jd * 16 + r] = y[r];
-      }
-      if (vectors) *reinterpret_cast<f16x4*>(out + jd * 16) = y;
+    for (int r = 0; r < 4; ++r) {
+      y[r] = attn_result(a, (f16)((KV8 ? o[jd][r] * kv_mul : o[jd][r]) / run_l));
+      if (!vectors) out[jd * 16 + r] = y[r];
     }
+    if (vectors) *reinterpret_cast<f16x4*>(out + jd * 16) = y;
   }
 }
 
@@ -1053,24 +1032,16 @@ static int attention_rows(const char* name, const pta_half* q, const void* kv_ri
   a.kv_scale = kv_scale;
   a.use_scale = use_scale; a.scale = (f16)(1.0 / sqrt((double)D));
   if (rows >= 16) {        // many rows: on the matrix unit, no splits, no workspace
-    int dev = 0, cus = 256;
-    if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0) cus = 256;
-    const bool two = !(kv8 && D == 128) && (long)((rows + 127) / 128) * Hq * B >= 2L * cus;
     a.per_head = 1.0f / (float)Hq; a.per_group = (float)Hkv / (float)Hq;
     auto go = [&](auto kernel) {
       for (; a.head0 < B * Hq; a.head0 += 8 * 65535) {                // (as many heads as a grid's z holds)
         const int eights = (B * Hq - a.head0 + 7) / 8;
-        const dim3 grid(8, two ? (rows + 127) / 128 : (rows + 63) / 64, eights < 65535 ? eights : 65535);
+        const dim3 grid(8, (rows + PA_ROWS - 1) / PA_ROWS, eights < 65535 ? eights : 65535);
         hipLaunchKernelGGL(kernel, grid, dim3(PA_THREADS), 0, (hipStream_t)stream, a);
       }
     };
-    if (D == 128) {
-      if (kv8) go(prompt_attention_mfma_kernel<128, 1, true>);           // (two groups: more registers than two waves a SIMD have)
-      else { if (two) go(prompt_attention_mfma_kernel<128, 2, false>); else go(prompt_attention_mfma_kernel<128, 1, false>); }
-    } else {
-      if (kv8) { if (two) go(prompt_attention_mfma_kernel<64, 2, true>); else go(prompt_attention_mfma_kernel<64, 1, true>); }
-      else { if (two) go(prompt_attention_mfma_kernel<64, 2, false>); else go(prompt_attention_mfma_kernel<64, 1, false>); }
-    }
+    if (D == 128) { if (kv8) go(prompt_attention_mfma_kernel<128, true>); else go(prompt_attention_mfma_kernel<128, false>); }
+    else { if (kv8) go(prompt_attention_mfma_kernel<64, true>); else go(prompt_attention_mfma_kernel<64, false>); }
     PTA_CHECK_LAUNCH(name);
     return PTA_OK;
   }
