@@ -1324,7 +1324,7 @@ __device__ __forceinline__ const unsigned char* uniform_pointer(const unsigned c
 constexpr int OWN_WAVES = 8;
 // weight streams of a workgroup that the registers hold (F152's decoding takes more of them), and channel blocks
 template <class Fmt> struct OwnStreams { static constexpr int cap = Fmt::kVec == 4 ? 3 : 4; };
-template <class Fmt, bool PAIR> constexpr int own_cap(int mt) { return (OwnStreams<Fmt>::cap + (Fmt::kVec == 1 && mt <= 2 ? 1 : 0)) / (PAIR ? 2 : 1); }
+template <class Fmt, bool PAIR> constexpr int own_cap(int mt) { return (OwnStreams<Fmt>::cap + (Fmt::kVec == 1 && mt <= 2 ? 2 : 0)) / (PAIR ? 2 : 1); }
 constexpr int own_ahead(int mt) { return mt <= 1 ? 2 : 1; }
 // tiles of weights in flight or in use: a tile of 16 rows takes less time than its weights' way from memory (13696 x 4096, 8 rows: F143
 // 17.4 -> 14.9 us, INT4 12.3 -> 10.9; at 32 rows no gain)
@@ -2536,6 +2536,7 @@ static int launch_gemm_panel(const GemmArgs& a, int unit0, int unit1, hipStream_
 template <class Fmt, int MT, bool PAIR>
 static int launch_gemm_own_for(const GemmArgs& a, int nb, hipStream_t s, const char* name) {
   constexpr int CAP = own_cap<Fmt, PAIR>(MT);
+  if (CAP >= 6 && nb == 6) return launch_gemm_own<Fmt, MT, CAP >= 6 ? 6 : 1, PAIR>(a, s, name);
   if (CAP >= 5 && nb == 5) return launch_gemm_own<Fmt, MT, CAP >= 5 ? 5 : 1, PAIR>(a, s, name);
   if (CAP >= 4 && nb == 4) return launch_gemm_own<Fmt, MT, CAP >= 4 ? 4 : 1, PAIR>(a, s, name);
   if (CAP >= 3 && nb == 3) return launch_gemm_own<Fmt, MT, CAP >= 3 ? 3 : 1, PAIR>(a, s, name);
@@ -2760,12 +2761,12 @@ static int dispatch_gemv(const GemmArgs& a, int total_nb, hipStream_t s, const c
       // 64 rows 9.6 against 19.5.
       // Several rounds: each begins with nothing on its way.  Weights of one vector a tile lose a little (32000 channels, 64 rows
       // 32.4 against 31.4), those of two win beyond 32 rows (F143 41.8 against 51.6), so does a pair of either (11008 channels, 64
-      // rows 29.2 against 39.7; F143 40.8 against 46.9), fp16 ones lose (72.5 against 68.3).  Pairs of up to 32 rows: 22.4 against
-      // 21.6.  9 to 16 rows, one round: 9.3 against 11.7 (4096 x 11008, 16 rows), K of 13696 13.5 against 17.8, pair of 2048 x 5632
+      // rows 29.2 against 39.7; F143 40.8 against 46.9), fp16 ones lose (72.5 against 68.3).  Pairs of up to 32 rows: INT4, one round and
+      // K of 3072 and more (11008 channels, 32 rows 16.9 against 21.5; 2048 x 5632 9.1 against 8.9).  9 to 16 rows, one round: 9.3 against 11.7 (4096 x 11008, 16 rows), K of 13696 13.5 against 17.8, pair of 2048 x 5632
       // 7.4 against 10.0; fp16 only where every compute unit has one block or none (11008 x 4096 22.5 against 26.4; 4096 x 4608 14.7
       // against 13.3).  5 to 8 rows: long K (13696 x 4096, 8 rows, INT4 10.9 against 13.5, F143 14.9 against 17.7, fp16 24.9 against 26.2;
       // 5632 x 2048, F143 7.7 against 8.3, but 5 rows 6.6 against 6.3 with INT4), INT4 pairs (2048 x 5632, 8.0 against 9.1) and many
-      // channels (4096 x 20480, 13.2 against 15.9); 4096 x 4096 is even or lost (F143 7.5 against 7.1).
+      // channels (4096 x 24576, 15.3 against 18.3); 4096 x 4096 is even or lost (F143 7.5 against 7.1).
       const int wgs4 = total_nb / (PAIR ? 2 : 4);
       const OwnPlan plan = plan_gemm_own<Fmt, PAIR>(a);
       const bool one_round = plan.rounds == 1;
@@ -2773,10 +2774,10 @@ static int dispatch_gemv(const GemmArgs& a, int total_nb, hipStream_t s, const c
       if (a.M <= 16) {
         own = !a.prefer_stream && a.KT >= 16 && one_round && (Fmt::kVec <= 2 || (!PAIR && total_nb <= cus));
         if (a.M <= 8)
-          own = own && ((a.KT >= 40 && a.M >= 7) || (a.KT >= 64 && Fmt::kVec <= 2) || (Fmt::kVec == 1 && (PAIR || total_nb > 4 * cus)));
+          own = own && ((a.KT >= 40 && a.M >= 7) || (a.KT >= 64 && Fmt::kVec <= 2) || (Fmt::kVec == 1 && (PAIR ? a.KT <= 24 : total_nb > 4 * cus)));
       } else {
         tile = tile_fits(a, PAIR ? 2 : 4, 4, PAIR) && 2 * wgs4 >= cus;
-        if (tile && PAIR) own = mt > 2 && Fmt::kVec <= 2;
+        if (tile && PAIR) own = (mt > 2 && Fmt::kVec <= 2) || (Fmt::kVec == 1 && one_round && a.KT >= 24);
         else if (tile) own = one_round || (mt > 2 && Fmt::kVec == 2);
         else own = a.KT >= 8 || mt > 2;
       }

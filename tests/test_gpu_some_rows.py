@@ -7,7 +7,7 @@ pytestmark = pytest.mark.gpu
 
 # rows at the ends of a row group; features one past, short of and on a tile of 128, with 1, 2 and an odd number of tiles for a wave and
 # with waves that have none; channels short of a block, of four and of a workgroup's blocks, and odd ones
-SHAPES = [(5, 8200, 250), (8, 5128, 40), (7, 13696, 72), (9, 2056, 40), (10, 3080, 264), (12, 4104, 24), (16, 5640, 1000), (16, 4096, 4112), (17, 8, 16), (31, 1000, 250), (32, 1160, 264), (33, 136, 1000), (48, 2048, 272), (47, 3080, 11),
+SHAPES = [(5, 8200, 250), (8, 5128, 40), (7, 13696, 72), (9, 2056, 40), (10, 3080, 264), (12, 4104, 24), (16, 5640, 1000), (16, 4096, 4112), (32, 1032, 20488), (17, 8, 16), (31, 1000, 250), (32, 1160, 264), (33, 136, 1000), (48, 2048, 272), (47, 3080, 11),
           (49, 520, 4100), (64, 4096, 2064), (63, 2176, 8200), (64, 24, 20),
           # row blocks of 48 and 64 rows, the last one with one row and full; groups of channels that are no multiple of eight
           (65, 1160, 264), (128, 4096, 4112), (129, 136, 1000), (205, 768, 2304), (256, 2056, 520), (1024, 768, 768)]
@@ -80,7 +80,7 @@ def test_several_matrices_with_inputs_and_biases_of_their_own(kind, M):
 
 
 @pytest.mark.parametrize("kind", ["int4", "f16", "f8"])
-@pytest.mark.parametrize("M, Kd, N", [(6, 2056, 72), (16, 2048, 40), (24, 1032, 44), (48, 128, 100), (64, 2048, 4128), (100, 1032, 44), (129, 264, 520)])
+@pytest.mark.parametrize("M, Kd, N", [(6, 2056, 72), (16, 2048, 40), (24, 1032, 44), (48, 128, 100), (64, 2048, 4128), (12, 3080, 10008), (32, 3072, 11008), (100, 1032, 44), (129, 264, 520)])
 def test_pair(kind, M, Kd, N):
     from poptransformer_amd import kernels as K
     x, w = operands(M, Kd, 2 * N, 7)
