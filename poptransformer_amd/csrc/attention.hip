@@ -580,12 +580,14 @@ __global__ __launch_bounds__(PA_THREADS) void prompt_attention_mfma_kernel(AttnA
 #pragma unroll
   for (int jd = 0; jd < D / 16; ++jd) o[jd] = f32x4{0.f, 0.f, 0.f, 0.f};
 
-  // cache rows p .. p + 63, requested one step ahead.  fp16: straight into the stage, rows past the last valid one past the
-  // descriptor's end: zeros.  KV8: into registers.
-  const __amdgpu_buffer_rsrc_t kr = __builtin_amdgcn_make_buffer_rsrc(const_cast<f16*>(a.kring + (KV8 ? 0 : ring)), 0, KV8 ? 0 : wg_valid * ROW, 0x00020000);
-  const __amdgpu_buffer_rsrc_t vr = __builtin_amdgcn_make_buffer_rsrc(const_cast<f16*>(a.vring + (KV8 ? 0 : ring)), 0, KV8 ? 0 : wg_valid * ROW, 0x00020000);
+  // cache rows p .. p + 63, requested one step ahead.  fp16: straight into the stage, by descriptors of the step's own rows (a head's
+  // rows may take more bytes than 32 bits count); rows past the last valid one lie past their end: zeros.  KV8: into registers.
   u32x2 kq[NV], vq[NV];       // KV8: the bytes as stored
   auto request = [&](int p, unsigned char* stage) {
+    const size_t first = ring + (size_t)p * D;
+    const int bytes = KV8 ? 0 : (wg_valid - p < PA_KEYS ? wg_valid - p : PA_KEYS) * ROW;
+    const __amdgpu_buffer_rsrc_t kr = __builtin_amdgcn_make_buffer_rsrc(const_cast<f16*>(a.kring + (KV8 ? 0 : first)), 0, bytes, 0x00020000);
+    const __amdgpu_buffer_rsrc_t vr = __builtin_amdgcn_make_buffer_rsrc(const_cast<f16*>(a.vring + (KV8 ? 0 : first)), 0, bytes, 0x00020000);
 #pragma unroll
     for (int i = 0; i < NV; ++i) {
       if constexpr (KV8) {
@@ -598,7 +600,7 @@ __global__ __launch_bounds__(PA_THREADS) void prompt_attention_mfma_kernel(AttnA
       } else {
         const int q = i * (PA_THREADS / 64) + wave;        // 64 places of 16 bytes: LDS receives them lane after lane
         const int row = (q * 64 + lane) / VPR, piece = (lane % VPR) ^ pa_key<D>(row);
-        const int from = (p + row) * ROW + piece * 16;
+        const int from = row * ROW + piece * 16;
         __builtin_amdgcn_raw_ptr_buffer_load_lds(kr, (__attribute__((address_space(3))) void*)(stage + q * 1024), 16, from, 0, 0, 0);
         __builtin_amdgcn_raw_ptr_buffer_load_lds(vr, (__attribute__((address_space(3))) void*)(stage + STAGE + q * 1024), 16, from, 0, 0, 0);
       }

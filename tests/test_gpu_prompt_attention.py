@@ -46,3 +46,24 @@ def test_against_float64(B, rows, Hq, Hkv, ring, step, D, kv8, offset):
     got = out.double().transpose(1, 2)
     assert torch.isfinite(got).all()
     assert ((got - ref).abs() <= bound).all(), ((got - ref).abs() / bound).max().item()
+
+
+def test_a_head_whose_cache_rows_take_more_than_4_gib():
+    """The last 16 of 2^25 + 200 positions: four rows of the ring, one of them past the first 4 GiB, share all of the weight (scores of 40
+    against 0: the others' weights, 2^25 * e^-40 of 4, lie below 2^-30), so the result is the mean of their V rows."""
+    from poptransformer_amd import kernels as K
+    D, rows, n = 64, 16, 2 ** 25 + 200
+    assert 2 ** 25 * D * 2 >= 2 ** 32
+    kv = torch.zeros((2, 1, 1, n, D), dtype=torch.float16, device="cuda")
+    at = torch.tensor([5, 2 ** 24 + 3, 2 ** 25 + 7, n - 20], device="cuda")
+    kv[0, 0, 0, at] = 5.0
+    v = torch.randn((4, D), generator=torch.Generator(device="cuda").manual_seed(1), device="cuda").half()
+    kv[1, 0, 0, at] = v
+    q = torch.ones((1, rows, 1, D), dtype=torch.float16, device="cuda")
+    out = torch.full((1, rows, 1, D), float("nan"), dtype=torch.float16, device="cuda")
+    K.prompt_attention(q, kv, torch.tensor(n - rows, dtype=torch.int32, device="cuda"), K.decode_attention_workspace(rows, 1, D, n, "cuda"), out,
+                       1, rows, 1, 1, D, n, True)
+    ref = v.double().mean(0)
+    # weights of exactly 1 (fp16), a sum of 4 in fp32, one rounding of the quotient; the rest of the weights
+    bound = 2.0 ** -11 * ref.abs() + 2.0 ** -24 + 2.0 ** -28 * v.double().abs().amax()
+    assert ((out.double().view(rows, D) - ref).abs() <= bound).all()
