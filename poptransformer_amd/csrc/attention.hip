@@ -243,7 +243,7 @@ struct AttnArgs {
   f16* out;           // [B, Hq*D]
   int B, Hq, Hkv, max_len, nsplit;
   float per_head, per_group;         // 1 / Hq, 1 / (query heads of a KV head), and
-  int head0;                         // the first of the launch's B * Hq heads: of prompt_attention_mfma_kernel
+  int head0, block0;                 // the first of the launch's B * Hq heads and of its blocks of rows: of prompt_attention_mfma_kernel
   int rows;           // consecutive positions per sequence (1 in the decode step): row r of a sequence sits at step + r
   int kv_scale;       // FP8 rings (KV8 kernels): rows hold F143 bytes of value * 2^-kv_scale
   int use_scale;
@@ -556,7 +556,7 @@ __global__ __launch_bounds__(PA_THREADS) void prompt_attention_mfma_kernel(AttnA
   const bool small = head < (1 << 20);
   const int b = small ? __builtin_amdgcn_readfirstlane((int)(((float)head + 0.5f) * a.per_head)) : head / a.Hq, h = head - b * a.Hq;
   const int kvh = small ? __builtin_amdgcn_readfirstlane((int)(((float)h + 0.5f) * a.per_group)) : h / (a.Hq / a.Hkv);
-  const int row_block = (int)(gridDim.y - 1 - blockIdx.y);
+  const int row_block = a.block0 + (int)(gridDim.y - 1 - blockIdx.y);
   const int step0 = *a.step;
   const int r0 = row_block * PA_ROWS + wave * 16;            // first row of this wave within the pass
   auto valid_of = [&](int row) { const int v = step0 + row + 1; return row < a.rows ? (v < a.max_len ? v : a.max_len) : 0; };
@@ -1035,12 +1035,15 @@ static int attention_rows(const char* name, const pta_half* q, const void* kv_ri
   a.use_scale = use_scale; a.scale = (f16)(1.0 / sqrt((double)D));
   if (rows >= 16) {        // many rows: on the matrix unit, no splits, no workspace
     a.per_head = 1.0f / (float)Hq; a.per_group = (float)Hkv / (float)Hq;
+    const int blocks = (rows + PA_ROWS - 1) / PA_ROWS;
     auto go = [&](auto kernel) {
-      for (; a.head0 < B * Hq; a.head0 += 8 * 65535) {                // (as many heads as a grid's z holds)
-        const int eights = (B * Hq - a.head0 + 7) / 8;
-        const dim3 grid(8, (rows + PA_ROWS - 1) / PA_ROWS, eights < 65535 ? eights : 65535);
-        hipLaunchKernelGGL(kernel, grid, dim3(PA_THREADS), 0, (hipStream_t)stream, a);
-      }
+      // (as many blocks of rows, and heads by eights, as a grid's y and z hold)
+      for (a.block0 = (blocks - 1) / 65535 * 65535; a.block0 >= 0; a.block0 -= 65535)
+        for (a.head0 = 0; a.head0 < B * Hq; a.head0 += 8 * 65535) {
+          const int here = blocks - a.block0, eights = (B * Hq - a.head0 + 7) / 8;
+          const dim3 grid(8, here < 65535 ? here : 65535, eights < 65535 ? eights : 65535);
+          hipLaunchKernelGGL(kernel, grid, dim3(PA_THREADS), 0, (hipStream_t)stream, a);
+        }
     };
     if (D == 128) { if (kv8) go(prompt_attention_mfma_kernel<128, true>); else go(prompt_attention_mfma_kernel<128, false>); }
     else { if (kv8) go(prompt_attention_mfma_kernel<64, true>); else go(prompt_attention_mfma_kernel<64, false>); }

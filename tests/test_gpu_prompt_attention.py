@@ -67,3 +67,29 @@ def test_a_head_whose_cache_rows_take_more_than_4_gib():
     # weights of exactly 1 (fp16), a sum of 4 in fp32, one rounding of the quotient; the rest of the weights
     bound = 2.0 ** -11 * ref.abs() + 2.0 ** -24 + 2.0 ** -28 * v.double().abs().amax()
     assert ((out.double().view(rows, D) - ref).abs() <= bound).all()
+
+
+def test_more_heads_than_a_grid_holds():
+    """Three launches (8 * 65535 heads each, the last one of 30), heads past 2^20 (whose quotients are integer divisions), grouped KV heads;
+    the heads on either side of the launches' ends and of 2^20, the first and last ones of a sequence, and every 9973rd."""
+    from poptransformer_amd import kernels as K
+    B, Hq, Hkv, D, rows = 3, 349530, 5, 64, 16
+    heads = B * Hq
+    assert heads == 2 * 8 * 65535 + 30 and heads > 2 ** 20
+    g = torch.Generator(device="cuda").manual_seed(3)
+    q = torch.randn((B, rows, Hq, D), generator=g, device="cuda", dtype=torch.float16)
+    kv = torch.randn((2, B, Hkv, rows, D), generator=g, device="cuda", dtype=torch.float16)
+    out = torch.full((B, rows, Hq, D), float("nan"), dtype=torch.float16, device="cuda")
+    K.prompt_attention(q, kv, torch.tensor(0, dtype=torch.int32, device="cuda"), K.decode_attention_workspace(B * rows, Hq, D, rows, "cuda"), out,
+                       B, rows, Hq, Hkv, D, rows, True)
+    assert torch.isfinite(out).all()
+    ends = [i * 8 * 65535 for i in range(3)] + [2 ** 20, Hq, 2 * Hq, heads]
+    at = torch.tensor(sorted({h for e in ends for h in range(e - 9, e + 9) if 0 <= h < heads} | set(range(0, heads, 9973))), device="cuda")
+    b, h = at // Hq, at % Hq
+    k, v = (t[b, h // (Hq // Hkv)].double() for t in kv)
+    s = (q[b, :, h].float() @ k.transpose(1, 2).contiguous().float()).half() * torch.tensor(1 / math.sqrt(D), dtype=torch.float16, device="cuda")
+    seen = torch.arange(rows, device="cuda")[None, :] <= torch.arange(rows, device="cuda")[:, None]
+    p = torch.softmax(s.double().masked_fill(~seen, -math.inf), dim=-1)
+    # the bound of test_against_float64
+    bound = (2.0 ** -11 * 2 + 4 * 2.0 ** -10 * s.double().abs().amax(-1, keepdim=True) + rows * 2.0 ** -20) * (p @ v.abs()) + rows * 2.0 ** -25 * v.abs().amax() + 2.0 ** -24
+    assert ((out[b, :, h].double() - p @ v).abs() <= bound).all()
