@@ -503,10 +503,12 @@ static int attn_splits(int B, int Hq, int max_len) {
 // What bounds it is a workgroup's chain of steps, the longest over all the positions: the last rows' workgroups are launched first, and a
 // step is kept short - 64 rows to a barrier, no transposition by 2-byte stores, no exchange between lanes but that of the maximum.
 // The heads of an XCD are its own (its L2 then holds their K and V): grid x is the head modulo eight.
-// Before (32 rows a step, V transposed by 2-byte stores, two barriers): us for one sequence of 32 heads of 128, 300 rows 17.4 -> 12.1,
-// 1000 59.2 -> 33.9, 2048 169 -> 87, 4000 593 -> 250; 64 rows behind 900 43.1 -> 24.1; F143, 1000 rows 63.9 -> 44.3; 8 x 12 heads of 64,
-// 1000 rows 84.9 -> 45.  17 rows 5.5 -> 6.2: a step of 64 where 32 would do (skipping its second half by a branch cost the long ones
-// a tenth).
+// Before (32 rows a step, V transposed by 2-byte stores, two barriers) and now: us for one sequence of 32 heads of 128, 17 rows 5.0, 5.5;
+// 64 rows 6.2, 6.1; 300 rows 16.6, 11.1; 1000 54.8, 31.0; 2048 160, 79; 4000 593, 227; 64 rows behind 900 42.5, 23.3; F143, 1000 rows
+// 62.6, 43.6; 8 x 12 heads of 64, 1000 rows 79, 44.
+// A wave whose rows end within a step's first 32 cache rows takes those alone, in code of its own: 17 rows 5.8 -> 5.5 (F143 6.3 -> 5.6),
+// 200 rows 10.0 -> 9.2, 17 rows behind 900 23.5 -> 21.8; 4000 rows 222 -> 227.  It does not touch V rows that none of its rows may see,
+// beyond its own 32: an infinity there times a weight of zero would be a NaN.
 // Row r of the pass sits at position step + r and attends to cache rows [0, min(step + r + 1, max_len)), as in
 // attn_partial_kernel.  Outputs differ from that kernel in the last bits (another summation order, fp16
 // probabilities); both are held to 1e-2 against the oracle.
@@ -583,6 +585,7 @@ __global__ __launch_bounds__(PA_THREADS) void prompt_attention_mfma_kernel(AttnA
   // cache rows p .. p + 63, requested one step ahead.  fp16: straight into the stage, by descriptors of the step's own rows (a head's
   // rows may take more bytes than 32 bits count); rows past the last valid one lie past their end: zeros.  KV8: into registers.
   u32x2 kq[NV], vq[NV];       // KV8: the bytes as stored
+  const bool one_half = wg_valid <= 32;                    // (nothing reads a second half then)
   auto request = [&](int p, unsigned char* stage) {
     const size_t first = ring + (size_t)p * D;
     const int bytes = KV8 ? 0 : (wg_valid - p < PA_KEYS ? wg_valid - p : PA_KEYS) * ROW;
@@ -590,6 +593,7 @@ __global__ __launch_bounds__(PA_THREADS) void prompt_attention_mfma_kernel(AttnA
     const __amdgpu_buffer_rsrc_t vr = __builtin_amdgcn_make_buffer_rsrc(const_cast<f16*>(a.vring + (KV8 ? 0 : first)), 0, bytes, 0x00020000);
 #pragma unroll
     for (int i = 0; i < NV; ++i) {
+      if (i == NV / 2 && (KV8 ? one_half : p + 32 >= wg_valid)) break;
       if constexpr (KV8) {
         const int c = (int)threadIdx.x + i * PA_THREADS, row = c / VPR, col = (c % VPR) * 8;
         kq[i] = u32x2{0, 0}; vq[i] = u32x2{0, 0};          // (the byte 0 is the value 0)
@@ -609,6 +613,7 @@ __global__ __launch_bounds__(PA_THREADS) void prompt_attention_mfma_kernel(AttnA
   auto decode = [&](unsigned char* stage) {
 #pragma unroll
     for (int i = 0; i < NV; ++i) {
+      if (i == NV / 2 && one_half) break;
       const int c = (int)threadIdx.x + i * PA_THREADS, row = c / VPR, at = row * ROW + ((c % VPR) ^ pa_key<D>(row)) * 16;
       *reinterpret_cast<f16x8*>(stage + at) = f143_decode8(kq[i][0], kq[i][1]);
       *reinterpret_cast<f16x8*>(stage + STAGE + at) = f143_decode8(vq[i][0], vq[i][1]);
@@ -619,18 +624,12 @@ __global__ __launch_bounds__(PA_THREADS) void prompt_attention_mfma_kernel(AttnA
   // V operands: sixteen lanes read four rows of sixteen features, four features a lane, and receive one feature of the four rows each
   const int v_at = ((lane >> 4) * 4 + ((lane & 15) >> 2)), v_row = v_at * ROW + (lane & 1) * 8, v_key = pa_key<D>(v_at), v_piece = (lane & 3) >> 1;
 
-  request(0, smem);
-  int turn = 0;
-  for (int p0 = 0; p0 < wg_valid; p0 += PA_KEYS, turn ^= 1) {
-    unsigned char* const stage = smem + turn * (2 * STAGE);
-    if constexpr (KV8) decode(stage);
-    else __builtin_amdgcn_s_waitcnt(0x0f70);               // vmcnt(0): this wave's share of the step's rows has landed
-    __syncthreads();                                       // (and every wave is done with the other stage)
-    if (p0 + PA_KEYS < wg_valid) request(p0 + PA_KEYS, smem + (turn ^ 1) * (2 * STAGE));
-    if (p0 >= wave_valid) continue;
-    f32x4 sc[4];
+  // the first PARTS * 32 cache rows of a step, which begins at row p0
+  auto attend = [&](unsigned char* stage, int p0, auto parts) {
+    constexpr int PARTS = decltype(parts)::value;
+    f32x4 sc[2 * PARTS];
 #pragma unroll
-    for (int hh = 0; hh < 4; ++hh) {
+    for (int hh = 0; hh < 2 * PARTS; ++hh) {
       sc[hh] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int m = 0; m < D / 32; ++m) {
@@ -638,21 +637,21 @@ __global__ __launch_bounds__(PA_THREADS) void prompt_attention_mfma_kernel(AttnA
         sc[hh] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kf, qf[m], sc[hh], 0, 0, 0);
       }
     }
-    float x[16];
+    float x[8 * PARTS];
 #pragma unroll
-    for (int e = 0; e < 16; ++e) {
+    for (int e = 0; e < 8 * PARTS; ++e) {
       f16 s16 = (f16)(KV8 ? sc[e >> 2][e & 3] * kv_mul : sc[e >> 2][e & 3]);      // fp16 output of the q.K^T MatMul
       if (a.use_scale) s16 = s16 * a.scale;       // fp16 multiply by fp16(1/sqrt(D))
       x[e] = (float)s16;
     }
-    if (p0 + PA_KEYS > all_valid) {
+    if (p0 + 32 * PARTS > all_valid) {
 #pragma unroll
-      for (int e = 0; e < 16; ++e)
+      for (int e = 0; e < 8 * PARTS; ++e)
         if (p0 + (e >> 2) * 16 + (lane >> 4) * 4 + (e & 3) >= my_valid) x[e] = -INFINITY;
     }
     float mx = x[0];
 #pragma unroll
-    for (int e = 1; e < 16; ++e) mx = fmaxf(mx, x[e]);
+    for (int e = 1; e < 8 * PARTS; ++e) mx = fmaxf(mx, x[e]);
     const float new_m = fmaxf(run_m, max_over_quarters(mx));
     const float base = new_m == -INFINITY ? 0.f : new_m;   // (nothing valid yet: the exponentials of -inf are zeros)
     if (__any(new_m > run_m)) {
@@ -664,10 +663,10 @@ __global__ __launch_bounds__(PA_THREADS) void prompt_attention_mfma_kernel(AttnA
         for (int r = 0; r < 4; ++r) o[jd][r] *= corr;
       run_m = new_m;
     }
-    f16x8 pa[2];
+    f16x8 pa[PARTS];
     float psum = 0.f;
 #pragma unroll
-    for (int e = 0; e < 16; ++e) {
+    for (int e = 0; e < 8 * PARTS; ++e) {
       const float pe = __expf(x[e] - base);
       psum += pe;
       pa[e >> 3][e & 7] = (f16)pe;
@@ -676,7 +675,7 @@ __global__ __launch_bounds__(PA_THREADS) void prompt_attention_mfma_kernel(AttnA
 #pragma unroll
     for (int jd = 0; jd < D / 16; ++jd) {
 #pragma unroll
-      for (int kg = 0; kg < 2; ++kg) {
+      for (int kg = 0; kg < PARTS; ++kg) {
         // cache rows (lane / 16) * 4 + 0..3 and 16 + the same of these 32, of feature jd * 16 + lane % 16
         unsigned char* const from = stage + STAGE + kg * 32 * ROW + v_row + (((jd * 2 + v_piece) ^ v_key) * 16);
         const f16x4 v0 = bitcast<f16x4>(__builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4*)(from)));
@@ -685,6 +684,18 @@ __global__ __launch_bounds__(PA_THREADS) void prompt_attention_mfma_kernel(AttnA
         o[jd] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vb, pa[kg], o[jd], 0, 0, 0);
       }
     }
+  };
+
+  request(0, smem);
+  int turn = 0;
+  for (int p0 = 0; p0 < wg_valid; p0 += PA_KEYS, turn ^= 1) {
+    unsigned char* const stage = smem + turn * (2 * STAGE);
+    if constexpr (KV8) decode(stage);
+    else __builtin_amdgcn_s_waitcnt(0x0f70);               // vmcnt(0): this wave's share of the step's rows has landed
+    __syncthreads();                                       // (and every wave is done with the other stage)
+    if (p0 + PA_KEYS < wg_valid) request(p0 + PA_KEYS, smem + (turn ^ 1) * (2 * STAGE));
+    if (p0 + 32 < wave_valid) attend(stage, p0, std::integral_constant<int, 2>{});
+    else if (p0 < wave_valid) attend(stage, p0, std::integral_constant<int, 1>{});
   }
   run_l += __shfl_xor(run_l, 16, 64);
   run_l += __shfl_xor(run_l, 32, 64);

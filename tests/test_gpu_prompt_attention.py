@@ -93,3 +93,26 @@ def test_more_heads_than_a_grid_holds():
     # the bound of test_against_float64
     bound = (2.0 ** -11 * 2 + 4 * 2.0 ** -10 * s.double().abs().amax(-1, keepdim=True) + rows * 2.0 ** -20) * (p @ v.abs()) + rows * 2.0 ** -25 * v.abs().amax() + 2.0 ** -24
     assert ((out[b, :, h].double() - p @ v).abs() <= bound).all()
+
+
+@pytest.mark.parametrize("kv8", [False, True])
+@pytest.mark.parametrize("step", [0, 64])
+def test_infinities_ahead_do_not_reach_rows_32_positions_behind(kv8, step):
+    """V holds an infinity (F143: its largest value) at position step + 40: rows whose waves end before the 32 cache rows that hold it are
+    what they are without it."""
+    from poptransformer_amd import kernels as K
+    D, rows, heads, ring = 64, 64, 3, 192
+    g = torch.Generator(device="cuda").manual_seed(5)
+    q = torch.randn((1, rows, heads, D), generator=g, device="cuda").half()
+    kv = torch.randn((2, 1, heads, ring, D), generator=g, device="cuda").half()
+    bad = kv.clone()
+    bad[1, :, :, step + 40] = float("inf")
+    outs = []
+    for t in (kv, bad):
+        t = K.half_to_fp8(t.view(-1, D), torch.tensor([0], dtype=torch.int32, device="cuda"), "F143").view(kv.shape) if kv8 else t
+        out = torch.full((1, rows, heads, D), float("nan"), dtype=torch.float16, device="cuda")
+        K.prompt_attention(q, t, torch.tensor(step, dtype=torch.int32, device="cuda"), K.decode_attention_workspace(rows, heads, D, ring, "cuda"),
+                           out, 1, rows, heads, heads, D, ring, True, kv_scale=0 if kv8 else None)
+        outs.append(out)
+    assert torch.isfinite(outs[1][:, :32]).all()
+    assert torch.equal(outs[0][:, :32], outs[1][:, :32])
