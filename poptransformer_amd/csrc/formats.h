@@ -153,12 +153,10 @@ struct FmtF8 : F16Product {
 
 // F143 weights for gemm_block_kernel.  Moved to fp16 bits 13..7 with their sign in bit 15 the seven magnitude bits are the
 // fp16 number decode(byte) * 2^-7, subnormals among them, which the matrix unit takes at their value: three instructions for two
-// weights (the 2^7 joins the exponent of the sum) where f143_pair, whose result is the number itself, has five.
+// weights where f143_pair, whose result is the number itself, has five.  The sum takes the 2^7 before the scale: one exponent for both
+// would be infinite from 2^121 on, and its product with a sum of zero a NaN.
 struct FmtF143Block : FmtF8<0> {
-  static __device__ __forceinline__ Scale load_scale(const void* scale, const int32_t* x_scale, int, int) {
-    const int e = reinterpret_cast<const int32_t*>(scale)[0] + (x_scale ? x_scale[0] : 0);
-    return Scale{ldexpf(1.0f, e + 7)};
-  }
+  static __device__ __forceinline__ float finish(float acc, Scale s) { return acc * 128.0f * s.mul; }
   static constexpr int kStage = 64;                          // (a vector holds 64 features of a channel)
   typedef u32x2 Piece;
   static constexpr int piece_at(int m) { return m * 8; }

@@ -1,4 +1,5 @@
 """Products of more than 128 rows by 16-bit and FP8 weights (gemm_block_kernel) at the edges of its tiles, against float64."""
+import math
 import numpy as np
 import pytest
 import torch
@@ -146,3 +147,27 @@ def test_rows_past_the_last_and_features_past_the_end_are_not_read():
     out = torch.empty((M, N), dtype=torch.float16, device="cuda")
     K.linear(store[:M], [K.F16Weight(w.half())], [out])
     close(out, x.half().double() @ w.half().double().T, x.half().double().abs() @ w.half().double().abs().T, Kd, 11)
+
+
+@pytest.mark.parametrize("slices", [False, True])
+@pytest.mark.parametrize("exponent", [-140, -30, 120, 121, 127])
+def test_fp8_exponents_at_the_ends_of_their_range(exponent, slices):
+    """Sums of zero are zeros at every exponent whose power of two is finite; the others overflow fp16, or vanish."""
+    from poptransformer_amd import kernels as K
+    M, Kd, N = 1000, 1032, 2056
+    x, w = operands(M, Kd, N, 19)
+    x = x.half()
+    x[3] = 0
+    codes = K.half_to_fp8(w.half(), torch.tensor([-3], dtype=torch.int32, device="cuda"))
+    codes[5] = 0
+    plain = K.fp8_to_half(codes, torch.tensor([0], dtype=torch.int32, device="cuda")).double()
+    out = torch.full((M, N), float("nan"), dtype=torch.float16, device="cuda")
+    K.linear(x, [K.F8Weight(codes, torch.tensor([exponent], dtype=torch.int32, device="cuda"))], [out],
+             workspace=K.linear_workspace(M, N, "cuda") if slices else None)
+    s, mag = x.double() @ plain.T, x.double().abs() @ plain.abs().T
+    assert (out[3] == 0).all() and (out[:, 5] == 0).all()
+    sure = s.abs() > (Kd + 2) * 2.0 ** -24 * mag * 2          # the others' signs and sizes are the rounding's
+    if exponent > 0:
+        assert torch.equal(out[sure], (s[sure].sign() * math.inf).half())
+    else:
+        close(out, s * 2.0 ** exponent, mag * 2.0 ** exponent, Kd, 11)
