@@ -326,6 +326,9 @@ __device__ __forceinline__ void gemm_put_pair(const GemmEpilogue& epi, const Gem
 static inline int device_compute_units();
 constexpr int GEMM_MAX_KSPLIT = 4;
 constexpr int GEMM_MAX_ROWS = 4096;
+// From so many features on the rows of a workgroup (up to 256, and 48 rows past the last one) take more bytes than the 32-bit offsets of
+// the kernels for more than 16 rows, and of gemm_own_kernel, reach.
+constexpr int GEMM_FAR = 1 << 22;
 
 template <class Fmt, int MT, int NW, bool PAIR>
 __global__ __launch_bounds__(NW * 64) void gemv_mfma_kernel(GemmArgs a) {
@@ -2633,6 +2636,27 @@ static void launch_gemv(const GemmArgs& a, int total_nb, hipStream_t s) {
 template <class Fmt, bool PAIR>
 static int dispatch_gemv(const GemmArgs& a, int total_nb, hipStream_t s, const char* name);
 
+// `chunk` rows at a time through the paths for so many
+template <class Fmt, bool PAIR>
+static int rows_in_turn(const GemmArgs& a, int chunk, int total_nb, hipStream_t s, const char* name) {
+  for (int m0 = 0; m0 < a.M; m0 += chunk) {
+    GemmArgs b = a;
+    b.M = a.M - m0 < chunk ? a.M - m0 : chunk;
+    if (b.X) b.X += (size_t)m0 * a.K;
+    for (int i = 0; i < a.count; ++i) {
+      if (b.mat[i].X) b.mat[i].X += (size_t)m0 * a.K;
+      if constexpr (Fmt::kWide) wide_skip_rows(b.mat[i], m0);
+      else if (!PAIR || i == 0) b.mat[i].Y += (size_t)m0 * a.mat[i].N;
+    }
+    if (PAIR) b.mat[1].Y = b.mat[0].Y;
+    if (b.epi.residual) b.epi.residual += (size_t)m0 * a.mat[0].N;
+    if (b.epi.mul) b.epi.mul += (size_t)m0 * a.mat[0].N;
+    const int rc = dispatch_gemv<Fmt, PAIR>(b, total_nb, s, name);
+    if (rc) return rc;
+  }
+  return PTA_OK;
+}
+
 template <class Fmt> struct BlockFormat { static constexpr bool ok = false; };
 
 // More than 64 rows.  Beyond 128 rows gemm_block_kernel or (INT4) gemm_panel_kernel, up to 128 gemm_rows_kernel, where
@@ -2714,27 +2738,12 @@ static int dispatch_many_rows(const GemmArgs& a, int total_nb, hipStream_t s, co
     PTA_CHECK_LAUNCH(name);
     return PTA_OK;
   }
-  const int chunk = 64;
-  for (int m0 = 0; m0 < a.M; m0 += chunk) {
-    GemmArgs b = a;
-    b.M = a.M - m0 < chunk ? a.M - m0 : chunk;
-    if (b.X) b.X += (size_t)m0 * a.K;
-    for (int i = 0; i < a.count; ++i) {
-      if (b.mat[i].X) b.mat[i].X += (size_t)m0 * a.K;
-      if constexpr (Fmt::kWide) wide_skip_rows(b.mat[i], m0);
-      else if (!PAIR || i == 0) b.mat[i].Y += (size_t)m0 * a.mat[i].N;
-    }
-    if (PAIR) b.mat[1].Y = b.mat[0].Y;
-    if (b.epi.residual) b.epi.residual += (size_t)m0 * a.mat[0].N;
-    if (b.epi.mul) b.epi.mul += (size_t)m0 * a.mat[0].N;
-    const int rc = dispatch_gemv<Fmt, PAIR>(b, total_nb, s, name);
-    if (rc) return rc;
-  }
-  return PTA_OK;
+  return rows_in_turn<Fmt, PAIR>(a, 64, total_nb, s, name);
 }
 
 template <class Fmt, bool PAIR>
 static int dispatch_gemv(const GemmArgs& a, int total_nb, hipStream_t s, const char* name) {
+  if (a.M > 16 && a.K >= GEMM_FAR && a.epi.norm == PTA_NORM_NONE) return rows_in_turn<Fmt, PAIR>(a, 16, total_nb, s, name);
   if (a.M > 64) return dispatch_many_rows<Fmt, PAIR>(a, total_nb, s, name);
   const size_t xbytes = (size_t)a.M * (a.KT * 128 + 8) * 2;
   bool all_shared_x = true;
@@ -2772,7 +2781,7 @@ static int dispatch_gemv(const GemmArgs& a, int total_nb, hipStream_t s, const c
       const bool one_round = plan.rounds == 1;
       bool own, tile = false;
       if (a.M <= 16) {
-        own = !a.prefer_stream && a.KT >= 16 && one_round && (Fmt::kVec <= 2 || (!PAIR && total_nb <= cus));
+        own = !a.prefer_stream && a.KT >= 16 && a.K < GEMM_FAR && one_round && (Fmt::kVec <= 2 || (!PAIR && total_nb <= cus));
         if (a.M <= 8)
           own = own && ((a.KT >= 40 && a.M >= 7) || (a.KT >= 64 && Fmt::kVec <= 2) || (Fmt::kVec == 1 && (PAIR ? a.KT <= 24 : total_nb > 4 * cus)));
       } else {

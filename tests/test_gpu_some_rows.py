@@ -126,3 +126,28 @@ def test_rows_past_the_last_and_features_past_the_end_are_not_read(kind):
     out = torch.empty((M, N), dtype=torch.float16, device="cuda")
     K.linear(store[:M], [tw], [out])
     close(out, x.half().double() @ plain.T, x.half().double().abs() @ plain.abs().T, Kd, 11)
+
+
+@pytest.mark.parametrize("kind, M, Kd, N", [("int4", 40, 2 ** 22 + 8, 40), ("f16", 130, 2 ** 22 + 8, 24), ("f16", 12, 2 ** 22, 24), ("int4", 64, 2 ** 25 + 8, 24)])
+def test_rows_further_apart_than_32_bits_count(kind, M, Kd, N):
+    """Rows of X of 8 and 64 MiB each (64 of the latter take 4 GiB): 65 features a row are +-1, so that the sums are whole numbers."""
+    from poptransformer_amd import kernels as K
+    g = torch.Generator(device="cuda").manual_seed(Kd)
+    at = torch.cat([torch.randint(0, Kd - 1, (M, 64), generator=g, device="cuda"), torch.full((M, 1), Kd - 1, device="cuda")], dim=1)
+    x = torch.zeros((M, Kd), dtype=torch.float16, device="cuda")
+    x.scatter_(1, at, (torch.randint(0, 2, (M, 65), generator=g, device="cuda") * 2 - 1).half())
+    if kind == "int4":
+        packed = torch.randint(-128, 128, (N, Kd // 2), generator=g, device="cuda", dtype=torch.int8)
+        tw, plain = K.W4Weight(packed, torch.ones(N, dtype=torch.float16, device="cuda")), K.int4_to_half(packed, torch.ones(N, dtype=torch.float16, device="cuda"))
+    else:
+        w = torch.randint(-8, 9, (N, Kd), generator=g, device="cuda", dtype=torch.int8).half()
+        tw, plain = K.F16Weight(w), w.T
+    out = torch.full((M, N), float("nan"), dtype=torch.float16, device="cuda")
+    K.linear(x, [tw], [out])
+    ref = (x.gather(1, at).float().unsqueeze(2) * plain[at.flatten()].view(M, 65, N).float())
+    # (a feature drawn twice is in x once)
+    once = torch.ones_like(at, dtype=torch.float32)
+    sorted_at, order = at.sort(dim=1, stable=True)
+    again = torch.cat([torch.zeros((M, 1), dtype=torch.bool, device="cuda"), sorted_at[:, 1:] == sorted_at[:, :-1]], dim=1)
+    once.scatter_(1, order, (~again).float())
+    assert torch.equal(out.float(), (ref * once.unsqueeze(2)).sum(1))
