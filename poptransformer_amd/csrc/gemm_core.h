@@ -1334,19 +1334,20 @@ constexpr int own_ahead(int mt) { return mt <= 1 ? 2 : 1; }
 constexpr int own_depth(int mt, int vectors) { return mt == 1 && vectors <= 4 ? 4 : 2; }
 
 template <class Fmt, int MT, int NB, bool PAIR>
-__global__ __launch_bounds__(OWN_WAVES * 64) __attribute__((amdgpu_waves_per_eu(2, 2))) void gemm_own_kernel(GemmArgs a, int groups) {
+__global__ __launch_bounds__(OWN_WAVES * 64) __attribute__((amdgpu_waves_per_eu(2, 2))) void gemm_own_kernel(GemmArgs a, int group0, int groups) {
   constexpr int NACC = PAIR ? 2 : 1, NS = NB * NACC;       // weight streams
   constexpr int KV = Fmt::kVec;
   extern __shared__ __align__(16) unsigned char smem[];
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int K = a.K;
-  // Grid: 8 groups of channels, the row blocks, the slices' groups by eights.  A group's row blocks are multiples of eight apart: on one
+  // Grid: 8 groups of channels (of the launch's, from group0 on), the row blocks, the slices' groups by eights.  A group's row blocks are multiples of eight apart: on one
   // XCD, whose L2 has its weights for all.  (One flat index, divided here, cost 1.5 us a launch.)
   const int row_block = blockIdx.y, eights = (groups + 7) / 8;
   int slice = 0, group = blockIdx.z;
   while (group >= eights) group -= eights, ++slice;
   group = group * 8 + blockIdx.x;
   if (group >= groups) return;
+  group += group0;
   const int row0 = row_block * (MT * 16), M = a.M - row0 < MT * 16 ? a.M - row0 : MT * 16;
   int mi = 0;
   if (!PAIR) {
@@ -1612,7 +1613,11 @@ static int launch_gemm_own(const GemmArgs& a, hipStream_t s, const char* name) {
   }
   const int nsl = a.ksplit > 1 ? a.ksplit : 1;
   const int groups = own_groups(a, NB, PAIR), row_blocks = (a.M + MT * 16 - 1) / (MT * 16);
-  hipLaunchKernelGGL((gemm_own_kernel<Fmt, MT, NB, PAIR>), dim3(8, row_blocks, (groups + 7) / 8 * nsl), dim3(OWN_WAVES * 64), smem, s, a, groups);
+  const int most = 65535 / nsl * 8;                // (as many groups as a grid's z holds)
+  for (int g = 0; g < groups; g += most) {
+    const int here = groups - g < most ? groups - g : most;
+    hipLaunchKernelGGL((gemm_own_kernel<Fmt, MT, NB, PAIR>), dim3(8, row_blocks, (here + 7) / 8 * nsl), dim3(OWN_WAVES * 64), smem, s, a, g, here);
+  }
   if (nsl > 1) launch_splitk_finish<Fmt>(a, s);
   return PTA_OK;
 }

@@ -151,3 +151,18 @@ def test_rows_further_apart_than_32_bits_count(kind, M, Kd, N):
     again = torch.cat([torch.zeros((M, 1), dtype=torch.bool, device="cuda"), sorted_at[:, 1:] == sorted_at[:, :-1]], dim=1)
     once.scatter_(1, order, (~again).float())
     assert torch.equal(out.float(), (ref * once.unsqueeze(2)).sum(1))
+
+
+def test_more_channels_than_a_grid_holds():
+    """Two launches: 8 * 65535 groups of three blocks of 16 channels, and the rest; channels at both ends of each, and every 100003rd."""
+    from poptransformer_amd import kernels as K
+    M, Kd, per = 33, 8, 8 * 65535 * 48
+    N = per + 1000
+    g = torch.Generator(device="cuda").manual_seed(7)
+    x = torch.randn((M, Kd), generator=g, device="cuda").half()
+    w = torch.randn((N, Kd), generator=g, device="cuda", dtype=torch.float16)
+    out = torch.full((M, N), float("nan"), dtype=torch.float16, device="cuda")
+    K.linear(x, [K.F16Weight(w)], [out])
+    assert torch.isfinite(out).all()
+    at = torch.tensor(sorted({n for e in (0, per, N) for n in range(e - 100, e + 100) if 0 <= n < N} | set(range(0, N, 100003))), device="cuda")
+    close(out[:, at], x.double() @ w[at].double().T, x.double().abs() @ w[at].double().abs().T, Kd, 11)
