@@ -109,6 +109,8 @@ typedef struct pta_fusion {
 } pta_fusion;
 
 size_t pta_linear_workspace_bytes(int M, int N);
+/* the name of the kernel that the calling thread's last product took, "" before the first (a product of several launches: the last one's) */
+const char* pta_linear_kernel(void);
 
 enum { PTA_NORM_NONE = 0, PTA_NORM_RMS = 1, PTA_NORM_LAYER = 2 };
 enum { PTA_ACT_NONE = 0, PTA_ACT_GELU_TANH = 1, PTA_ACT_RELU_SQUARE = 2, PTA_ACT_SIGMOID = 3 };

@@ -324,6 +324,9 @@ __device__ __forceinline__ void gemm_put_pair(const GemmEpilogue& epi, const Gem
 }
 
 static inline int device_compute_units();
+// The kernel that the calling thread's last product took (its last launch's, where it was several; without the finish of a K split): for
+// tests that are meant for one of them.
+inline thread_local const char* gemm_kernel_taken = "";
 constexpr int GEMM_MAX_KSPLIT = 4;
 constexpr int GEMM_MAX_ROWS = 4096;
 // From so many features on the rows of a workgroup (up to 256, and 48 rows past the last one) take more bytes than the 32-bit offsets of
@@ -836,6 +839,7 @@ static int launch_gemv_wide(const GemmArgs& a, int total_nb, hipStream_t s, cons
                 "%s: cannot reserve %zu bytes of LDS", name, smem);
     ready = true;
   }
+  gemm_kernel_taken = "gemv_wide_kernel";
   hipLaunchKernelGGL((gemv_wide_kernel<Fmt, NB, PAIR, NORM>), dim3((total_nb + NB - 1) / NB), dim3(WIDE_WAVES * 64), smem, s,
                      a, total_nb);
   return PTA_OK;
@@ -1072,6 +1076,7 @@ static int launch_gemv_stream(const GemmArgs& a, int total_nb, int cus, hipStrea
   // tiles per step, and four steps in the ring: 96 KiB on their way per compute unit, a ring of 64 registers
   constexpr int V = Fmt::kVec * (PAIR ? 2 : 1);
   constexpr int U = V >= 4 ? 1 : V >= 2 ? 2 : 4, D = 4;
+  gemm_kernel_taken = "gemv_stream_kernel";
   hipLaunchKernelGGL((gemv_stream_kernel<Fmt, U, D, PAIR>), dim3(total_nb < cus ? total_nb : cus), dim3(STREAM_WAVES * 64), 0, s, a,
                      total_nb);
   return PTA_OK;
@@ -1298,6 +1303,7 @@ static int launch_gemm_tile(const GemmArgs& a, int total_nb, hipStream_t s, cons
     ready = true;
   }
   const int per_wg = PAIR ? WPG : 2 * WPG;
+  gemm_kernel_taken = "gemm_tile_kernel";
   hipLaunchKernelGGL((gemm_tile_kernel<Fmt, MT, KQ, PAIR, NWV>), dim3(total_nb / per_wg), dim3(NWV * 64), smem, s, a);
   return PTA_OK;
 }
@@ -1613,6 +1619,7 @@ static int launch_gemm_own(const GemmArgs& a, hipStream_t s, const char* name) {
   }
   const int nsl = a.ksplit > 1 ? a.ksplit : 1;
   const int groups = own_groups(a, NB, PAIR), row_blocks = (a.M + MT * 16 - 1) / (MT * 16);
+  gemm_kernel_taken = "gemm_own_kernel";
   const int most = 65535 / nsl * 8;                // (as many groups as a grid's z holds)
   for (int g = 0; g < groups; g += most) {
     const int here = groups - g < most ? groups - g : most;
@@ -1871,6 +1878,7 @@ static int launch_gemm_listed(const GemmArgs& a, int total_nb, int max_tiles, co
   if (rc) return rc;
   constexpr int per_wg = PAIR ? ROWS_CB / 2 : ROWS_CB;
   const int groups = (total_nb + per_wg - 1) / per_wg;
+  gemm_kernel_taken = "gemm_rows_kernel";
   hipLaunchKernelGGL((gemm_rows_kernel<Fmt, RG, PAIR, ListedRows>), dim3((groups * max_tiles + 7) / 8 * 8), dim3(ROWS_WAVES * 64), smem, s, a,
                      groups, max_tiles, rows);
   return PTA_OK;
@@ -1885,6 +1893,7 @@ static int launch_gemm_rows(const GemmArgs& a, int total_nb, hipStream_t s, cons
   const int row_blocks = (a.M + ROWS_WAVES * RG * 16 - 1) / (ROWS_WAVES * RG * 16);
   const int nsl = a.ksplit > 1 ? a.ksplit : 1;
   const int per = (groups * row_blocks + 7) / 8;
+  gemm_kernel_taken = "gemm_rows_kernel";
   hipLaunchKernelGGL((gemm_rows_kernel<Fmt, RG, PAIR>), dim3(per * 8, nsl), dim3(ROWS_WAVES * 64), smem, s, a, groups, row_blocks, AllRows{});
   if (nsl > 1) launch_splitk_finish<Fmt>(a, s);
   return PTA_OK;
@@ -2446,6 +2455,7 @@ static int launch_gemm_block(const GemmArgs& a, int group0, int group1, hipStrea
   const int groups = group1 - group0, row_blocks = (a.M + RG * 32 - 1) / (RG * 32);
   const int nsl = a.ksplit > 1 ? a.ksplit : 1;
   const int per = (groups * row_blocks + 7) / 8;
+  gemm_kernel_taken = "gemm_block_kernel";
   hipLaunchKernelGGL((gemm_block_kernel<Fmt, RG, PAIR>), dim3(per * 8, nsl), dim3(BLOCK_WAVES * 64), block_stages<Fmt>(RG) * block_stage_bytes<Fmt>(RG), s, a,
                      group0, groups, row_blocks, AllRows{});
   if (nsl > 1) launch_splitk_finish<Fmt>(a, s);
@@ -2460,6 +2470,7 @@ static int launch_gemm_block_listed(const GemmArgs& a, size_t x_rows, int max_ti
   const int rc = reserve_gemm_block<Fmt, RG, PAIR, ListedRows>(name);
   if (rc) return rc;
   const int groups = block_groups(a, PAIR);
+  gemm_kernel_taken = "gemm_block_kernel";
   hipLaunchKernelGGL((gemm_block_kernel<Fmt, RG, PAIR, ListedRows>), dim3((groups * max_tiles + 7) / 8 * 8), dim3(BLOCK_WAVES * 64),
                      block_stages<Fmt>(RG) * block_stage_bytes<Fmt>(RG), s, a, 0, groups, max_tiles, rows);
   return PTA_OK;
@@ -2536,6 +2547,7 @@ static int launch_gemm_panel(const GemmArgs& a, int unit0, int unit1, hipStream_
   const int row_blocks = (a.M + RG * 16 - 1) / (RG * 16);
   const int nsl = a.ksplit > 1 ? a.ksplit : 1;
   const int per = (groups * row_blocks + 7) / 8;
+  gemm_kernel_taken = "gemm_panel_kernel";
   hipLaunchKernelGGL((gemm_panel_kernel<Fmt, NST, RG, KH, PAIR>), dim3(per * 8, nsl), dim3(PANEL_WAVES * 64), smem, s, a, groups, row_blocks, unit0, unit1);
   if (nsl > 1) launch_splitk_finish<Fmt>(a, s);
   return PTA_OK;
@@ -2621,6 +2633,7 @@ template <class Fmt, int NW, bool PAIR>
 static void launch_gemv_lds(const GemmArgs& a, int total_nb, hipStream_t s) {
   const size_t xbytes = (((size_t)a.M * (a.KT * 128 + 8) * 2) + 15) & ~(size_t)15;
   const size_t smem = xbytes + (size_t)NW * (PAIR ? 2 : 1) * 256 * sizeof(float);
+  gemm_kernel_taken = "gemv_lds_kernel";
   hipLaunchKernelGGL((gemv_lds_kernel<Fmt, NW, PAIR>), dim3(total_nb), dim3(NW * 64), smem, s, a);
 }
 
@@ -2628,6 +2641,7 @@ template <class Fmt, int MT, bool PAIR>
 static void launch_gemv(const GemmArgs& a, int total_nb, hipStream_t s) {
   // Waves per block: enough to split K finely when there are few channel blocks, fewer when
   // the grid alone already fills the machine.  The LDS reduction buffer caps the wide cases.
+  gemm_kernel_taken = "gemv_mfma_kernel";
   if constexpr (PAIR) {
     hipLaunchKernelGGL((gemv_mfma_kernel<Fmt, MT, 8, PAIR>), dim3(total_nb), dim3(8 * 64), 0, s, a);
   } else {

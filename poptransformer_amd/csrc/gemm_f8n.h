@@ -242,6 +242,7 @@ static int launch_gemv_f8n(const GemmArgs& a, int total_nb, hipStream_t s, const
                 "%s: cannot reserve %zu bytes of LDS", name, smem);
     ready = true;
   }
+  gemm_kernel_taken = "gemv_f8n_kernel";
   hipLaunchKernelGGL((gemv_f8n_kernel<NB, PAIR, XBYTES>), dim3((total_nb + NB - 1) / NB), dim3(WIDE_WAVES * 64), smem, s, a,
                      total_nb);
   return PTA_OK;
@@ -605,6 +606,7 @@ static int launch_gemm_f8n_panel(const GemmArgs& a, int unit0, int unit1, hipStr
   const int row_blocks = (a.M + RG * 16 - 1) / (RG * 16);
   const int nsl = a.ksplit > 1 ? a.ksplit : 1;
   const int per = (groups * row_blocks + 7) / 8;
+  gemm_kernel_taken = "gemm_f8n_panel_kernel";
   hipLaunchKernelGGL((gemm_f8n_panel_kernel<NST, RG, KH, PAIR>), dim3(per * 8, nsl), dim3(PANEL_WAVES * 64), smem, s, a, groups, row_blocks, unit0, unit1);
   if (nsl > 1) launch_splitk_finish<FmtF8<0>>(a, s);
   return PTA_OK;

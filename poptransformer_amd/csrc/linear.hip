@@ -128,6 +128,8 @@ extern "C" int pta_linear(const pta_half* X, const int32_t* x_scale, int count, 
   return linear_impl(X, x_scale, 0, count, host_w, host_bias, host_Y, M, swiglu, fuse, stream);
 }
 
+extern "C" const char* pta_linear_kernel(void) { return gemm_kernel_taken; }
+
 extern "C" size_t pta_linear_workspace_bytes(int M, int N) {
   if (M <= 0 || N <= 0) return 0;
   return (size_t)GEMM_MAX_KSPLIT * M * N * sizeof(float);

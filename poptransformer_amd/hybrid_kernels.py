@@ -67,6 +67,11 @@ def linear_workspace(rows, channels, device):
     return torch.empty(H.load().pta_wide_linear_workspace_bytes(rows, channels), dtype=torch.uint8, device=device)
 
 
+def linear_kernel():
+    """The name of the kernel that this thread's last bf16 product took."""
+    return H.load().pta_wide_linear_kernel().decode()
+
+
 def _linear_args(x, w, out, rows, ld=None, tail=None, cap=0.0, up=None, pair=H.PAIR_NONE, limit=0.0, slope=0.0, workspace=None, bias=None,
                  bias2=None, act=H.ACT_NONE, mul=None, accumulate=False):
     _need(x, w.dtype, "x", rows * w.K)

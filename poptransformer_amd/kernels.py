@@ -74,6 +74,11 @@ def linear_workspace(M, N, device):
     return torch.empty(_lib.load().pta_linear_workspace_bytes(M, N), dtype=torch.uint8, device=device)
 
 
+def linear_kernel():
+    """The name of the kernel that this thread's last product took."""
+    return _lib.load().pta_linear_kernel().decode()
+
+
 # ------------------------------------------------------------------ INT4 -----------------
 def int4_to_half(packed, scale, axis=1):
     """ops.int4_to_half (reference: poptransformer/ops/customized.py:115-125)."""
