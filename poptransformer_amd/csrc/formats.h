@@ -191,7 +191,7 @@ struct FmtBF16 {
 };
 
 // the formats of gemm_block_kernel
-template <> struct OwnStreams<FmtF8<1>> { static constexpr int cap = 3; };
+template <> struct OwnStreams<FmtF8<1>> { static constexpr int cap = 3; static constexpr bool long_decode = true; };
 template <> struct BlockFormat<FmtF16> { static constexpr bool ok = true; typedef FmtF16 type; };
 template <> struct BlockFormat<FmtBF16> { static constexpr bool ok = true; typedef FmtBF16 type; };
 template <> struct BlockFormat<FmtF8<0>> { static constexpr bool ok = true; typedef FmtF143Block type; };

@@ -1332,7 +1332,7 @@ __device__ __forceinline__ const unsigned char* uniform_pointer(const unsigned c
 // ------------------------------------------------------------------------------------------
 constexpr int OWN_WAVES = 8;
 // weight streams of a workgroup that the registers hold (F152's decoding takes more of them), and channel blocks
-template <class Fmt> struct OwnStreams { static constexpr int cap = Fmt::kVec == 4 ? 3 : 4; };
+template <class Fmt> struct OwnStreams { static constexpr int cap = Fmt::kVec == 4 ? 3 : 4; static constexpr bool long_decode = false; };
 template <class Fmt, bool PAIR> constexpr int own_cap(int mt) { return (OwnStreams<Fmt>::cap + (Fmt::kVec == 1 && mt <= 2 ? 2 : 0)) / (PAIR ? 2 : 1); }
 constexpr int own_ahead(int mt) { return mt <= 1 ? 2 : 1; }
 // tiles of weights in flight or in use: a tile of 16 rows takes less time than its weights' way from memory (13696 x 4096, 8 rows: F143
@@ -2760,6 +2760,37 @@ static int dispatch_many_rows(const GemmArgs& a, int total_nb, hipStream_t s, co
   return rows_in_turn<Fmt, PAIR>(a, 64, total_nb, s, name);
 }
 
+// 5 to 16 rows without a norm: gemm_own_kernel, or (false) gemv_wide_kernel and gemv_stream_kernel.  Where its workgroups are one round and
+// there are 16 feature tiles and more.  gemv_wide_kernel takes 16 or 32 tiles a step and is at its best where they fill its steps (K about
+// 4096, 8192, 12288); gemm_own_kernel's lead grows with the rows and with K.  Ratios of its time to theirs, K of 2048 to 13696 by 1024 to
+// 12288 channels, medians of four runs in turn at the lines:
+//   9 to 16 rows: INT4 0.71 to 1.04.  F143 0.74 to 1.02; K of 3300 to 5000, and more than two blocks a compute unit, from 12 rows on 0.88 to
+//   1.01 (9 rows 1.08).  16-bit weights, up to a block a compute unit (4096 x 12288 1.06): 0.79 to 1.04; K of 3300 to 5120 from 14 rows on
+//   0.92 to 1.06 (9 rows 1.13), about 8192 and 12288 from 12 rows on 0.91 to 1.01 (9 rows 1.06).  Pairs 0.81 to 1.04; K of 3300 to 5000
+//   from 14 rows on (9 rows 1.12).
+//   7 and 8 rows, K past 5120 (pairs 6000): 0.83 to 1.02; not 16-bit and single F143 weights about 8192 and 12288 (1.05 to 1.07).
+//   5 and 6 rows: K from 8192 on INT4 0.89 to 0.99, from 10240 on F143 and pairs 0.87 to 1.02 (8192 1.07); not 16-bit weights.
+//   5 to 8 rows, INT4: short K and pairs of up to two blocks a compute unit 0.89 to 1.02 (2048 x 11008 1.11), single weights of more than
+//   four blocks a compute unit (4096 x 24576 0.84).
+//   F152 (16 instructions a decoded operand): 9 rows and more, K up to 3072, two blocks a compute unit 0.74 to 1.0; else up to 1.21.
+template <class Fmt, bool PAIR>
+static bool own_takes_few_rows(const GemmArgs& a, int total_nb, int cus, bool one_round) {
+  const int KT = a.KT;
+  if (a.prefer_stream || !one_round || KT < 16 || a.K >= GEMM_FAR) return false;
+  if (OwnStreams<Fmt>::long_decode) return a.M > 8 && !PAIR && KT <= 24 && total_nb <= 2 * cus;
+  if (Fmt::kVec > 2 && (PAIR || total_nb > cus)) return false;
+  const bool full = KT > 40 && ((KT + 4) & 31) <= 8;         // whole steps of gemv_wide_kernel, or nearly
+  if (a.M <= 8) {
+    if (Fmt::kVec == 1 && (PAIR ? KT <= 24 && total_nb <= 2 * cus : total_nb > 4 * cus)) return true;
+    if (a.M <= 6) return Fmt::kVec == 1 && !PAIR ? KT >= 64 : Fmt::kVec <= 2 && KT >= 80 && (PAIR || !full);
+    return KT > (PAIR ? 47 : 40) && (Fmt::kVec == 1 || PAIR || !full);
+  }
+  if (Fmt::kVec > 2) return a.M >= (KT > 24 && KT <= 40 ? 14 : full ? 12 : 9);
+  const bool middle = KT > 24 && KT < 40;
+  if (PAIR) return !middle || a.M >= 14;
+  return Fmt::kVec == 1 || a.M >= 12 || (!middle && total_nb <= 2 * cus);
+}
+
 template <class Fmt, bool PAIR>
 static int dispatch_gemv(const GemmArgs& a, int total_nb, hipStream_t s, const char* name) {
   if (a.M > 16 && a.K >= GEMM_FAR && a.epi.norm == PTA_NORM_NONE) return rows_in_turn<Fmt, PAIR>(a, 16, total_nb, s, name);
@@ -2782,7 +2813,7 @@ static int dispatch_gemv(const GemmArgs& a, int total_nb, hipStream_t s, const c
     const int per_cu = (total_nb + cus - 1) / cus;
     const int mt = (a.M + 15) / 16;
     if (a.epi.norm == PTA_NORM_NONE && a.M > 4) {
-      // gemm_own_kernel or gemm_tile_kernel (16 rows: gemv_wide_kernel, gemv_stream_kernel).  Both sides in us, INT4 unless named.
+      // gemm_own_kernel or gemm_tile_kernel (up to 16 rows: own_takes_few_rows).  Both sides in us, INT4 unless named.
       // One round of gemm_own_kernel's workgroups: it.  64 rows, 4096 x 11008: 14.5 against 21.8, 4096 x 4096 11.1 against 15.2,
       // 2048 x 2048 7.1 against 11.8; 32 rows 11.1 against 14.3, 8.0 against 11.2, 5.6 against 9.4; F143, 64 rows, 4096 x 4096
       // 11.9 against 16.2; bf16 14.5 against 18.2; with odd channel counts, which gemm_tile_kernel cannot take, 1000 channels at
@@ -2790,19 +2821,13 @@ static int dispatch_gemv(const GemmArgs& a, int total_nb, hipStream_t s, const c
       // Several rounds: each begins with nothing on its way.  Weights of one vector a tile lose a little (32000 channels, 64 rows
       // 32.4 against 31.4), those of two win beyond 32 rows (F143 41.8 against 51.6), so does a pair of either (11008 channels, 64
       // rows 29.2 against 39.7; F143 40.8 against 46.9), fp16 ones lose (72.5 against 68.3).  Pairs of up to 32 rows: INT4, one round and
-      // K of 3072 and more (11008 channels, 32 rows 16.9 against 21.5; 2048 x 5632 9.1 against 8.9).  9 to 16 rows, one round: 9.3 against 11.7 (4096 x 11008, 16 rows), K of 13696 13.5 against 17.8, pair of 2048 x 5632
-      // 7.4 against 10.0; fp16 only where every compute unit has one block or none (11008 x 4096 22.5 against 26.4; 4096 x 4608 14.7
-      // against 13.3).  5 to 8 rows: long K (13696 x 4096, 8 rows, INT4 10.9 against 13.5, F143 14.9 against 17.7, fp16 24.9 against 26.2;
-      // 5632 x 2048, F143 7.7 against 8.3, but 5 rows 6.6 against 6.3 with INT4), INT4 pairs (2048 x 5632, 8.0 against 9.1) and many
-      // channels (4096 x 24576, 15.3 against 18.3); 4096 x 4096 is even or lost (F143 7.5 against 7.1).
+      // K of 3072 and more (11008 channels, 32 rows 16.9 against 21.5; 2048 x 5632 9.1 against 8.9).
       const int wgs4 = total_nb / (PAIR ? 2 : 4);
       const OwnPlan plan = plan_gemm_own<Fmt, PAIR>(a);
       const bool one_round = plan.rounds == 1;
       bool own, tile = false;
       if (a.M <= 16) {
-        own = !a.prefer_stream && a.KT >= 16 && a.K < GEMM_FAR && one_round && (Fmt::kVec <= 2 || (!PAIR && total_nb <= cus));
-        if (a.M <= 8)
-          own = own && ((a.KT >= 40 && a.M >= 7) || (a.KT >= 64 && Fmt::kVec <= 2) || (Fmt::kVec == 1 && (PAIR ? a.KT <= 24 : total_nb > 4 * cus)));
+        own = own_takes_few_rows<Fmt, PAIR>(a, total_nb, cus, one_round);
       } else {
         tile = tile_fits(a, PAIR ? 2 : 4, 4, PAIR) && 2 * wgs4 >= cus;
         if (tile && PAIR) own = (mt > 2 && Fmt::kVec <= 2) || (Fmt::kVec == 1 && one_round && a.KT >= 24);

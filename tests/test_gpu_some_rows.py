@@ -166,3 +166,36 @@ def test_more_channels_than_a_grid_holds():
     assert torch.isfinite(out).all()
     at = torch.tensor(sorted({n for e in (0, per, N) for n in range(e - 100, e + 100) if 0 <= n < N} | set(range(0, N, 100003))), device="cuda")
     close(out[:, at], x.double() @ w[at].double().T, x.double().abs() @ w[at].double().abs().T, Kd, 11)
+
+
+@pytest.mark.parametrize("kind, M, Kd, N, pair, own", [
+    # full steps of gemv_wide_kernel, and either side of them; channels past two blocks a compute unit; short K and long
+    ("f8", 9, 4096, 4096, False, False), ("f8", 11, 4096, 1024, False, False), ("f8", 12, 4096, 4096, False, True), ("f8", 9, 3072, 4096, False, True),
+    ("f8", 9, 5120, 4096, False, True), ("f8", 8, 4096, 4096, False, False), ("f8", 8, 5632, 2048, False, True), ("f8", 8, 5632, 5632, True, False),
+    ("f8", 6, 8192, 4096, False, False), ("f8", 6, 11008, 4096, False, True), ("f8", 9, 4096, 5632, True, False), ("f8", 9, 4096, 2048, True, False), ("f8", 14, 4096, 2048, True, True), ("f8", 9, 9216, 2048, True, True), ("f8", 8, 1024, 2048, False, False),
+    ("f16", 9, 4096, 4096, False, False), ("f16", 13, 4096, 2048, False, False), ("f16", 14, 4096, 4096, False, True), ("f16", 9, 2048, 2048, False, True),
+    ("f16", 9, 5632, 2048, False, True), ("f16", 16, 4096, 4608, False, False), ("f16", 16, 2048, 2048, True, False), ("f16", 6, 11008, 4096, False, False), ("f16", 8, 8192, 2048, False, False), ("f16", 11, 12288, 1024, False, False), ("f16", 12, 8192, 2048, False, True),
+    ("f16", 8, 11008, 4096, False, True), ("f8", 8, 8192, 4096, False, False), ("f8", 9, 8192, 4096, False, True), ("f8", 7, 5120, 2048, False, False),
+    ("f8", 9, 2560, 12288, False, False), ("f8", 12, 2560, 12288, False, True), ("f16", 9, 5120, 4096, False, False),
+    ("f152", 16, 4096, 4096, False, False), ("f152", 9, 2048, 4096, False, True), ("f152", 16, 2048, 12288, False, False), ("f152", 8, 2048, 2048, False, False),
+    ("f152", 16, 11008, 4096, False, False),
+    ("int4", 9, 4096, 4096, False, True), ("int4", 12, 4096, 5632, True, False), ("int4", 16, 4096, 5632, True, True), ("int4", 5, 2048, 5632, True, True),
+    ("int4", 8, 2048, 11008, True, False), ("int4", 5, 4096, 24576, False, True), ("int4", 5, 4096, 12288, False, False), ("int4", 5, 8192, 2048, False, True),
+    ("int4", 6, 8192, 5632, True, False)])
+def test_which_few_rows_the_kernel_takes(kind, M, Kd, N, pair, own):
+    from poptransformer_amd import kernels as K
+    x, w = operands(M, Kd, N, 3)
+    x = (x * 0.02 if pair else x).half()
+    tw, plain = weight_of(kind, w)
+    out = torch.full((M, N), float("nan"), dtype=torch.float16, device="cuda")
+    K.linear(x, [tw, tw] if pair else [tw], [out, out] if pair else [out], swiglu=pair)
+    assert (K.linear_kernel() == "gemm_own_kernel") == own, K.linear_kernel()
+    y = x.double() @ plain.T
+    if not pair:
+        close(out, y, x.double().abs() @ plain.abs().T, Kd, 11)
+    else:
+        # as in test_pair
+        d = 2.0 ** -11 * y.abs() + (Kd + 2) * 2.0 ** -24 * (x.double().abs() @ plain.abs().T)
+        silu = torch.nn.functional.silu(y)
+        bound = 1.1 * d * (y.abs() + d) + d * silu.abs() + 2.5 * 2.0 ** -11 * (silu * y).abs() + 2.0 ** -20 * (1 + y.abs())
+        assert ((out.double() - silu * y).abs() <= bound).all()
