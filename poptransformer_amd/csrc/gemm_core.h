@@ -2641,15 +2641,17 @@ template <class Fmt, int MT, bool PAIR>
 static void launch_gemv(const GemmArgs& a, int total_nb, hipStream_t s) {
   // Waves per block: enough to split K finely when there are few channel blocks, fewer when
   // the grid alone already fills the machine.  The LDS reduction buffer caps the wide cases.
+  // (more than 16 rows of 16 feature tiles and more: F152 weights only)
+  constexpr bool FINE = !PAIR && (MT == 1 || (MT == 2 && OwnStreams<Fmt>::long_decode));
   gemm_kernel_taken = "gemv_mfma_kernel";
-  if constexpr (PAIR) {
-    hipLaunchKernelGGL((gemv_mfma_kernel<Fmt, MT, 8, PAIR>), dim3(total_nb), dim3(8 * 64), 0, s, a);
-  } else {
-    if (a.KT >= 16 && total_nb <= 1024)
+  if constexpr (FINE) {
+    if (a.KT >= 16 && total_nb <= 1024) {
       hipLaunchKernelGGL((gemv_mfma_kernel<Fmt, MT, 16, PAIR>), dim3(total_nb), dim3(16 * 64), 0, s, a);
-    else
-      hipLaunchKernelGGL((gemv_mfma_kernel<Fmt, MT, 8, PAIR>), dim3(total_nb), dim3(8 * 64), 0, s, a);
+      return;
+    }
   }
+  constexpr int NW = MT == 4 && PAIR ? 4 : 8;
+  hipLaunchKernelGGL((gemv_mfma_kernel<Fmt, MT, NW, PAIR>), dim3(total_nb), dim3(NW * 64), 0, s, a);
 }
 
 template <class Fmt, bool PAIR>
@@ -2688,10 +2690,13 @@ static int dispatch_many_rows(const GemmArgs& a, int total_nb, hipStream_t s, co
   // 256 rows 36 against 49.  fp16: 768 x 3072, 205 rows 9.8 against 15.5; 2048 x 2048, 256 rows 11.2 against 19.4; F143 4096 x 4096,
   // 256 rows 20.6 against 29.6.  More rounds: to 128 rows two (4096 x 11008, 128 rows, INT4 29.8 against 40.9, F143 35.8 against 44.3,
   // fp16 44 against 47), of INT4 weights three (their pair of 11008 channels 41.5 against 48.0), and small launches (768 x 3072,
-  // 512 rows, INT4 16.0 against 25.1); beyond, these lose: 4096 x 11008, 160 rows, INT4 42.8 against 39.8, fp16 60 against 44.
+  // 512 rows, INT4 16.0 against 25.1); beyond, these lose: 4096 x 11008, 160 rows, INT4 42.8 against 39.8, fp16 60 against 44.  The plan's
+  // time does not see what a round's begin and end take, so with short K the rounds are counted too: INT4 768 x 32000, 65 rows, four rounds
+  // 26.8 against 21.3; pair 768 x 11008, three, 17.7 against 13.7; 512 x 4096, 1000 rows, four, 1.14 times; 1024 x 6144, 768 rows, five, 1.10.
   if (a.epi.norm == PTA_NORM_NONE) {
     const OwnPlan plan = plan_gemm_own<Fmt, PAIR>(a);
-    if (plan.rounds == 1 || (a.M <= 128 && plan.rounds <= (Fmt::kVec == 1 ? 3 : 2)) || plan.us <= (Fmt::kVec == 1 ? 22.0 : 11.0))
+    const int most = a.M <= 128 ? (Fmt::kVec == 1 && a.KT >= 12 ? 3 : 2) : a.KT >= 8 || PAIR ? 4 : 3;
+    if (plan.rounds == 1 || (plan.rounds <= most && (a.M <= 128 || plan.us <= (Fmt::kVec == 1 ? 22.0 : 11.0))))
       return launch_gemm_own_plan<Fmt, PAIR>(a, plan, s, name);
   }
   const int cus = device_compute_units();
@@ -2830,9 +2835,18 @@ static int dispatch_gemv(const GemmArgs& a, int total_nb, hipStream_t s, const c
         own = own_takes_few_rows<Fmt, PAIR>(a, total_nb, cus, one_round);
       } else {
         tile = tile_fits(a, PAIR ? 2 : 4, 4, PAIR) && 2 * wgs4 >= cus;
-        if (tile && PAIR) own = (mt > 2 && Fmt::kVec <= 2) || (Fmt::kVec == 1 && one_round && a.KT >= 24);
+        constexpr bool F152 = OwnStreams<Fmt>::long_decode;
+        if (tile && PAIR) own = mt > 2 ? Fmt::kVec <= 2 && !(F152 && a.KT <= 16 && wgs4 <= cus) : Fmt::kVec == 1 && one_round && a.KT >= 24;
         else if (tile) own = one_round || (mt > 2 && Fmt::kVec == 2);
-        else own = a.KT >= 8 || mt > 2;
+        // Launches that gemm_tile_kernel cannot take (odd numbers of blocks, few of them, few feature tiles): gemm_own_kernel or
+        // gemv_mfma_kernel, whose workgroups of one block come and go.  Few feature tiles, more than 32 rows: a wave has one or none, and
+        // the end is all (us, 33 rows: 128 features 1.17 times; pairs 256 x 1024 fp16 4.4 against 5.5, 768 x 11008 13.3 against 19.0, F143 11.8
+        // against 16.2; 768 x 2048 it wins).  Up to 32 rows, against the kernel before them: 16-bit pairs of several rounds 1024 x 5608 0.88
+        // and 1.19, 2048 x 5608 0.93 and 1.09, 3072 x 5608 0.96 and 1.0, one round of 1024 features 0.92 and 1.03; F152 singles 1024 x 4104
+        // 0.9 and 1.1, 3072 x 1000 1.08 and 1.2, pairs 2048 x 4104 0.73 and 0.99, 4096 x 2056 0.97 and 0.9.
+        else if (mt > 2) own = PAIR ? a.KT >= 8 || (one_round && a.KT > 4) : a.KT > 2;
+        else if (F152) own = a.KT > (PAIR ? 16 : 24) && (!PAIR || total_nb <= cus);
+        else own = a.KT >= 8 && !(PAIR && Fmt::kVec > 2 && (a.KT == 8 || (!one_round && a.KT < 24)));
       }
       if (own) return launch_gemm_own_plan<Fmt, PAIR>(a, plan, s, name);
       int rc = 1;
@@ -2856,7 +2870,7 @@ static int dispatch_gemv(const GemmArgs& a, int total_nb, hipStream_t s, const c
           }
         }
         if (!wide && a.M <= 32) rc = launch_gemm_tile<Fmt, 2, 4, PAIR>(a, total_nb, s, name);
-        else if constexpr (PAIR ? Fmt::kVec > 2 : Fmt::kVec != 2) {
+        else if constexpr (PAIR ? Fmt::kVec > 2 || OwnStreams<Fmt>::long_decode : Fmt::kVec != 2) {
           if (!wide) rc = launch_gemm_tile<Fmt, 4, 4, PAIR>(a, total_nb, s, name);
         }
       }
@@ -2879,7 +2893,8 @@ static int dispatch_gemv(const GemmArgs& a, int total_nb, hipStream_t s, const c
       else rc = launch_gemv_wide_for<Fmt, PAIR, false>(a, total_nb, per_cu, s, name);
       if (rc) return rc;
     } else if (a.M <= 16) launch_gemv<Fmt, 1, PAIR>(a, total_nb, s);
-    else launch_gemv<Fmt, 2, PAIR>(a, total_nb, s);        // (17 to 32 rows of fewer than 8 feature tiles)
+    else if (a.M <= 32) launch_gemv<Fmt, 2, PAIR>(a, total_nb, s);
+    else launch_gemv<Fmt, 4, PAIR>(a, total_nb, s);
   }
   PTA_CHECK_LAUNCH(name);
   return PTA_OK;

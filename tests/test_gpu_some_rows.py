@@ -183,19 +183,64 @@ def test_more_channels_than_a_grid_holds():
     ("int4", 8, 2048, 11008, True, False), ("int4", 5, 4096, 24576, False, True), ("int4", 5, 4096, 12288, False, False), ("int4", 5, 8192, 2048, False, True),
     ("int4", 6, 8192, 5632, True, False)])
 def test_which_few_rows_the_kernel_takes(kind, M, Kd, N, pair, own):
+    taken = product(kind, M, Kd, N, pair)
+    assert (taken == "gemm_own_kernel") == own, taken
+
+
+def product(kind, M, Kd, N, pair):
+    """A product, checked; the kernel that it took."""
     from poptransformer_amd import kernels as K
     x, w = operands(M, Kd, N, 3)
     x = (x * 0.02 if pair else x).half()
     tw, plain = weight_of(kind, w)
     out = torch.full((M, N), float("nan"), dtype=torch.float16, device="cuda")
     K.linear(x, [tw, tw] if pair else [tw], [out, out] if pair else [out], swiglu=pair)
-    assert (K.linear_kernel() == "gemm_own_kernel") == own, K.linear_kernel()
-    y = x.double() @ plain.T
+    taken = K.linear_kernel()
+    y, mag = x.double() @ plain.T, x.double().abs() @ plain.abs().T
     if not pair:
-        close(out, y, x.double().abs() @ plain.abs().T, Kd, 11)
+        close(out, y, mag, Kd, 11)
     else:
         # as in test_pair
-        d = 2.0 ** -11 * y.abs() + (Kd + 2) * 2.0 ** -24 * (x.double().abs() @ plain.abs().T)
+        d = 2.0 ** -11 * y.abs() + (Kd + 2) * 2.0 ** -24 * mag
         silu = torch.nn.functional.silu(y)
         bound = 1.1 * d * (y.abs() + d) + d * silu.abs() + 2.5 * 2.0 ** -11 * (silu * y).abs() + 2.0 ** -20 * (1 + y.abs())
         assert ((out.double() - silu * y).abs() <= bound).all()
+    return taken
+
+
+@pytest.mark.parametrize("kind, M, Kd, N, pair, kernel", [
+    # few feature tiles and several rounds, or next to none; either side of the lines
+    ("f16", 33, 768, 5632, True, "gemv_mfma"), ("f16", 64, 768, 5608, True, "gemv_mfma"), ("int4", 63, 512, 8192, True, "gemv_mfma"), ("f8", 48, 768, 11008, True, "gemv_mfma"),
+    ("f152", 64, 768, 8200, True, "gemv_mfma"), ("f16", 40, 512, 1000, True, "gemv_mfma"), ("f16", 48, 768, 2048, True, "gemm_own"), ("f16", 33, 1024, 5632, True, "gemm_tile"), ("f16", 33, 1024, 5608, True, "gemm_own"),
+    ("f16", 40, 256, 40, False, "gemv_mfma"), ("int4", 64, 128, 1000, False, "gemv_mfma"), ("f8", 33, 8, 4104, False, "gemv_mfma"), ("f152", 49, 256, 250, False, "gemv_mfma"),
+    ("f16", 33, 264, 1000, False, "gemm_own"), ("int4", 64, 768, 50257, False, "gemm_own"),
+    # what gemm_tile_kernel cannot take
+    ("f16", 20, 1024, 5608, True, "gemv_mfma"), ("f16", 32, 2048, 5608, True, "gemv_mfma"), ("f16", 32, 3072, 5608, True, "gemm_own"), ("f16", 17, 2048, 2056, True, "gemm_own"),
+    ("int4", 20, 1024, 5608, True, "gemm_own"), ("f152", 24, 2048, 1000, False, "gemv_mfma"), ("f152", 17, 3072, 4104, False, "gemv_mfma"), ("f152", 32, 4096, 1000, False, "gemm_own"),
+    ("f152", 20, 4096, 5608, True, "gemv_mfma"), ("f152", 31, 2048, 2056, True, "gemv_mfma"), ("f152", 32, 4096, 2056, True, "gemm_own"),
+    ("f152", 64, 2048, 5632, True, "gemm_tile"), ("f152", 33, 1024, 5632, True, "gemm_tile"), ("f152", 40, 4096, 5632, True, "gemm_own"),
+    # rounds of gemm_own_kernel beyond 64 rows
+    ("int4", 65, 768, 11008, True, "gemm_rows"), ("int4", 128, 1024, 32000, False, "gemm_rows"), ("int4", 128, 2048, 5632, True, "gemm_own"),
+    ("int4", 1000, 512, 4096, False, "gemm_panel"), ("int4", 700, 512, 4096, False, "gemm_own"), ("int4", 768, 1024, 6144, False, "gemm_panel")])
+def test_which_kernel_more_rows_take(kind, M, Kd, N, pair, kernel):
+    assert product(kind, M, Kd, N, pair) == kernel + "_kernel"
+
+
+@pytest.mark.parametrize("M, Kd, N, pair, kernel", [(33, 256, 250, False, "gemv_mfma"), (64, 72, 1000, False, "gemv_mfma"), (40, 768, 5632, True, "gemv_mfma"),
+                                                    (24, 520, 5632, True, "gemv_mfma"), (33, 520, 250, False, "gemm_own")])
+def test_which_kernel_more_rows_of_bf16_take(M, Kd, N, pair, kernel):
+    from poptransformer_amd import hybrid_kernels as HK
+    x, w = operands(M, Kd, N, 11)
+    x, w = (x * 0.1).to(torch.bfloat16), w.to(torch.bfloat16)
+    W = HK.WideWeight(w, torch.bfloat16)
+    out = torch.full((M, HK.pad8(N)), float("nan"), dtype=torch.float32, device="cuda")
+    HK.linear(x, W, out, M, ld=HK.pad8(N), **(dict(up=W, pair=1) if pair else {}))
+    assert HK.linear_kernel() == kernel + "_kernel"
+    y, mag = x.double() @ w.double().T, x.double().abs() @ w.double().abs().T
+    if not pair:
+        return close(out[:, :N], y, mag, Kd, 24)
+    d = (Kd + 2) * 2.0 ** -24 * mag
+    silu = torch.nn.functional.silu(y)
+    # the sums' errors (silu multiplies the gate's by 1.1 at most), the exponential and the quotient in fp32
+    bound = 1.1 * d * (y.abs() + d) + d * silu.abs() + 2.0 ** -20 * (silu * y).abs() + 2.0 ** -24
+    assert ((out[:, :N].double() - silu * y).abs() <= bound).all()
