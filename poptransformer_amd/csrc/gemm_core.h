@@ -1900,10 +1900,10 @@ static int launch_gemm_rows(const GemmArgs& a, int total_nb, hipStream_t s, cons
 }
 
 // The sums of a wave's tile (RG row groups x NST channel blocks; lane l holds channels st * 16 + (l / 16) * 4 + r of
-// row l % 16 of each row group) go out: unit cw of the workgroup, first block blk0 of matrix mi, rows from row0 of M,
+// row l % 16 of each row group) go out: unit cw of the workgroup, first block blk0 of matrix `mat`, rows from row0 of M,
 // to the rows of Y that `order` lists (null: the same).
 template <class Fmt, int NST, int RG, bool PAIR>
-__device__ __forceinline__ void panel_store(const GemmArgs& a, f32x4 (&acc)[RG][NST], unsigned char* smem, int cw, int mi, int blk0,
+__device__ __forceinline__ void panel_store(const GemmMat& mat, const GemmEpilogue& epi, float* part, f32x4 (&acc)[RG][NST], unsigned char* smem, int cw, int blk0,
                                             int row0, int nsl, typename Fmt::Scale s0, typename Fmt::Scale s1, int M, const int32_t* order = nullptr) {
   constexpr int SW = NST * 16 + 4;                // floats per row of a wave's epilogue strip
   const int lane = threadIdx.x & 63;
@@ -1912,10 +1912,9 @@ __device__ __forceinline__ void panel_store(const GemmArgs& a, f32x4 (&acc)[RG][
   // back with eight consecutive channels of one row per lane: one 16-byte store per lane, whole 128-byte stretches
   // of a row per wave.  (A wave's LDS accesses complete in order.)
   float* strip = reinterpret_cast<float*>(smem) + (size_t)cw * (16 * SW);
-  const GemmMat& mat = a.mat[PAIR ? 0 : mi];
   const int N = mat.N;
-  const bool direct = !mat.bias && mat.act == PTA_ACT_NONE && !a.epi.bias && a.epi.act == PTA_ACT_NONE && !a.epi.mul &&
-                      a.epi.post_scale == 0.0f && !a.epi.out_fp8_scale;
+  const bool direct = !mat.bias && mat.act == PTA_ACT_NONE && !epi.bias && epi.act == PTA_ACT_NONE && !epi.mul &&
+                      epi.post_scale == 0.0f && !epi.out_fp8_scale;
   auto put = [&](const f32x4 (&sums)[NST]) {
 #pragma unroll
     for (int st = 0; st < NST; ++st)
@@ -1946,7 +1945,7 @@ __device__ __forceinline__ void panel_store(const GemmArgs& a, f32x4 (&acc)[RG][
         f16x8 y;
 #pragma unroll
         for (int j = 0; j < 8; ++j)
-          y[j] = swiglu_out(a.epi, (f16)Fmt::finish(j < 4 ? g0[j & 3] : g1[j & 3], s0), (f16)Fmt::finish(j < 4 ? u0[j & 3] : u1[j & 3], s1));
+          y[j] = swiglu_out(epi, (f16)Fmt::finish(j < 4 ? g0[j & 3] : g1[j & 3], s0), (f16)Fmt::finish(j < 4 ? u0[j & 3] : u1[j & 3], s1));
         if (n + 8 <= N && (N & 7) == 0) {
           *reinterpret_cast<f16x8*>(mat.Y + (size_t)m * N + n) = y;
         } else {
@@ -1966,7 +1965,7 @@ __device__ __forceinline__ void panel_store(const GemmArgs& a, f32x4 (&acc)[RG][
         const f32x4 v0 = *reinterpret_cast<const f32x4*>(strip + rr * SW + c0), v1 = *reinterpret_cast<const f32x4*>(strip + rr * SW + c0 + 4);
         if (m >= M) continue;
         if (nsl > 1) {
-          float* p = a.part + ((size_t)blockIdx.y * M + m) * N + n;
+          float* p = part + ((size_t)blockIdx.y * M + m) * N + n;
           if (n + 8 <= N && (N & 3) == 0) {
             *reinterpret_cast<f32x4*>(p) = v0;
             *reinterpret_cast<f32x4*>(p + 4) = v1;
@@ -1984,11 +1983,11 @@ __device__ __forceinline__ void panel_store(const GemmArgs& a, f32x4 (&acc)[RG][
         f16x8 y;
         if (direct && n + 8 <= N && (N & 7) == 0) {                // nothing but the residual stream to add: whole vectors
           f16x8 res;
-          if (a.epi.residual) res = *reinterpret_cast<const f16x8*>(a.epi.residual + (size_t)m * N + n);
+          if (epi.residual) res = *reinterpret_cast<const f16x8*>(epi.residual + (size_t)m * N + n);
 #pragma unroll
           for (int j = 0; j < 8; ++j) {
             y[j] = (f16)Fmt::finish(j < 4 ? v0[j & 3] : v1[j & 3], s0);
-            if (a.epi.residual) y[j] = y[j] + res[j];
+            if (epi.residual) y[j] = y[j] + res[j];
           }
           *reinterpret_cast<f16x8*>(mat.Y + (size_t)m * N + n) = y;
           continue;
@@ -1999,7 +1998,7 @@ __device__ __forceinline__ void panel_store(const GemmArgs& a, f32x4 (&acc)[RG][
           if (n + j < N) {
             if (mat.bias) y0 = y0 + mat.bias[n + j];
             y0 = apply_act(mat.act, y0);
-            y0 = apply_epilogue(a.epi, y0, m, n + j, N);
+            y0 = apply_epilogue(epi, y0, m, n + j, N);
           }
           y[j] = y0;
         }
@@ -2220,7 +2219,7 @@ __global__ __launch_bounds__(PANEL_WAVES * 64) __attribute__((amdgpu_waves_per_e
 
   const typename Fmt::Scale s0 = Fmt::load_scale(a.mat[PAIR ? 0 : mi].scale, a.x_scale, 0, 1);   // no format's finish uses the per-channel part
   const typename Fmt::Scale s1 = Fmt::load_scale(a.mat[PAIR ? 1 : mi].scale, a.x_scale, 0, 1);
-  panel_store<Fmt, NST, RG, PAIR>(a, acc, smem, cw, mi, blk0, row0, nsl, s0, s1, M);
+  panel_store<Fmt, NST, RG, PAIR>(a.mat[PAIR ? 0 : mi], a.epi, a.part, acc, smem, cw, blk0, row0, nsl, s0, s1, M);
 }
 
 // ------------------------------------------------------------------------------------------
@@ -2382,6 +2381,14 @@ __global__ __launch_bounds__(BLOCK_WAVES * 64) __attribute__((amdgpu_waves_per_e
   for (int n = 0; n < NS; ++n)
 #pragma unroll
     for (int q = 0; q < LOADS; ++q) bring(first * (64 / SF) + n, n * STAGE, q);
+  // (the wide epilogue's many arguments, read while the first stages are on their way: 1024 x 4096, 512 rows, bf16 22.7 -> 19.0 us; the
+  // fp16 one's few gain nothing)
+  GemmMat wide;
+  GemmEpilogue none{};
+  if constexpr (Fmt::kWide) {
+    wide = a.mat[PAIR ? 0 : mi];
+    read_end<Fmt, PAIR>(wide, none);
+  }
   __builtin_amdgcn_s_waitcnt(0x0f70);             // vmcnt(0)
   __syncthreads();
 #pragma unroll
@@ -2424,7 +2431,7 @@ __global__ __launch_bounds__(BLOCK_WAVES * 64) __attribute__((amdgpu_waves_per_e
   __syncthreads();                                // (what follows reuses the stages)
   const typename Fmt::Scale s0 = Fmt::load_scale(a.mat[PAIR ? 0 : mi].scale, a.x_scale, 0, 1);   // no format's finish uses the per-channel part
   const typename Fmt::Scale s1 = Fmt::load_scale(a.mat[PAIR ? 1 : mi].scale, a.x_scale, 0, 1);
-  panel_store<Fmt, NST, RG, PAIR>(a, acc, smem, wave, mi, blk0 + wc * (PAIR ? 2 : 4), row0 + wr * (RG * 16), nsl, s0, s1, M, order);
+  panel_store<Fmt, NST, RG, PAIR>(Fmt::kWide ? wide : a.mat[PAIR ? 0 : mi], a.epi, a.part, acc, smem, wave, blk0 + wc * (PAIR ? 2 : 4), row0 + wr * (RG * 16), nsl, s0, s1, M, order);
 }
 
 template <class Fmt, int RG, bool PAIR, class Rows>
@@ -2768,12 +2775,13 @@ static int dispatch_many_rows(const GemmArgs& a, int total_nb, hipStream_t s, co
 // 5 to 16 rows without a norm: gemm_own_kernel, or (false) gemv_wide_kernel and gemv_stream_kernel.  Where its workgroups are one round and
 // there are 16 feature tiles and more.  gemv_wide_kernel takes 16 or 32 tiles a step and is at its best where they fill its steps (K about
 // 4096, 8192, 12288); gemm_own_kernel's lead grows with the rows and with K.  Ratios of its time to theirs, K of 2048 to 13696 by 1024 to
-// 12288 channels, medians of four runs in turn at the lines:
-//   9 to 16 rows: INT4 0.71 to 1.04.  F143 0.74 to 1.02; K of 3300 to 5000, and more than two blocks a compute unit, from 12 rows on 0.88 to
-//   1.01 (9 rows 1.08).  16-bit weights, up to a block a compute unit (4096 x 12288 1.06): 0.79 to 1.04; K of 3300 to 5120 from 14 rows on
-//   0.92 to 1.06 (9 rows 1.13), about 8192 and 12288 from 12 rows on 0.91 to 1.01 (9 rows 1.06).  Pairs 0.81 to 1.04; K of 3300 to 5000
-//   from 14 rows on (9 rows 1.12).
-//   7 and 8 rows, K past 5120 (pairs 6000): 0.83 to 1.02; not 16-bit and single F143 weights about 8192 and 12288 (1.05 to 1.07).
+// 12288 channels, medians of runs in turn, weights from HBM and from the last cache alike:
+//   9 to 16 rows: INT4 0.71 to 1.05.  F143 0.74 to 1.02; K of 3300 to 5000, and more than two blocks a compute unit, from 12 rows on 0.88 to
+//   1.01 (9 rows 1.08).  16-bit weights, up to a block a compute unit (4096 x 12288 1.06): 0.79 to 1.04; K of 3300 to 5000 from 16 rows on
+//   0.92 to 1.02 (14 rows 1.08, 9 rows 1.14), about 8192 and 12288 from 12 rows on 0.91 to 1.01 (9 rows 1.06).  Pairs 0.81 to 1.04; K of
+//   3300 to 5000 from 14 rows on (9 rows 1.12).
+//   7 and 8 rows, K past 5120 (pairs and 16-bit weights 6000): 0.83 to 1.02; not 16-bit and single F143 weights about 8192 and 12288 (1.05 to
+//   1.07).
 //   5 and 6 rows: K from 8192 on INT4 0.89 to 0.99, from 10240 on F143 and pairs 0.87 to 1.02 (8192 1.07); not 16-bit weights.
 //   5 to 8 rows, INT4: short K and pairs of up to two blocks a compute unit 0.89 to 1.02 (2048 x 11008 1.11), single weights of more than
 //   four blocks a compute unit (4096 x 24576 0.84).
@@ -2788,10 +2796,10 @@ static bool own_takes_few_rows(const GemmArgs& a, int total_nb, int cus, bool on
   if (a.M <= 8) {
     if (Fmt::kVec == 1 && (PAIR ? KT <= 24 && total_nb <= 2 * cus : total_nb > 4 * cus)) return true;
     if (a.M <= 6) return Fmt::kVec == 1 && !PAIR ? KT >= 64 : Fmt::kVec <= 2 && KT >= 80 && (PAIR || !full);
-    return KT > (PAIR ? 47 : 40) && (Fmt::kVec == 1 || PAIR || !full);
+    return KT > (PAIR || Fmt::kVec > 2 ? 47 : 40) && (Fmt::kVec == 1 || PAIR || !full);
   }
-  if (Fmt::kVec > 2) return a.M >= (KT > 24 && KT <= 40 ? 14 : full ? 12 : 9);
   const bool middle = KT > 24 && KT < 40;
+  if (Fmt::kVec > 2) return a.M >= (middle ? 16 : full ? 12 : 9);
   if (PAIR) return !middle || a.M >= 14;
   return Fmt::kVec == 1 || a.M >= 12 || (!middle && total_nb <= 2 * cus);
 }

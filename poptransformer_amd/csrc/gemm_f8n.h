@@ -577,7 +577,7 @@ __global__ __launch_bounds__(PANEL_WAVES * 64) __attribute__((amdgpu_waves_per_e
   }
   if (!active) return;
   const Fmt::Scale s0 = Fmt::load_scale(m0.scale, a.x_scale, 0, 1), s1 = Fmt::load_scale(m1.scale, a.x_scale, 0, 1);
-  panel_store<Fmt, NST, RG, PAIR>(a, acc, smem, cw, mi, blk0, row0, nsl, s0, s1, M);
+  panel_store<Fmt, NST, RG, PAIR>(a.mat[PAIR ? 0 : mi], a.epi, a.part, acc, smem, cw, blk0, row0, nsl, s0, s1, M);
 }
 
 // LDS of gemm_f8n_panel_kernel: two stages of both operands and their flags; the parts' meeting; the epilogue strips

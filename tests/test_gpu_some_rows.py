@@ -173,10 +173,10 @@ def test_more_channels_than_a_grid_holds():
     ("f8", 9, 4096, 4096, False, False), ("f8", 11, 4096, 1024, False, False), ("f8", 12, 4096, 4096, False, True), ("f8", 9, 3072, 4096, False, True),
     ("f8", 9, 5120, 4096, False, True), ("f8", 8, 4096, 4096, False, False), ("f8", 8, 5632, 2048, False, True), ("f8", 8, 5632, 5632, True, False),
     ("f8", 6, 8192, 4096, False, False), ("f8", 6, 11008, 4096, False, True), ("f8", 9, 4096, 5632, True, False), ("f8", 9, 4096, 2048, True, False), ("f8", 14, 4096, 2048, True, True), ("f8", 9, 9216, 2048, True, True), ("f8", 8, 1024, 2048, False, False),
-    ("f16", 9, 4096, 4096, False, False), ("f16", 13, 4096, 2048, False, False), ("f16", 14, 4096, 4096, False, True), ("f16", 9, 2048, 2048, False, True),
+    ("f16", 9, 4096, 4096, False, False), ("f16", 15, 4096, 2048, False, False), ("f16", 16, 4096, 4096, False, True), ("f16", 9, 2048, 2048, False, True),
     ("f16", 9, 5632, 2048, False, True), ("f16", 16, 4096, 4608, False, False), ("f16", 16, 2048, 2048, True, False), ("f16", 6, 11008, 4096, False, False), ("f16", 8, 8192, 2048, False, False), ("f16", 11, 12288, 1024, False, False), ("f16", 12, 8192, 2048, False, True),
     ("f16", 8, 11008, 4096, False, True), ("f8", 8, 8192, 4096, False, False), ("f8", 9, 8192, 4096, False, True), ("f8", 7, 5120, 2048, False, False),
-    ("f8", 9, 2560, 12288, False, False), ("f8", 12, 2560, 12288, False, True), ("f16", 9, 5120, 4096, False, False),
+    ("f8", 9, 2560, 12288, False, False), ("f8", 12, 2560, 12288, False, True), ("f16", 9, 5120, 4096, False, True), ("f16", 8, 5632, 2048, False, False),
     ("f152", 16, 4096, 4096, False, False), ("f152", 9, 2048, 4096, False, True), ("f152", 16, 2048, 12288, False, False), ("f152", 8, 2048, 2048, False, False),
     ("f152", 16, 11008, 4096, False, False),
     ("int4", 9, 4096, 4096, False, True), ("int4", 12, 4096, 5632, True, False), ("int4", 16, 4096, 5632, True, True), ("int4", 5, 2048, 5632, True, True),
