@@ -2687,7 +2687,25 @@ static int rows_in_turn(const GemmArgs& a, int chunk, int total_nb, hipStream_t 
 
 template <class Fmt> struct BlockFormat { static constexpr bool ok = false; };
 
-// More than 64 rows.  Beyond 128 rows gemm_block_kernel or (INT4) gemm_panel_kernel, up to 128 gemm_rows_kernel, where
+// More than 128 rows, 16-bit weights: whether one round of gemm_rows_kernel's workgroups (128 rows, and half the channels of
+// gemm_block_kernel's) is the faster launch.  gemm_block_kernel's time follows the rows that its blocks hold, gemm_rows_kernel's does not,
+// and with few tiles half the chip has none; a single weight's K can be split instead, a pair's cannot.  Ratios gemm_block_kernel to
+// gemm_rows_kernel, weights from HBM, pairs 2048 x 2048 to 5632: 129 rows 0.95, 160 1.04, 200 1.17, 256 1.26, 320 1.1, 400 0.9, 512 1.14, 768
+// 1.08, 1000 0.95; 8192 x 5632, 256 rows 1.26.  The fp32 epilogue adds to the former (it passes through LDS in one copy of the code): with K
+// of 1024 1.03 to 1.31 (pairs) and 1.0 to 1.23 for up to 192 workgroups of the latter, 2048 x 6144, 512 rows 1.18.
+template <class Fmt, bool PAIR>
+static bool rows_before_blocks(const GemmArgs& a, int total_nb, int cus) {
+  if (Fmt::kVec < 4) return false;
+  const int blocks = (a.M + 127) / 128, wgs = total_nb / (PAIR ? ROWS_CB / 2 : ROWS_CB) * blocks;
+  if (wgs > cus) return false;
+  const double held = a.M / (128.0 * blocks), line = 0.75 + 0.04 * (blocks - 2);
+  if (Fmt::kWide && a.KT <= 8) return PAIR || wgs <= cus * 3 / 4 || held >= line;
+  if (Fmt::kWide && a.KT <= 16) return PAIR ? held >= line - 0.15 : wgs >= cus * 5 / 8 && held >= line;
+  return PAIR && held >= line;
+}
+
+// More than 64 rows: gemm_own_kernel where its workgroups are few rounds; beyond 128 rows gemm_block_kernel (16-bit and F143 weights) or
+// gemm_panel_kernel (INT4, F152), and up to 128, or by rows_before_blocks, gemm_rows_kernel, where
 // the channel blocks divide into their workgroup tiles; a single matrix with few channels also splits K when a workspace is at hand.  Otherwise
 // the rows go through the smaller paths in turn, 64 at a time.
 template <class Fmt, bool PAIR>
@@ -2713,13 +2731,14 @@ static int dispatch_many_rows(const GemmArgs& a, int total_nb, hipStream_t s, co
   // More than 128 rows (measured on whole prompt passes of the 7B shape, gemm_rows_kernel against this: 6.5 against
   // 7.2 ms at 128 rows, 7.7 against 7.3 at 192, 8.1 against 7.5 at 256): 128-row panels through LDS, the weights
   // straight into registers.
-  // Formats with a form of gemm_block_kernel: all launches of more than 128 rows.  Measured against the kernels they had before (us):
+  // Formats with a form of gemm_block_kernel: launches of more than 128 rows.  Measured against the kernels they had before (us):
   // FP8, 1000 rows: 4096 x 2 x 13696 pair 500 -> 198, 13696 x 4096 311 -> 110, 4096 x 4608 145 -> 60 (gemm_panel_kernel, whose two
   // vectors per tile spill); bf16, 2048 rows: 4096 x 4096 102 -> 70, 11008 x 4096 261 -> 190; fp16 4096 x 2 x 11008 pair, 2048
   // rows 564 -> 326, 512 rows 176 -> 103, 160 rows 83 -> 60 (gemm_rows_kernel).  At 65 to 128 rows the pair and 11008 features
   // lose (0.75 to 0.9) what small matrices win (1.3): those stay.
   if constexpr (BlockFormat<Fmt>::ok) {
-    if (a.M > 128 && a.epi.norm == PTA_NORM_NONE) return dispatch_gemm_block<typename BlockFormat<Fmt>::type, PAIR>(a, s, name);
+    if (a.M > 128 && a.epi.norm == PTA_NORM_NONE && !(tiles && rows_before_blocks<Fmt, PAIR>(a, total_nb, cus)))
+      return dispatch_gemm_block<typename BlockFormat<Fmt>::type, PAIR>(a, s, name);
   }
   if constexpr (Fmt::kVec <= 2 && !BlockFormat<Fmt>::ok) {
     if (a.M > 128 && panel_fits(a, 4, PAIR)) {

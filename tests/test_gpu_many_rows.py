@@ -1,4 +1,5 @@
-"""Products of more than 128 rows by 16-bit and FP8 weights (gemm_block_kernel) at the edges of its tiles, against float64."""
+"""Products of more than 128 rows by 16-bit and FP8 weights, against float64.  Launches of one or few rounds go to gemm_own_kernel: the
+sizes that are meant for gemm_block_kernel and gemm_rows_kernel, at the edges of their tiles, assert that they reach them (BLOCK and below)."""
 import math
 import numpy as np
 import pytest
@@ -10,6 +11,11 @@ SHAPES = [  # rows, features, channels: one past and one short of a tile of 128 
     (129, 8, 16), (255, 72, 250), (256, 64, 256), (257, 136, 264), (384, 200, 520), (1000, 1000, 48), (513, 4096, 272),
     # more workgroups than gemm_own_kernel takes
     (129, 2056, 8200), (255, 4104, 4100), (513, 2056, 2056), (1000, 1032, 1040)]
+
+# gemm_block_kernel: remainders of its stages of 32 and 64 features (fewer of them than it has stages, one, and past the last whole one), rows
+# one past and short of 128 and 256, channels short of a block, of eight and of its groups of 256
+BLOCK = [(1000, 8, 2056), (999, 24, 2050), (1000, 32, 2056), (1000, 56, 2047), (1000, 64, 2056), (897, 72, 2304), (1000, 88, 2300), (896, 96, 2560), (1000, 120, 2056),
+         (129, 136, 8200), (255, 152, 8200), (256, 160, 8192), (257, 184, 8200), (383, 192, 8200), (385, 200, 8195), (1025, 520, 2056), (4096, 40, 1000)]
 
 
 def close(got, ref, magnitude, K, bits):
@@ -171,3 +177,142 @@ def test_fp8_exponents_at_the_ends_of_their_range(exponent, slices):
         assert torch.equal(out[sure], (s[sure].sign() * math.inf).half())
     else:
         close(out, s * 2.0 ** exponent, mag * 2.0 ** exponent, Kd, 11)
+
+
+@pytest.mark.parametrize("kind", ["f16", "f8"])
+@pytest.mark.parametrize("M, Kd, N", BLOCK)
+@pytest.mark.parametrize("slices", [False, True])
+def test_tiles_of_both_operands_through_lds(kind, M, Kd, N, slices):
+    from poptransformer_amd import kernels as K
+    x, w = operands(M, Kd, N, 3)
+    x = x.half()
+    tw, plain = weight_of(kind, w)
+    out = torch.full((M, N), float("nan"), dtype=torch.float16, device="cuda")
+    K.linear(x, [tw], [out], workspace=K.linear_workspace(M, N, "cuda") if slices else None)
+    assert K.linear_kernel() == "gemm_block_kernel"
+    close(out, x.double() @ plain.T, x.double().abs() @ plain.abs().T, Kd, 11)
+
+
+def test_slices_of_k_of_tiles_through_lds():
+    """More slices than steps would have work for, and slices whose last one is short: the fp32 parts are added and the epilogue applied."""
+    from poptransformer_amd import kernels as K
+    for kind, M, Kd, N in (("f16", 1000, 4104, 1032), ("f8", 1000, 6152, 1500), ("f16", 513, 2056, 2056), ("f8", 900, 13704, 1301)):
+        x, w = operands(M, Kd, N, 23)
+        x = x.half()
+        tw, plain = weight_of(kind, w)
+        workspace = K.linear_workspace(M, N, "cuda")
+        workspace.fill_(0xFF)
+        bias, res = torch.randn(N, device="cuda").half(), torch.randn((M, N), device="cuda").half()
+        out = res.clone()
+        K.linear(x, [tw], [out], bias=bias, residual=out, workspace=workspace)
+        assert K.linear_kernel() == "gemm_block_kernel"
+        assert not torch.equal(workspace, torch.full_like(workspace, 0xFF))
+        ref, mag = x.double() @ plain.T, x.double().abs() @ plain.abs().T
+        # three roundings: the sum, with the bias, with the residual
+        bound = 2.0 ** -11 * 1.001 * (ref.abs() + (ref + bias.double()).abs() + (ref + bias.double() + res.double()).abs()) + (Kd + 2) * 2.0 ** -24 * mag * 1.01 + 2.0 ** -22
+        assert ((out.double() - ref - bias.double() - res.double()).abs() <= bound).all()
+
+
+@pytest.mark.parametrize("kind", ["f16", "f8"])
+@pytest.mark.parametrize("own_inputs", [False, True])
+@pytest.mark.parametrize("M, Kd", [(1000, 200), (300, 24)])
+def test_several_matrices_through_lds(kind, own_inputs, M, Kd):
+    from poptransformer_amd import kernels as K
+    sizes = (40, 256, 270, 8200)
+    xs, tws, plains, biases, outs = [], [], [], [], []
+    for i, n in enumerate(sizes):
+        x, w = operands(M, Kd, n, 10 + i)
+        tw, plain = weight_of(kind, w)
+        xs.append(x.half()), tws.append(tw), plains.append(plain)
+        biases.append(torch.randn(n, device="cuda").half())
+        outs.append(torch.empty((M, n), dtype=torch.float16, device="cuda"))
+    if own_inputs:
+        K.linear(None, tws, outs, biases=biases, xs=xs)
+    else:
+        xs = xs[:1] * len(sizes)
+        K.linear(xs[0], tws, outs, biases=biases)
+    assert K.linear_kernel() == "gemm_block_kernel"
+    for x, out, plain, b in zip(xs, outs, plains, biases):
+        ref, mag = x.double() @ plain.T, x.double().abs() @ plain.abs().T
+        # the sum is rounded, then its sum with the bias
+        bound = 2.0 ** -11 * (ref.abs() + (ref + b.double()).abs()) * 1.001 + (Kd + 2) * 2.0 ** -24 * mag + 2.0 ** -23
+        assert ((out.double() - ref - b.double()).abs() <= bound).all()
+
+
+@pytest.mark.parametrize("kind", ["f16", "f8"])
+@pytest.mark.parametrize("M, Kd", [(1000, 24), (999, 104), (259, 1032)])
+def test_tiles_through_lds_read_nothing_past_the_rows_and_features(kind, M, Kd):
+    """NaN around the rows of X: the rows that the last tile misses, and (the next row's) what lies behind a row's last feature."""
+    from poptransformer_amd import kernels as K
+    N = 8200
+    store = torch.full((M + 300, Kd), float("nan"), dtype=torch.float16, device="cuda")
+    x, w = operands(M, Kd, N, 17)
+    x[::2] = x[::2].abs()
+    store[:M] = x.half()
+    store[M // 2] = float("nan")
+    tw, plain = weight_of(kind, w)
+    out = torch.empty((M, N), dtype=torch.float16, device="cuda")
+    K.linear(store[:M], [tw], [out])
+    assert K.linear_kernel() == "gemm_block_kernel"
+    assert torch.isnan(out[M // 2]).all()
+    rows = torch.arange(M, device="cuda") != M // 2
+    close(out[rows], x[rows].half().double() @ plain.T, x[rows].half().double().abs() @ plain.abs().T, Kd, 11)
+
+
+@pytest.mark.parametrize("kind, M, Kd, N, kernel", [
+    ("f16", 129, 2048, 5632, "block"), ("f16", 160, 2048, 5632, "block"), ("f16", 200, 2056, 5632, "rows"), ("f16", 256, 2048, 2048, "rows"), ("f16", 255, 2120, 5632, "rows"),
+    ("f16", 320, 2048, 3072, "rows"), ("f16", 400, 2048, 4096, "block"), ("f16", 512, 2048, 4096, "rows"), ("f16", 512, 2048, 4160, "block"), ("f16", 512, 520, 4100, "block"),
+    ("f16", 1000, 2048, 2048, "block"), ("f8", 256, 2048, 5632, "block"),
+    ("f8", 515, 1032, 4104, "block"), ("f8", 130, 72, 8200, "block"), ("f16", 2048, 24, 1000, "block")])
+def test_which_kernel_pairs_take(kind, M, Kd, N, kernel):
+    from poptransformer_amd import kernels as K
+    x, w = operands(M, Kd, 2 * N, 7)
+    x = (x * 0.02 if kind == "f8" else x).half()              # (as in test_pair)
+    (g, gp), (u, up) = weight_of(kind, w[:N].contiguous()), weight_of(kind, w[N:].contiguous())
+    out = torch.empty((M, N), dtype=torch.float16, device="cuda")
+    K.linear(x, [g, u], [out, out], swiglu=True)
+    assert K.linear_kernel() == f"gemm_{kernel}_kernel"
+    gate, upv = x.double() @ gp.T, x.double() @ up.T
+    ref = torch.nn.functional.silu(gate) * upv
+    mag_g, mag_u = x.double().abs() @ gp.abs().T, x.double().abs() @ up.abs().T
+    dg, du = 2.0 ** -11 * gate.abs() + (Kd + 2) * 2.0 ** -24 * mag_g, 2.0 ** -11 * upv.abs() + (Kd + 2) * 2.0 ** -24 * mag_u
+    bound = 1.1 * dg * (upv.abs() + du) + du * torch.nn.functional.silu(gate).abs() + 2.5 * 2.0 ** -11 * ref.abs() + 2.0 ** -20 * (1 + upv.abs())
+    assert ((out.double() - ref).abs() <= bound).all()
+
+
+@pytest.mark.parametrize("M, Kd, main, tail, kernel", [
+    (129, 72, 16005, 5, "block"), (257, 1000, 10990, 18, "block"), (1100, 264, 3000, 0, "block"), (300, 2048, 8200, 0, "block"), (400, 2056, 6144, 0, "block"), (1000, 40, 3200, 3, "block"),
+    # short K, and one round of workgroups with whole blocks of rows
+    (512, 512, 4096, 0, "rows"), (129, 1024, 6016, 128, "rows"), (512, 2048, 6140, 4, "rows"), (1000, 1000, 4096, 0, "block"), (768, 1032, 1024, 0, "block")])
+@pytest.mark.parametrize("slices", [False, True])
+def test_which_kernel_wide_products_take(M, Kd, main, tail, kernel, slices):
+    from poptransformer_amd import hybrid_kernels as HK
+    x, w = operands(M, Kd, main + tail, 11)
+    x, w = x.to(torch.bfloat16), w.to(torch.bfloat16)
+    W = HK.WideWeight(w, torch.bfloat16, tail=tail)
+    out = torch.full((M, main), float("nan"), device="cuda")
+    t = torch.full((M * max(tail, 1),), float("nan"), device="cuda")
+    HK.linear(x, W, out, M, ld=main, tail=t if tail else None, workspace=HK.linear_workspace(M, W.N, "cuda") if slices else None)
+    assert HK.linear_kernel() == f"gemm_{kernel}_kernel"
+    ref, mag = x.double() @ w.double().T, x.double().abs() @ w.double().abs().T
+    close(out, ref[:, :main], mag[:, :main], Kd, 24)
+    if tail:
+        close(t[:M * tail].view(M, tail), ref[:, main:], mag[:, main:], Kd, 24)
+
+
+@pytest.mark.parametrize("M, Kd, N, kernel", [(256, 1024, 4096, "rows"), (129, 512, 7168, "rows"), (160, 2048, 5632, "rows"), (129, 2048, 5632, "block"), (160, 4096, 4096, "block"), (256, 4104, 4096, "rows"), (515, 136, 4100, "block")])
+def test_which_kernel_wide_pairs_take(M, Kd, N, kernel):
+    from poptransformer_amd import hybrid_kernels as HK
+    x, w = operands(M, Kd, 2 * N, 29)
+    x, w = (x * 0.1).to(torch.bfloat16), w.to(torch.bfloat16)
+    g, u = (HK.WideWeight(t.contiguous(), torch.bfloat16) for t in (w[:N], w[N:]))
+    out = torch.full((M, HK.pad8(N)), float("nan"), dtype=torch.bfloat16, device="cuda")
+    HK.linear(x, g, out, M, ld=HK.pad8(N), up=u, pair=1)
+    assert HK.linear_kernel() == f"gemm_{kernel}_kernel"
+    xd, gd, ud = x.double(), w[:N].double(), w[N:].double()
+    gate, upv = xd @ gd.T, xd @ ud.T
+    ref = torch.nn.functional.silu(gate) * upv
+    dg, du = (Kd + 2) * 2.0 ** -24 * (xd.abs() @ gd.abs().T), (Kd + 2) * 2.0 ** -24 * (xd.abs() @ ud.abs().T)
+    # the sums' errors, the exponential and the quotient in fp32, one rounding to bf16
+    bound = 1.1 * dg * (upv.abs() + du) + du * torch.nn.functional.silu(gate).abs() + (2.0 ** -8 + 2.0 ** -20) * ref.abs() + 2.0 ** -24
+    assert ((out[:, :N].double() - ref).abs() <= bound).all()
