@@ -2717,10 +2717,12 @@ static int dispatch_many_rows(const GemmArgs& a, int total_nb, hipStream_t s, co
   // fp16 44 against 47), of INT4 weights three (their pair of 11008 channels 41.5 against 48.0), and small launches (768 x 3072,
   // 512 rows, INT4 16.0 against 25.1); beyond, these lose: 4096 x 11008, 160 rows, INT4 42.8 against 39.8, fp16 60 against 44.  The plan's
   // time does not see what a round's begin and end take, so with short K the rounds are counted too: INT4 768 x 32000, 65 rows, four rounds
-  // 26.8 against 21.3; pair 768 x 11008, three, 17.7 against 13.7; 512 x 4096, 1000 rows, four, 1.14 times; 1024 x 6144, 768 rows, five, 1.10.
+  // 26.8 against 21.3; pair 768 x 11008, three, 17.7 against 13.7; bf16 256 x 11008, 65 rows, two, 1.14 times; 512 x 4096, 1000 rows, four,
+  // 1.14 times; 1024 x 6144, 768 rows, five, 1.10.  And 16-bit weights of long K, two rounds: 8192 x 8192, 65 to 128 rows, 1.08 to 1.18 times,
+  // 11008 x 8192 1.2 to 1.34 (4096 x 8192 0.83 to 0.97).
   if (a.epi.norm == PTA_NORM_NONE) {
     const OwnPlan plan = plan_gemm_own<Fmt, PAIR>(a);
-    const int most = a.M <= 128 ? (Fmt::kVec == 1 && a.KT >= 12 ? 3 : 2) : a.KT >= 8 || PAIR ? 4 : 3;
+    const int most = a.M <= 128 ? ((Fmt::kWide && a.KT <= 2) || (Fmt::kVec > 2 && a.KT >= 56) ? 1 : Fmt::kVec == 1 && a.KT >= 12 ? 3 : 2) : a.KT >= 8 || PAIR ? 4 : 3;
     if (plan.rounds == 1 || (plan.rounds <= most && (a.M <= 128 || plan.us <= (Fmt::kVec == 1 ? 22.0 : 11.0))))
       return launch_gemm_own_plan<Fmt, PAIR>(a, plan, s, name);
   }

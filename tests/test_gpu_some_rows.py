@@ -221,13 +221,16 @@ def product(kind, M, Kd, N, pair):
     ("f152", 64, 2048, 5632, True, "gemm_tile"), ("f152", 33, 1024, 5632, True, "gemm_tile"), ("f152", 40, 4096, 5632, True, "gemm_own"),
     # rounds of gemm_own_kernel beyond 64 rows
     ("int4", 65, 768, 11008, True, "gemm_rows"), ("int4", 128, 1024, 32000, False, "gemm_rows"), ("int4", 128, 2048, 5632, True, "gemm_own"),
+    ("f16", 65, 8192, 8192, False, "gemm_rows"), ("f16", 65, 6144, 8192, False, "gemm_own"), ("f16", 128, 8192, 4096, False, "gemm_own"), ("f8", 100, 8192, 8192, False, "gemm_own"),
+    ("int4", 65, 256, 11008, False, "gemm_own"),
     ("int4", 1000, 512, 4096, False, "gemm_panel"), ("int4", 700, 512, 4096, False, "gemm_own"), ("int4", 768, 1024, 6144, False, "gemm_panel")])
 def test_which_kernel_more_rows_take(kind, M, Kd, N, pair, kernel):
     assert product(kind, M, Kd, N, pair) == kernel + "_kernel"
 
 
 @pytest.mark.parametrize("M, Kd, N, pair, kernel", [(33, 256, 250, False, "gemv_mfma"), (64, 72, 1000, False, "gemv_mfma"), (40, 768, 5632, True, "gemv_mfma"),
-                                                    (24, 520, 5632, True, "gemv_mfma"), (33, 520, 250, False, "gemm_own")])
+                                                    (24, 520, 5632, True, "gemv_mfma"), (33, 520, 250, False, "gemm_own"), (65, 256, 11008, False, "gemm_rows"),
+                                                    (65, 384, 11008, False, "gemm_own")])
 def test_which_kernel_more_rows_of_bf16_take(M, Kd, N, pair, kernel):
     from poptransformer_amd import hybrid_kernels as HK
     x, w = operands(M, Kd, N, 11)
