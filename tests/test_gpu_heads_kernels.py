@@ -326,6 +326,37 @@ def test_lists_of_the_experts_rows(tile):
             assert np.array_equal(mine[:, 1], begin[e] + tile * np.arange(len(mine)))
 
 
+@pytest.mark.parametrize("tile", [128, 256])
+def test_experts_whose_rows_take_more_than_2_gib(tile):
+    """The down product of 8 experts of 65544 features for 2049 rows: the rows of its input take 2^31 bytes and more, which 32-bit offsets do
+    not reach (gemm_rows_kernel; with 65528 features gemm_block_kernel).  64 features of a row are +-1: the sums are whole numbers."""
+    HK, T = _hk()
+    rows, experts, d = 2049, 8, 48
+    for ff, kernel in ((65544, "gemm_rows_kernel"), (65496, "gemm_block_kernel")):
+        assert (rows * experts * ff * 2 > 2 ** 31 - 1) == (kernel == "gemm_rows_kernel")
+        rng = np.random.default_rng(ff)
+        r = HK.Routing(rows, experts, experts, False, 1.0, "cuda")
+        chosen = _choices(rng, rows, experts, experts, "")
+        r.chosen[:, :experts] = _dev(chosen, torch.int32)
+        lists = HK.expert_lists(rows, experts, experts, tile, "cuda")
+        HK.group_experts(r, rows, tile, lists)
+        w = [torch.from_numpy(rng.integers(-3, 4, size=(d, ff)).astype(np.float32)).to("cuda") for _ in range(experts)]
+        at = torch.from_numpy(rng.integers(0, ff // 64, size=(rows * experts, 64)) + np.arange(64) * (ff // 64)).to("cuda")     # (64 different ones)
+        x = torch.zeros((rows * experts, ff), dtype=torch.bfloat16, device="cuda")
+        sign = torch.from_numpy(rng.integers(0, 2, size=at.shape) * 2 - 1).to("cuda")
+        x.scatter_(1, at, sign.to(torch.bfloat16))
+        out = torch.full((rows * experts, d), float("nan"), dtype=torch.float32, device="cuda")
+        HK.experts(x, r, rows, dict(w=HK.ExpertWeight(w, T["bfloat16"])), out, lists=lists, tile_rows=tile)
+        assert HK.linear_kernel() == kernel
+        which = r.chosen[:, :experts].reshape(-1)
+        want = torch.empty_like(out)
+        for e in range(experts):
+            mine = torch.nonzero(which == e)[:, 0]
+            want[mine] = (w[e].T[at[mine]] * sign[mine].unsqueeze(2)).sum(1)
+        assert torch.equal(out, want)
+        del x, at, sign
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("rows", [1, 2, 7, 16, 17, 130, 600])
 def test_experts(dtype, rows):
