@@ -1,3 +1,8 @@
+    """More than 64 rows, with and without the K split that a workspace allows.  Small launches (all of up to 256 rows here, and 100
+    channels) go to the kernel whose waves have feature tiles of their own, the larger ones to the one that takes 128-row panels through
+    LDS and the weights straight into registers; 1160 features = a ragged last tile; 200 and 600 rows = a ragged last row block.  (The
+    other kernels for so many rows: tests/test_gpu_many_rows.py.)  Bias and a residual that aliases the output; the residual alone (the
+    epilogue that moves whole vectors)."""
 """Parity of each HIP kernel, called through the C ABI, against the numpy oracle."""
 import numpy as np
 import pytest
@@ -1441,8 +1446,8 @@ def test_w4a16_gemm_up_to_256_rows(K, M, Kdim, N):
 
 
 def test_w4a16_gemm_most_rows_few_channels_exact_integers(K):
-    """4096 rows (the most a launch takes) and 256 channels: a workgroup of the panel kernel in which half the waves
-    have no channel blocks and only help to bring the rows in; 3000 rows = a ragged last panel."""
+    """4096 rows (the most a launch takes) and 256 channels: 64 row blocks of few workgroups each; 3000 rows = a ragged last one.  (Panels
+    in which half the waves have no channel blocks: tests/test_gpu_many_rows.py.)"""
     rng = np.random.default_rng(77)
     for M in (4096, 3000):
         Kdim, N = 512, 256

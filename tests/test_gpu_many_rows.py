@@ -316,3 +316,72 @@ def test_which_kernel_wide_pairs_take(M, Kd, N, kernel):
     # the sums' errors, the exponential and the quotient in fp32, one rounding to bf16
     bound = 1.1 * dg * (upv.abs() + du) + du * torch.nn.functional.silu(gate).abs() + (2.0 ** -8 + 2.0 ** -20) * ref.abs() + 2.0 ** -24
     assert ((out[:, :N].double() - ref).abs() <= bound).all()
+
+
+def int4_weight(Kd, N, seed):
+    from poptransformer_amd import kernels as K
+    g = torch.Generator(device="cuda").manual_seed(seed)
+    packed = torch.randint(-128, 128, (N, Kd // 2), generator=g, device="cuda", dtype=torch.int8)
+    scale = (torch.rand(N, generator=g, device="cuda") * 0.01 + 0.002).half()
+    return K.W4Weight(packed, scale), K.int4_to_half(packed, scale).double().T.contiguous()
+
+
+@pytest.mark.parametrize("kind, M, Kd, N, kernel", [
+    # registers for the rows, up to 128 of them: more rounds of gemm_own_kernel than it takes; K in slices (16-bit, few groups of channels)
+    ("int4", 100, 1032, 32000, "gemm_rows_kernel"), ("int4", 128, 520, 32000, "gemm_rows_kernel"), ("int4", 65, 4096, 50304, "gemm_rows_kernel"),
+    ("f16", 100, 8200, 8192, "gemm_rows_kernel"), ("f16", 128, 13704, 7168, "gemm_rows_kernel"), ("f8", 70, 1032, 40960, "gemm_rows_kernel"), ("f152", 128, 2056, 14336, "gemm_rows_kernel"),
+    # panels of 128 rows: units of 64 channels that are no multiple of a workgroup's eight, or four with K in halves, so that waves have none
+    ("int4", 1000, 1032, 8384, "gemm_panel_kernel"), ("int4", 1000, 2056, 6464, "gemm_panel_kernel"), ("int4", 4096, 4096, 320, "gemm_panel_kernel"), ("int4", 3000, 8200, 448, "gemm_panel_kernel"),
+    ("int4", 1025, 4104, 2112, "gemm_panel_kernel"), ("f152", 600, 2056, 4160, "gemm_panel_kernel"),
+    # blocks that do not divide: 64 rows in turn, the last eight
+    ("int4", 200, 1032, 32008, "gemv_"), ("f152", 136, 520, 32040, "gemv_")])
+@pytest.mark.parametrize("slices", [False, True])
+def test_kernels_of_many_rounds(kind, M, Kd, N, kernel, slices):
+    from poptransformer_amd import kernels as K
+    x, w = operands(M, Kd, 8 if kind == "int4" else N, 31)
+    x = x.half()
+    if kind == "int4":
+        tw, plain = int4_weight(Kd, N, 33)
+    elif kind == "f152":
+        scale = torch.tensor([-1], dtype=torch.int32, device="cuda")
+        codes = K.half_to_fp8(w.half(), scale, "F152")
+        tw, plain = K.F8Weight(codes, scale, "F152"), K.fp8_to_half(codes, scale, "F152").double()
+    else:
+        tw, plain = weight_of(kind, w)
+    workspace = K.linear_workspace(M, N, "cuda") if slices else None
+    out = torch.full((M, N), float("nan"), dtype=torch.float16, device="cuda")
+    K.linear(x, [tw], [out], workspace=workspace)
+    assert K.linear_kernel().startswith(kernel), K.linear_kernel()
+    ref, mag = x.double() @ plain.T, x.double().abs() @ plain.abs().T
+    close(out, ref, mag, Kd, 11)
+    # in place on the residual, behind a bias
+    bias, res = torch.randn(N, device="cuda").half(), torch.randn((M, N), device="cuda").half()
+    out = res.clone()
+    K.linear(x, [tw], [out], bias=bias, residual=out, workspace=workspace)
+    bound = 2.0 ** -11 * 1.001 * (ref.abs() + (ref + bias.double()).abs() + (ref + bias.double() + res.double()).abs()) + (Kd + 2) * 2.0 ** -24 * mag * 1.01 + 2.0 ** -22
+    assert ((out.double() - ref - bias.double() - res.double()).abs() <= bound).all()
+
+
+def test_panels_of_a_pair_and_of_several_matrices():
+    """Units of pairs and of matrices that share a workgroup with idle waves; the last round of tiles in a launch of its own."""
+    from poptransformer_amd import kernels as K
+    for M, Kd, N in ((1000, 1032, 4192), (600, 2056, 2080)):
+        x = (operands(M, Kd, 1, 35)[0] * 0.02).half()
+        (g, gp), (u, up) = int4_weight(Kd, N, 36), int4_weight(Kd, N, 37)
+        out = torch.full((M, N), float("nan"), dtype=torch.float16, device="cuda")
+        K.linear(x, [g, u], [out, out], swiglu=True)
+        assert K.linear_kernel() == "gemm_panel_kernel"
+        gate, upv = x.double() @ gp.T, x.double() @ up.T
+        silu = torch.nn.functional.silu(gate)
+        dg, du = (2.0 ** -11 * t.abs() + (Kd + 2) * 2.0 ** -24 * (x.double().abs() @ p.abs().T) for t, p in ((gate, gp), (upv, up)))
+        # as in test_pair
+        bound = 1.1 * dg * (upv.abs() + du) + du * silu.abs() + 2.5 * 2.0 ** -11 * (silu * upv).abs() + 2.0 ** -20 * (1 + upv.abs())
+        assert ((out.double() - silu * upv).abs() <= bound).all()
+    M, Kd, sizes = 900, 1032, (4160, 320, 4096, 192)
+    x = operands(M, Kd, 1, 38)[0].half()
+    ws = [int4_weight(Kd, n, 40 + i) for i, n in enumerate(sizes)]
+    outs = [torch.full((M, n), float("nan"), dtype=torch.float16, device="cuda") for n in sizes]
+    K.linear(x, [w for w, _ in ws], outs)
+    assert K.linear_kernel() == "gemm_panel_kernel"
+    for (_, p), out in zip(ws, outs):
+        close(out, x.double() @ p.T, x.double().abs() @ p.abs().T, Kd, 11)
