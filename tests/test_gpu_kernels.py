@@ -1,8 +1,3 @@
-    """More than 64 rows, with and without the K split that a workspace allows.  Small launches (all of up to 256 rows here, and 100
-    channels) go to the kernel whose waves have feature tiles of their own, the larger ones to the one that takes 128-row panels through
-    LDS and the weights straight into registers; 1160 features = a ragged last tile; 200 and 600 rows = a ragged last row block.  (The
-    other kernels for so many rows: tests/test_gpu_many_rows.py.)  Bias and a residual that aliases the output; the residual alone (the
-    epilogue that moves whole vectors)."""
 """Parity of each HIP kernel, called through the C ABI, against the numpy oracle."""
 import numpy as np
 import pytest
@@ -1421,12 +1416,11 @@ def test_fp8_products_of_many_rows_pair_multi_and_nan(K, M):
 @pytest.mark.parametrize("M", [65, 128, 200, 256, 600, 1024])
 @pytest.mark.parametrize("Kdim,N", [(4096, 4096), (1160, 8192), (11008, 4096), (512, 100)])
 def test_w4a16_gemm_up_to_256_rows(K, M, Kdim, N):
-    """More than 64 rows: up to 128 the kernel that keeps the activation fragments in registers, beyond them the
-    kernel that takes 128-row panels through LDS and the weights straight into registers;
-    with and without the K split that a workspace allows; 1160 features = a ragged last tile; 200 and 600 rows = a
-    ragged last row block, and for channel counts that do not divide into the workgroup tiles (100) the 64-row
-    paths over the rows in turn.  Bias and a residual that aliases the output; the residual alone (the epilogue
-    that moves whole vectors)."""
+    """More than 64 rows, with and without the K split that a workspace allows.  Small launches (all of up to 256 rows here, and 100
+    channels) go to the kernel whose waves have feature tiles of their own, the larger ones to the one that takes 128-row panels through
+    LDS and the weights straight into registers; 1160 features = a ragged last tile; 200 and 600 rows = a ragged last row block.  (The
+    other kernels for so many rows: tests/test_gpu_many_rows.py.)  Bias and a residual that aliases the output; the residual alone (the
+    epilogue that moves whole vectors)."""
     x, packed, scale = _w4_case(M + Kdim + N, M, Kdim, N)
     rng = np.random.default_rng(M * N)
     bias = rng.standard_normal(N).astype(np.float16)
