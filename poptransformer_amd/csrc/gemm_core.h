@@ -270,7 +270,7 @@ struct GemmArgs {
   int M, K, KT;
   GemmEpilogue epi;
   // PAIR mode (SwiGLU): mat[0] is the gate weight, mat[1] the up weight, output in mat[0].Y.
-  // K split across workgroups (gemm_own_kernel and the kernels for more rows, one matrix): slice blockIdx.y of `ksplit` writes its fp32
+  // K split across workgroups (gemm_own_kernel and the kernels for more rows, one matrix): one of `ksplit` slices (blockIdx.y; gemm_own_kernel: part of blockIdx.z) writes its fp32
   // sums to part[slice][M][N]; splitk_finish_kernel adds the slices and applies the epilogue.
   float* part;
   size_t part_bytes;
@@ -1083,10 +1083,10 @@ static int launch_gemv_stream(const GemmArgs& a, int total_nb, int cus, hipStrea
 }
 
 // ------------------------------------------------------------------------------------------
-// Variant for 16 < M <= 64 and launches of more workgroups than compute units (and pairs of up to 32 rows): the activation rows of a feature tile are staged in LDS once per
-// workgroup and shared by its waves, so that the B operands (4 KiB per 16 rows and tile, against
+// Variant for 16 < M <= 64 and launches that gemm_own_kernel's workgroups would be several rounds of (dispatch_gemv has the lines): the
+// activation rows of a feature tile are staged in LDS once per workgroup and shared by its waves, so that the B operands (4 KiB per 16 rows and tile, against
 // 1 KiB of INT4 weights) come from LDS and not from the L2.
-// A workgroup of 8 waves owns 2 * (8 / KQ) weight streams of 16 channels (consecutive channel blocks
+// A workgroup of 8 (NWV; 16 where the dispatch says so) waves owns 2 * (8 / KQ) weight streams of 16 channels (consecutive channel blocks
 // of one matrix; or, for a SwiGLU pair, the gate and the up weights of 8 / KQ channel blocks) and
 // all rows; its waves form KQ groups that take the feature tiles g, g + KQ, ... each; a wave
 // multiplies two streams, so every B fragment it reads from LDS feeds two MFMAs.  The X tiles of
@@ -1316,17 +1316,18 @@ __device__ __forceinline__ const unsigned char* uniform_pointer(const unsigned c
 }
 
 // ------------------------------------------------------------------------------------------
-// Variant for more than 8 rows and few workgroups: each wave multiplies feature tiles of its own.
+// Variant for 5 rows and more (own_takes_few_rows, dispatch_gemv, dispatch_many_rows) and few workgroups: each wave multiplies feature
+// tiles of its own.
 // A workgroup of 8 waves owns NB blocks of 16 channels (of one matrix; for a SwiGLU pair of both) and MT * 16 rows (all of up to
 // 64, else a row block); its wave w takes
-// the feature tiles w, w + 8, ... of its slice of K.  A wave's rows travel global -> registers -> LDS -> registers: the loads take
+// the feature tiles w, w + 8, ... of its slice of K.  A wave's rows are loaded straight into LDS: the loads take
 // 256 bytes of 4 rows each (in the matrix unit's operand order, 64 bytes of 16 rows, the same bytes take twice as long), the LDS
-// area belongs to the wave alone and turns them into operands, so that nothing in the loop waits for another wave, and the rows
+// area belongs to the wave alone and is read in operand order, so that nothing in the loop waits for another wave, and the rows
 // and weights of the next tile are in flight (16 KiB and NB KiB a wave at 64 rows) while one is multiplied.  The waves' sums meet
 // in LDS at the end.
 // What bounds it is the rows: every workgroup reads all of them, and a compute unit gets 112 GB/s out of its L2 when all read
 // (4.6 us for 64 rows of 4096 features).  Parts of a launch of 64 rows, 4096 x 11008 INT4 (15.5 us before the end's arguments were
-// read ahead, 14.2 with it): 3 us an empty one, 4.1 the rows, 2 the weights, 1 products and decoding, 2 to 3 the end.
+// read ahead, 14.2 with it, weights from the last cache; 15.5 from HBM): 3 us an empty one, 4.1 the rows, 2 the weights, 1 products and decoding, 2 to 3 the end.
 // Before (gemm_tile_kernel, whose waves wait for one another at every step): 21.8 us.  16 requests in flight a wave are enough;
 // twice as many at 32 rows were slower by 0.6 us.
 // ------------------------------------------------------------------------------------------
@@ -2381,7 +2382,7 @@ __global__ __launch_bounds__(BLOCK_WAVES * 64) __attribute__((amdgpu_waves_per_e
   for (int n = 0; n < NS; ++n)
 #pragma unroll
     for (int q = 0; q < LOADS; ++q) bring(first * (64 / SF) + n, n * STAGE, q);
-  // (the wide epilogue's many arguments, read while the first stages are on their way: 1024 x 4096, 512 rows, bf16 22.7 -> 19.0 us; the
+  // (the wide epilogue's many arguments, read while the first stages are on their way: bf16, 1024 x 8192, 1000 rows 29.5 -> 28.1 us; 2048 x 8192 46.9 -> 45.4; the
   // fp16 one's few gain nothing)
   GemmMat wide;
   GemmEpilogue none{};
@@ -2648,7 +2649,7 @@ template <class Fmt, int MT, bool PAIR>
 static void launch_gemv(const GemmArgs& a, int total_nb, hipStream_t s) {
   // Waves per block: enough to split K finely when there are few channel blocks, fewer when
   // the grid alone already fills the machine.  The LDS reduction buffer caps the wide cases.
-  // (more than 16 rows of 16 feature tiles and more: F152 weights only)
+  // (more than 16 rows in 16 waves: F152 weights only, which go to gemm_own_kernel later than the others)
   constexpr bool FINE = !PAIR && (MT == 1 || (MT == 2 && OwnStreams<Fmt>::long_decode));
   gemm_kernel_taken = "gemv_mfma_kernel";
   if constexpr (FINE) {
@@ -2883,8 +2884,9 @@ static int dispatch_gemv(const GemmArgs& a, int total_nb, hipStream_t s, const c
         // What bounds these launches is the bytes through the busiest compute unit: a workgroup reads all rows of X
         // beside its weights.  More workgroups than compute units (20480 channels: 320 of 64 channels): workgroups
         // of 16 waves and 128 channels where their rounds come out shorter - 160 of 768 KiB against two rounds of
-        // 640 at 64 rows.  Measured, 4096 x 20480: 26.0 against 40.7 us at 64 rows, 24.7 against 38.2 at 48, 18.8
-        // against 20.8 at 32.
+        // 640 at 64 rows.  INT4, weights from HBM: 4096 x 20480, 64 rows 28.0 against 41.9 us, 48 rows 26.6 against 40.3; 4096 x
+        // 32000, 64 rows 32.0 against 44.9, 32 rows 23.3 against 24.3, 17 rows 21.8 against 22.4; F143, 4096 x 20480, 32 rows 27.5
+        // against 28.4.
         bool wide = false;
         if constexpr (!PAIR && Fmt::kVec <= 2) {
           // (beyond 32 rows with INT4 weights only: with two vectors per tile the 16 waves' registers do not hold it)
