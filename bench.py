@@ -778,9 +778,7 @@ def main():
         launches = reps * len(weights.blocks)
         kernel_s = e0.elapsed_time(e1) * 1e-3 / launches
         kernel_bytes = 2 * (d * f // 2 + 2 * f) + B * d * 2 + B * f * 2
-        kernel_name = ("gemv_lds_kernel<FmtW4, 8, true>" if B <= 4 else
-                       "gemv_wide_kernel<FmtW4, 3, true>" if B <= 16 else "gemv_mfma_kernel<FmtW4, MT, 8, true>") + \
-            " (INT4 gate/up + SwiGLU)"
+        kernel_name = f"{K.linear_kernel()} (INT4 gate/up + SwiGLU)"
     achieved = kernel_bytes / kernel_s / 1e9
 
     out = {
