@@ -134,8 +134,8 @@ def test_persistent_step_at_7b_width_matches_oracle(wide, B, plen):
 
 @pytest.mark.timeout(600)
 def test_per_operator_path_at_7b_width_batch_16_matches_oracle(wide):
-    """Batch 16 on the per-operator path: gemv_wide_kernel with three channel blocks per workgroup (q/k/v in one
-    launch, gate/up + SwiGLU, and the lm_head), one attention workgroup per (sequence, head)."""
+    """Batch 16 on the per-operator path: one round of gemm_own_kernel's workgroups (q/k/v in one launch, gate/up +
+    SwiGLU), gemv_stream_kernel (the lm_head), one attention workgroup per (sequence, head)."""
     from poptransformer_amd.engine import fused, loader
     B, L, pad, eos, plen = 16, 48, 0, 2, 8
     steps = plen - 1 + 32
