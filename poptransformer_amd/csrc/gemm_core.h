@@ -630,7 +630,7 @@ __global__ __launch_bounds__(NW * 64) void gemv_lds_kernel(GemmArgs a) {
 }
 
 // ------------------------------------------------------------------------------------------
-// Variant for 4 < M <= 16 when all matrices of the launch share X: one workgroup of 16 waves per
+// Variant for 4 < M <= 16 (F152 weights: up to 32) when all matrices of the launch share X: one workgroup of 16 waves per
 // compute unit's worth of work.  A workgroup owns NB 16-channel blocks (blocks g, g + G, ... of
 // the launch's G workgroups); wave w takes the feature tiles w, w + 16, ... of ALL of them, so the
 // activation fragments of a tile (the B operands: 4 KiB per 16 rows, against 1 KiB of INT4
@@ -639,12 +639,13 @@ __global__ __launch_bounds__(NW * 64) void gemv_lds_kernel(GemmArgs a) {
 // ------------------------------------------------------------------------------------------
 constexpr int WIDE_WAVES = 16;
 
-template <class Fmt, int NB, bool PAIR, bool NORM = false>
+template <class Fmt, int MT, int NB, bool PAIR, bool NORM = false>
 __global__ __launch_bounds__(WIDE_WAVES * 64) void gemv_wide_kernel(GemmArgs a, int total_nb) {
+  static_assert(!NORM || MT == 1, "the fused norm covers up to 16 rows");
   constexpr int NACC = PAIR ? 2 : 1;
   constexpr int KV = Fmt::kVec;
   extern __shared__ __align__(16) unsigned char smem[];
-  float* red = reinterpret_cast<float*>(smem);          // [WIDE_WAVES][NB][NACC][256]
+  float* red = reinterpret_cast<float*>(smem);          // [WIDE_WAVES][NB][NACC][MT][256]
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int G = gridDim.x;
   const int K = a.K, KT = a.KT;
@@ -672,15 +673,21 @@ __global__ __launch_bounds__(WIDE_WAVES * 64) void gemv_wide_kernel(GemmArgs a, 
       wp[b][g] = reinterpret_cast<const u32x4*>(m.tiled) + (size_t)nb[b] * KT * (64 * KV) + lane;
     }
   }
-  int row = lane & 15;
-  row = row < a.M ? row : a.M - 1;                      // padding rows compute values that are never stored
-  const f16* xrow = a.X + (size_t)row * K + (lane >> 4) * 8;
+  const f16* xrow[MT];
+#pragma unroll
+  for (int mt = 0; mt < MT; ++mt) {
+    int row = mt * 16 + (lane & 15);
+    row = row < a.M ? row : a.M - 1;                    // padding rows compute values that are never stored
+    xrow[mt] = a.X + (size_t)row * K + (lane >> 4) * 8;
+  }
 
-  f32x4 acc[NB][NACC];
+  f32x4 acc[NB][NACC][MT];
 #pragma unroll
   for (int b = 0; b < NB; ++b)
 #pragma unroll
-    for (int g = 0; g < NACC; ++g) acc[b][g] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int g = 0; g < NACC; ++g)
+#pragma unroll
+      for (int mt = 0; mt < MT; ++mt) acc[b][g][mt] = f32x4{0.f, 0.f, 0.f, 0.f};
 
   // Fused norm: a first pass over this wave's activation fragments gives the row sums (lane l
   // holds row l % 16, features (l / 16) * 8 + 0..7 of every 32), they meet over the lane groups and, in
@@ -694,7 +701,7 @@ __global__ __launch_bounds__(WIDE_WAVES * 64) void gemv_wide_kernel(GemmArgs a, 
       for (int j = 0; j < 4; ++j) {
         const int k = kt * 128 + j * 32;
         if (k + (lane >> 4) * 8 < K) {
-          const f16x8 v = *reinterpret_cast<const f16x8*>(xrow + k);
+          const f16x8 v = *reinterpret_cast<const f16x8*>(xrow[0] + k);
 #pragma unroll
           for (int e = 0; e < 8; ++e) { const float f = (float)v[e]; s1 += f; s2 = __builtin_fmaf(f, f, s2); }
         }
@@ -749,7 +756,7 @@ __global__ __launch_bounds__(WIDE_WAVES * 64) void gemv_wide_kernel(GemmArgs a, 
         const int k = kt * 128 + j * 32;
         const f16x8 z = {0, 0, 0, 0, 0, 0, 0, 0};
         const bool in = there && k + (lane >> 4) * 8 < K;
-        xb[u][j] = in ? *reinterpret_cast<const f16x8*>(xrow + k) : z;
+        xb[u][j] = in ? *reinterpret_cast<const f16x8*>(xrow[0] + k) : z;
         if (NORM && in) {
           const f16x8 gm = *reinterpret_cast<const f16x8*>(a.epi.norm_weight + k + (lane >> 4) * 8);
           if (a.epi.norm == PTA_NORM_RMS) {
@@ -773,8 +780,8 @@ __global__ __launch_bounds__(WIDE_WAVES * 64) void gemv_wide_kernel(GemmArgs a, 
         for (int b = 0; b < NB; ++b)
 #pragma unroll
           for (int g = 0; g < NACC; ++g)
-            acc[b][g] = Fmt::mma(Fmt::a_operand(w[u][b][g], j, sc[b][g]), xb[u][j],
-                                                                  acc[b][g]);
+            acc[b][g][0] = Fmt::mma(Fmt::a_operand(w[u][b][g], j, sc[b][g]), xb[u][j],
+                                                                     acc[b][g][0]);
   };
   int kt0 = wave;
   if constexpr (NORM) {
@@ -791,37 +798,68 @@ __global__ __launch_bounds__(WIDE_WAVES * 64) void gemv_wide_kernel(GemmArgs a, 
       kt0 += WIDE_WAVES * UN;
     }
   }
-  for (; kt0 < KT; kt0 += WIDE_WAVES * UN) {
-    load_w(kt0);
-    load_x(kt0);
-    products();
+  if constexpr (MT == 1) {
+    for (; kt0 < KT; kt0 += WIDE_WAVES * UN) {
+      load_w(kt0);
+      load_x(kt0);
+      products();
+    }
+  } else {
+    // several row groups: the activations of 32 features at a time, each used for all blocks; a weight operand is decoded once for all rows
+    for (; kt0 < KT; kt0 += WIDE_WAVES) {
+      u32x4 wt[NB][NACC][KV];
+#pragma unroll
+      for (int b = 0; b < NB; ++b)
+#pragma unroll
+        for (int g = 0; g < NACC; ++g)
+#pragma unroll
+          for (int v = 0; v < KV; ++v) wt[b][g][v] = __builtin_nontemporal_load(wp[b][g] + ((size_t)kt0 * KV + v) * 64);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const int k = kt0 * 128 + j * 32;
+        f16x8 xs[MT];
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt) xs[mt] = k + (lane >> 4) * 8 < K ? *reinterpret_cast<const f16x8*>(xrow[mt] + k) : f16x8{};
+#pragma unroll
+        for (int b = 0; b < NB; ++b)
+#pragma unroll
+          for (int g = 0; g < NACC; ++g) {
+            const f16x8 av = Fmt::a_operand(wt[b][g], j, sc[b][g]);
+#pragma unroll
+            for (int mt = 0; mt < MT; ++mt) acc[b][g][mt] = Fmt::mma(av, xs[mt], acc[b][g][mt]);
+          }
+      }
+    }
   }
 
-  // The accumulator of lane l holds channels (l/16)*4 + r, r = 0..3, for activation row l%16.
+  // The accumulator of lane l holds channels (l/16)*4 + r, r = 0..3, for activation row l%16 of its group.
 #pragma unroll
   for (int b = 0; b < NB; ++b)
 #pragma unroll
     for (int g = 0; g < NACC; ++g)
 #pragma unroll
-      for (int r = 0; r < 4; ++r) red[(((wave * NB + b) * NACC + g) * 4 + r) * 64 + lane] = acc[b][g][r];
+      for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) red[((((wave * NB + b) * NACC + g) * MT + mt) * 4 + r) * 64 + lane] = acc[b][g][mt][r];
   __syncthreads();
-  // The 256 outputs (16 rows x 16 channels) of block b are finished by quarter b of the workgroup, thread t of it taking row
-  // (t / 16) % 16, channel t % 16.
+  // The 256 outputs (16 rows x 16 channels) of row group mt of block b are finished by quarter (b * MT + mt) % 4 of the workgroup,
+  // thread t of it taking row (t / 16) % 16, channel t % 16.
   const int quarter = threadIdx.x >> 8;
 #pragma unroll
-  for (int b = 0; b < NB; ++b) {
-    if (b != quarter) continue;
-    const int nn = threadIdx.x & 15, m = (threadIdx.x >> 4) & 15;
+  for (int i = 0; i < NB * MT; ++i) {
+    if ((i & 3) != quarter) continue;
+    const int b = i / MT, mt = i % MT;
+    const int nn = threadIdx.x & 15, m = mt * 16 + ((threadIdx.x >> 4) & 15);
     const GemmMat& mat = a.mat[PAIR ? 0 : mi[b]];
     const int N = mat.N, n = nb[b] * 16 + nn;
     if ((int)blockIdx.x + b * G >= total_nb || m >= a.M || n >= N) continue;
-    const int r = nn & 3, ln = (nn >> 2) * 16 + m;
+    const int r = nn & 3, ln = (nn >> 2) * 16 + (m & 15);
     float sum[NACC];
 #pragma unroll
     for (int g = 0; g < NACC; ++g) {
       float t = 0.f;
 #pragma unroll
-      for (int w = 0; w < WIDE_WAVES; ++w) t += red[(((w * NB + b) * NACC + g) * 4 + r) * 64 + ln];
+      for (int w = 0; w < WIDE_WAVES; ++w) t += red[((((w * NB + b) * NACC + g) * MT + mt) * 4 + r) * 64 + ln];
       sum[g] = Fmt::finish(t, sc[b][g]);      // no format's finish uses the per-channel part of the scale
     }
     if (PAIR) gemm_put_pair<Fmt>(a.epi, mat, m, n, N, sum[0], sum[NACC - 1]);
@@ -829,18 +867,18 @@ __global__ __launch_bounds__(WIDE_WAVES * 64) void gemv_wide_kernel(GemmArgs a, 
   }
 }
 
-template <class Fmt, int NB, bool PAIR, bool NORM>
+template <class Fmt, int MT, int NB, bool PAIR, bool NORM>
 static int launch_gemv_wide(const GemmArgs& a, int total_nb, hipStream_t s, const char* name) {
   static bool ready = false;
-  const size_t smem = (size_t)WIDE_WAVES * NB * (PAIR ? 2 : 1) * 256 * sizeof(float);
+  const size_t smem = (size_t)WIDE_WAVES * NB * (PAIR ? 2 : 1) * MT * 256 * sizeof(float);
   if (!ready) {
-    PTA_REQUIRE(hipFuncSetAttribute((const void*)gemv_wide_kernel<Fmt, NB, PAIR, NORM>,
+    PTA_REQUIRE(hipFuncSetAttribute((const void*)gemv_wide_kernel<Fmt, MT, NB, PAIR, NORM>,
                                     hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem) == hipSuccess,
                 "%s: cannot reserve %zu bytes of LDS", name, smem);
     ready = true;
   }
   gemm_kernel_taken = "gemv_wide_kernel";
-  hipLaunchKernelGGL((gemv_wide_kernel<Fmt, NB, PAIR, NORM>), dim3((total_nb + NB - 1) / NB), dim3(WIDE_WAVES * 64), smem, s,
+  hipLaunchKernelGGL((gemv_wide_kernel<Fmt, MT, NB, PAIR, NORM>), dim3((total_nb + NB - 1) / NB), dim3(WIDE_WAVES * 64), smem, s,
                      a, total_nb);
   return PTA_OK;
 }
@@ -849,12 +887,12 @@ static int launch_gemv_wide(const GemmArgs& a, int total_nb, hipStream_t s, cons
 template <class Fmt, bool PAIR>
 constexpr int wide_cap() { return Fmt::kVec * (PAIR ? 2 : 1) <= 4 ? 3 : 2; }
 
-template <class Fmt, bool PAIR, bool NORM>
+template <class Fmt, int MT, bool PAIR, bool NORM>
 static int launch_gemv_wide_for(const GemmArgs& a, int total_nb, int per_cu, hipStream_t s, const char* name) {
   constexpr int cap = wide_cap<Fmt, PAIR>();
-  if (per_cu <= 1) return launch_gemv_wide<Fmt, 1, PAIR, NORM>(a, total_nb, s, name);
-  if (per_cu == 2 || cap == 2) return launch_gemv_wide<Fmt, 2, PAIR, NORM>(a, total_nb, s, name);
-  return launch_gemv_wide<Fmt, cap, PAIR, NORM>(a, total_nb, s, name);
+  if (per_cu <= 1) return launch_gemv_wide<Fmt, MT, 1, PAIR, NORM>(a, total_nb, s, name);
+  if (per_cu == 2 || cap == 2) return launch_gemv_wide<Fmt, MT, 2, PAIR, NORM>(a, total_nb, s, name);
+  return launch_gemv_wide<Fmt, MT, cap, PAIR, NORM>(a, total_nb, s, name);
 }
 
 // the longest chain of channel blocks a compute unit multiplies under launch_gemv_wide_for
@@ -2826,6 +2864,16 @@ static bool own_takes_few_rows(const GemmArgs& a, int total_nb, int cus, bool on
   return Fmt::kVec == 1 || a.M >= 12 || (!middle && total_nb <= 2 * cus);
 }
 
+// 17 to 32 rows by single F152 weights over one X: gemv_wide_kernel, whose 16 waves decode side by side where gemm_own_kernel has eight, as
+// long as its workgroups (of up to three blocks) are one round and K is not split.  Ratios of its time to that of the other kernels
+// (gemm_own_kernel, gemm_tile_kernel, up to 3072 features gemv_mfma_kernel), weights from HBM, 496 to 11008 channels: 1920 features 0.83 to
+// 1.05, 2048 0.82 to 0.98, 3072 0.76 to 0.95, 4096 to 13696 0.86 to 0.99; 1024 0.91 to 1.12, 1664 0.86 to 1.17, 1792 0.86 to 1.12; 29 rows and more, a block a compute unit, 5120 features 1.0, 8192 and
+// more 1.03 to 1.09.  Two rounds: 14336 and 16384 channels 1.17 to 1.35, 32000 1.13 to 1.28 (20480 0.77 to 0.92).  K in slices: 11008 x 1000 to
+// 4104 1.07 to 1.55.
+static inline bool wide_takes_some_rows(const GemmArgs& a, int total_nb, int cus, int blocks, bool split) {
+  return a.M > 16 && a.M <= 32 && a.KT >= 15 && !split && total_nb <= blocks * cus && !(a.M > 28 && a.KT > 40 && total_nb <= cus);
+}
+
 template <class Fmt, bool PAIR>
 static int dispatch_gemv(const GemmArgs& a, int total_nb, hipStream_t s, const char* name) {
   if (a.M > 16 && a.K >= GEMM_FAR && a.epi.norm == PTA_NORM_NONE) return rows_in_turn<Fmt, PAIR>(a, 16, total_nb, s, name);
@@ -2873,10 +2921,18 @@ static int dispatch_gemv(const GemmArgs& a, int total_nb, hipStream_t s, const c
         // the end is all (us, 33 rows: 128 features 1.17 times; pairs 256 x 1024 fp16 4.4 against 5.5, 768 x 11008 13.3 against 19.0, F143 11.8
         // against 16.2; 768 x 2048 it wins).  Up to 32 rows, against the kernel before them: 16-bit pairs of several rounds 1024 x 5608 0.88
         // and 1.19, 2048 x 5608 0.93 and 1.09, 3072 x 5608 0.96 and 1.0, one round of 1024 features 0.92 and 1.03; F152 singles 1024 x 4104
-        // 0.9 and 1.1, 3072 x 1000 1.08 and 1.2, pairs 2048 x 4104 0.73 and 0.99, 4096 x 2056 0.97 and 0.9.
+        // 0.9 and 1.1, pairs 2048 x 4104 0.73 and 0.99, 4096 x 2056 0.97 and 0.9.
         else if (mt > 2) own = PAIR ? a.KT >= 8 || (one_round && a.KT > 4) : a.KT > 2;
         else if (F152) own = a.KT > (PAIR ? 16 : 24) && (!PAIR || total_nb <= cus);
         else own = a.KT >= 8 && !(PAIR && Fmt::kVec > 2 && (a.KT == 8 || (!one_round && a.KT < 24)));
+      }
+      if constexpr (OwnStreams<Fmt>::long_decode && !PAIR) {
+        if (all_shared_x && wide_takes_some_rows(a, total_nb, cus, wide_cap<Fmt, PAIR>(), plan.slices > 1)) {
+          const int rc = launch_gemv_wide_for<Fmt, 2, PAIR, false>(a, total_nb, per_cu, s, name);
+          if (rc) return rc;
+          PTA_CHECK_LAUNCH(name);
+          return PTA_OK;
+        }
       }
       if (own) return launch_gemm_own_plan<Fmt, PAIR>(a, plan, s, name);
       int rc = 1;
@@ -2920,8 +2976,8 @@ static int dispatch_gemv(const GemmArgs& a, int total_nb, hipStream_t s, const c
         }
       }
       if (streamed) {}
-      else if (a.epi.norm != PTA_NORM_NONE) rc = launch_gemv_wide_for<Fmt, PAIR, true>(a, total_nb, per_cu, s, name);
-      else rc = launch_gemv_wide_for<Fmt, PAIR, false>(a, total_nb, per_cu, s, name);
+      else if (a.epi.norm != PTA_NORM_NONE) rc = launch_gemv_wide_for<Fmt, 1, PAIR, true>(a, total_nb, per_cu, s, name);
+      else rc = launch_gemv_wide_for<Fmt, 1, PAIR, false>(a, total_nb, per_cu, s, name);
       if (rc) return rc;
     } else if (a.M <= 16) launch_gemv<Fmt, 1, PAIR>(a, total_nb, s);
     else if (a.M <= 32) launch_gemv<Fmt, 2, PAIR>(a, total_nb, s);

@@ -216,7 +216,11 @@ def product(kind, M, Kd, N, pair):
     ("f16", 33, 264, 1000, False, "gemm_own"), ("int4", 64, 768, 50257, False, "gemm_own"),
     # what gemm_tile_kernel cannot take
     ("f16", 20, 1024, 5608, True, "gemv_mfma"), ("f16", 32, 2048, 5608, True, "gemv_mfma"), ("f16", 32, 3072, 5608, True, "gemm_own"), ("f16", 17, 2048, 2056, True, "gemm_own"),
-    ("int4", 20, 1024, 5608, True, "gemm_own"), ("f152", 24, 2048, 1000, False, "gemv_mfma"), ("f152", 17, 3072, 4104, False, "gemv_mfma"), ("f152", 32, 4096, 1000, False, "gemm_own"),
+    ("int4", 20, 1024, 5608, True, "gemm_own"), 
+    # F152 weights of up to 32 rows: one round of workgroups of one, two and three blocks (the last one's short of them), and the lines round it
+    ("f152", 24, 2048, 1000, False, "gemv_wide"), ("f152", 17, 3072, 4104, False, "gemv_wide"), ("f152", 32, 4096, 1000, False, "gemv_wide"), ("f152", 31, 1928, 40, False, "gemv_wide"),
+    ("f152", 20, 2056, 11000, False, "gemv_wide"), ("f152", 18, 4104, 12288, False, "gemv_wide"), ("f152", 32, 8200, 4104, False, "gemv_wide"), ("f152", 28, 8200, 1000, False, "gemv_wide"),
+    ("f152", 29, 8200, 1000, False, "gemm_own"), ("f152", 24, 1792, 1000, False, "gemv_mfma"), ("f152", 24, 1800, 1000, False, "gemv_wide"), ("f152", 24, 4096, 12304, False, "gemm_own"), ("f152", 33, 4096, 1000, False, "gemm_own"),
     ("f152", 20, 4096, 5608, True, "gemv_mfma"), ("f152", 31, 2048, 2056, True, "gemv_mfma"), ("f152", 32, 4096, 2056, True, "gemm_own"),
     ("f152", 64, 2048, 5632, True, "gemm_tile"), ("f152", 33, 1024, 5632, True, "gemm_tile"), ("f152", 40, 4096, 5632, True, "gemm_own"),
     # rounds of gemm_own_kernel beyond 64 rows
@@ -247,3 +251,35 @@ def test_which_kernel_more_rows_of_bf16_take(M, Kd, N, pair, kernel):
     # the sums' errors (silu multiplies the gate's by 1.1 at most), the exponential and the quotient in fp32
     bound = 1.1 * d * (y.abs() + d) + d * silu.abs() + 2.0 ** -20 * (silu * y).abs() + 2.0 ** -24
     assert ((out[:, :N].double() - silu * y).abs() <= bound).all()
+
+
+@pytest.mark.parametrize("M, Kd", [(17, 2056), (32, 4104), (27, 1928)])
+def test_f152_weights_over_one_input(M, Kd):
+    """gemv_wide_kernel with two groups of rows: blocks of several matrices (the last workgroup's beyond them) with biases, NaN behind the last
+    row; with inputs of their own and with slices of K other kernels."""
+    from poptransformer_amd import kernels as K
+    sizes = (40, 4096, 270, 16)
+    store = torch.full((M + 32, Kd), float("nan"), dtype=torch.float16, device="cuda")
+    tws, plains, biases = [], [], []
+    for i, n in enumerate(sizes):
+        x, w = operands(M, Kd, n, 50 + i)
+        if i == 0:
+            store[:M] = x.half()
+        tw, plain = weight_of("f152", w)
+        tws.append(tw), plains.append(plain), biases.append(torch.randn(n, device="cuda").half())
+    x = store[:M]
+    for xs in (None, [x] * 4):
+        outs = [torch.full((M, n), float("nan"), dtype=torch.float16, device="cuda") for n in sizes]
+        K.linear(None if xs else x, tws, outs, biases=biases, **(dict(xs=xs) if xs else {}))
+        assert (K.linear_kernel() == "gemv_wide_kernel") == (xs is None)
+        for out, plain, b in zip(outs, plains, biases):
+            ref, mag = x.double() @ plain.T, x.double().abs() @ plain.abs().T
+            # the sum is rounded, then its sum with the bias
+            bound = 2.0 ** -11 * (ref.abs() + (ref + b.double()).abs()) * 1.001 + (Kd + 2) * 2.0 ** -24 * mag + 2.0 ** -23
+            assert ((out.double() - ref - b.double()).abs() <= bound).all()
+    long, w = operands(M, 11008, 1000, 60)
+    tw, plain = weight_of("f152", w)
+    out = torch.full((M, 1000), float("nan"), dtype=torch.float16, device="cuda")
+    K.linear(long.half(), [tw], [out], workspace=K.linear_workspace(M, 1000, "cuda"))
+    assert K.linear_kernel() == "gemm_own_kernel"
+    close(out, long.half().double() @ plain.T, long.half().double().abs() @ plain.abs().T, 11008, 11)
