@@ -503,10 +503,10 @@ static int attn_splits(int B, int Hq, int max_len) {
 // What bounds it is a workgroup's chain of steps, the longest over all the positions: the last rows' workgroups are launched first, and a
 // step is kept short - 64 rows to a barrier, no transposition by 2-byte stores, no exchange between lanes but that of the maximum.
 // The heads of an XCD are its own (its L2 then holds their K and V): grid x is the head modulo eight.
-// Before (32 rows a step, V transposed by 2-byte stores, two barriers) and now: us for one sequence of 32 heads of 128, 17 rows 5.0, 5.5;
-// 64 rows 6.2, 6.1; 300 rows 16.6, 11.1; 1000 54.8, 31.0; 2048 160, 79; 4000 593, 227; 64 rows behind 900 42.5, 23.3; F143, 1000 rows
-// 62.6, 43.6; 8 x 12 heads of 64, 1000 rows 79, 44.
-// A wave whose rows end within a step's first 32 cache rows takes those alone, in code of its own: 17 rows 5.8 -> 5.5 (F143 6.3 -> 5.6),
+// Before (32 rows a step, V transposed by 2-byte stores, two barriers) and now: us for one sequence of 32 heads of 128, 17 rows 4.8, 4.8;
+// 64 rows 6.0, 5.5; 65 rows 6.0, 6.3 (F143 6.5, 7.3); 300 rows 16.6, 11.1; 1000 53.8, 30.7; 2048 160, 79; 4000 593, 227; 64 rows behind 900
+// 42.5, 23.3; F143, 1000 rows 61.6, 43.9; 8 x 12 heads of 64, 1000 rows 78, 44.
+// A wave whose rows end within a step's first 32 cache rows takes those alone, in code of its own: 17 rows -0.3 us (F143 -0.7),
 // 200 rows 10.0 -> 9.2, 17 rows behind 900 23.5 -> 21.8; 4000 rows 222 -> 227.  It does not touch V rows that none of its rows may see,
 // beyond its own 32: an infinity there times a weight of zero would be a NaN.
 // Row r of the pass sits at position step + r and attends to cache rows [0, min(step + r + 1, max_len)), as in
@@ -686,16 +686,30 @@ __global__ __launch_bounds__(PA_THREADS) void prompt_attention_mfma_kernel(AttnA
     }
   };
 
-  request(0, smem);
-  int turn = 0;
-  for (int p0 = 0; p0 < wg_valid; p0 += PA_KEYS, turn ^= 1) {
-    unsigned char* const stage = smem + turn * (2 * STAGE);
+  auto landed = [&](unsigned char* stage) {
     if constexpr (KV8) decode(stage);
     else __builtin_amdgcn_s_waitcnt(0x0f70);               // vmcnt(0): this wave's share of the step's rows has landed
     __syncthreads();                                       // (and every wave is done with the other stage)
-    if (p0 + PA_KEYS < wg_valid) request(p0 + PA_KEYS, smem + (turn ^ 1) * (2 * STAGE));
-    if (p0 + 32 < wave_valid) attend(stage, p0, std::integral_constant<int, 2>{});
-    else if (p0 < wave_valid) attend(stage, p0, std::integral_constant<int, 1>{});
+  };
+  request(0, smem);
+  // One step: code of its own, in the order it runs in.  A short launch's time is that of its instructions' way from memory, and with the
+  // steps' loop round them 17 rows took 5.2 us against 4.8, 64 rows 5.8 against 5.5 (F143 5.4, 5.0 and 6.4, 6.0).
+  if (__builtin_expect(wg_valid <= PA_KEYS, 1)) {
+    landed(smem);
+    if (__builtin_expect(wave_valid <= 32, 1)) {
+      if (wave_valid > 0) attend(smem, 0, std::integral_constant<int, 1>{});
+    } else {
+      attend(smem, 0, std::integral_constant<int, 2>{});
+    }
+  } else {
+    int turn = 0;
+    for (int p0 = 0; p0 < wg_valid; p0 += PA_KEYS, turn ^= 1) {
+      unsigned char* const stage = smem + turn * (2 * STAGE);
+      landed(stage);
+      if (p0 + PA_KEYS < wg_valid) request(p0 + PA_KEYS, smem + (turn ^ 1) * (2 * STAGE));
+      if (p0 + 32 < wave_valid) attend(stage, p0, std::integral_constant<int, 2>{});
+      else if (p0 < wave_valid) attend(stage, p0, std::integral_constant<int, 1>{});
+    }
   }
   run_l += __shfl_xor(run_l, 16, 64);
   run_l += __shfl_xor(run_l, 32, 64);

@@ -7,7 +7,9 @@ pytestmark = pytest.mark.gpu
 
 CASES = [  # sequences, rows, query heads, KV heads, ring, step
     (1, 16, 1, 1, 16, 0), (1, 17, 8, 8, 64, 0), (2, 63, 5, 5, 128, 0), (1, 64, 9, 3, 130, 65), (3, 65, 12, 4, 200, 63), (1, 129, 16, 2, 192, 40),
-    (2, 128, 7, 7, 100, 20), (1, 300, 32, 32, 512, 1)]
+    (2, 128, 7, 7, 100, 20), (1, 300, 32, 32, 512, 1),
+    # one step: of 20, 32, 33 and 64 cache rows, and one row more than that; a ring that is full before the pass
+    (1, 20, 3, 3, 20, 30), (1, 32, 3, 3, 40, 0), (2, 33, 4, 2, 64, 0), (1, 17, 9, 3, 64, 47), (1, 64, 3, 3, 64, 9), (2, 16, 3, 3, 80, 49)]
 
 
 @pytest.mark.parametrize("kv8", [False, True])
