@@ -2867,11 +2867,11 @@ static bool own_takes_few_rows(const GemmArgs& a, int total_nb, int cus, bool on
 // 17 to 32 rows by single F152 weights over one X: gemv_wide_kernel, whose 16 waves decode side by side where gemm_own_kernel has eight, as
 // long as its workgroups (of up to three blocks) are one round and K is not split.  Ratios of its time to that of the other kernels
 // (gemm_own_kernel, gemm_tile_kernel, up to 3072 features gemv_mfma_kernel), weights from HBM, 496 to 11008 channels: 1920 features 0.83 to
-// 1.05, 2048 0.82 to 0.98, 3072 0.76 to 0.95, 4096 to 13696 0.86 to 0.99; 1024 0.91 to 1.12, 1664 0.86 to 1.17, 1792 0.86 to 1.12; 29 rows and more, a block a compute unit, 5120 features 1.0, 8192 and
-// more 1.03 to 1.09.  Two rounds: 14336 and 16384 channels 1.17 to 1.35, 32000 1.13 to 1.28 (20480 0.77 to 0.92).  K in slices: 11008 x 1000 to
-// 4104 1.07 to 1.55.
+// 1.05, 2048 0.82 to 0.98, 3072 0.76 to 0.95, 4096 to 13696 0.86 to 0.99; 1536 to 1792 with a block a compute unit 0.94 to 1.02, with more
+// 0.86 to 1.17; 1024 0.91 to 1.12; 29 rows and more, a block a compute unit, 5120 features 1.0, 8192 and more 1.03 to 1.09.  Two rounds: 14336
+// and 16384 channels 1.17 to 1.35, 32000 1.13 to 1.28 (20480 0.77 to 0.92).  K in slices: 11008 x 1000 to 4104 1.07 to 1.55.
 static inline bool wide_takes_some_rows(const GemmArgs& a, int total_nb, int cus, int blocks, bool split) {
-  return a.M > 16 && a.M <= 32 && a.KT >= 15 && !split && total_nb <= blocks * cus && !(a.M > 28 && a.KT > 40 && total_nb <= cus);
+  return a.M > 16 && a.M <= 32 && a.KT >= (total_nb <= cus ? 12 : 15) && !split && total_nb <= blocks * cus && !(a.M > 28 && a.KT > 40 && total_nb <= cus);
 }
 
 template <class Fmt, bool PAIR>

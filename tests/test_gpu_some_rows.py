@@ -220,7 +220,7 @@ def product(kind, M, Kd, N, pair):
     # F152 weights of up to 32 rows: one round of workgroups of one, two and three blocks (the last one's short of them), and the lines round it
     ("f152", 24, 2048, 1000, False, "gemv_wide"), ("f152", 17, 3072, 4104, False, "gemv_wide"), ("f152", 32, 4096, 1000, False, "gemv_wide"), ("f152", 31, 1928, 40, False, "gemv_wide"),
     ("f152", 20, 2056, 11000, False, "gemv_wide"), ("f152", 18, 4104, 12288, False, "gemv_wide"), ("f152", 32, 8200, 4104, False, "gemv_wide"), ("f152", 28, 8200, 1000, False, "gemv_wide"),
-    ("f152", 29, 8200, 1000, False, "gemm_own"), ("f152", 24, 1792, 1000, False, "gemv_mfma"), ("f152", 24, 1800, 1000, False, "gemv_wide"), ("f152", 24, 4096, 12304, False, "gemm_own"), ("f152", 33, 4096, 1000, False, "gemm_own"),
+    ("f152", 29, 8200, 1000, False, "gemm_own"), ("f152", 24, 1408, 1000, False, "gemv_mfma"), ("f152", 24, 1416, 1000, False, "gemv_wide"), ("f152", 32, 1792, 4104, False, "gemv_mfma"), ("f152", 32, 1800, 4104, False, "gemv_wide"), ("f152", 24, 4096, 12304, False, "gemm_own"), ("f152", 33, 4096, 1000, False, "gemm_own"),
     ("f152", 20, 4096, 5608, True, "gemv_mfma"), ("f152", 31, 2048, 2056, True, "gemv_mfma"), ("f152", 32, 4096, 2056, True, "gemm_own"),
     ("f152", 64, 2048, 5632, True, "gemm_tile"), ("f152", 33, 1024, 5632, True, "gemm_tile"), ("f152", 40, 4096, 5632, True, "gemm_own"),
     # rounds of gemm_own_kernel beyond 64 rows
