@@ -2732,14 +2732,24 @@ template <class Fmt> struct BlockFormat { static constexpr bool ok = false; };
 // gemm_rows_kernel, weights from HBM, pairs 2048 x 2048 to 5632: 129 rows 0.95, 160 1.04, 200 1.17, 256 1.26, 320 1.1, 400 0.9, 512 1.14, 768
 // 1.08, 1000 0.95; 8192 x 5632, 256 rows 1.26.  The fp32 epilogue adds to the former (it passes through LDS in one copy of the code): with K
 // of 1024 1.03 to 1.31 (pairs) and 1.0 to 1.23 for up to 192 workgroups of the latter, 2048 x 6144, 512 rows 1.18.
+// Single weights whose K is not split (no workspace, or several of them), 2048 to 12288 channels: fp16, K of 8192: 160 rows 0.9, 200 1.05 to
+// 1.08, 250 1.2 to 1.26, 320 1.0, 384 1.2, 500 1.11 to 1.19, 742 1.1, 1000 1.12; of 4096: 200 1.0, 250 1.12 to 1.16, 320 0.96, 384 1.1, 500
+// 1.06, 742 1.0 (1000 rows, 4096 channels, a workgroup a compute unit: 0.91); of 2048: 250 1.08, 384 1.05, 500 1.0.  bf16, K from 4096 on: 160 rows 0.95 to 1.0, 200 1.15, 250 1.3, 320 1.08, 384 1.28, 500
+// 1.2, 742 1.13, 1000 1.11 to 1.19; of 2048: 129 1.04, 160 1.12, 200 1.26, 250 1.33, 320 1.18, 500 1.25 (2048 channels 0.95 to 0.99).
 template <class Fmt, bool PAIR>
 static bool rows_before_blocks(const GemmArgs& a, int total_nb, int cus) {
   if (Fmt::kVec < 4) return false;
   const int blocks = (a.M + 127) / 128, wgs = total_nb / (PAIR ? ROWS_CB / 2 : ROWS_CB) * blocks;
   if (wgs > cus) return false;
   const double held = a.M / (128.0 * blocks), line = 0.75 + 0.04 * (blocks - 2);
+  const bool whole = !PAIR && (a.count > 1 || !a.part || a.part_bytes < 2 * (size_t)a.M * a.mat[0].N * sizeof(float));      // K is not split
   if (Fmt::kWide && a.KT <= 8) return PAIR || wgs <= cus * 3 / 4 || held >= line;
-  if (Fmt::kWide && a.KT <= 16) return PAIR ? held >= line - 0.15 : wgs >= cus * 5 / 8 && held >= line;
+  if (Fmt::kWide && a.KT <= 16) return PAIR || (whole && wgs >= cus / 4) ? held >= line - 0.15 : wgs >= cus * 5 / 8 && held >= line;
+  if (whole) {
+    if (Fmt::kWide) return held >= 0.75 + 0.03 * (blocks - 2);
+    if (a.KT < 24) return a.KT >= 16 && blocks <= 3 && held >= 0.9 && wgs >= cus / 4;
+    return wgs <= cus * 3 / 4 && held >= (a.KT >= 48 ? 0.77 + 0.03 * (blocks - 2) : 0.85 + 0.02 * (blocks - 2));
+  }
   return PAIR && held >= line;
 }
 

@@ -281,7 +281,7 @@ def test_which_kernel_pairs_take(kind, M, Kd, N, kernel):
 
 
 @pytest.mark.parametrize("M, Kd, main, tail, kernel", [
-    (129, 72, 16005, 5, "block"), (257, 1000, 10990, 18, "block"), (1100, 264, 3000, 0, "block"), (300, 2048, 8200, 0, "block"), (400, 2056, 6144, 0, "block"), (1000, 40, 3200, 3, "block"),
+    (129, 72, 16005, 5, "block"), (257, 1000, 10990, 18, "block"), (1100, 264, 3000, 0, "block"), (520, 2048, 8200, 0, "block"), (400, 2056, 6144, 0, "block"), (1000, 40, 3200, 3, "block"),
     # short K, and one round of workgroups with whole blocks of rows
     (512, 512, 4096, 0, "rows"), (129, 1024, 6016, 128, "rows"), (512, 2048, 6140, 4, "rows"), (1000, 1000, 4096, 0, "block"), (768, 1032, 1024, 0, "block")])
 @pytest.mark.parametrize("slices", [False, True])
@@ -298,6 +298,31 @@ def test_which_kernel_wide_products_take(M, Kd, main, tail, kernel, slices):
     close(out, ref[:, :main], mag[:, :main], Kd, 24)
     if tail:
         close(t[:M * tail].view(M, tail), ref[:, main:], mag[:, main:], Kd, 24)
+
+
+@pytest.mark.parametrize("kind, M, Kd, N, kernel", [
+    # K of 8192 and more, of 3072, of 2048; bf16 K past 2048 and up to it; either side of the lines
+    ("f16", 200, 8192, 4096, "rows"), ("f16", 196, 8200, 4096, "block"), ("f16", 742, 6152, 2048, "rows"), ("f16", 1000, 8192, 2048, "rows"), ("f16", 1000, 4096, 4096, "block"), ("f16", 250, 3080, 4096, "rows"),
+    ("f16", 320, 4096, 4096, "block"), ("f16", 250, 2056, 4096, "rows"), ("f16", 500, 2048, 4096, "block"), ("f16", 256, 1920, 12288, "block"), ("f8", 256, 8192, 12288, "block"),
+    ("bf16", 192, 2056, 12288, "rows"), ("bf16", 191, 2056, 12288, "block"), ("bf16", 1000, 4096, 4096, "rows"), ("bf16", 160, 2048, 6144, "rows"), ("bf16", 129, 2048, 6144, "block"),
+    ("bf16", 384, 1544, 2048, "block"), ("bf16", 250, 11008, 4096, "rows")])
+def test_which_kernel_weights_take_whose_k_is_not_split(kind, M, Kd, N, kernel):
+    x, w = operands(M, Kd, N, 41)
+    if kind == "bf16":
+        from poptransformer_amd import hybrid_kernels as HK
+        x, plain = x.to(torch.bfloat16), w.to(torch.bfloat16).double()
+        out = torch.full((M, N), float("nan"), device="cuda")
+        HK.linear(x, HK.WideWeight(w.to(torch.bfloat16), torch.bfloat16), out, M, ld=N)
+        taken, bits = HK.linear_kernel(), 24
+    else:
+        from poptransformer_amd import kernels as K
+        x = x.half()
+        tw, plain = weight_of(kind, w)
+        out = torch.full((M, N), float("nan"), dtype=torch.float16, device="cuda")
+        K.linear(x, [tw], [out])
+        taken, bits = K.linear_kernel(), 11
+    assert taken == f"gemm_{kernel}_kernel"
+    close(out, x.double() @ plain.T, x.double().abs() @ plain.abs().T, Kd, bits)
 
 
 @pytest.mark.parametrize("M, Kd, N, kernel", [(256, 1024, 4096, "rows"), (129, 512, 7168, "rows"), (160, 2048, 5632, "rows"), (129, 2048, 5632, "block"), (160, 4096, 4096, "block"), (256, 4104, 4096, "rows"), (515, 136, 4100, "block")])
