@@ -515,6 +515,40 @@ int pta_decode_step_failed(const void* workspace, int* failed, pta_stream_t stre
 int pta_llama_decode_step_static(const pta_decode_model* model, const pta_decode_state* state, int clear_failure,
                                  pta_stream_t stream);
 
+/* ----------------------------------------------------------------------------------
+ * One iteration of the decode loop of a GPT-2 model with fp16 weights in one launch
+ * (models/gpt2/model.py, models/base_model.py:271-355).  The workgroups of all products and attentions are one
+ * grid; each waits for the values that it reads, always of workgroups that started before it, so that
+ * launches may run beside anything else, each other included (with workspaces of their own).
+ * Results are those of the per-operator entry points up to the order of fp32 sums.
+ * ---------------------------------------------------------------------------------- */
+
+typedef struct pta_gpt2_layer {
+  const void *qkv, *out, *fc, *down;                  /* weights tiled by pta_f16_tile: [3 hidden, hidden], [hidden, hidden], [ffn, hidden], [hidden, ffn] */
+  const pta_half *qkv_bias, *out_bias, *fc_bias, *down_bias;
+  const pta_half *norm1_weight, *norm1_bias, *norm2_weight, *norm2_bias;      /* 16-byte aligned */
+  pta_half* kv_ring;                                  /* ring of pta_qkv_rope_append for this layer */
+} pta_gpt2_layer;
+
+typedef struct pta_gpt2_model {
+  const pta_gpt2_layer* layers;                       /* DEVICE array [n_layer]                       */
+  int n_layer;
+  const pta_half *embed, *positions;                  /* [vocab, hidden], [n_positions, hidden]       */
+  const pta_half *norm_weight, *norm_bias;            /* the final norm's                             */
+  const void* head;                                   /* lm_head [vocab, hidden] tiled by pta_f16_tile */
+  int batch, hidden, n_head, ffn, vocab, max_len, n_positions;
+  float eps;
+  int pad_id, eos_id, early_stop;                     /* as pta_step_update                           */
+} pta_gpt2_model;
+
+/* Bytes of the workspace of pta_gpt2_step; 0 for unsupported shapes (supported: batch up to 8, heads of 64, hidden up to 2048, ffn
+ * up to 8192 and a multiple of 8, n_positions >= max_len; with 8 rows less, where LDS does not hold them).  The caller zeroes it once after allocating it (256-byte aligned). */
+size_t pta_gpt2_step_workspace_bytes(const pta_gpt2_model* model);
+
+/* Enqueues one loop iteration.  Launches with one workspace must follow each other in stream order.  Every wait is bounded: if one gives up,
+ * the loop state is left untouched and later launches do nothing (pta_decode_step_failed). */
+int pta_gpt2_step(const pta_gpt2_model* model, const pta_decode_state* state, void* workspace, pta_stream_t stream);
+
 #ifdef __cplusplus
 }
 #endif

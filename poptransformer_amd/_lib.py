@@ -49,6 +49,17 @@ class DecodeState(ctypes.Structure):
     _fields_ = [(n, c_void_p) for n in ("container", "mask", "stop_mask", "step", "keep_going", "next_ids", "logits")]
 
 
+class Gpt2Layer(ctypes.Structure):
+    _fields_ = [(n, c_void_p) for n in ("qkv", "out", "fc", "down", "qkv_bias", "out_bias", "fc_bias", "down_bias", "norm1_weight", "norm1_bias",
+                                        "norm2_weight", "norm2_bias", "kv_ring")]
+
+
+class Gpt2Model(ctypes.Structure):
+    _fields_ = [("layers", c_void_p), ("n_layer", c_int), ("embed", c_void_p), ("positions", c_void_p), ("norm_weight", c_void_p), ("norm_bias", c_void_p),
+                ("head", c_void_p), ("batch", c_int), ("hidden", c_int), ("n_head", c_int), ("ffn", c_int), ("vocab", c_int), ("max_len", c_int),
+                ("n_positions", c_int), ("eps", c_float), ("pad_id", c_int), ("eos_id", c_int), ("early_stop", c_int)]
+
+
 class Fusion(ctypes.Structure):
     _fields_ = [("bias", c_void_p), ("residual", c_void_p), ("act", c_int), ("mul", c_void_p), ("post_scale", c_float),
                 ("norm", c_int),
@@ -132,6 +143,8 @@ SIGNATURES = {
     "pta_llama_decode_step_f8": (c_int, [POINTER(DecodeModel), POINTER(DecodeState), c_int, c_void_p, c_void_p]),
     "pta_decode_step_failed": (c_int, [c_void_p, POINTER(c_int), c_void_p]),
     "pta_llama_decode_step_static": (c_int, [POINTER(DecodeModel), POINTER(DecodeState), c_int, c_void_p]),
+    "pta_gpt2_step_workspace_bytes": (c_size_t, [POINTER(Gpt2Model)]),
+    "pta_gpt2_step": (c_int, [POINTER(Gpt2Model), POINTER(DecodeState), c_void_p, c_void_p]),
 }
 
 _lib = None

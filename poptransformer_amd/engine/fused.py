@@ -295,7 +295,34 @@ class FusedDecoder(DecodeLoop, LayerOps):
         self.graph = None
         self._stream = torch.cuda.Stream()
         self.persistent = None
+        self.chained = self._gpt2_step()     # GPT-2: an iteration as one launch, where the kernel has the shape (None: per operator)
         self.probe = None                # callable(name, block index, tensor or tensors): looks into eager iterations of the per-operator path
+
+    def _gpt2_step(self):
+        """pta_gpt2_step over this decoder's buffers, or None: another family or selection, other weights, or a shape that it does not cover."""
+        s, w = self.spec, self.w
+        if s.family != "gpt2" or s.topk != 1 or s.fp8_cache or s.head_dim != 64 or s.n_kv_head != s.n_head:
+            return None
+        if w.pos_embed is None or not isinstance(w.head.w, K.F16Weight) or w.head.bias is not None:
+            return None
+        lins = [lw for b in w.blocks for lw in (b.qkv[0], b.out, b.mlp_in[0], b.mlp_out)]
+        if any(len(b.qkv) != 1 or len(b.mlp_in) != 1 for b in w.blocks) or not all(isinstance(lw.w, K.F16Weight) and lw.bias is not None for lw in lins):
+            return None
+        norms = [g for b in w.blocks for g in (b.norm1, b.norm2)] + [w.final_norm]
+        if any(t is None or t.data_ptr() % 16 for g in norms for t in g):
+            return None
+        layers = []
+        for b, ring in zip(w.blocks, self.rings):
+            names = {"qkv": b.qkv[0], "out": b.out, "fc": b.mlp_in[0], "down": b.mlp_out}
+            layers.append(dict({n: lw.w.tiled for n, lw in names.items()}, **{n + "_bias": lw.bias for n, lw in names.items()}, norm1_weight=b.norm1[0],
+                               norm1_bias=b.norm1[1], norm2_weight=b.norm2[0], norm2_bias=b.norm2[1], kv_ring=ring))
+        state = dict(container=self.container, mask=self.mask, stop_mask=self.stop_mask, step=self.step, keep_going=self.keep_going,
+                     next_ids=self.next_ids, logits=self.logits)
+        try:
+            return K.Gpt2Step(layers, w.embed, w.pos_embed, w.final_norm, w.head.w.tiled, s.batch, s.d_model, s.n_head, w.blocks[0].mlp_out.K, s.vocab,
+                              s.max_len, s.eps, s.pad_id, s.eos_id, s.early_stop, state)
+        except NotImplementedError:
+            return None
 
     def enable_persistent(self):
         """Run each loop iteration as one persistent launch (pta_llama_decode_step) instead of one
@@ -329,6 +356,9 @@ class FusedDecoder(DecodeLoop, LayerOps):
     def step_fn(self):
         if self.persistent is not None:
             self.persistent.launch()
+            return
+        if self.chained is not None and self.probe is None:
+            self.chained.launch()
             return
         s, w = self.spec, self.w
         B = s.batch
@@ -418,3 +448,5 @@ class FusedDecoder(DecodeLoop, LayerOps):
             raise RuntimeError("persistent decode step: a workgroup gave up waiting (the kernel needs every compute unit "
                                "of the device for itself while it runs); the loop state was not advanced past the failing "
                                "iteration.  The failure word is sticky: persistent.clear_failure() re-arms the decoder")
+        if self.chained is not None and self.chained.failed():
+            raise RuntimeError("GPT-2 step: a workgroup gave up waiting; the loop state was not advanced past the failing iteration")

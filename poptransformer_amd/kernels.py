@@ -681,3 +681,32 @@ class DecodeStep:
         flag = ctypes.c_int(0)
         check(_lib.load().pta_decode_step_failed(_p(self.workspace), ctypes.byref(flag), _stream()))
         return bool(flag.value)
+
+
+class Gpt2Step:
+    """One whole loop iteration of a GPT-2 decoder with fp16 weights in a single launch (pta_gpt2_step).  Holds the device copies of the layer
+    descriptors and the workspace; raises NotImplementedError for shapes the kernel does not cover."""
+
+    def __init__(self, layers, embed, positions, norm, head, batch, hidden, n_head, ffn, vocab, max_len, eps, pad_id, eos_id, early_stop, state):
+        lib = _lib.load()
+        arr = (_lib.Gpt2Layer * len(layers))()
+        for dst, src in zip(arr, layers):
+            for name, t in src.items():
+                setattr(dst, name, t.data_ptr())
+        self.layers = torch.frombuffer(bytearray(bytes(arr)), dtype=torch.uint8).to(embed.device)
+        self._keep = (layers, embed, positions, norm, head, state)
+        self.model = _lib.Gpt2Model(self.layers.data_ptr(), len(layers), embed.data_ptr(), positions.data_ptr(), norm[0].data_ptr(), norm[1].data_ptr(),
+                                    head.data_ptr(), batch, hidden, n_head, ffn, vocab, max_len, positions.shape[0], eps, pad_id, eos_id, 1 if early_stop else 0)
+        nbytes = lib.pta_gpt2_step_workspace_bytes(ctypes.byref(self.model))
+        if nbytes == 0:
+            raise NotImplementedError(f"GPT-2 step kernel: unsupported shape (batch {batch}, {n_head} heads, hidden {hidden}, ffn {ffn})")
+        self.workspace = torch.zeros(nbytes, dtype=torch.uint8, device=embed.device)
+        self.state = _lib.DecodeState(**{k: v.data_ptr() for k, v in state.items()})
+
+    def launch(self):
+        check(_lib.load().pta_gpt2_step(ctypes.byref(self.model), ctypes.byref(self.state), _p(self.workspace), _stream()))
+
+    def failed(self):
+        flag = ctypes.c_int(0)
+        check(_lib.load().pta_decode_step_failed(_p(self.workspace), ctypes.byref(flag), _stream()))
+        return bool(flag.value)
