@@ -1938,12 +1938,223 @@ static int launch_gemm_rows(const GemmArgs& a, int total_nb, hipStream_t s, cons
   return PTA_OK;
 }
 
+// a's second and fourth sixteen lanes change places with b's first and third
+__device__ __forceinline__ void swap_sixteens(uint32_t& a, uint32_t& b) {
+  const auto r = __builtin_amdgcn_permlane16_swap(a, b, false, false);
+  a = r[0];
+  b = r[1];
+}
+
+// Of sums of two neighbouring channel blocks (as panel_store has them, four channels a lane) rounded to 16 bits, eight consecutive channels
+// a lane: of block (lane / 16) % 2, from lane / 32 * 8 on.
+template <class T4>
+__device__ __forceinline__ u32x4 eight_channels(T4 first, T4 second) {
+  u32x2 a = bitcast<u32x2>(first), b = bitcast<u32x2>(second);
+  uint32_t a0 = a[0], a1 = a[1], b0 = b[0], b1 = b[1];
+  swap_sixteens(a0, b0);
+  swap_sixteens(a1, b1);
+  return u32x4{a0, a1, b0, b1};
+}
+
+// What is rounded to 16 bits: sigmoid and swish by the hardware's exponential and reciprocal (2 to 4 units of the 24-bit result).
+__device__ __forceinline__ float quick_sigmoid(float v) { return __builtin_amdgcn_rcpf(1.0f + __expf(-v)); }
+__device__ __forceinline__ float quick_swish(float v) { return v * quick_sigmoid(v); }
+
+// The ends of a tile that most products have, straight from the registers and without a loop; false: another one (panel_store).  What bounds
+// them is what they wait for: through LDS, row group by row group, each stretch of a residual, a gate or an old sum was a round trip to memory
+// of its own behind the one before, and swish by a division of eleven instructions kept a unit's vector ALU for 8 us a tile; here
+// all that a tile adds is requested together.  A launch of 2048 x 4096 without its products 10.3 -> 8.2 us (an empty one 2.6), 2048 x 8192 11.0 ->
+// 9.2; with them, weights from HBM: fp16, 2048 rows, 4096 x 8192 117 -> 114, 4096 x 4096 74 -> 72; bf16, 2048 rows, 11008 x 4096 with gate and
+// fp32 residual 215 -> 201, a pair of 4096 x 11008 341 -> 300, two of 4096 x 4096 with biases and sigmoids 137 -> 113.
+template <class Fmt, int NST, int RG, bool PAIR>
+__device__ __forceinline__ bool straight_store(const GemmMat& mat, const GemmEpilogue& epi, float* part, const f32x4 (&acc)[RG][NST], int blk0, int row0, int nsl,
+                                               typename Fmt::Scale s0, typename Fmt::Scale s1, int M, const int32_t* order) {
+  static_assert(NST == 4 && RG % 2 == 0, "tile");
+  const int lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4;
+  const int N = mat.N, n0 = blk0 * 16;
+  if (!PAIR && nsl > 1) {                                   // a slice of K: the sums as they are
+    if (N & 3) return false;
+    float* p = part + ((size_t)blockIdx.y * M + row0 + r) * N + n0 + g * 4;
+#pragma unroll
+    for (int rg = 0; rg < RG; ++rg) {
+      if (row0 + rg * 16 + r < M) {
+#pragma unroll
+        for (int st = 0; st < NST; ++st)
+          if (n0 + st * 16 + g * 4 < N) *reinterpret_cast<f32x4*>(p + (size_t)rg * 16 * N + st * 16) = acc[rg][st];
+      }
+    }
+    return true;
+  }
+  const int c8 = (g & 1) * 16 + (g >> 1) * 8;               // a lane's eight channels of two blocks
+  if constexpr (!Fmt::kWide) {
+    if ((N & 7) || epi.out_fp8_scale || (reinterpret_cast<uintptr_t>(mat.Y) & 15)) return false;
+    if constexpr (PAIR) {
+      f16* y = mat.Y + (size_t)(row0 + r) * N + n0 + c8;
+      const bool in = n0 + c8 < N;
+#pragma unroll
+      for (int rg = 0; rg < RG; ++rg) {
+        f16x4 v[2];
+#pragma unroll
+        for (int st = 0; st < 2; ++st)
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            v[st][e] = (f16)Fmt::finish(acc[rg][2 + st][e], s1) * (f16)quick_swish((float)(f16)Fmt::finish(acc[rg][st][e], s0));
+        const u32x4 out = eight_channels(v[0], v[1]);
+        if (in && row0 + rg * 16 + r < M) *reinterpret_cast<u32x4*>(y + (size_t)rg * 16 * N) = out;
+      }
+    } else {
+      const f16* bias = mat.bias ? mat.bias : epi.bias;
+      if ((mat.bias && epi.bias) || mat.act != PTA_ACT_NONE || epi.act != PTA_ACT_NONE || epi.mul || epi.post_scale != 0.0f ||
+          ((reinterpret_cast<uintptr_t>(bias) | reinterpret_cast<uintptr_t>(epi.residual)) & 15))
+        return false;
+      const size_t at = (size_t)(row0 + r) * N + n0 + c8;
+      const f16* from = epi.residual + at;
+      f16x8 b[2], res[RG][2];
+#pragma unroll
+      for (int p = 0; p < 2; ++p) {
+        const bool in = n0 + p * 32 + c8 < N;
+        b[p] = f16x8{0, 0, 0, 0, 0, 0, 0, 0};
+        if (bias && in) b[p] = *reinterpret_cast<const f16x8*>(bias + n0 + p * 32 + c8);
+        if (epi.residual) {
+#pragma unroll
+          for (int rg = 0; rg < RG; ++rg)
+            if (in && row0 + rg * 16 + r < M) res[rg][p] = *reinterpret_cast<const f16x8*>(from + (size_t)rg * 16 * N + p * 32);
+        }
+      }
+#pragma unroll
+      for (int rg = 0; rg < RG; ++rg)
+#pragma unroll
+        for (int p = 0; p < 2; ++p) {
+          f16x4 v[2];
+#pragma unroll
+          for (int st = 0; st < 2; ++st)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) v[st][e] = (f16)Fmt::finish(acc[rg][p * 2 + st][e], s0);
+          f16x8 out = bitcast<f16x8>(eight_channels(v[0], v[1]));
+          if (bias) out = out + b[p];
+          if (epi.residual) out = out + res[rg][p];
+          if (n0 + p * 32 + c8 < N && row0 + rg * 16 + r < M) *reinterpret_cast<f16x8*>(mat.Y + at + (size_t)rg * 16 * N + p * 32) = out;
+        }
+    }
+  } else {
+    const WideOut& w = mat.wide;
+    const bool tail = !PAIR && w.tail_count && n0 + NST * 16 > w.n_main;
+    if ((w.ld & 7) || (w.n_main & 7) || w.mul_f32 ||
+        (tail && ((w.tail_count & 3) || ((reinterpret_cast<uintptr_t>(w.tail) | reinterpret_cast<uintptr_t>(w.tail_bias)) & 15))) ||
+        ((reinterpret_cast<uintptr_t>(mat.Y) | reinterpret_cast<uintptr_t>(w.bias) | reinterpret_cast<uintptr_t>(w.mul) | (PAIR ? reinterpret_cast<uintptr_t>(w.bias2) : 0)) & 15))
+      return false;
+    int m[RG];
+    bool on[RG];
+#pragma unroll
+    for (int rg = 0; rg < RG; ++rg) {
+      on[rg] = row0 + rg * 16 + r < M;
+      m[rg] = on[rg] ? (order ? order[row0 + rg * 16 + r] : row0 + rg * 16 + r) : 0;
+    }
+    const int c4 = n0 + g * 4;
+    auto channels = [&](const float* p, int c) { return p && c < w.n_main ? *reinterpret_cast<const f32x4*>(p + c) : f32x4{0.f, 0.f, 0.f, 0.f}; };
+    if constexpr (PAIR) {
+      if (w.out_f32 || w.mul) return false;
+      f32x4 b1[2], b2[2];
+#pragma unroll
+      for (int st = 0; st < 2; ++st) { b1[st] = channels(w.bias, c4 + st * 16); b2[st] = channels(w.bias2, c4 + st * 16); }
+      auto all = [&](auto value) {
+#pragma unroll
+        for (int rg = 0; rg < RG; ++rg) {
+          bf16x4 v[2];
+#pragma unroll
+          for (int st = 0; st < 2; ++st)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) v[st][e] = (bf16)value(acc[rg][st][e] + b1[st][e], acc[rg][2 + st][e] + b2[st][e]);
+          const u32x4 out = eight_channels(v[0], v[1]);
+          if (on[rg] && n0 + c8 < w.n_main) *reinterpret_cast<u32x4*>(reinterpret_cast<bf16*>(mat.Y) + (size_t)m[rg] * w.ld + n0 + c8) = out;
+        }
+      };
+      const float limit = w.limit, slope = w.slope;
+      if (w.clamped) all([=](float a, float b) {
+        a = fminf(a, limit);
+        b = fminf(fmaxf(b, -limit), limit);
+        return a * quick_sigmoid(slope * a) * (b + 1.0f);
+      });
+      else all([](float a, float b) { return b * quick_swish(a); });
+    } else {
+      if (w.cap > 0.f || (w.act != PTA_ACT_NONE && (w.act != PTA_ACT_SIGMOID || w.out_f32))) return false;
+      if (!w.out_f32 && (w.mul || w.accumulate)) return false;
+      if (tail) {
+#pragma unroll
+        for (int st = 0; st < NST; ++st) {
+          const int c = c4 + st * 16 - w.n_main;
+          if (c < 0 || c >= w.tail_count) continue;
+          f32x4 add = {0.f, 0.f, 0.f, 0.f};
+          if (w.tail_bias) add = *reinterpret_cast<const f32x4*>(w.tail_bias + c);
+#pragma unroll
+          for (int rg = 0; rg < RG; ++rg)
+            if (on[rg]) *reinterpret_cast<f32x4*>(w.tail + (size_t)m[rg] * w.tail_count + c) = acc[rg][st] + add;
+        }
+      }
+      f32x4 b[NST];
+#pragma unroll
+      for (int st = 0; st < NST; ++st) b[st] = channels(w.bias, c4 + st * 16);
+      if (!w.out_f32) {
+        auto all = [&](auto value) {
+#pragma unroll
+          for (int rg = 0; rg < RG; ++rg)
+#pragma unroll
+            for (int p = 0; p < 2; ++p) {
+              bf16x4 v[2];
+#pragma unroll
+              for (int st = 0; st < 2; ++st)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) v[st][e] = (bf16)value(acc[rg][p * 2 + st][e] + b[p * 2 + st][e]);
+              const u32x4 out = eight_channels(v[0], v[1]);
+              if (on[rg] && n0 + p * 32 + c8 < w.n_main)
+                *reinterpret_cast<u32x4*>(reinterpret_cast<bf16*>(mat.Y) + (size_t)m[rg] * w.ld + n0 + p * 32 + c8) = out;
+            }
+        };
+        if (w.act == PTA_ACT_SIGMOID) all([](float v) { return quick_sigmoid(v); });
+        else all([](float v) { return v; });
+      } else {
+        // (some row groups at a time, as many as the registers hold: what they are multiplied by and added to is requested together)
+        constexpr int AT = RG == 4 ? 4 : 2;
+#pragma unroll
+        for (int h = 0; h < RG; h += AT) {
+          f32x4 old[AT][NST];
+          bf16x4 by[AT][NST];
+#pragma unroll
+          for (int i = 0; i < AT; ++i)
+#pragma unroll
+            for (int st = 0; st < NST; ++st) {
+              const bool in = on[h + i] && c4 + st * 16 < w.n_main;
+              const size_t at = (size_t)m[h + i] * w.ld + c4 + st * 16;
+              if (w.accumulate && in) old[i][st] = *reinterpret_cast<const f32x4*>(reinterpret_cast<const float*>(mat.Y) + at);
+              if (w.mul && in) by[i][st] = *reinterpret_cast<const bf16x4*>(reinterpret_cast<const bf16*>(w.mul) + at);
+            }
+#pragma unroll
+          for (int i = 0; i < AT; ++i)
+#pragma unroll
+            for (int st = 0; st < NST; ++st) {
+              f32x4 v;
+#pragma unroll
+              for (int e = 0; e < 4; ++e) {
+                v[e] = acc[h + i][st][e] + b[st][e];
+                if (w.mul) v[e] *= (float)by[i][st][e];
+                if (w.accumulate) v[e] += old[i][st][e];
+              }
+              if (on[h + i] && c4 + st * 16 < w.n_main) *reinterpret_cast<f32x4*>(reinterpret_cast<float*>(mat.Y) + (size_t)m[h + i] * w.ld + c4 + st * 16) = v;
+            }
+        }
+      }
+    }
+  }
+  return true;
+}
+
 // The sums of a wave's tile (RG row groups x NST channel blocks; lane l holds channels st * 16 + (l / 16) * 4 + r of
 // row l % 16 of each row group) go out: unit cw of the workgroup, first block blk0 of matrix `mat`, rows from row0 of M,
 // to the rows of Y that `order` lists (null: the same).
 template <class Fmt, int NST, int RG, bool PAIR>
 __device__ __forceinline__ void panel_store(const GemmMat& mat, const GemmEpilogue& epi, float* part, f32x4 (&acc)[RG][NST], unsigned char* smem, int cw, int blk0,
                                             int row0, int nsl, typename Fmt::Scale s0, typename Fmt::Scale s1, int M, const int32_t* order = nullptr) {
+  if (straight_store<Fmt, NST, RG, PAIR>(mat, epi, part, acc, blk0, row0, nsl, s0, s1, M, order)) return;
   constexpr int SW = NST * 16 + 4;                // floats per row of a wave's epilogue strip
   const int lane = threadIdx.x & 63;
   // Lane l holds channels st * 16 + (l / 16) * 4 + r of row l % 16 of each row group.  Row group by row group the

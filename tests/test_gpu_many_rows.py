@@ -410,3 +410,79 @@ def test_panels_of_a_pair_and_of_several_matrices():
     assert K.linear_kernel() == "gemm_panel_kernel"
     for (_, p), out in zip(ws, outs):
         close(out, x.double() @ p.T, x.double().abs() @ p.abs().T, Kd, 11)
+
+
+# The ends of gemm_block_kernel and gemm_panel_kernel: sizes that are stored straight from the registers (channels in eights, few kinds of ends) and
+# beside each one that is not; rows one past and one short of a row group, channels short of a wave's tile.
+ENDS = [(1025, 520, 2056), (1009, 520, 2052), (1039, 200, 2050), (4096, 40, 1000)]
+
+
+@pytest.mark.parametrize("kind", ["f16", "f8", "int4"])
+@pytest.mark.parametrize("M, Kd, N", ENDS)
+@pytest.mark.parametrize("bias, residual, act", [(0, 1, 0), (1, 0, 0), (1, 1, 0), (1, 1, 1)])
+def test_ends_of_half_results(kind, M, Kd, N, bias, residual, act):
+    from poptransformer_amd import _lib
+    from poptransformer_amd import kernels as K
+    x, w = operands(M, Kd, N, 41)
+    # (a channel of the FP8 weight holds +-120 and more five times: the sum stays below 5 * 240 * 5.5 * 0.02 = 132 and the square of it and a bias below 20000, where
+    # with x fifty times that it passes 65504)
+    x = (x * 0.02 if kind == "f8" else x).half()
+    if kind == "int4":
+        N = N // 8 * 8
+        w = w[:N]
+        scale = (w.abs().amax(1) / 7.0).half()
+        q = torch.clamp(torch.round(w / scale.float()[:, None]), -8, 7).to(torch.int8)
+        u = (q & 0xF).to(torch.uint8)
+        tw, plain = K.W4Weight(((u[:, 0::2] << 4) | u[:, 1::2]).view(torch.int8).contiguous(), scale), (q.half() * scale[:, None]).double()
+    else:
+        tw, plain = weight_of(kind, w)
+    b, r = torch.randn(N, device="cuda").half(), torch.randn((M, N), device="cuda").half()
+    out = torch.full((M, N), float("nan"), dtype=torch.float16, device="cuda")
+    K.linear(x, [tw], [out], bias=b if bias else None, residual=r if residual else None, act=_lib.ACT_RELU_SQUARE if act else _lib.ACT_NONE)
+    ref, mag = x.double() @ plain.T, x.double().abs() @ plain.abs().T
+    error = 2.0 ** -11 * ref.abs() + (Kd + 2) * 2.0 ** -24 * mag + 2.0 ** -24              # of the rounded sum, then of each step on it
+    if bias:
+        ref = ref + b.double()
+        error = error + 2.0 ** -11 * (ref.abs() + error)
+    if act:
+        ref, slope = torch.relu(ref) ** 2, 2 * torch.relu(ref)
+        error = error * (slope + error) + 2.0 ** -11 * (ref + error)
+    if residual:
+        ref = ref + r.double()
+        error = error + 2.0 ** -11 * (ref.abs() + error)
+    assert ((out.double() - ref).abs() <= error * 1.001 + 2.0 ** -23).all()
+
+
+@pytest.mark.parametrize("M, Kd, N", ENDS)
+@pytest.mark.parametrize("end", ["plain", "sigmoid", "gelu", "fp32", "added", "product", "cap", "pair", "clamped", "pair_biases"])
+def test_ends_of_wide_results(M, Kd, N, end):
+    from poptransformer_amd import _hybrid_lib as H
+    from poptransformer_amd import hybrid_kernels as HK
+    x, w = operands(M, Kd, 2 * N, 43)
+    x, w, F = x.bfloat16(), w.bfloat16(), torch.nn.functional
+    ld = HK.pad8(N)
+    made = [HK.WideWeight(w[i * N:(i + 1) * N].float(), torch.bfloat16, main_to=ld if "pair" in end or end == "clamped" else None) for i in (0, 1)]
+    g, u = (x.double() @ w[i * N:(i + 1) * N].double().T for i in (0, 1))
+    b1, b2 = torch.randn(ld, device="cuda"), torch.randn(ld, device="cuda")
+    f32 = end in ("fp32", "added", "product", "cap")
+    out = torch.randn((M, ld), device="cuda").to(torch.float32 if f32 else torch.bfloat16)
+    by, before = torch.randn((M, ld), device="cuda").bfloat16(), out.double()
+    kw = {"plain": {}, "sigmoid": dict(bias=b1, act=H.ACT_SIGMOID), "gelu": dict(act=H.ACT_GELU_TANH), "fp32": dict(bias=b1), "cap": dict(cap=1.5),
+          "added": dict(bias=b1, accumulate=True), "product": dict(mul=by, accumulate=True), "pair": dict(up=made[1], pair=H.PAIR_SWIGLU),
+          "clamped": dict(up=made[1], pair=H.PAIR_CLAMPED, limit=1.25, slope=1.7), "pair_biases": dict(up=made[1], pair=H.PAIR_SWIGLU, bias=b1, bias2=b2)}[end]
+    if N % 8 and end in ("sigmoid", "fp32", "added"):                                       # (a bias has a number for every main channel)
+        kw["bias"] = b1[:N].contiguous()
+    HK.linear(x, made[0], out, M, ld=ld, **kw)
+    v, up, B1, B2 = g, u, b1[:N].double(), b2[:N].double()
+    ref = {"plain": lambda: v, "sigmoid": lambda: torch.sigmoid(v + B1), "gelu": lambda: F.gelu(v, approximate="tanh"), "fp32": lambda: v + B1,
+           "cap": lambda: 1.5 * torch.tanh(v / 1.5), "added": lambda: before[:, :N] + v + B1, "product": lambda: before[:, :N] + v * by[:, :N].double(),
+           "pair": lambda: F.silu(v) * up, "pair_biases": lambda: F.silu(v + B1) * (up + B2),
+           "clamped": lambda: v.clamp(max=1.25) * torch.sigmoid(1.7 * v.clamp(max=1.25)) * (up.clamp(-1.25, 1.25) + 1)}[end]()
+    # sums of K products (numbers of about 0.05 sqrt(K)) in fp32, at most multiplied by the other factor; one rounding to bf16
+    factor = 1 + (by[:, :N].double().abs() if end == "product" else (v.abs() + up.abs() + 4) if "pair" in end or end == "clamped" else 1)
+    mag = (x.double().abs() @ w[:N].double().abs().T).amax()
+    bound = (0 if f32 else 2.0 ** -8) * ref.abs() + (Kd + 8) * 2.0 ** -24 * mag * factor + 4 * 2.0 ** -24 * ref.abs() + 2.0 ** -24
+    worst = ((out[:, :N].double() - ref).abs() / bound).max().item()
+    assert worst <= 1.0, worst
+    if ld > N and "pair" not in end and end != "clamped":
+        assert torch.equal(out[:, N:].double(), before[:, N:])                              # columns past the last channel are left alone
