@@ -70,8 +70,7 @@ class LatentMixing(Angles):
                 places.append(np.arange(first, first + n, dtype=np.int32))
                 zero += [at - first] * -(-count // H.LATENT_TILE)
                 at += n
-            flat = torch.from_numpy(np.concatenate(slots + places + [np.array(zero, np.int32)])).to(self.dev)
-            slot, pos, tile_key = torch.split(flat, [at, at, len(zero)])
+            slot, pos, tile_key = self._on_device(np.concatenate(slots), np.concatenate(places), np.array(zero, np.int32))
             lists[window] = ((slot, pos), (*rows.tiles[:2], tile_key))
         return lists[window]
 

@@ -93,10 +93,9 @@ class SequenceStore:
 
     def restart(self, slots):
         """The given slots hold a sequence without tokens."""
-        for layer, store in zip(self.spec.layers, self.stores):
-            if layer.mixer.kind in ("mlstm", "ssd"):
-                for slot in slots:
-                    store[0][slot].zero_()
+        states = [store[0][slot] for layer, store in zip(self.spec.layers, self.stores) if layer.mixer.kind in ("mlstm", "ssd") for slot in slots]
+        if states:
+            torch._foreach_zero_(states)     # (a launch for all layers of a slot, or of several)
         for slot in slots:
             self.length[slot] = 0
 
