@@ -2474,8 +2474,8 @@ __global__ __launch_bounds__(PANEL_WAVES * 64) __attribute__((amdgpu_waves_per_e
 
 // ------------------------------------------------------------------------------------------
 // Variant for hundreds of rows of formats with more than one vector per tile (16-bit and FP8 weights): both operands
-// through LDS.  A workgroup of 8 waves (2 row halves x 4 channel quarters) owns 32 * RG rows and 256 channels (a
-// pair: 128 gate and 128 up channels); loads that write LDS directly bring stages of Fmt::kStage features of both.
+// through LDS.  A workgroup of 8 waves owns 256, 192 or 128 rows and 256 channels (a pair: 128 gate and 128 up channels), or 128 rows and
+// 128 channels; loads that write LDS directly bring stages of Fmt::kStage features of both.
 // At 256 x 256 a 64-feature step is 64 KiB for 8.4 MFLOP, a quarter of the bytes per product that gemm_rows_kernel's
 // workgroups (256 x 128, weights through registers) take.
 // What bounds it: the matrix unit at the clock that the power leaves (1.7 GHz in long launches), and the loads.  A step of 64
@@ -2485,8 +2485,14 @@ __global__ __launch_bounds__(PANEL_WAVES * 64) __attribute__((amdgpu_waves_per_e
 // Channels need not divide: blocks past a matrix's last one lie past its descriptor and read as zeros.
 // ------------------------------------------------------------------------------------------
 constexpr int BLOCK_WAVES = 8;
-constexpr int BLOCK_CB = 16;                 // channel blocks of a workgroup
-constexpr double BLOCK_STEP_256 = 1.6, BLOCK_STEP_128 = 0.92;      // us of a step of 64 features (measured, all compute units at work)
+// The tile of a wave's RG row groups x 4 channel blocks: 2 x 4 waves of 8, 6 or 4 groups (256, 192 or 128 rows by 256 channels), or 4 x 2 of 2 (128 x 128)
+constexpr int block_row_parts(int rg) { return rg == 2 ? 4 : 2; }
+constexpr int block_rows(int rg) { return block_row_parts(rg) * rg * 16; }
+constexpr int block_cb(int rg) { return 8 / block_row_parts(rg) * 4; }         // channel blocks of a workgroup
+// us of a step of 64 features (measured, all compute units at work; the smaller tiles of weights that are decoded read their operands more often),
+// and of a tile's begin and end
+constexpr double block_step_us(int rg, bool decoded) { return rg == 8 ? 1.6 : rg == 6 ? (decoded ? 1.3 : 1.25) : rg == 4 ? 0.92 : decoded ? 0.74 : 0.6; }
+constexpr double block_ends_us(int rg) { return rg == 8 ? 9.0 : rg == 6 ? 7.5 : rg == 4 ? 6.0 : 5.0; }
 
 // v, of which the compiler no longer knows where it is from
 __device__ __forceinline__ u32x4 as_computed(u32x4 v) {
@@ -2499,30 +2505,37 @@ __device__ __forceinline__ u32x4 as_computed(u32x4 v) {
   return v;
 }
 
+// row loads (of 1 KiB) per wave and stage
 template <class Fmt>
-constexpr int block_stage_bytes(int rg) { return rg * 32 * Fmt::kStage * 2 + BLOCK_CB * Fmt::kVec * 8 * Fmt::kStage; }
+constexpr int block_row_loads(int rg) { return (block_rows(rg) * Fmt::kStage * 2 + BLOCK_WAVES * 1024 - 1) / (BLOCK_WAVES * 1024); }
 template <class Fmt>
-constexpr int block_stages(int rg) { return 160 * 1024 / block_stage_bytes<Fmt>(rg) < 5 ? 160 * 1024 / block_stage_bytes<Fmt>(rg) : 5; }
+constexpr int block_stage_bytes(int rg) { return block_row_loads<Fmt>(rg) * BLOCK_WAVES * 1024 + block_cb(rg) * Fmt::kVec * 8 * Fmt::kStage; }
+template <class Fmt>
+constexpr int block_stages(int rg) {
+  const int most = rg == 2 ? 8 : 5, fit = 160 * 1024 / block_stage_bytes<Fmt>(rg);      // (a small tile's stages go by in half the time)
+  return fit < most ? fit : most;
+}
 
 template <class Fmt, int RG, bool PAIR, class Rows = AllRows>
 __global__ __launch_bounds__(BLOCK_WAVES * 64) __attribute__((amdgpu_waves_per_eu(2, 2))) void gemm_block_kernel(GemmArgs a, int group0, int groups, int row_blocks, Rows rows) {
   constexpr int KV = Fmt::kVec, NST = 4;
   constexpr int SF = Fmt::kStage;                 // features of a stage: 32 or 64
   constexpr int WVEC = KV * 8 * SF;               // bytes of a channel block's features of a stage
-  constexpr int ROWS = RG * 32;
-  constexpr int XB = ROWS * SF * 2;               // bytes of a stage's rows
-  constexpr int STAGE = XB + BLOCK_CB * WVEC;
+  constexpr int ROWS = block_rows(RG), WR = block_row_parts(RG), WC = BLOCK_WAVES / WR;
+  constexpr int CB = block_cb(RG), BPW = CB / BLOCK_WAVES;      // channel blocks of the workgroup, and how many a wave brings
+  constexpr int XL = block_row_loads<Fmt>(RG);    // row loads per wave and stage
+  constexpr int XB = XL * BLOCK_WAVES * 1024;     // bytes of a stage's rows (rounded up to whole loads)
+  constexpr int STAGE = XB + CB * WVEC;
   constexpr int NS = block_stages<Fmt>(RG);
   constexpr int PPR = SF / 8;                     // 16-byte pieces of a row
   constexpr int RPL = 64 / PPR;                   // rows of a load
-  constexpr int XL = ROWS / RPL / BLOCK_WAVES;    // row loads per wave and stage
-  constexpr int WL = WVEC / 1024;                 // loads per channel block; a wave brings two blocks
-  constexpr int LOADS = XL + 2 * WL;
+  constexpr int WL = WVEC / 1024;                 // loads per channel block
+  constexpr int LOADS = XL + BPW * WL;
   constexpr int WAIT = (NS - 2) * LOADS;          // loads that may be on their way when a stage must have landed
-  static_assert((SF == 32 || SF == 64) && WVEC % 1024 == 0 && XL >= 1 && NS >= 2 && WAIT < 16, "stages");
+  static_assert((SF == 32 || SF == 64) && WVEC % 1024 == 0 && NS >= 2 && WAIT < 16 && STAGE == block_stage_bytes<Fmt>(RG), "stages");
   extern __shared__ __align__(16) unsigned char smem[];
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int wr = wave >> 2, wc = wave & 3;
+  const int wr = wave / WC, wc = wave % WC;
   const int K = a.K;
   // workgroup id -> tile as in gemm_panel_kernel: contiguous stretches of the tile list per die, the row block fastest
   int per = (int)gridDim.x / 8;
@@ -2549,11 +2562,11 @@ __global__ __launch_bounds__(BLOCK_WAVES * 64) __attribute__((amdgpu_waves_per_e
   if constexpr (!PAIR) {
 #pragma unroll
     for (int i = 0; i < 3; ++i) {
-      const int g = i < a.count ? (a.mat[i].N + 255) / 256 : 0;
+      const int g = i < a.count ? (a.mat[i].N + CB * 16 - 1) / (CB * 16) : 0;
       if (mi == i && i + 1 < a.count && group >= g) { group -= g; mi = i + 1; }
     }
   }
-  const int blk0 = group * (PAIR ? BLOCK_CB / 2 : BLOCK_CB);      // first block within its matrix
+  const int blk0 = group * (PAIR ? CB / 2 : CB);  // first block within its matrix
   // the slice's features in steps of 64
   const int nsl = a.ksplit > 1 ? a.ksplit : 1;
   const int all = (K + 63) / 64, per_slice = ((a.KT + nsl - 1) / nsl) * 2;
@@ -2561,12 +2574,12 @@ __global__ __launch_bounds__(BLOCK_WAVES * 64) __attribute__((amdgpu_waves_per_e
   const int last = first + per_slice < all ? first + per_slice : all;
   const int steps = last > first ? last - first : 0;
 
-  // this wave brings blocks 2 wave and 2 wave + 1 of the workgroup's sixteen (of a pair: eight gate, then eight up blocks)
+  // this wave brings blocks BPW * wave and on of the workgroup's (of a pair: first the gate's, then the up blocks)
   const GemmMat& wm = a.mat[PAIR ? wave >> 2 : mi];
-  const int wb = blk0 + 2 * (PAIR ? wave & 3 : wave);
+  const int wb = blk0 + BPW * (PAIR ? wave & 3 : wave);
   const uint32_t blk_bytes = (uint32_t)a.KT * (KV * 1024);
   int there = (wm.N + 15) / 16 - wb;
-  there = __builtin_amdgcn_readfirstlane(there < 0 ? 0 : there < 2 ? there : 2);
+  there = __builtin_amdgcn_readfirstlane(there < 0 ? 0 : there < BPW ? there : BPW);
   const unsigned char* wp = uniform_pointer(reinterpret_cast<const unsigned char*>(wm.tiled) + weight_at + (size_t)(there ? wb : 0) * blk_bytes);
   const __amdgpu_buffer_rsrc_t wres = __builtin_amdgcn_make_buffer_rsrc(const_cast<unsigned char*>(wp), 0, (int)(there * blk_bytes), 0x00020000);
   const f16* X = a.mat[mi].X ? a.mat[mi].X : a.X;
@@ -2593,12 +2606,13 @@ __global__ __launch_bounds__(BLOCK_WAVES * 64) __attribute__((amdgpu_waves_per_e
   auto bring = [&](int s, int at, int q) {
     const bool in = s < end;
     if (q < XL) {
-      const int off = Rows::kListed ? listed[q] : x0 + q * (BLOCK_WAVES * RPL * 2) * K;
+      int off = Rows::kListed ? listed[q] : x0 + q * (BLOCK_WAVES * RPL * 2) * K;
+      if (XL * BLOCK_WAVES * RPL > ROWS && (q * BLOCK_WAVES + wave) * RPL >= ROWS) off = -1;      // (rows that the tile does not have)
       __builtin_amdgcn_raw_ptr_buffer_load_lds(xres, (__attribute__((address_space(3))) void*)(smem + at + (q * BLOCK_WAVES + wave) * 1024), 16,
                                                in && s * SF + piece * 8 < K ? off : -1, s * (SF * 2), 0, 0);
     } else {
       const int b = (q - XL) / WL, v = (q - XL) % WL;
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(wres, (__attribute__((address_space(3))) void*)(smem + at + XB + (2 * wave + b) * WVEC + v * 1024), 16,
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(wres, (__attribute__((address_space(3))) void*)(smem + at + XB + (BPW * wave + b) * WVEC + v * 1024), 16,
                                                in ? (int)(b * blk_bytes) + lane * 16 : -1, s * WVEC + v * 1024, 0, 0);
     }
   };
@@ -2613,7 +2627,7 @@ __global__ __launch_bounds__(BLOCK_WAVES * 64) __attribute__((amdgpu_waves_per_e
   typedef typename Fmt::Piece Piece;              // a lane's bytes of a weight operand
   const int a_at = XB + (PAIR ? wc * 2 : wc * 4) * WVEC + lane * 16;
   auto a_piece = [&](int at, int m, int st) {
-    const int blk = PAIR ? st % 2 + (st / 2) * (BLOCK_CB / 2) : st;
+    const int blk = PAIR ? st % 2 + (st / 2) * (CB / 2) : st;
     return *reinterpret_cast<const Piece*>(smem + at + a_at + blk * WVEC + (SF == 64 ? Fmt::piece_at(m) : 0));
   };
   const int b_row = (wr * (RG * 16) + (lane & 15)) * (SF * 2);
@@ -2668,7 +2682,7 @@ __global__ __launch_bounds__(BLOCK_WAVES * 64) __attribute__((amdgpu_waves_per_e
         const f16x8 av = Fmt::operand(ahead[st]);
         ahead[st] = a_piece(nx, 1 - m, st);
 #pragma unroll
-        for (int r = 0; r < RG / 4; ++r) xf[1 - m][st * (RG / 4) + r] = b_operand(nx, 1 - m, st * (RG / 4) + r);
+        for (int r = st * RG / NST; r < (st + 1) * RG / NST; ++r) xf[1 - m][r] = b_operand(nx, 1 - m, r);
 #pragma unroll
         for (int rg = 0; rg < RG; ++rg) acc[rg][st] = Fmt::mma(av, xf[m][rg], acc[rg][st]);
         __builtin_amdgcn_sched_barrier(0);        // (the requests stay where they are)
@@ -2697,10 +2711,10 @@ static int reserve_gemm_block(const char* name) {
   return PTA_OK;
 }
 
-// channel groups of the launch
-static inline int block_groups(const GemmArgs& a, bool pair) {
+// channel groups of the launch, of `channels` each (of a pair: of half as many of both)
+static inline int block_groups(const GemmArgs& a, bool pair, int channels = 256) {
   int g = 0;
-  for (int i = 0; i < (pair ? 1 : a.count); ++i) g += pair ? (a.mat[i].N + 127) / 128 : (a.mat[i].N + 255) / 256;
+  for (int i = 0; i < (pair ? 1 : a.count); ++i) g += pair ? (a.mat[i].N + channels / 2 - 1) / (channels / 2) : (a.mat[i].N + channels - 1) / channels;
   return g;
 }
 
@@ -2709,7 +2723,7 @@ template <class Fmt, int RG, bool PAIR>
 static int launch_gemm_block(const GemmArgs& a, int group0, int group1, hipStream_t s, const char* name) {
   const int rc = reserve_gemm_block<Fmt, RG, PAIR, AllRows>(name);
   if (rc) return rc;
-  const int groups = group1 - group0, row_blocks = (a.M + RG * 32 - 1) / (RG * 32);
+  const int groups = group1 - group0, row_blocks = (a.M + block_rows(RG) - 1) / block_rows(RG);
   const int nsl = a.ksplit > 1 ? a.ksplit : 1;
   const int per = (groups * row_blocks + 7) / 8;
   gemm_kernel_taken = "gemm_block_kernel";
@@ -2733,43 +2747,57 @@ static int launch_gemm_block_listed(const GemmArgs& a, size_t x_rows, int max_ti
   return PTA_OK;
 }
 
-// How a launch is cut: the cheapest of 256 or 128 rows per workgroup, K in slices of workgroups (one matrix, a
-// workspace at hand), or the channel groups of the whole rounds with 256 rows and the rest with 128 - twice the workgroups, each half as long.
+// How a launch is cut: the cheapest of the four tiles, K in slices of workgroups (one matrix, a workspace at hand; tiles of 256 and 128 rows by 256
+// channels), or the channel groups of the whole rounds with 256 rows and the rest with a smaller tile - more workgroups, each shorter.
+// What bounds most launches of one to three rounds is the compute units that the last round leaves idle: 144 tiles of 256 x 256 keep 112 of
+// them from work, the same rows in 198 of 192 x 256 58; 64 tiles of 128 x 256 192, in 128 x 128 128 of them.  A smaller tile reads more
+// bytes of LDS a product (a step of 64 features, MFMAs alone 1.2, 0.9, 0.6, 0.3 us), so it wins by its rounds only.
+// us, with two tiles (256 and 128 by 256) and with four, weights from HBM: fp16, 1960 rows, 2048 x 2048 33.4 -> 25.0, 2048 x 4608 50.6 -> 45.0,
+// 5632 x 2048 73.2 -> 58.2; 300 rows, 4096 x 4096 53.1 -> 38.2; 1656 rows, 11008 x 2048 117 -> 90; pair of 5632 x 5632, 791 rows 126 -> 109;
+// bf16 pair of 11008 x 1024, 1100 rows 111 -> 76; F143, 2040 rows, 4096 x 4608 83.6 -> 77.9, 1601 rows, 5632 x 5632 118 -> 104.  Of 215 launches
+// of 140 to 2000 rows that changed their tile, the slowest ratio was 0.98 (bf16, 1837 rows, 3072 x 11008: 136 -> 139), the middle one 1.1.
+// Not kept: 192 rows with K in slices (F143, 1583 rows, 11008 x 2304 94 -> 146), 192 rows for the rest at 4 us (0.97 to 1.04; hence 8), as many
+// tiles of 192 as of 256 rows (three fp16 weights, 372 rows, 4288 x 7744 92 -> 99).
 template <class Fmt, bool PAIR>
 static int dispatch_gemm_block(const GemmArgs& a, hipStream_t s, const char* name) {
-  const int cus = device_compute_units(), groups = block_groups(a, PAIR);
-  const int blocks8 = (a.M + 255) / 256, blocks4 = (a.M + 127) / 128;
+  const int cus = device_compute_units(), groups = block_groups(a, PAIR), narrow = block_groups(a, PAIR, 128);
   const double steps = (a.K + 63) / 64;
-  auto cost = [&](bool tall, int tiles, int nsl) {
+  auto blocks = [&](int rg) { return (a.M + block_rows(rg) - 1) / block_rows(rg); };
+  auto cost = [&](int rg, int tiles, int nsl) {
     const double finish = nsl > 1 ? 5.0 + (double)a.M * a.mat[0].N * (4.0 * nsl + 6.0) / 4.5e6 : 0.0;
-    return ((tiles * nsl + cus - 1) / cus) * ((tall ? BLOCK_STEP_256 : BLOCK_STEP_128) * steps / nsl + (tall ? 9.0 : 6.0)) + finish;
+    return ((tiles * nsl + cus - 1) / cus) * (block_step_us(rg, Fmt::kVec == 2) * steps / nsl + block_ends_us(rg)) + finish;
   };
-  double best = cost(true, groups * blocks8, 1);
-  int how = 0, slices = 1;                        // 0: 256 rows, 1: 128 rows, 2: both
-  const double low = cost(false, groups * blocks4, 1);
-  if (low < best) { best = low; how = 1; }
-  const int whole = (groups * blocks8 / cus) * cus / blocks8;
-  if (whole > 0 && whole < groups) {
-    const double both = cost(true, whole * blocks8, 1) + cost(false, (groups - whole) * blocks4, 1) + 4.0;
-    if (both < best) { best = both; how = 2; }
+  const int whole = (groups * blocks(8) / cus) * cus / blocks(8);               // channel groups within whole rounds
+  double best = cost(8, groups * blocks(8), 1);
+  int rg = 8, rest = 0, slices = 1;               // the tile; that of the channel groups beyond the whole rounds (0: the same)
+  for (int r = 6; r >= 2; r -= 2) {
+    const double c = cost(r, (r == 2 ? narrow : groups) * blocks(r), 1);
+    if (r == 6 && blocks(8) > 1 && blocks(6) == blocks(8)) continue;            // (as many tiles: what a tile of 256 rows lacks it does not load either)
+    if (c < best) { best = c; rg = r; rest = 0; }
+    if (whole == 0 || whole >= groups || (r == 2 && !PAIR && a.count > 1)) continue;      // (several matrices: their groups are counted differently)
+    const double both = cost(8, whole * blocks(8), 1) + cost(r, (r == 2 ? narrow - 2 * whole : groups - whole) * blocks(r), 1) + (r == 6 ? 8.0 : 4.0);
+    if (both < best) { best = both; rg = 8; rest = r; }
   }
   if (!PAIR && a.count == 1 && a.part)
     for (int nsl = 2; nsl <= GEMM_MAX_KSPLIT; ++nsl) {
       if (a.KT < nsl * 4 || a.part_bytes < (size_t)nsl * a.M * a.mat[0].N * sizeof(float)) break;
-      for (int low_rows = 0; low_rows < 2; ++low_rows) {
-        const double c = cost(!low_rows, groups * (low_rows ? blocks4 : blocks8), nsl);
-        if (c < best) { best = c; how = low_rows; slices = nsl; }
+      for (int r = 8; r >= 4; r -= 4) {
+        const double c = cost(r, groups * blocks(r), nsl);
+        if (c < best) { best = c; rg = r; rest = 0; slices = nsl; }
       }
     }
   GemmArgs b = a;
   b.ksplit = slices;
-  int rc;
-  if (how == 2) {
-    rc = launch_gemm_block<Fmt, 8, PAIR>(b, 0, whole, s, name);
-    if (!rc) rc = launch_gemm_block<Fmt, 4, PAIR>(b, whole, groups, s, name);
-  } else {
-    rc = how == 0 ? launch_gemm_block<Fmt, 8, PAIR>(b, 0, groups, s, name) : launch_gemm_block<Fmt, 4, PAIR>(b, 0, groups, s, name);
-  }
+  auto launch = [&](int r, int group0, int group1) {                            // groups of 256 channels; to the last one: -1
+    switch (r) {
+      case 8: return launch_gemm_block<Fmt, 8, PAIR>(b, group0, group1 < 0 ? groups : group1, s, name);
+      case 6: return launch_gemm_block<Fmt, 6, PAIR>(b, group0, group1 < 0 ? groups : group1, s, name);
+      case 4: return launch_gemm_block<Fmt, 4, PAIR>(b, group0, group1 < 0 ? groups : group1, s, name);
+      default: return launch_gemm_block<Fmt, 2, PAIR>(b, 2 * group0, group1 < 0 ? narrow : 2 * group1, s, name);
+    }
+  };
+  int rc = launch(rg, 0, rest ? whole : -1);
+  if (!rc && rest) rc = launch(rest, whole, -1);
   if (rc) return rc;
   PTA_CHECK_LAUNCH(name);
   return PTA_OK;

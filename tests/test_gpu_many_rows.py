@@ -486,3 +486,48 @@ def test_ends_of_wide_results(M, Kd, N, end):
     assert worst <= 1.0, worst
     if ld > N and "pair" not in end and end != "clamped":
         assert torch.equal(out[:, N:].double(), before[:, N:])                              # columns past the last channel are left alone
+
+
+# gemm_block_kernel's tiles of 192 rows and of 128 x 128, alone and behind whole rounds of 256 rows: rows one past a tile, channels short of a block and of a tile
+TILES = [("one", 1537, 200, 5000), ("one", 385, 72, 5003), ("one", 1921, 1032, 8195), ("pair", 257, 200, 11000), ("pair", 385, 520, 1500),
+         ("pair", 1537, 1032, 5000), ("pair", 1921, 2056, 6152), ("three", 1153, 200, 2051), ("three", 577, 136, 1030), ("three", 1921, 2056, 4100)]
+
+
+@pytest.mark.parametrize("kind", ["f16", "f8", "bf16"])
+@pytest.mark.parametrize("form, M, Kd, N", TILES)
+def test_tiles_of_other_sizes(kind, form, M, Kd, N):
+    from poptransformer_amd import hybrid_kernels as HK
+    from poptransformer_amd import kernels as K
+    if kind == "bf16" and form == "three":
+        pytest.skip("the wide entry point takes several weights of few rows only")
+    x, w = operands(M, Kd, {"one": 1, "pair": 2, "three": 3}[form] * N, 51)
+    parts = [w[i * N:(i + 1) * N] for i in range(w.shape[0] // N)]
+    if kind == "bf16":
+        x, ld = x.bfloat16(), HK.pad8(N)
+        plains = [p.bfloat16().double() for p in parts]
+        tws = [HK.WideWeight(p, torch.bfloat16, main_to=ld if form == "pair" else None) for p in parts]
+        out = torch.full((M, ld), float("nan"), dtype=torch.bfloat16 if form == "pair" else torch.float32, device="cuda")
+        if form == "pair":
+            from poptransformer_amd import _hybrid_lib as H
+            HK.linear(x, tws[0], out, M, ld=ld, up=tws[1], pair=H.PAIR_SWIGLU)
+        else:
+            HK.linear(x, tws[0], out, M, ld=ld)
+        outs = [out[:, :N]]
+    else:
+        x = (x * 0.02 if kind == "f8" and form == "pair" else x).half()                     # (as in test_pair: the product stays far below 65504)
+        tws, plains = zip(*(weight_of(kind, p) for p in parts))
+        outs = [torch.full((M, N), float("nan"), dtype=torch.float16, device="cuda") for _ in range(3 if form == "three" else 1)]
+        K.linear(x, list(tws), outs * 2 if form == "pair" else outs, swiglu=form == "pair")
+        assert K.linear_kernel() == "gemm_block_kernel"
+    if form != "pair":
+        for out, plain in zip(outs, plains):
+            close(out, x.double() @ plain.T, x.double().abs() @ plain.abs().T, Kd, 24 if kind == "bf16" else 11)
+        return
+    gate, upv = (x.double() @ p.T for p in plains)
+    silu = torch.nn.functional.silu(gate)
+    unit = 0.0 if kind == "bf16" else 2.0 ** -11                                            # (fp16 results are rounded before the activation as well)
+    dg, du = (unit * t.abs() + (Kd + 2) * 2.0 ** -24 * (x.double().abs() @ p.abs().T) for t, p in ((gate, plains[0]), (upv, plains[1])))
+    # as in test_pair: the slope of silu is below 1.1; swish and the product are rounded
+    last = 2.0 ** -8 if kind == "bf16" else 2.5 * 2.0 ** -11
+    bound = 1.1 * dg * (upv.abs() + du) + du * silu.abs() + last * (silu * upv).abs() + 2.0 ** -20 * (1 + upv.abs())
+    assert ((outs[0].double() - silu * upv).abs() <= bound).all()
