@@ -109,6 +109,20 @@ typedef struct pta_fusion {
 } pta_fusion;
 
 size_t pta_linear_workspace_bytes(int M, int N);
+
+/* The norm of a product's rows that pta_linear_then_norm does behind it. */
+typedef struct pta_row_norm {
+  int norm;                    /* PTA_NORM_RMS or PTA_NORM_LAYER                                              */
+  const pta_half* weight;      /* [N]                                                                         */
+  const pta_half* bias;        /* [N], PTA_NORM_LAYER only                                                    */
+  float eps;
+  pta_half* y;                 /* [M, N]: the normed rows; with a shift it may be NULL                         */
+  const int32_t* grid_scale;   /* NULL, or (PTA_NORM_RMS) the cast of pta_rmsnorm_fp8_grid                     */
+  int grid_format;
+  pta_half* prev;              /* NULL, or (PTA_NORM_LAYER) the shift of pta_layer_norm_ce_mix: [M, N],        */
+  const pta_half* mix[3];      /* its mixing vectors [N] (the first one is needed)                             */
+  pta_half* mixed[3];          /* and their results [M, N]                                                     */
+} pta_row_norm;
 /* the name of the kernel that the calling thread's last product took, "" before the first (a product of several launches: the last one's) */
 const char* pta_linear_kernel(void);
 
@@ -404,6 +418,11 @@ typedef struct pta_weight {
 int pta_linear(const pta_half* X, const int32_t* x_scale, int count, const pta_weight* host_w,
                const pta_half* const* host_bias, pta_half* const* host_Y, int M, int swiglu,
                const pta_fusion* fuse, pta_stream_t stream);
+
+/* pta_linear of one weight, then pta_rmsnorm, pta_rmsnorm_fp8_grid, pta_layer_norm_ce or pta_layer_norm_ce_mix of Y's rows: bit-identical to the
+ * two calls.  Where the product's K is split across workgroups (fuse->workspace), adding the slices and the norm are one launch. */
+int pta_linear_then_norm(const pta_half* X, const int32_t* x_scale, const pta_weight* host_w, const pta_half* bias, pta_half* Y, int M,
+                         const pta_fusion* fuse, const pta_row_norm* host_norm, pta_stream_t stream);
 
 /* out = up * swish(gate), two fp16 ops (models/llama2/mlp.py:22-26): the unfused form of the
  * SwiGLU pair, for gate/up weights that cannot share a launch. */

@@ -69,6 +69,11 @@ class Fusion(ctypes.Structure):
                 ("mix_state", c_void_p), ("mix_step", c_void_p)]
 
 
+class RowNorm(ctypes.Structure):
+    _fields_ = [("norm", c_int), ("weight", c_void_p), ("bias", c_void_p), ("eps", c_float), ("y", c_void_p), ("grid_scale", c_void_p),
+                ("grid_format", c_int), ("prev", c_void_p), ("mix", c_void_p * 3), ("mixed", c_void_p * 3)]
+
+
 # name -> (restype, argtypes); the order follows include/poptransformer_hip.h
 SIGNATURES = {
     "pta_version": (c_int, []),
@@ -132,6 +137,7 @@ SIGNATURES = {
     "pta_half_to_fp8_grid": (c_int, [c_void_p, c_void_p, c_void_p, c_size_t, c_int, c_void_p]),
     "pta_linear": (c_int, [c_void_p, c_void_p, c_int, POINTER(Weight), POINTER(c_void_p), POINTER(c_void_p), c_int, c_int,
                            POINTER(Fusion), c_void_p]),
+    "pta_linear_then_norm": (c_int, [c_void_p, c_void_p, POINTER(Weight), c_void_p, c_void_p, c_int, POINTER(Fusion), POINTER(RowNorm), c_void_p]),
     "pta_swiglu": (c_int, [c_void_p, c_void_p, c_void_p, c_size_t, c_void_p]),
     "pta_rwkv_mix": (c_int, [c_void_p] * 8 + [c_int, c_int, c_void_p]),
     "pta_layer_norm_ce_mix": (c_int, [c_void_p] * 11 + [c_int, c_int, c_float, c_void_p]),

@@ -7,6 +7,7 @@
 #pragma once
 #include "common.h"
 #include "f8codec.h"
+#include "norm_core.h"
 
 // Where and how a product of a "wide" format goes: one fp32 value per output, rounded once where it is stored.
 struct WideOut {
@@ -262,6 +263,15 @@ static inline void wide_skip_rows(GemmMat& mat, int m0) {
   if (w.mul) w.mul = reinterpret_cast<const unsigned char*>(w.mul) + (size_t)m0 * w.ld * (w.mul_f32 ? 4 : 2);
 }
 
+// A norm of the result's rows behind the product: where K was split the launch that adds the slices does it (done), else whoever asked for it.
+struct FinishNorm {
+  NormArgs norm;
+  NormMix mix;
+  int mode;            // of norm_row
+  bool shifted;        // with the mix
+  bool done;
+};
+
 struct GemmArgs {
   GemmMat mat[4];
   int count;
@@ -276,6 +286,7 @@ struct GemmArgs {
   size_t part_bytes;
   int ksplit;          // 0 or 1: no split
   int prefer_stream;   // host side: up to 16 rows go to gemv_stream_kernel wherever it fits
+  FinishNorm* then;    // host side: see there, or null
 };
 // v, read from memory at this point and kept in scalar registers
 template <class T>
@@ -1316,9 +1327,91 @@ __global__ __launch_bounds__(256) void splitk_finish_kernel(GemmArgs a) {
   }
 }
 
+// The same with the norm of the finished rows behind it, a row a workgroup: the rows' sums are read once, and the norm's launch and its reading of
+// the rows are gone.  What bounds it at few rows is the chain of a row (32 rows of 4096, four slices, residual, gate and three mixes: 9.6 -> 6.1 us), at many the
+// bytes (1000 rows, two slices: 17.1 -> 11.0).  Every operation is that of the two kernels, in their order.
+template <class Fmt, int VECS>
+struct FinishedRow {
+  const GemmArgs& a;
+  size_t total, at;                               // numbers of a slice, and the row's first
+  typename Fmt::Scale scale;
+  f32x4 sums[VECS][GEMM_MAX_KSPLIT][2];
+  f16x8 add[VECS][4];                             // bias of the weight, of the epilogue, factor, residual
+  // (Loads without a branch round them, where paths meet the compiler waits for what is in flight: a slice that there is not reads the last one
+  // again, what is not added the old result.)
+  __device__ __forceinline__ void request(int i, int c) {
+    const size_t n = (size_t)c * 8;
+#pragma unroll
+    for (int sl = 0; sl < GEMM_MAX_KSPLIT; ++sl) {
+      const float* from = a.part + (sl < a.ksplit ? sl : a.ksplit - 1) * total + at + n;
+      sums[i][sl][0] = *reinterpret_cast<const f32x4*>(from);
+      sums[i][sl][1] = *reinterpret_cast<const f32x4*>(from + 4);
+    }
+    const f16* const old = a.mat[0].Y + at;
+    const f16* const from[4] = {a.mat[0].bias ? a.mat[0].bias : old, a.epi.bias ? a.epi.bias : old, a.epi.mul ? a.epi.mul + at : old,
+                                a.epi.residual ? a.epi.residual + at : old};
+#pragma unroll
+    for (int k = 0; k < 4; ++k) add[i][k] = *reinterpret_cast<const f16x8*>(from[k] + n);
+  }
+  __device__ __forceinline__ f16x8 value(int i, int c) const {
+    const GemmMat& mat = a.mat[0];
+    f16x8 out;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      float t = 0.f;
+#pragma unroll
+      for (int sl = 0; sl < GEMM_MAX_KSPLIT; ++sl)
+        if (sl < a.ksplit) t += sums[i][sl][e >> 2][e & 3];
+      f16 y = (f16)Fmt::finish(t, scale);
+      if (mat.bias) y = y + add[i][0][e];
+      if (a.epi.bias) y = y + add[i][1][e];
+      if (a.epi.mul) y = y * add[i][2][e];
+      if (a.epi.residual) y = y + add[i][3][e];
+      if (a.epi.post_scale != 0.0f) y = y * (f16)a.epi.post_scale;
+      out[e] = y;
+    }
+    *reinterpret_cast<f16x8*>(mat.Y + at + (size_t)c * 8) = out;
+    return out;
+  }
+};
+
+template <class Fmt, int MODE, bool MIX, int VECS>
+__global__ __launch_bounds__(NORM_THREADS) void splitk_finish_norm_kernel(GemmArgs a, NormArgs norm, NormMix mix) {
+  const int N = a.mat[0].N;
+  // (no format's finish uses the per-channel part of its scale)
+  FinishedRow<Fmt, VECS> row{a, (size_t)a.M * N, (size_t)blockIdx.x * N, Fmt::load_scale(a.mat[0].scale, a.x_scale, 0, 1)};
+  norm_row<MODE, MIX, VECS>(norm, mix, blockIdx.x, row);
+}
+
+template <class Fmt, int VECS>
+static void launch_finish_norm(const GemmArgs& a, const FinishNorm& t, hipStream_t s) {
+  if (t.mode == 0) hipLaunchKernelGGL((splitk_finish_norm_kernel<Fmt, 0, false, VECS>), dim3(a.M), dim3(NORM_THREADS), 0, s, a, t.norm, t.mix);
+  else if (t.shifted) hipLaunchKernelGGL((splitk_finish_norm_kernel<Fmt, 2, true, VECS>), dim3(a.M), dim3(NORM_THREADS), 0, s, a, t.norm, t.mix);
+  else hipLaunchKernelGGL((splitk_finish_norm_kernel<Fmt, 2, false, VECS>), dim3(a.M), dim3(NORM_THREADS), 0, s, a, t.norm, t.mix);
+}
+
+template <class Fmt>
+static bool launch_splitk_finish_norm(const GemmArgs& a, hipStream_t s) {
+  const GemmMat& mat = a.mat[0];
+  FinishNorm* t = a.then;
+  const void* whole[] = {mat.Y, mat.bias, a.epi.bias, a.epi.mul, a.epi.residual};
+  for (const void* p : whole)
+    if (p && !pta_aligned(p, 16)) return false;
+  // (no activation: a row's sixteen of each kind are more instructions than the rest of the kernel)
+  if (t->norm.cols != mat.N || a.epi.out_fp8_scale || mat.act != PTA_ACT_NONE || a.epi.act != PTA_ACT_NONE || t->mode == 1 || a.ksplit > GEMM_MAX_KSPLIT) return false;
+  // (as few pieces of a thread as the row needs: what a row is made of stays in registers)
+  if (mat.N <= 8 * NORM_THREADS) launch_finish_norm<Fmt, 1>(a, *t, s);
+  else if (mat.N <= 16 * NORM_THREADS) launch_finish_norm<Fmt, 2>(a, *t, s);
+  else launch_finish_norm<Fmt, 4>(a, *t, s);
+  return t->done = true;
+}
+
 template <class Fmt>
 static void launch_splitk_finish(const GemmArgs& a, hipStream_t s) {
   const size_t total = (size_t)a.M * a.mat[0].N;
+  if constexpr (!Fmt::kWide) {
+    if (a.then && launch_splitk_finish_norm<Fmt>(a, s)) return;
+  }
   // (four channels of a row at once where no four cross its end and Y's vectors are whole)
   if (a.mat[0].N % 4 == 0 && (Fmt::kWide || pta_aligned(a.mat[0].Y, 8)))
     hipLaunchKernelGGL((splitk_finish_kernel<Fmt, 4>), dim3((unsigned)((total / 4 + 255) / 256)), dim3(256), 0, s, a);
@@ -2947,6 +3040,7 @@ template <class Fmt, bool PAIR>
 static int rows_in_turn(const GemmArgs& a, int chunk, int total_nb, hipStream_t s, const char* name) {
   for (int m0 = 0; m0 < a.M; m0 += chunk) {
     GemmArgs b = a;
+    b.then = nullptr;
     b.M = a.M - m0 < chunk ? a.M - m0 : chunk;
     if (b.X) b.X += (size_t)m0 * a.K;
     for (int i = 0; i < a.count; ++i) {

@@ -42,7 +42,7 @@ static int f8n_panel_min_rows() {
 // an exponent (x_scale) that are not known to lie on the F143 grid (they keep to the fp16 instruction)
 static int linear_impl(const void* X, const int32_t* x_scale, int x_bytes, int count, const pta_weight* host_w,
                        const pta_half* const* host_bias, pta_half* const* host_Y, int M, int swiglu,
-                       const pta_fusion* fuse, pta_stream_t stream) {
+                       const pta_fusion* fuse, pta_stream_t stream, FinishNorm* then = nullptr) {
   PTA_REQUIRE(host_w && host_Y, "pta_linear: null pointer");
   PTA_REQUIRE(count >= 1 && count <= 4, "pta_linear: count must be in [1, 4], got %d", count);
   PTA_REQUIRE(!swiglu || count == 2, "pta_linear: a SwiGLU pair is exactly two weights (gate, up)");
@@ -52,6 +52,7 @@ static int linear_impl(const void* X, const int32_t* x_scale, int x_bytes, int c
   for (int i = 0; i < count; ++i) PTA_REQUIRE(X || host_w[i].x, "pta_linear: entry %d has no input", i);
   PTA_REQUIRE(kind >= PTA_W_INT4 && kind <= PTA_W_F152, "pta_linear: unknown weight kind %d", kind);
   GemmArgs a{};
+  a.then = then;
   a.count = count; a.X = (const f16*)X; a.x_scale = x_scale; a.M = M; a.K = K; a.KT = (K + 127) / 128;
   PTA_REQUIRE(!x_scale || kind == PTA_W_F143 || kind == PTA_W_F152, "pta_linear: x_scale is only meaningful with FP8 weights");
   int nb = 0;
@@ -126,6 +127,33 @@ extern "C" int pta_linear(const pta_half* X, const int32_t* x_scale, int count, 
                           const pta_half* const* host_bias, pta_half* const* host_Y, int M, int swiglu,
                           const pta_fusion* fuse, pta_stream_t stream) {
   return linear_impl(X, x_scale, 0, count, host_w, host_bias, host_Y, M, swiglu, fuse, stream);
+}
+
+extern "C" int pta_linear_then_norm(const pta_half* X, const int32_t* x_scale, const pta_weight* host_w, const pta_half* bias, pta_half* Y, int M,
+                                    const pta_fusion* fuse, const pta_row_norm* host_norm, pta_stream_t stream) {
+  const char* name = "pta_linear_then_norm";
+  PTA_REQUIRE(host_w && Y && host_norm, "%s: null pointer", name);
+  const pta_row_norm& n = *host_norm;
+  const bool shifted = n.prev != nullptr;
+  PTA_REQUIRE(n.norm == PTA_NORM_RMS || n.norm == PTA_NORM_LAYER, "%s: unknown norm %d", name, n.norm);
+  PTA_REQUIRE(!shifted || n.norm == PTA_NORM_LAYER, "%s: a token shift follows a LayerNorm", name);
+  PTA_REQUIRE(!n.grid_scale || n.norm == PTA_NORM_RMS, "%s: the FP8 grid follows an RMSNorm", name);
+  PTA_REQUIRE(!(fuse && fuse->out_fp8_scale), "%s: the rows to be normed are left as they are", name);
+  const int cols = host_w->N;
+  int rc = check_norm(name, Y, n.weight, shifted ? n.prev : n.y, M, cols);
+  if (rc) return rc;
+  if (n.norm == PTA_NORM_LAYER) rc = check_layer_norm(name, n.bias, cols);
+  if (!rc && n.grid_scale) rc = check_grid(name, n.grid_scale, n.grid_format);
+  if (!rc && shifted) rc = check_norm_mix(name, n.y, n.mix, n.mixed);
+  if (rc) return rc;
+  FinishNorm then{NormArgs{(const f16*)n.weight, (const f16*)n.bias, (f16*)n.y, cols, n.eps, n.grid_scale, n.grid_format}, NormMix{},
+                  n.norm == PTA_NORM_RMS ? 0 : M == 1 ? 1 : 2, shifted, false};
+  if (shifted) then.mix = NormMix{(f16*)n.prev, {(const f16*)n.mix[0], (const f16*)n.mix[1], (const f16*)n.mix[2]}, {(f16*)n.mixed[0], (f16*)n.mixed[1], (f16*)n.mixed[2]}};
+  rc = linear_impl(X, x_scale, 0, 1, host_w, &bias, &Y, M, 0, fuse, stream, &then);
+  if (rc || then.done) return rc;
+  launch_norm((const f16*)Y, M, then.mode, then.norm, shifted ? &then.mix : nullptr, (hipStream_t)stream);
+  PTA_CHECK_LAUNCH(name);
+  return PTA_OK;
 }
 
 extern "C" const char* pta_linear_kernel(void) { return gemm_kernel_taken; }

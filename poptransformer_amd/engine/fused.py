@@ -165,6 +165,21 @@ class LayerOps:
         self._norm(x, gb, self.h)
         return self.h, None
 
+    def _added_and_normed(self, x, lw, gb, consumers):
+        """self.x += lw(x); then as `_normed` of self.x.  One call where lw's K may be split: adding the slices and the norm are one launch there."""
+        if self._lin_ws is None or self.fuse_norm:
+            self._linear(x, lw, self.x, residual=self.x)
+            return self._normed(self.x, gb, consumers)
+        xin, xs, _ = self._lhs(x, lw, None)
+        self._on_grid.pop(self.x.data_ptr(), None)
+        grid = self._common_grid(consumers) if self.spec.norm == "rms" else None
+        out = self.h if grid is None else self._fp8_buf[self.x.shape[1]]
+        K.linear_then_norm(xin, lw.w, self.x, K.RowNorm(gb[0], gb[1] if self.spec.norm == "ln" else None, self.spec.eps, out=out, grid=grid), x_scale=xs,
+                           bias=lw.bias, residual=self.x, workspace=self._lin_ws)
+        if grid is not None:
+            self._on_grid[out.data_ptr()] = self._grid_id(consumers[0])
+        return out, None
+
     @staticmethod
     def _grid_id(lw):
         """Identifies the FP8 grid an FP8 Linear casts its input to: format and exponent (by value when the
@@ -364,13 +379,13 @@ class FusedDecoder(DecodeLoop, LayerOps):
         B = s.batch
         K.embedding(w.embed, self.container, self.x, pos_table=w.pos_embed,
                     pos=self.step if w.pos_embed is not None else None, ids_index=self.step)
+        h, nrm = self._normed(self.x, w.blocks[0].norm1, w.blocks[0].qkv)
         for li, blk in enumerate(w.blocks):
             if not hasattr(self, "_qkv_views"):
                 self._prepare_qkv_views(blk)
             probe = self.probe                           # diagnostics of eager iterations: callable(name, block, tensor(s))
             if probe is not None:
                 probe("block_in", li, self.x)
-            h, nrm = self._normed(self.x, blk.norm1, blk.qkv)
             self._linear_group(h, blk.qkv, self._qkv_bufs, nrm)
             if probe is not None:
                 probe("projections", li, self._qkv_bufs)
@@ -383,18 +398,17 @@ class FusedDecoder(DecodeLoop, LayerOps):
                                    kv_scale=self.kv_scale, out_grid=grid)
             if grid is not None:
                 self._on_grid[self.ctx.data_ptr()] = self._grid_id(blk.out)
-            self._linear(self.ctx, blk.out, self.x, residual=self.x)
+            h, nrm = self._added_and_normed(self.ctx, blk.out, blk.norm2, blk.mlp_in)
             if probe is not None:
                 probe("after_attention", li, self.x)
-            h, nrm = self._normed(self.x, blk.norm2, blk.mlp_in)
             if len(blk.mlp_in) == 2:
                 self._linear_group(h, blk.mlp_in, [self.act, self.act], nrm, swiglu=True, consumer=blk.mlp_out)
             else:
                 self._linear(h, blk.mlp_in[0], self.act, act=_lib.ACT_GELU_TANH, norm=nrm)
-            self._linear(self.act, blk.mlp_out, self.x, residual=self.x)
+            last = li + 1 == len(w.blocks)
+            h, nrm = self._added_and_normed(self.act, blk.mlp_out, w.final_norm if last else w.blocks[li + 1].norm1, [w.head] if last else w.blocks[li + 1].qkv)
         if self.probe is not None:                       # ... and the stream leaving the last block
             self.probe("block_in", len(w.blocks), self.x)
-        h, nrm = self._normed(self.x, w.final_norm, [w.head])
         self._linear(h, w.head, self.logits, norm=nrm)
         self.select(self.logits, self.next_ids)
         K.step_update(self.container, self.mask, self.stop_mask, self.step, self.next_ids, None, self.keep_going,

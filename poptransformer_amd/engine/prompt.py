@@ -62,20 +62,22 @@ class PromptPass(LayerOps):
         K.embedding(w.embed, ids, self.x)
         if w.pos_embed is not None:        # GPT-2: learned positions, one table row per position
             self.x.add_(w.pos_embed.index_select(0, positions).repeat(B, 1))
+        h, nrm = self._normed(self.x, w.blocks[0].norm1, w.blocks[0].qkv)
         for li, blk in enumerate(w.blocks):
             if not hasattr(self, "_qkv_views"):
                 self._prepare_qkv_views(blk)
-            h, nrm = self._normed(self.x, blk.norm1, blk.qkv)
             self._linear_group(h, blk.qkv, self._qkv_bufs, nrm)
             qp, kp, vp, qs, ks, vs = self._qkv_views
             K.prompt_rope_append(qp, kp, vp, self.q_rot, dec.rings[li], self.first, w.inv_freq, B, R, s.n_head,
                                  s.n_kv_head, s.head_dim, s.max_len, s.rope, qs, ks, vs, kv_scale=dec.kv_scale)
             K.prompt_attention(self.q_rot, dec.rings[li], self.first, self.attn_ws, self.ctx, B, R, s.n_head,
                                s.n_kv_head, s.head_dim, s.max_len, s.scale_scores, kv_scale=dec.kv_scale)
-            self._linear(self.ctx, blk.out, self.x, residual=self.x)
-            h, nrm = self._normed(self.x, blk.norm2, blk.mlp_in)
+            h, nrm = self._added_and_normed(self.ctx, blk.out, blk.norm2, blk.mlp_in)
             if len(blk.mlp_in) == 2:
                 self._linear_group(h, blk.mlp_in, [self.act, self.act], nrm, swiglu=True, consumer=blk.mlp_out)
             else:
                 self._linear(h, blk.mlp_in[0], self.act, act=_lib.ACT_GELU_TANH, norm=nrm)
-            self._linear(self.act, blk.mlp_out, self.x, residual=self.x)
+            if li + 1 < len(w.blocks):
+                h, nrm = self._added_and_normed(self.act, blk.mlp_out, w.blocks[li + 1].norm1, w.blocks[li + 1].qkv)
+            else:
+                self._linear(self.act, blk.mlp_out, self.x, residual=self.x)

@@ -136,23 +136,30 @@ class RWKVDecoder(DecodeLoop):
                 self._shifted(x, blk.ln1, [blk.att_key, blk.att_value, blk.att_receptance], blk.att_mix, self.st_att[i],
                               [self.k, self.v, self.r], [_lib.ACT_NONE, _lib.ACT_NONE, _lib.ACT_SIGMOID])
             else:
-                K.layer_norm_ce_mix(x, blk.ln1[0], blk.ln1[1], s.eps, self.st_att[i], blk.att_mix, self.mix)
+                if i == 0 or blk.pre_ln is not None:         # (else with the product before)
+                    K.layer_norm_ce_mix(x, blk.ln1[0], blk.ln1[1], s.eps, self.st_att[i], blk.att_mix, self.mix)
                 self._group(self.mix, [blk.att_key, blk.att_value, blk.att_receptance], [self.k, self.v, self.r],
                             [_lib.ACT_NONE, _lib.ACT_NONE, _lib.ACT_SIGMOID])
             K.rwkv_wkv(self.k, self.v, self.r, blk.time_decay, blk.time_first, self.st_num[i], self.st_den[i],
                        self.st_max[i], self.y)
-            K.linear(self.y, [blk.att_output.w], [x], residual=x, workspace=self._lin_ws)
             if self.fuse_shift:
+                K.linear(self.y, [blk.att_output.w], [x], residual=x, workspace=self._lin_ws)
                 self._shifted(x, blk.ln2, [blk.ffn_key, blk.ffn_receptance], blk.ffn_mix, self.st_ffn[i], [self.fk, self.fr],
                               [_lib.ACT_RELU_SQUARE, _lib.ACT_SIGMOID])
             else:
-                K.layer_norm_ce_mix(x, blk.ln2[0], blk.ln2[1], s.eps, self.st_ffn[i], blk.ffn_mix, self.mix[:2])
+                K.linear_then_norm(self.y, blk.att_output.w, x, K.RowNorm(blk.ln2[0], blk.ln2[1], s.eps, shift=(self.st_ffn[i], blk.ffn_mix, self.mix[:2])),
+                                   residual=x, workspace=self._lin_ws)
                 self._group(self.mix[:2], [blk.ffn_key, blk.ffn_receptance], [self.fk, self.fr],
                             [_lib.ACT_RELU_SQUARE, _lib.ACT_SIGMOID])
             halve = s.rescale_every > 0 and (i + 1) % s.rescale_every == 0
-            K.linear(self.fk, [blk.ffn_value.w], [x], mul=self.fr, residual=x, post_scale=0.5 if halve else 0.0,
-                     workspace=self._lin_ws)
-        K.layer_norm_ce(x, w.ln_out[0], w.ln_out[1], s.eps, self.h)
+            end = dict(mul=self.fr, residual=x, post_scale=0.5 if halve else 0.0, workspace=self._lin_ws)
+            if i + 1 == s.n_layer:
+                K.linear_then_norm(self.fk, blk.ffn_value.w, x, K.RowNorm(w.ln_out[0], w.ln_out[1], s.eps, out=self.h), **end)
+            elif self.fuse_shift or w.blocks[i + 1].pre_ln is not None:
+                K.linear(self.fk, [blk.ffn_value.w], [x], **end)
+            else:
+                ln, mixes = w.blocks[i + 1].ln1, w.blocks[i + 1].att_mix
+                K.linear_then_norm(self.fk, blk.ffn_value.w, x, K.RowNorm(ln[0], ln[1], s.eps, shift=(self.st_att[i + 1], mixes, self.mix)), **end)
         K.linear(self.h, [w.head.w], [self.logits])
         self.select(self.logits, self.next_ids)
         K.step_update(self.container, None, self.stop_mask, self.step, self.next_ids, None, self.keep_going,

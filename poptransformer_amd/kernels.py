@@ -310,6 +310,37 @@ def linear(x, weights, outs, biases=None, x_scale=None, swiglu=False, bias=None,
     return outs
 
 
+class RowNorm:
+    """The norm that `linear_then_norm` does behind a product: `rmsnorm`, `rmsnorm_fp8_grid` (grid = (exponent, format)), `layer_norm_ce` (beta) or
+    `layer_norm_ce_mix` (shift = (previous rows, mixing vectors, results)), into `out`."""
+
+    def __init__(self, gamma, beta, eps, out=None, grid=None, shift=None):
+        prev, mixes, mixed = shift if shift is not None else (None, (), ())
+        for t, what in [(gamma, "gamma"), (beta, "beta"), (out, "out"), (prev, "previous rows")] + [(t, "mixing vector") for t in mixes] + [(t, "mixed rows") for t in mixed]:
+            if t is not None:
+                _need(t, torch.float16, what)
+        self.cols = gamma.numel()
+        self.rows = [t for t in (out, prev, *mixed) if t is not None]
+        V = ctypes.c_void_p * 3
+        self.args = _lib.RowNorm(_lib.NORM_RMS if beta is None else _lib.NORM_LAYER, _p(gamma), _p(beta), eps, _p(out), _p(grid[0]) if grid else None,
+                                 _fmt(grid[1]) if grid else 0, _p(prev), V(*[_p(t) for t in mixes]), V(*[_p(t) for t in mixed]))
+        self._keep = (gamma, beta, out, grid, shift)
+
+
+def linear_then_norm(x, w, out, then, x_scale=None, bias=None, residual=None, act=_lib.ACT_NONE, mul=None, post_scale=0.0, workspace=None):
+    """`linear` of one weight, then the norm `then` (a RowNorm) of its result's rows: one launch does the end of both where K is split."""
+    _need(x, torch.float16, "x", 2)
+    M = x.shape[0]
+    if w.K != x.shape[1]:
+        raise ValueError(f"matmul: contracting dimensions differ ({x.shape[1]} vs {w.K})")
+    if then.cols != w.N or any(t.numel() < M * w.N for t in then.rows):
+        raise ValueError(f"linear_then_norm: a norm of {then.cols} columns behind [{M}, {w.N}], or too few rows for its results")
+    desc = _desc(w, None, _lib.ACT_NONE, None)
+    check(_lib.load().pta_linear_then_norm(_p(x), _p(x_scale), ctypes.byref(desc), None, _p(out), M, _fusion(bias, residual, act, None, mul, post_scale, workspace),
+                                           ctypes.byref(then.args), _stream()))
+    return out
+
+
 def swiglu(gate, up, out=None):
     _need(gate, torch.float16, "gate")
     _need(up, torch.float16, "up")

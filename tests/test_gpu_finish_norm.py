@@ -1,0 +1,74 @@
+"""pta_linear_then_norm against pta_linear and the norm's own entry point, bit for bit: products whose K is split (the slices are added and the rows
+normed by one launch) and products whose K is not."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def weight(kind, N, Kd, g):
+    from poptransformer_amd import kernels as K
+    w = torch.randn((N, Kd), generator=g, device="cuda") * 0.05
+    if kind == "f16":
+        return K.F16Weight(w.half())
+    if kind == "int4":
+        return K.W4Weight(torch.randint(-128, 128, (N, Kd // 2), generator=g, device="cuda").to(torch.int8), (torch.rand(N, generator=g, device="cuda") * 0.01).half())
+    scale = torch.tensor([-1], dtype=torch.int32, device="cuda")
+    return K.F8Weight(K.half_to_fp8(w.half(), scale, kind), scale, kind)
+
+
+# rows, features, channels, whether K is split where there is a workspace: the fewest and the most columns of a row, rows one past a tile, no split
+SHAPES = {"int4": [(32, 16384, 4096, True), (17, 8192, 8, None), (257, 8192, 2048, None), (1000, 11008, 4096, True), (20, 256, 4096, False)],
+          "f16": [(33, 8192, 1032, None), (300, 4104, 1024, None), (129, 16384, 8184, None), (5, 4096, 4096, False)],
+          "F143": [(1020, 13704, 4096, True), (40, 13696, 4096, None), (200, 4096, 2048, None)],
+          "F152": [(64, 8192, 2056, None)]}
+
+
+@pytest.mark.parametrize("kind, M, Kd, N, split", [(k, *s) for k, shapes in SHAPES.items() for s in shapes])
+@pytest.mark.parametrize("form", ["rms", "grid", "layer", "shift"])
+def test_as_the_two_calls(kind, M, Kd, N, split, form):
+    from poptransformer_amd import kernels as K
+    g = torch.Generator(device="cuda").manual_seed(61)
+    x = torch.randn((M, Kd), generator=g, device="cuda").half() * 0.1
+    w = weight(kind, N, Kd, g)
+
+    def rows(*shape):
+        return torch.randn(shape, generator=g, device="cuda").half()
+    gamma, beta, bias, mul, res, prev = rows(N), rows(N), rows(N), rows(M, N), rows(M, N), rows(M, N)
+    mixes, exponent = [rows(N) for _ in range(3)], torch.tensor([-2], dtype=torch.int32, device="cuda")
+    ends = {"rms": dict(residual=res), "grid": dict(bias=bias, residual=res), "layer": dict(bias=bias), "shift": dict(mul=mul, residual=res, post_scale=0.5)}[form]
+    got, ref, out, one = (torch.full((M, N), float("nan"), dtype=torch.float16, device="cuda") for _ in range(4))
+    mixed, plain, before = [torch.empty_like(got) for _ in range(3)], [torch.empty_like(got) for _ in range(3)], prev.clone()
+    workspace = K.linear_workspace(M, N, "cuda")
+    workspace.fill_(0xFF)
+    then = {"rms": lambda: K.RowNorm(gamma, None, 1e-5, out=out), "grid": lambda: K.RowNorm(gamma, None, 1e-5, out=out, grid=(exponent, "F143")),
+            "layer": lambda: K.RowNorm(gamma, beta, 1e-5, out=out), "shift": lambda: K.RowNorm(gamma, beta, 1e-5, out=out, shift=(prev, mixes[:2], mixed[:2]))}[form]()
+    K.linear_then_norm(x, w, got, then, workspace=workspace, **ends)
+    if split is not None:
+        assert split == (not torch.equal(workspace, torch.full_like(workspace, 0xFF)))
+    K.linear(x, [w], [ref], workspace=workspace, **ends)
+    if form == "rms":
+        K.rmsnorm(ref, gamma, 1e-5, one)
+    elif form == "grid":
+        K.rmsnorm_fp8_grid(ref, gamma, 1e-5, exponent, "F143", out=one)
+    elif form == "layer":
+        K.layer_norm_ce(ref, gamma, beta, 1e-5, one)
+    else:
+        K.layer_norm_ce_mix(ref, gamma, beta, 1e-5, before, mixes[:2], plain[:2], out=one)
+        assert torch.equal(prev, before) and all(torch.equal(a, b) for a, b in zip(mixed[:2], plain[:2]))
+    assert not torch.isnan(got).any() and torch.equal(got, ref) and torch.equal(out, one)
+
+
+def test_what_is_refused():
+    from poptransformer_amd import kernels as K
+    g = torch.Generator(device="cuda").manual_seed(3)
+    x, w = torch.randn((20, 256), generator=g, device="cuda").half(), weight("f16", 64, 256, g)
+    out, gamma = torch.empty((20, 64), dtype=torch.float16, device="cuda"), torch.ones(64, dtype=torch.float16, device="cuda")
+    with pytest.raises(ValueError):
+        K.linear_then_norm(x, w, out, K.RowNorm(gamma[:56].contiguous(), None, 1e-5, out=torch.empty_like(out)))
+    with pytest.raises(ValueError):
+        K.linear_then_norm(x, w, out, K.RowNorm(gamma, None, 1e-5, out=torch.empty((19, 64), dtype=torch.float16, device="cuda")))
+    with pytest.raises(ValueError):
+        K.linear_then_norm(x, w, out, K.RowNorm(gamma, None, 1e-5))
+    with pytest.raises(ValueError):
+        K.linear_then_norm(x, w, out, K.RowNorm(gamma, gamma, 1e-5, out=torch.empty_like(out), grid=(torch.zeros(1, dtype=torch.int32, device="cuda"), "F143")))
