@@ -581,6 +581,24 @@ typedef struct pta_add_parts_args {
 
 int pta_add_parts(const pta_add_parts_args* host_args, pta_stream_t stream);
 
+/* pta_add_parts, own := gelu(h gate^T) * own, y = own' proj^T and pta_depth_norm with that y as one launch, for few bf16 rows (h stays inside).
+ * add.h and norm.y are not used; add.x is the newest depth of norm's history. */
+typedef struct pta_depth_end_args {
+  pta_add_parts_args add;
+  pta_depth_norm_args norm;
+  int side;               /* features of the token's own part: a multiple of 8                                     */
+  const void* gate;       /* [side, width] tiled by pta_bf16_tile                                                  */
+  const void* own;        /* [rows, side] bf16                                                                     */
+  const void* proj;       /* [width, side] tiled by pta_bf16_tile                                                  */
+  void* workspace;        /* 64-byte aligned, zeroed once after it is allocated; launches with it follow each other */
+  size_t workspace_bytes;
+} pta_depth_end_args;
+
+/* Bytes of the workspace; 0 for what pta_depth_end does not take (up to 4 rows of up to 8192, up to 1024 features).  Rows, width and
+ * features of all launches with one workspace are the same. */
+size_t pta_depth_end_workspace_bytes(int rows, int width, int side);
+int pta_depth_end(const pta_depth_end_args* host_args, pta_stream_t stream);
+
 /* ---- Next-token selection over fp32 logits, and the loop's bookkeeping -------------------------------------------- */
 int pta_argmax_f32(const float* logits, int32_t* ids, float* values, int rows, int n, pta_stream_t stream);
 int pta_topk_f32(const float* logits, int32_t* ids, float* values, int rows, int n, int k, pta_stream_t stream);

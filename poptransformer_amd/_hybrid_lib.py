@@ -87,6 +87,8 @@ DepthNormArgs = _struct("DepthNormArgs", [
 AddPartsArgs = _struct("AddPartsArgs", [
     ("dtype", _I), ("rows", _I), ("width", _I), ("x", _P), ("parts", _P), ("n_parts", _I), ("parts_ld", _I), ("part_f32", _I),
     ("part_weight", _P), ("weights_ld", _I), ("h", _P), ("h_ld", _I)])
+DepthEndArgs = _struct("DepthEndArgs", [
+    ("add", AddPartsArgs), ("norm", DepthNormArgs), ("side", _I), ("gate", _P), ("own", _P), ("proj", _P), ("workspace", _P), ("workspace_bytes", c_size_t)])
 ExpertWeights = _struct("ExpertWeights", [("W", _P), ("W2", _P), ("K", _I), ("N", _I), ("n_main", _I), ("pair", _I), ("limit", _F), ("slope", _F)])
 ExpertsArgs = _struct("ExpertsArgs", [
     ("dtype", _I), ("rows", _I), ("experts", _I), ("top", _I), ("choices", _I), ("chosen", _P), ("X", _P), ("ld_x", _I),
@@ -123,6 +125,8 @@ SIGNATURES = {
     "pta_gated_norm": (_I, [POINTER(GatedNormArgs), _P]),
     "pta_depth_norm": (_I, [POINTER(DepthNormArgs), _P]),
     "pta_add_parts": (_I, [POINTER(AddPartsArgs), _P]),
+    "pta_depth_end_workspace_bytes": (c_size_t, [_I, _I, _I]),
+    "pta_depth_end": (_I, [POINTER(DepthEndArgs), _P]),
     "pta_mlstm_state_floats": (c_size_t, [_I, _I, _I]),
     "pta_mlstm_workspace_bytes": (c_size_t, [POINTER(MlstmArgs)]),
     "pta_mlstm": (_I, [POINTER(MlstmArgs), _P]),

@@ -116,6 +116,7 @@ class DepthBuffers(LatentBuffers, ExpertBuffers):
         self.logits = {n: buf(rows, n, dtype=F32) for n in {lw.router.shape[0] for lw in layers if lw.router is not None}}
         channels = max([spec.width] + [w.N for lw in layers for w in lw.linears()])
         self.workspace = HK.linear_workspace(rows, channels, device) if rows > 16 else None
+        self.end_workspace = HK.depth_end_workspace(rows, spec.width, weights.side.shape[2], dtype, device)      # (None: more rows than a layer's end takes at once)
 
 
 class DepthDecoder(HeadMixing, LatentMixing, StateSpaceMixing, ExpertMixing, HybridDecoder):
@@ -178,12 +179,15 @@ class DepthDecoder(HeadMixing, LatentMixing, StateSpaceMixing, ExpertMixing, Hyb
                 parts = self._mixture(i, b, n, logits)
             elif layer.mlp is not None:
                 HK.linear(b.act[lw.up.n_main], lw.down, x, n, **add)
-            HK.add_parts(x, n, b.rounded, **parts)
-            HK.linear(b.rounded, lw.side_gate, b.side_act, n, act=H.ACT_GELU_TANH, mul=b.side[i], workspace=b.workspace)
-            HK.linear(b.side_act, lw.side_proj, b.y, n, ld=spec.width, workspace=b.workspace)
             going_on = i + 1 < depths or self.probe is not None
-            HK.depth_norm(b.history, i + 2, weights=lw.average, y=b.y, y_weight=lw.side_norm, next=i + 2 if going_on else None,
-                          **ahead(i + 1), **common)
+            end = dict(weights=lw.average, y_weight=lw.side_norm, next=i + 2 if going_on else None, **ahead(i + 1), **common)
+            if b.end_workspace is not None and n == b.rows:
+                HK.depth_end(x, n, b.rounded, parts, lw.side_gate, b.side[i], lw.side_proj, (b.history, i + 2, end), b.end_workspace)
+            else:
+                HK.add_parts(x, n, b.rounded, **parts)
+                HK.linear(b.rounded, lw.side_gate, b.side_act, n, act=H.ACT_GELU_TANH, mul=b.side[i], workspace=b.workspace)
+                HK.linear(b.side_act, lw.side_proj, b.y, n, ld=spec.width, workspace=b.workspace)
+                HK.depth_norm(b.history, i + 2, y=b.y, **end)
             if self.probe is not None:
                 self.probe(i, b.history[i + 2, :n].clone())
         return b, None

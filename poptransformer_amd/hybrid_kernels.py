@@ -472,8 +472,8 @@ def result_norm(x, rows, eps, h, weight=None, table=None, embed_scale=1.0, ids=N
 
 
 def depth_norm(history, depth, rows, eps, h, norm_weight, centred=True, weights=None, y=None, y_weight=None, next=None, table=None, embed_scale=1.0,
-               ids=None, ids_index=None, pos_out=None, side_table=None, side=None, router=None, routing=None, correction=None):
-    """The end of a layer (pta_depth_norm).  history fp32 [depths, R, width], of which the first `depth` count; next: the index in it
+               ids=None, ids_index=None, pos_out=None, side_table=None, side=None, router=None, routing=None, correction=None, launch=True):
+    """The end of a layer (pta_depth_norm; launch False: its arguments).  history fp32 [depths, R, width], of which the first `depth` count; next: the index in it
     that gets the average; side_table [vocab, layers, ld], side [layers, R, ld]."""
     width = history.shape[-1]
     _need(history, F32, "history")
@@ -482,6 +482,9 @@ def depth_norm(history, depth, rows, eps, h, norm_weight, centred=True, weights=
     _need(h, h.dtype, "h", rows * h.shape[-1])
     _need(norm_weight, F32, "norm_weight", width)
     a = H.DepthNormArgs(_CODE[h.dtype], rows, width, _p(history), history.shape[1] * width, depth)
+    if y is None and y_weight is not None and not launch:
+        _need(y_weight, F32, "y_weight", width)
+        a.y_weight = _p(y_weight)
     if weights is not None:
         _need(weights, F32, "weights", depth)
         a.weights = _p(weights)
@@ -506,11 +509,13 @@ def depth_norm(history, depth, rows, eps, h, norm_weight, centred=True, weights=
     if router is not None:
         _need(router, h.dtype, "router", (routing.experts + routing.shared) * h.shape[-1])
         a.router, a.routing = _p(router), routing.args(rows, correction)
+    if not launch:
+        return a
     H.check(H.load().pta_depth_norm(ctypes.byref(a), _stream()))
 
 
-def add_parts(x, rows, h, parts=None, n_parts=0, parts_ld=None, part_weight=None):
-    """x [R, width] fp32 += the weighted parts [rows, parts_ld, width]; h = x (pta_add_parts)."""
+def add_parts(x, rows, h, parts=None, n_parts=0, parts_ld=None, part_weight=None, launch=True):
+    """x [R, width] fp32 += the weighted parts [rows, parts_ld, width]; h = x (pta_add_parts; launch False: its arguments)."""
     width = x.shape[-1]
     _need(x, F32, "x", rows * width)
     _need(h, h.dtype, "h", rows * h.shape[-1])
@@ -524,7 +529,27 @@ def add_parts(x, rows, h, parts=None, n_parts=0, parts_ld=None, part_weight=None
         a.parts, a.n_parts, a.parts_ld, a.part_f32 = _p(parts), n_parts, parts_ld, int(parts.dtype == F32)
         a.part_weight, a.weights_ld = _p(part_weight), part_weight.shape[-1]
     a.h, a.h_ld = _p(h), h.shape[-1]
+    if not launch:
+        return a
     H.check(H.load().pta_add_parts(ctypes.byref(a), _stream()))
+
+
+def depth_end_workspace(rows, width, side, dtype, device):
+    """The workspace of `depth_end` for such rows (zeroed), or None where it does not take them."""
+    n = H.load().pta_depth_end_workspace_bytes(rows, width, side) if dtype == torch.bfloat16 else 0
+    return torch.zeros(n, dtype=torch.uint8, device=device) if n else None
+
+
+def depth_end(x, rows, h, parts, gate, own, proj, norm, workspace):
+    """`add_parts` (its keywords: parts), gelu(h gate^T) * own, the product of that with proj, and `depth_norm` (its arguments: norm, without y) in one launch."""
+    width, side = x.shape[-1], own.shape[-1]
+    if (gate.K, proj.K) != (h.shape[-1], side) or gate.n_main != side or proj.n_main != width or gate.dtype != torch.bfloat16 or proj.dtype != torch.bfloat16:
+        raise ValueError(f"the token's own part: weights [{gate.n_main}, {gate.K}] and [{proj.n_main}, {proj.K}] for rows of {width} and {side}")
+    _need(own, torch.bfloat16, "own", rows * side)
+    history, depth, kw = norm
+    a = H.DepthEndArgs(add_parts(x, rows, h, launch=False, **parts), depth_norm(history, depth, launch=False, **kw), side, _p(gate.data), _p(own), _p(proj.data),
+                       _p(workspace), workspace.numel())
+    H.check(H.load().pta_depth_end(ctypes.byref(a), _stream()))
 
 
 class ExpertWeight:
