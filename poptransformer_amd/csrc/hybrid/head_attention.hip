@@ -380,8 +380,8 @@ __global__ __launch_bounds__(256) void head_merge_kernel(HA a, const float* part
 }
 
 // ------------------------------------------------------------------------------------------
-// Many rows on the matrix unit (bf16, D and E up to 256): a workgroup of four waves takes 128 rows of one head, a wave 2 groups
-// of 16 queries - of two maps: 64 rows, the groups being the two maps of the same 16 rows, so that the values are read once.
+// Many rows on the matrix unit (bf16, D and E up to 256): a workgroup of four waves takes 64 rows of one head, a wave 16
+// queries - of two maps both, so that the values are read once.
 // 64 keys at a time pass through LDS.  S^T = K Q^T, O^T = V^T P^T.  A lane holds scores of ONE query, keys 16 t + 4 (lane / 16) +
 // 0..3 of every 16-key group t; two groups are the eight values of a B operand as they stand, and the transposed reads of V take
 // the keys in that order.
@@ -393,14 +393,15 @@ constexpr size_t head_tile_smem() { return (size_t)HT_KEYS * (MAPS * (DKT * 32 +
 
 template <int DKT, int DVT, int MAPS>
 __global__ __launch_bounds__(256) void head_tile_kernel(HA a) {
-  constexpr int QW = 2, RW = QW / MAPS * 16, KS = DKT * 32 + 8, VIT = (DVT + 1) / 2, VS = VIT * 32 + 8;
+  constexpr int QW = MAPS, RW = 16, KS = DKT * 32 + 8, VIT = (DVT + 1) / 2, VS = VIT * 32 + 8;
   extern __shared__ __align__(16) unsigned char head_tile_lds[];
   bf16* sk = reinterpret_cast<bf16*>(head_tile_lds);                   // [MAPS][HT_KEYS][KS]
   bf16* sv = sk + MAPS * HT_KEYS * KS;                                 // [HT_KEYS][VS]
   // of the distance from row n of the workgroup's to key k of a step, at k - n + (rows - 1): what is taken off the score
   __shared__ float far[HT_KEYS + 4 * RW];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, lg = lane >> 4, lc = lane & 15;
-  const int head = blockIdx.x, tile = blockIdx.y, skip = (int)blockIdx.z * 4 * RW;
+  // (a sequence's last rows, whose chain is the longest, first)
+  const int head = blockIdx.x, tile = (int)(gridDim.y - 1 - blockIdx.y), skip = (int)(gridDim.z - 1 - blockIdx.z) * 4 * RW;
   const int D = a.D, E = a.E, g = head / (a.H / a.G);
   int count = a.tile_count[tile] - skip;
   if (count <= 0) return;
@@ -537,31 +538,7 @@ __global__ __launch_bounds__(256) void head_tile_kernel(HA a) {
     }
     bf16x8 p[QW][2];
 #pragma unroll
-    for (int w = 0; w < QW; ++w) {
-      float top = mx[w];
-#pragma unroll
-      for (int t = 0; t < 4; ++t)
-#pragma unroll
-        for (int e = 0; e < 4; ++e) top = fmaxf(top, s[w][t][e]);
-      top = fmaxf(top, __shfl_xor(top, 16, 64));
-      top = fmaxf(top, __shfl_xor(top, 32, 64));
-      const float keep = exp2f(mx[w] - top);
-      mx[w] = top;
-      float sum = 0.f;
-#pragma unroll
-      for (int t = 0; t < 4; ++t)
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const float x = exp2f(s[w][t][e] - top);
-          sum += x;
-          p[w][t >> 1][(t & 1) * 4 + e] = (bf16)x;
-        }
-      l[w] = l[w] * keep + sum;
-#pragma unroll
-      for (int t = 0; t < DVT; ++t)
-#pragma unroll
-        for (int e = 0; e < 4; ++e) o[w][t][e] *= keep;
-    }
+    for (int w = 0; w < QW; ++w) softmax_step(s[w], mx[w], l[w], p[w], o[w]);
 #pragma unroll
     for (int kg = 0; kg < 2; ++kg) {
       const bf16* v = sv + (kg * 32 + lg * 4 + (lc >> 2)) * VS + (lc & 3) * 4;
@@ -701,7 +678,7 @@ static int launch_tiles(const HA& a, hipStream_t s) {
   static_assert(smem <= 160 * 1024, "LDS");
   PTA_REQUIRE(smem <= 64 * 1024 || hipFuncSetAttribute((const void*)head_tile_kernel<DKT, DVT, MAPS>, hipFuncAttributeMaxDynamicSharedMemorySize,
                                                        (int)smem) == hipSuccess, "pta_head_attention: %zu bytes of LDS refused", smem);
-  hipLaunchKernelGGL((head_tile_kernel<DKT, DVT, MAPS>), dim3(a.H, a.tiles, MAPS), dim3(256), smem, s, a);
+  hipLaunchKernelGGL((head_tile_kernel<DKT, DVT, MAPS>), dim3(a.H, a.tiles, 2), dim3(256), smem, s, a);
   return PTA_OK;
 }
 

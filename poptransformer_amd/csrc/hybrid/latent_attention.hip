@@ -500,23 +500,25 @@ __global__ __launch_bounds__(256) void latent_gather_kernel(LA a, int pieces, in
 }
 
 // ------------------------------------------------------------------------------------------
-// Many rows over per-head keys and values (bf16): a workgroup of four waves takes up to 128 rows of one head, a wave 2
-// groups of 16; 64 keys at a time pass through LDS.  S^T = K Q^T, O^T = V^T P^T.  A lane holds scores of ONE query, keys
+// Many rows over per-head keys and values (bf16): a workgroup of four waves takes up to 64 rows of one head, a wave a
+// group of 16; 64 keys at a time pass through LDS.  S^T = K Q^T, O^T = V^T P^T.  A lane holds scores of ONE query, keys
 // 16 t + 4 (lane / 16) + 0..3 of every 16-key group t; two groups are the eight values of a B operand as they stand, and
-// the transposed reads of V take the keys in that order.
+// the transposed reads of V take the keys in that order.  (128 rows a workgroup, two groups a wave: 2048 rows of 32 heads 108 us, now 94.)
 // ------------------------------------------------------------------------------------------
 constexpr int LT_KEYS = 64;
 
 template <int DKT, int DVT>
 __global__ __launch_bounds__(256) void latent_tile_kernel(LA a) {
-  constexpr int QW = 2, KS = DKT * 32 + 8, VS = DVT * 16 + 8, VIT = (DVT + 1) / 2;
+  constexpr int QW = 1, KS = DKT * 32 + 8, VS = DVT * 16 + 8, VIT = (DVT + 1) / 2;
   __shared__ __align__(16) bf16 sk[LT_KEYS * KS];
   __shared__ __align__(16) bf16 sv[LT_KEYS * (VIT * 32 + 8)];
   static_assert(VS == VIT * 32 + 8, "value blocks come in pairs");
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, lg = lane >> 4, lc = lane & 15;
-  const int head = blockIdx.x, tile = blockIdx.y;
+  const int head = blockIdx.x, tile = (int)(gridDim.y - 1 - blockIdx.y);      // (a sequence's last rows, whose chain is the longest, first)
   const int D = a.D, QD = a.D + a.P, E = a.E, ld = a.H * (D + E);
-  const int count = a.tile_count[tile], row0 = a.tile_row[tile], key0 = a.tile_key[tile];
+  const int skip = (int)(gridDim.z - 1 - blockIdx.z) * 64 * QW;
+  const int count = (a.tile_count[tile] - skip < 64 * QW ? a.tile_count[tile] - skip : 64 * QW), row0 = a.tile_row[tile] + skip, key0 = a.tile_key[tile];
+  if (count <= 0) return;
   const int p0 = position_of(a, row0);
   const bf16* kb = reinterpret_cast<const bf16*>(a.kv) + head * D;
   const bf16* vb = reinterpret_cast<const bf16*>(a.kv) + a.H * D + head * E;
@@ -584,6 +586,7 @@ __global__ __launch_bounds__(256) void latent_tile_kernel(LA a) {
     __syncthreads();
     if (jt + LT_KEYS <= i_last) fetch(jt + LT_KEYS);
     if (jt > w_last || jt + LT_KEYS - 1 < w_first - a.window + 1) continue;       // nothing this wave's rows see
+    const bool whole = jt + LT_KEYS - 1 <= w_first && jt > w_last - a.window;     // all of it, all of them
     f32x4 s[QW][4];
 #pragma unroll
     for (int t = 0; t < 4; ++t) {
@@ -599,33 +602,20 @@ __global__ __launch_bounds__(256) void latent_tile_kernel(LA a) {
     bf16x8 p[QW][2];
 #pragma unroll
     for (int w = 0; w < QW; ++w) {
-      float top = mx[w];
 #pragma unroll
       for (int t = 0; t < 4; ++t)
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const int dist = qi[w] - (jt + t * 16 + lg * 4 + e);
-          s[w][t][e] = dist >= 0 && dist < a.window ? s[w][t][e] * scale2 : -INFINITY;
-          top = fmaxf(top, s[w][t][e]);
-        }
-      top = fmaxf(top, __shfl_xor(top, 16, 64));
-      top = fmaxf(top, __shfl_xor(top, 32, 64));
-      const float keep = exp2f(mx[w] - top);
-      mx[w] = top;
-      float sum = 0.f;
+        for (int e = 0; e < 4; ++e) s[w][t][e] *= scale2;
+      if (!whole) {
 #pragma unroll
-      for (int t = 0; t < 4; ++t)
+        for (int t = 0; t < 4; ++t)
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const float x = exp2f(s[w][t][e] - top);
-          sum += x;
-          p[w][t >> 1][(t & 1) * 4 + e] = (bf16)x;
-        }
-      l[w] = l[w] * keep + sum;
-#pragma unroll
-      for (int t = 0; t < DVT; ++t)
-#pragma unroll
-        for (int e = 0; e < 4; ++e) o[w][t][e] *= keep;
+          for (int e = 0; e < 4; ++e) {
+            const int dist = qi[w] - (jt + t * 16 + lg * 4 + e);
+            if (!(dist >= 0 && dist < a.window)) s[w][t][e] = -INFINITY;
+          }
+      }
+      softmax_step(s[w], mx[w], l[w], p[w], o[w]);
     }
 #pragma unroll
     for (int kg = 0; kg < 2; ++kg) {
@@ -791,7 +781,7 @@ extern "C" int pta_latent_tiles_fit(int dtype, int D, int P, int E) { return dty
 
 template <int DKT>
 static void launch_latent_tiles(const LA& a, hipStream_t s) {
-  const dim3 grid(a.H, a.tiles);
+  const dim3 grid(a.H, a.tiles, PTA_LATENT_TILE / 64);
   if (a.E <= 64) hipLaunchKernelGGL((latent_tile_kernel<DKT, 4>), grid, dim3(256), 0, s, a);
   else if (a.E <= 128) hipLaunchKernelGGL((latent_tile_kernel<DKT, 8>), grid, dim3(256), 0, s, a);
   else hipLaunchKernelGGL((latent_tile_kernel<DKT, 16>), grid, dim3(256), 0, s, a);

@@ -251,30 +251,30 @@ __global__ __launch_bounds__(64) void window_merge_kernel(WA a, const float* par
 }
 
 // ------------------------------------------------------------------------------------------
-// Many rows on the matrix unit (bf16, D <= 32 * DT): a workgroup of four waves takes 64 * QW rows of one query head, a
-// wave QW groups of 16; 64 keys at a time pass through LDS, once as they are (the A operand of S^T = K Q^T) and once
-// transposed (the A operand of O^T = K^T P^T: the values are the keys).  A lane holds scores of ONE query, keys
-// 16 t + 4 (lane / 16) + 0..3 of every 16-key group t; two groups are the eight values of a B operand as they stand if
-// the transposed copy keeps its keys in that order: key 4 x + e of the first group of 32 goes to place 8 x + e, of the
-// second to 8 x + 4 + e.
+// Many rows on the matrix unit (bf16, D <= 32 * DT): a workgroup of four waves takes 64 rows of one query head, a
+// wave a group of 16; 64 keys at a time pass through LDS: the A operand of S^T = K Q^T as they are, of O^T = K^T P^T (the values are the keys) by
+// transposing reads.  A lane holds scores of ONE query, keys 16 t + 4 (lane / 16) + 0..3 of every 16-key group t; two groups are the eight
+// values of a B operand as they stand, and the transposed reads take the keys in that order.
+// What bounds it is a workgroup's chain, from its queries through the steps of the longest sequence: loads without branches round them (each such
+// branch waits for its load), softmax_step, no masks where a step is seen whole, no transposed copy (16 heads of 128, sequences of 700, 560, 420 and 280 rows:
+// 56 us with them, 43 without; 34 with 64 rows a workgroup, each operand read for one group of queries, where 128 rows were two: more chains side by side
+// are worth more than fewer reads, also at 2048 rows of 32 heads).
 // ------------------------------------------------------------------------------------------
 constexpr int WT_KEYS = 64;
-constexpr int WT_VSTRIDE = WT_KEYS + 8;
 
-template <int DT, int QW>
+template <int DT>
 __global__ __launch_bounds__(256) void window_tile_kernel(WA a, bool vec) {
-  constexpr int DM = DT * 32;
+  constexpr int QW = 1, DM = DT * 32;
   constexpr int KS = DM + 8;
   constexpr int CH = DM / 8;                              // 16-byte pieces of a key row
   constexpr int ITEMS = WT_KEYS / 2 * CH;                 // (pair of keys, piece)
   constexpr int IPT = (ITEMS + 255) / 256;
   __shared__ __align__(16) bf16 sk[WT_KEYS * KS];
-  __shared__ __align__(16) bf16 sv[DM * WT_VSTRIDE + DM];   // row d starts at d * WT_VSTRIDE + (d / 8) * 8
   __shared__ float sr[WT_KEYS];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, lg = lane >> 4, lc = lane & 15;
-  const int head = blockIdx.x, tile = blockIdx.y;
+  const int head = blockIdx.x, tile = (int)(gridDim.y - 1 - blockIdx.y);      // (a sequence's last rows, whose chain is the longest, first)
   const int D = a.D, Dp = padded8(D), g = head / (a.H / a.G);
-  const int skip = (int)blockIdx.z * 64 * QW;
+  const int skip = (int)(gridDim.z - 1 - blockIdx.z) * 64 * QW;
   const int count = a.tile_count[tile] - skip;
   if (count <= 0) return;
   const int row0 = a.tile_row[tile] + skip;
@@ -286,46 +286,69 @@ __global__ __launch_bounds__(256) void window_tile_kernel(WA a, bool vec) {
   // queries: lane holds features 32 m + 8 lg + 0..7 of row lc of each of its groups
   bf16x8 qf[QW][DT];
   int qi[QW];
+  const bf16* qrow[QW];
+  float rq[QW];
 #pragma unroll
   for (int w = 0; w < QW; ++w) {
     int n = (wave * QW + w) * 16 + lc;
     qi[w] = p0 + n;
     n = n < count ? n : count - 1;
-    const bf16* q = reinterpret_cast<const bf16*>(a.q) + (size_t)(row0 + n) * a.ld + head * D;
-    const float rq = a.q_scale[row0 + n] * a.scale * 1.4426950408889634f;
+    qrow[w] = reinterpret_cast<const bf16*>(a.q) + (size_t)(row0 + n) * a.ld + head * D;
+    rq[w] = a.q_scale[row0 + n] * a.scale * 1.4426950408889634f;
+  }
+  if (vec && D == DM) {                                   // whole pieces: requested without a branch, together
+    u32x4 raw[QW][DT];
+#pragma unroll
+    for (int w = 0; w < QW; ++w)
+#pragma unroll
+      for (int m = 0; m < DT; ++m) raw[w][m] = *reinterpret_cast<const u32x4*>(qrow[w] + m * 32 + lg * 8);
+    float wq[DT][8], wk[DT][8];
 #pragma unroll
     for (int m = 0; m < DT; ++m) {
-      const int d = m * 32 + lg * 8, left = D - d;
-      float v[8], wq[8], wk[8];
-      load8(q + (left > 0 ? d : 0), vec && left >= 8, left, v);
-      load8(a.q_norm + head * D + (left > 0 ? d : 0), vec && left >= 8, left, wq);
-      load8(a.k_norm + g * D + (left > 0 ? d : 0), vec && left >= 8, left, wk);
-#pragma unroll
-      for (int e = 0; e < 8; ++e) qf[w][m][e] = (bf16)(v[e] * rq * wq[e] * wk[e]);
+      load8(a.q_norm + head * D + m * 32 + lg * 8, true, 8, wq[m]);
+      load8(a.k_norm + g * D + m * 32 + lg * 8, true, 8, wk[m]);
     }
+#pragma unroll
+    for (int w = 0; w < QW; ++w)
+#pragma unroll
+      for (int m = 0; m < DT; ++m)
+#pragma unroll
+        for (int e = 0; e < 8; ++e) qf[w][m][e] = (bf16)((float)bitcast<bf16x8>(raw[w][m])[e] * rq[w] * wq[m][e] * wk[m][e]);
+  } else {
+#pragma unroll
+    for (int w = 0; w < QW; ++w)
+#pragma unroll
+      for (int m = 0; m < DT; ++m) {
+        const int d = m * 32 + lg * 8, left = D - d;
+        float v[8], wq[8], wk[8];
+        load8(qrow[w] + (left > 0 ? d : 0), vec && left >= 8, left, v);
+        load8(a.q_norm + head * D + (left > 0 ? d : 0), vec && left >= 8, left, wq);
+        load8(a.k_norm + g * D + (left > 0 ? d : 0), vec && left >= 8, left, wk);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) qf[w][m][e] = (bf16)(v[e] * rq[w] * wq[e] * wk[e]);
+      }
   }
   const int i_last = p0 + (count < 64 * QW ? count : 64 * QW) - 1;
   const int lo = p0 - a.window + 1 > 0 ? p0 - a.window + 1 : 0;
   const int w_first = p0 + wave * QW * 16, w_last = w_first + QW * 16 - 1;
 
   u32x4 pf[IPT][2];
-  float pr = 0.f;
+  float pr;
+  // (Loads without a branch round them, which would be waited for at its end, one after another: keys past the last one repeat it, and nobody sees
+  // them; columns past the row's repeat its first ones, where the queries hold zeros and nothing is stored.)
   auto fetch = [&](int jt) {
+    const int first = jt % a.ring_len;
+    auto place = [&](int k) {
+      k = first + (jt + k < i_last ? k : i_last - jt);
+      return k < a.ring_len ? k : a.ring_len >= WT_KEYS ? k - a.ring_len : k % a.ring_len;
+    };
 #pragma unroll
     for (int it = 0; it < IPT; ++it) {
       const int idx = threadIdx.x + it * 256, c = idx % CH, kp = idx / CH;
 #pragma unroll
-      for (int t = 0; t < 2; ++t) {
-        const int j = jt + kp * 2 + t;
-        pf[it][t] = u32x4{0, 0, 0, 0};
-        if (idx < ITEMS && j <= i_last && c * 8 < Dp)
-          pf[it][t] = *reinterpret_cast<const u32x4*>(ring + (size_t)(j % a.ring_len) * Dp + c * 8);
-      }
+      for (int t = 0; t < 2; ++t) pf[it][t] = *reinterpret_cast<const u32x4*>(ring + (size_t)place(kp * 2 + t) * Dp + (c * 8 < Dp ? c * 8 : 0));
     }
-    if (threadIdx.x < WT_KEYS) {
-      const int j = jt + threadIdx.x;
-      pr = j <= i_last ? rinv[j % a.ring_len] : 0.f;
-    }
+    pr = rinv[place(threadIdx.x & (WT_KEYS - 1))];
   };
   auto stage = [&]() {
 #pragma unroll
@@ -334,14 +357,6 @@ __global__ __launch_bounds__(256) void window_tile_kernel(WA a, bool vec) {
       if (idx >= ITEMS) break;
       *reinterpret_cast<u32x4*>(sk + (kp * 2) * KS + c * 8) = pf[it][0];
       *reinterpret_cast<u32x4*>(sk + (kp * 2 + 1) * KS + c * 8) = pf[it][1];
-      const int k32 = (kp * 2) & 31, place = ((kp * 2) & 32) + ((k32 & 15) >> 2) * 8 + (k32 >> 4) * 4 + (k32 & 3);
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const uint32_t x = pf[it][0][e], y = pf[it][1][e];
-        bf16* base = sv + (c * 8 + 2 * e) * WT_VSTRIDE + c * 8 + place;
-        *reinterpret_cast<uint32_t*>(base) = (x & 0xffffu) | (y << 16);
-        *reinterpret_cast<uint32_t*>(base + WT_VSTRIDE) = (x >> 16) | (y & 0xffff0000u);
-      }
     }
     if (threadIdx.x < WT_KEYS) sr[threadIdx.x] = pr;
   };
@@ -363,6 +378,7 @@ __global__ __launch_bounds__(256) void window_tile_kernel(WA a, bool vec) {
     __syncthreads();
     if (jt + WT_KEYS <= i_last) fetch(jt + WT_KEYS);
     if (jt > w_last || jt + WT_KEYS - 1 < w_first - a.window + 1) continue;       // nothing this wave's rows see
+    const bool whole = jt + WT_KEYS - 1 <= w_first && jt > w_last - a.window;     // all of it, all of them
     f32x4 s[QW][4];
 #pragma unroll
     for (int t = 0; t < 4; ++t) {
@@ -378,46 +394,35 @@ __global__ __launch_bounds__(256) void window_tile_kernel(WA a, bool vec) {
     bf16x8 p[QW][2];
 #pragma unroll
     for (int w = 0; w < QW; ++w) {
-      float top = m[w];
+      const int near = qi[w] - (jt + lg * 4);                                      // distance of the lane's first key
+      const float far = (float)near;
 #pragma unroll
       for (int t = 0; t < 4; ++t) {
         const f32x4 ri = *reinterpret_cast<const f32x4*>(sr + t * 16 + lg * 4);
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const int dist = qi[w] - (jt + t * 16 + lg * 4 + e);
-          const float v = s[w][t][e] * ri[e] - slope * (float)dist;
-          s[w][t][e] = dist >= 0 && dist < a.window ? v : -INFINITY;
-          top = fmaxf(top, s[w][t][e]);
-        }
+        for (int e = 0; e < 4; ++e) s[w][t][e] = s[w][t][e] * ri[e] - slope * (far - (float)(t * 16 + e));
       }
-      top = fmaxf(top, __shfl_xor(top, 16, 64));
-      top = fmaxf(top, __shfl_xor(top, 32, 64));
-      const float keep = exp2f(m[w] - top);
-      m[w] = top;
-      float sum = 0.f;
+      if (!whole) {
 #pragma unroll
-      for (int t = 0; t < 4; ++t)
+        for (int t = 0; t < 4; ++t)
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const float x = exp2f(s[w][t][e] - top);
-          sum += x;
-          p[w][t >> 1][(t & 1) * 4 + e] = (bf16)x;
-        }
-      l[w] = l[w] * keep + sum;
-#pragma unroll
-      for (int t = 0; t < DT * 2; ++t)
-#pragma unroll
-        for (int e = 0; e < 4; ++e) o[w][t][e] *= keep;
+          for (int e = 0; e < 4; ++e) {
+            const int dist = near - (t * 16 + e);
+            if (!(dist >= 0 && dist < a.window)) s[w][t][e] = -INFINITY;
+          }
+      }
+      softmax_step(s[w], m[w], l[w], p[w], o[w]);
     }
 #pragma unroll
-    for (int t = 0; t < DT * 2; ++t)
+    for (int kg = 0; kg < 2; ++kg) {
+      const bf16* v = sk + (kg * 32 + lg * 4 + (lc >> 2)) * KS + (lc & 3) * 4;
 #pragma unroll
-      for (int kg = 0; kg < 2; ++kg) {
-        const int d = t * 16 + lc;
-        const bf16x8 vf = *reinterpret_cast<const bf16x8*>(sv + d * WT_VSTRIDE + (d >> 3) * 8 + kg * 32 + lg * 8);
+      for (int t = 0; t < DT * 2; ++t) {
+        const bf16x8 vf = join(read_transposed(v + t * 16), read_transposed(v + t * 16 + 16 * KS));
 #pragma unroll
         for (int w = 0; w < QW; ++w) o[w][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf, p[w][kg], o[w][t], 0, 0, 0);
       }
+    }
   }
 #pragma unroll
   for (int w = 0; w < QW; ++w) {
@@ -515,12 +520,12 @@ extern "C" int pta_window_attention(const WA* args, pta_stream_t stream) {
     PTA_REQUIRE(a.tiles > 0 && a.tile_row && a.tile_count, "pta_window_attention: the rows' tiles are missing");
     PTA_REQUIRE(a.tiles <= 65535, "pta_window_attention: %d tiles (at most 65535)", a.tiles);
     const bool vec = vectors_fit(a);
-    const dim3 one(a.H, a.tiles, 1), two(a.H, a.tiles, 2);
-    if (a.D <= 32) hipLaunchKernelGGL((window_tile_kernel<1, 2>), one, dim3(256), 0, s, a, vec);
-    else if (a.D <= 64) hipLaunchKernelGGL((window_tile_kernel<2, 2>), one, dim3(256), 0, s, a, vec);
-    else if (a.D <= 96) hipLaunchKernelGGL((window_tile_kernel<3, 2>), one, dim3(256), 0, s, a, vec);
-    else if (a.D <= 128) hipLaunchKernelGGL((window_tile_kernel<4, 2>), one, dim3(256), 0, s, a, vec);
-    else hipLaunchKernelGGL((window_tile_kernel<8, 1>), two, dim3(256), 0, s, a, vec);
+    const dim3 grid(a.H, a.tiles, PTA_WINDOW_TILE / 64);
+    if (a.D <= 32) hipLaunchKernelGGL((window_tile_kernel<1>), grid, dim3(256), 0, s, a, vec);
+    else if (a.D <= 64) hipLaunchKernelGGL((window_tile_kernel<2>), grid, dim3(256), 0, s, a, vec);
+    else if (a.D <= 96) hipLaunchKernelGGL((window_tile_kernel<3>), grid, dim3(256), 0, s, a, vec);
+    else if (a.D <= 128) hipLaunchKernelGGL((window_tile_kernel<4>), grid, dim3(256), 0, s, a, vec);
+    else hipLaunchKernelGGL((window_tile_kernel<8>), grid, dim3(256), 0, s, a, vec);
   }
   PTA_CHECK_LAUNCH("pta_window_attention");
   return PTA_OK;
