@@ -1328,7 +1328,7 @@ __global__ __launch_bounds__(256) void splitk_finish_kernel(GemmArgs a) {
 }
 
 // The same with the norm of the finished rows behind it, a row a workgroup: the rows' sums are read once, and the norm's launch and its reading of
-// the rows are gone.  What bounds it at few rows is the chain of a row (32 rows of 4096, four slices, residual, gate and three mixes: 9.6 -> 6.1 us), at many the
+// the rows are gone.  What bounds it at few rows is the chain of a row (32 rows of 4096, four slices, residual, gate and three mixes: 9.6 -> 5.7 us), at many the
 // bytes (1000 rows, two slices: 17.1 -> 11.0).  Every operation is that of the two kernels, in their order.
 template <class Fmt, int VECS>
 struct FinishedRow {
@@ -1353,7 +1353,7 @@ struct FinishedRow {
 #pragma unroll
     for (int k = 0; k < 4; ++k) add[i][k] = *reinterpret_cast<const f16x8*>(from[k] + n);
   }
-  __device__ __forceinline__ f16x8 value(int i, int c) const {
+  __device__ __forceinline__ f16x8 value(int i) const {
     const GemmMat& mat = a.mat[0];
     f16x8 out;
 #pragma unroll
@@ -1370,9 +1370,9 @@ struct FinishedRow {
       if (a.epi.post_scale != 0.0f) y = y * (f16)a.epi.post_scale;
       out[e] = y;
     }
-    *reinterpret_cast<f16x8*>(mat.Y + at + (size_t)c * 8) = out;
     return out;
   }
+  __device__ __forceinline__ void keep(int c, f16x8 v) const { *reinterpret_cast<f16x8*>(a.mat[0].Y + at + (size_t)c * 8) = v; }
 };
 
 template <class Fmt, int MODE, bool MIX, int VECS>

@@ -7,26 +7,38 @@
 // there are several.  One workgroup normalises one row in a single pass over registers.
 #include "norm_core.h"
 
+template <int VECS>
 struct RowInMemory {
   const f16* from;
-  f16x8 v[NORM_MAX_VEC];
+  f16x8 v[VECS];
   __device__ __forceinline__ void request(int i, int c) { v[i] = *reinterpret_cast<const f16x8*>(from + (size_t)c * 8); }
-  __device__ __forceinline__ f16x8 value(int i, int) const { return v[i]; }
+  __device__ __forceinline__ f16x8 value(int i) const { return v[i]; }
+  __device__ __forceinline__ void keep(int, f16x8) const {}
 };
 
-template <int MODE, bool MIX = false>
+template <int MODE, bool MIX, int VECS>
 __global__ __launch_bounds__(NORM_THREADS) void norm_kernel(const f16* __restrict__ x, NormArgs a, NormMix mix) {
-  RowInMemory row{x + (size_t)blockIdx.x * a.cols};
-  norm_row<MODE, MIX, NORM_MAX_VEC>(a, mix, blockIdx.x, row);
+  RowInMemory<VECS> row{x + (size_t)blockIdx.x * a.cols};
+  norm_row<MODE, MIX, VECS>(a, mix, blockIdx.x, row);
 }
 
 void launch_norm(const f16* x, int rows, int mode, const NormArgs& a, const NormMix* mix, hipStream_t s) {
   const NormMix m = mix ? *mix : NormMix{};
-  if (mode == 0) hipLaunchKernelGGL((norm_kernel<0>), dim3(rows), dim3(NORM_THREADS), 0, s, x, a, m);
-  else if (mode == 1 && mix) hipLaunchKernelGGL((norm_kernel<1, true>), dim3(rows), dim3(NORM_THREADS), 0, s, x, a, m);
-  else if (mode == 1) hipLaunchKernelGGL((norm_kernel<1>), dim3(rows), dim3(NORM_THREADS), 0, s, x, a, m);
-  else if (mix) hipLaunchKernelGGL((norm_kernel<2, true>), dim3(rows), dim3(NORM_THREADS), 0, s, x, a, m);
-  else hipLaunchKernelGGL((norm_kernel<2>), dim3(rows), dim3(NORM_THREADS), 0, s, x, a, m);
+  auto launch = [&](auto vecs) {
+    constexpr int V = decltype(vecs)::value;
+    if (mode == 0) hipLaunchKernelGGL((norm_kernel<0, false, V>), dim3(rows), dim3(NORM_THREADS), 0, s, x, a, m);
+    else if (mode == 1 && mix) hipLaunchKernelGGL((norm_kernel<1, true, V>), dim3(rows), dim3(NORM_THREADS), 0, s, x, a, m);
+    else if (mode == 1) hipLaunchKernelGGL((norm_kernel<1, false, V>), dim3(rows), dim3(NORM_THREADS), 0, s, x, a, m);
+    else if (mix) hipLaunchKernelGGL((norm_kernel<2, true, V>), dim3(rows), dim3(NORM_THREADS), 0, s, x, a, m);
+    else hipLaunchKernelGGL((norm_kernel<2, false, V>), dim3(rows), dim3(NORM_THREADS), 0, s, x, a, m);
+  };
+  // (as few pieces of a thread as the row needs)
+  switch ((a.cols + 8 * NORM_THREADS - 1) / (8 * NORM_THREADS)) {
+    case 1: launch(std::integral_constant<int, 1>{}); break;
+    case 2: launch(std::integral_constant<int, 2>{}); break;
+    case 3: launch(std::integral_constant<int, 3>{}); break;
+    default: launch(std::integral_constant<int, NORM_MAX_VEC>{});
+  }
 }
 
 int check_norm(const char* name, const void* x, const void* g, const void* y, int rows, int cols) {
