@@ -5,6 +5,7 @@
 // mean square of the token's keys; the key norm's weight, the query norm and the score scale are folded into the query:
 //   score(i, j) = rinv_j * (q'_i . k_j) - slope * (i - j),   q' = q * rinv_q * w_q * w_k * scale.
 #include "attention.h"
+#include "ring.h"
 
 typedef pta_window_attention_args WA;
 
@@ -267,8 +268,8 @@ __global__ __launch_bounds__(256) void window_tile_kernel(WA a, bool vec) {
   constexpr int QW = 1, DM = DT * 32;
   constexpr int KS = DM + 8;
   constexpr int CH = DM / 8;                              // 16-byte pieces of a key row
-  constexpr int ITEMS = WT_KEYS / 2 * CH;                 // (pair of keys, piece)
-  constexpr int IPT = (ITEMS + 255) / 256;
+  typedef KeyPairs<WT_KEYS, CH> Items;                    // (pair of keys, piece)
+  constexpr int ITEMS = Items::ITEMS, IPT = Items::PER_THREAD;
   __shared__ __align__(16) bf16 sk[WT_KEYS * KS];
   __shared__ float sr[WT_KEYS];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, lg = lane >> 4, lc = lane & 15;
@@ -338,13 +339,10 @@ __global__ __launch_bounds__(256) void window_tile_kernel(WA a, bool vec) {
   // them; columns past the row's repeat its first ones, where the queries hold zeros and nothing is stored.)
   auto fetch = [&](int jt) {
     const int first = jt % a.ring_len;
-    auto place = [&](int k) {
-      k = first + (jt + k < i_last ? k : i_last - jt);
-      return k < a.ring_len ? k : a.ring_len >= WT_KEYS ? k - a.ring_len : k % a.ring_len;
-    };
+    auto place = [&](int k) { return ring_row<WT_KEYS>(first, jt, k, i_last, a.ring_len); };
 #pragma unroll
     for (int it = 0; it < IPT; ++it) {
-      const int idx = threadIdx.x + it * 256, c = idx % CH, kp = idx / CH;
+      const int idx = threadIdx.x + it * 256, c = Items::piece(idx), kp = Items::pair(idx);
 #pragma unroll
       for (int t = 0; t < 2; ++t) pf[it][t] = *reinterpret_cast<const u32x4*>(ring + (size_t)place(kp * 2 + t) * Dp + (c * 8 < Dp ? c * 8 : 0));
     }
@@ -353,7 +351,7 @@ __global__ __launch_bounds__(256) void window_tile_kernel(WA a, bool vec) {
   auto stage = [&]() {
 #pragma unroll
     for (int it = 0; it < IPT; ++it) {
-      const int idx = threadIdx.x + it * 256, c = idx % CH, kp = idx / CH;
+      const int idx = threadIdx.x + it * 256, c = Items::piece(idx), kp = Items::pair(idx);
       if (idx >= ITEMS) break;
       *reinterpret_cast<u32x4*>(sk + (kp * 2) * KS + c * 8) = pf[it][0];
       *reinterpret_cast<u32x4*>(sk + (kp * 2 + 1) * KS + c * 8) = pf[it][1];

@@ -216,6 +216,19 @@ def test_attention_prompt_decode_and_portions(dtype, H, G, D, window):
         assert _rel(got, want) < a.tol(), how
 
 
+@pytest.mark.parametrize("D", [20, 32, 72, 96])
+@pytest.mark.parametrize("window,rows", [(7, 59), (24, 48), (64, 62), (63, 64)])
+def test_prompt_portions_through_rings_of_one_to_two_steps(D, window, rows):
+    """Rings of 65 to 126 rows, as few as the window and a portion need, in the last slot: portions begin at all kinds of places of the ring."""
+    rng = np.random.default_rng(window)
+    T, H, G = 320, 2, 1
+    a = Attention("bfloat16", H, G, D, window, 2, window - 1 + rows, seed=D)
+    proj = a.project(*(rng.standard_normal((T, c)) for c in (H * D, G * D, H * D)))
+    print(f"attention D {D} window {window}: portions of {rows} through a ring of {window - 1 + rows}", flush=True)
+    got = np.concatenate([a.run(proj[p:p + rows].contiguous(), [(1, p, min(rows, T - p))]) for p in range(0, T, rows)])
+    assert _rel(got, a.want(proj)) < a.tol()
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
 def test_attention_batch_of_unequal_sequences(dtype):
     rng = np.random.default_rng(3)
