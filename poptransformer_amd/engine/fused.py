@@ -314,17 +314,26 @@ class FusedDecoder(DecodeLoop, LayerOps):
         self.probe = None                # callable(name, block index, tensor or tensors): looks into eager iterations of the per-operator path
 
     def _gpt2_step(self):
-        """pta_gpt2_step over this decoder's buffers, or None: another family or selection, other weights, or a shape that it does not cover."""
+        """pta_gpt2_step over this decoder's buffers, or None: another family or selection, other weights, or a shape that it does not cover.  It reads
+        by pointers and the spec's sizes, so tensors that are not what those say stay with the operators, which refuse them or take them as they are."""
         s, w = self.spec, self.w
         if s.family != "gpt2" or s.topk != 1 or s.fp8_cache or s.head_dim != 64 or s.n_kv_head != s.n_head:
             return None
-        if w.pos_embed is None or not isinstance(w.head.w, K.F16Weight) or w.head.bias is not None:
+        if any(len(b.qkv) != 1 or len(b.mlp_in) != 1 for b in w.blocks) or len(w.blocks) != s.n_layer:
             return None
-        lins = [lw for b in w.blocks for lw in (b.qkv[0], b.out, b.mlp_in[0], b.mlp_out)]
-        if any(len(b.qkv) != 1 or len(b.mlp_in) != 1 for b in w.blocks) or not all(isinstance(lw.w, K.F16Weight) and lw.bias is not None for lw in lins):
+        d, ffn = s.d_model, w.blocks[0].mlp_out.K
+
+        def plain(t, *shape):
+            return t is not None and t.is_cuda and t.dtype == torch.float16 and t.is_contiguous() and tuple(t.shape) == shape and t.data_ptr() % 16 == 0
+
+        def fits(lw, n, k, bias=True):
+            return isinstance(lw.w, K.F16Weight) and (lw.w.N, lw.w.K) == (n, k) and (plain(lw.bias, n) if bias else lw.bias is None)
+        # (an embedding's ids end where its table does, the step's where the vocabulary does: they are one)
+        if not (plain(w.embed, s.vocab, d) and w.pos_embed is not None and plain(w.pos_embed, w.pos_embed.shape[0], d) and fits(w.head, s.vocab, d, bias=False)):
             return None
-        norms = [g for b in w.blocks for g in (b.norm1, b.norm2)] + [w.final_norm]
-        if any(t is None or t.data_ptr() % 16 for g in norms for t in g):
+        if not all(fits(b.qkv[0], 3 * d, d) and fits(b.out, d, d) and fits(b.mlp_in[0], ffn, d) and fits(b.mlp_out, d, ffn) for b in w.blocks):
+            return None
+        if not all(len(g) == 2 and plain(g[0], d) and plain(g[1], d) for b in w.blocks for g in (b.norm1, b.norm2, w.final_norm)):
             return None
         layers = []
         for b, ring in zip(w.blocks, self.rings):
@@ -334,7 +343,7 @@ class FusedDecoder(DecodeLoop, LayerOps):
         state = dict(container=self.container, mask=self.mask, stop_mask=self.stop_mask, step=self.step, keep_going=self.keep_going,
                      next_ids=self.next_ids, logits=self.logits)
         try:
-            return K.Gpt2Step(layers, w.embed, w.pos_embed, w.final_norm, w.head.w.tiled, s.batch, s.d_model, s.n_head, w.blocks[0].mlp_out.K, s.vocab,
+            return K.Gpt2Step(layers, w.embed, w.pos_embed, w.final_norm, w.head.w.tiled, s.batch, d, s.n_head, ffn, s.vocab,
                               s.max_len, s.eps, s.pad_id, s.eos_id, s.early_stop, state)
         except NotImplementedError:
             return None

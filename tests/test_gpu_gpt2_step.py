@@ -130,3 +130,41 @@ def test_shapes_and_options_that_stay_per_operator():
     assert made(B=9) is None and made(topk=4) is None and made(fp8_cache=True) is None and made(max_len=701) is None
     one = made()
     assert isinstance(one, K.Gpt2Step) and not one.failed()
+
+
+def test_tensors_that_are_not_what_the_spec_says_stay_per_operator():
+    """What the operators refuse is refused, and what they take is computed as they do."""
+    import dataclasses
+    from poptransformer_amd import kernels as K
+    from poptransformer_amd.engine import fused, loader
+    cfg = _cfg(4)
+    w = loader.gpt2_weights(OM.make_gpt2_state_dict(cfg, seed=3), cfg)
+    ids = np.random.default_rng(2).integers(2, 500, size=(2, 24)).astype(np.int32)
+    ids[:, 0] = 450, 7
+
+    def made(**kw):
+        dec = fused.FusedDecoder(loader.gpt2_spec(cfg, 24, 2, 0, 1), dataclasses.replace(w, **kw))
+        dec.reset(ids)
+        assert dec.chained is None
+        return dec
+
+    def block(**kw):
+        return [w.blocks[0], dataclasses.replace(w.blocks[1], **kw)]
+    b, d = w.blocks[1], w.embed.shape[1]
+    narrow = fused.LinearWeights(K.F16Weight(torch.zeros((d, d - 64), dtype=torch.float16, device="cuda")), b.out.bias)
+    wide = torch.zeros((w.embed.shape[0], 2 * d), dtype=torch.float16, device="cuda")
+    wide[:, ::2] = w.embed
+    for kw in (dict(embed=w.embed.float()), dict(embed=wide[:, ::2]), dict(blocks=block(out=narrow)), dict(blocks=block(mlp_out=narrow))):
+        with pytest.raises(ValueError):
+            made(**kw).step_fn()
+    # a table of fewer tokens than the head has: ids past its end are its last row's
+    short, last = made(embed=w.embed[:400].contiguous()), fused.FusedDecoder(loader.gpt2_spec(cfg, 24, 2, 0, 1), w)
+    last.reset(np.minimum(ids, 399))
+    last.chained = None
+    for dec in (short, last):
+        dec.step_fn()
+    assert torch.equal(short.logits, last.logits)
+    # (no result of these is looked at: the operators do not check them either)
+    made(pos_embed=w.pos_embed.float()), made(blocks=block(norm1=(b.norm1[0].float(), b.norm1[1]))), made(final_norm=(w.final_norm[0], w.final_norm[1][:-8].clone()))
+    made(blocks=block(qkv=[fused.LinearWeights(K.F16Weight(torch.zeros((2 * d, d), dtype=torch.float16, device="cuda")), b.qkv[0].bias)]))
+    made(blocks=block(out=fused.LinearWeights(b.out.w, b.out.bias.float())))
