@@ -565,7 +565,7 @@ typedef struct pta_gpt2_model {
 size_t pta_gpt2_step_workspace_bytes(const pta_gpt2_model* model);
 
 /* Enqueues one loop iteration.  Launches with one workspace must follow each other in stream order.  Every wait is bounded: if one gives up,
- * the loop state is left untouched and later launches do nothing (pta_decode_step_failed). */
+ * the loop state is left untouched and later launches do nothing (pta_decode_step_failed) until the caller has zeroed the workspace again. */
 int pta_gpt2_step(const pta_gpt2_model* model, const pta_decode_state* state, void* workspace, pta_stream_t stream);
 
 #ifdef __cplusplus

@@ -513,8 +513,11 @@ __global__ __launch_bounds__(G2_THREADS) void gpt2_step_kernel(G2Args a) {
   int id = __builtin_amdgcn_readfirstlane((int)start[0]);
   const int step = __builtin_amdgcn_readfirstlane((int)start[3]);
   G2Wait wait{(__builtin_amdgcn_readfirstlane(start[2]) + 1) & 0xffffu, a.ctl + 1};     // (a workspace begins with zeros, which are no iteration)
-  if (__builtin_amdgcn_readfirstlane(start[1])) {                // a wait of an earlier launch gave up: nothing is done until that is cleared
-    if (id == a.total - 1 && threadIdx.x == 0) a.ctl[0] = 0;
+  if (__builtin_amdgcn_readfirstlane(start[1])) {                // a wait gave up: nothing is done until that is cleared
+    if (id == a.total - 1 && threadIdx.x == 0) {                 // (nor is this iteration's number used again: words of it may be there)
+      a.ctl[0] = 0;
+      a.ctl[2] = wait.tag;
+    }
     return;
   }
   if (id == a.total - 1) {

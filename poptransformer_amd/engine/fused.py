@@ -473,4 +473,5 @@ class FusedDecoder(DecodeLoop, LayerOps):
                                "of the device for itself while it runs); the loop state was not advanced past the failing "
                                "iteration.  The failure word is sticky: persistent.clear_failure() re-arms the decoder")
         if self.chained is not None and self.chained.failed():
-            raise RuntimeError("GPT-2 step: a workgroup gave up waiting; the loop state was not advanced past the failing iteration")
+            raise RuntimeError("GPT-2 step: a workgroup gave up waiting; the loop state was not advanced past the failing iteration.  The failure word is "
+                               "sticky: chained.clear_failure() re-arms the decoder")

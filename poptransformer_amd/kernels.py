@@ -737,6 +737,12 @@ class Gpt2Step:
     def launch(self):
         check(_lib.load().pta_gpt2_step(ctypes.byref(self.model), ctypes.byref(self.state), _p(self.workspace), _stream()))
 
+    def clear_failure(self):
+        """Re-arms the workspace after a launch has set its failure word (the word is sticky: until then every launch returns at once)."""
+        torch.cuda.synchronize()
+        self.workspace.zero_()
+        torch.cuda.synchronize()
+
     def failed(self):
         flag = ctypes.c_int(0)
         check(_lib.load().pta_decode_step_failed(_p(self.workspace), ctypes.byref(flag), _stream()))

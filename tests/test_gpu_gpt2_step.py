@@ -168,3 +168,32 @@ def test_tensors_that_are_not_what_the_spec_says_stay_per_operator():
     made(pos_embed=w.pos_embed.float()), made(blocks=block(norm1=(b.norm1[0].float(), b.norm1[1]))), made(final_norm=(w.final_norm[0], w.final_norm[1][:-8].clone()))
     made(blocks=block(qkv=[fused.LinearWeights(K.F16Weight(torch.zeros((2 * d, d), dtype=torch.float16, device="cuda")), b.qkv[0].bias)]))
     made(blocks=block(out=fused.LinearWeights(b.out.w, b.out.bias.float())))
+
+
+@pytest.mark.parametrize("clear", ["all", "word"])
+def test_a_wait_that_gave_up_is_reported_and_cleared(clear):
+    """The word that a wait sets when it gives up, set by hand, where words of the next iteration's number lie about: launches do nothing, `run` raises, and
+    once cleared - by the decoder, or the word alone behind a launch that found it - no such word is taken for one that has arrived."""
+    one, per_op = _decoders(_cfg(4), 24, 2)
+    ids = np.random.default_rng(4).integers(2, 500, size=(2, 24)).astype(np.int32)
+    per_op.run(ids, 12)
+    for graph in (False, True):
+        if graph:
+            one.capture()
+        one.run(ids, 3)
+        words = one.chained.workspace.view(torch.int32)
+        assert int(words[0]) == 0 and int(words[1]) == 0
+        words[64:] = (int(words[2]) + 1 & 0xFFFF) << 16 | 0x3C00                  # ones that seem to have arrived
+        words[1] = 1
+        torch.cuda.synchronize()
+        with pytest.raises(RuntimeError, match="clear_failure"):
+            one.run(ids, 3)
+        assert int(one.step.item()) == 0
+        if clear == "all":
+            one.chained.clear_failure()
+        else:
+            words[1] = 0
+            torch.cuda.synchronize()
+        got, step = one.run(ids, 12)
+        assert step == 12
+        _close(one.logits, per_op.logits)
