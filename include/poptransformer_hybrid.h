@@ -599,6 +599,10 @@ typedef struct pta_depth_end_args {
 size_t pta_depth_end_workspace_bytes(int rows, int width, int side);
 int pta_depth_end(const pta_depth_end_args* host_args, pta_stream_t stream);
 
+/* Whether a wait of a launch with this workspace gave up: every wait is bounded, and if one ends without what it waited for, h of that launch and of all
+ * later ones is NaN (routing, next and the newest depth stay as they are) until the caller has zeroed the workspace again.  Synchronises the stream. */
+int pta_depth_end_failed(const void* workspace, int* failed, pta_stream_t stream);
+
 /* ---- Next-token selection over fp32 logits, and the loop's bookkeeping -------------------------------------------- */
 int pta_argmax_f32(const float* logits, int32_t* ids, float* values, int rows, int n, pta_stream_t stream);
 int pta_topk_f32(const float* logits, int32_t* ids, float* values, int rows, int n, int k, pta_stream_t stream);

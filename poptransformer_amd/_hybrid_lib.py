@@ -127,6 +127,7 @@ SIGNATURES = {
     "pta_add_parts": (_I, [POINTER(AddPartsArgs), _P]),
     "pta_depth_end_workspace_bytes": (c_size_t, [_I, _I, _I]),
     "pta_depth_end": (_I, [POINTER(DepthEndArgs), _P]),
+    "pta_depth_end_failed": (_I, [_P, POINTER(_I), _P]),
     "pta_mlstm_state_floats": (c_size_t, [_I, _I, _I]),
     "pta_mlstm_workspace_bytes": (c_size_t, [POINTER(MlstmArgs)]),
     "pta_mlstm": (_I, [POINTER(MlstmArgs), _P]),

@@ -565,3 +565,16 @@ extern "C" int pta_depth_end(const DE* args, pta_stream_t stream) {
   PTA_CHECK_LAUNCH(name);
   return PTA_OK;
 }
+
+extern "C" int pta_depth_end_failed(const void* workspace, int* failed, pta_stream_t stream) {
+  PTA_REQUIRE(workspace && failed, "pta_depth_end_failed: null pointer");
+  uint32_t word = 0;
+  hipError_t e = hipMemcpyAsync(&word, reinterpret_cast<const uint32_t*>(workspace) + 2, sizeof(word), hipMemcpyDeviceToHost, (hipStream_t)stream);
+  if (e == hipSuccess) e = hipStreamSynchronize((hipStream_t)stream);
+  if (e != hipSuccess) {
+    pta_set_error("pta_depth_end_failed: %s", hipGetErrorString(e));
+    return PTA_EHIP;
+  }
+  *failed = word != 0;
+  return PTA_OK;
+}

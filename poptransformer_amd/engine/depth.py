@@ -192,6 +192,23 @@ class DepthDecoder(HeadMixing, LatentMixing, StateSpaceMixing, ExpertMixing, Hyb
                 self.probe(i, b.history[i + 2, :n].clone())
         return b, None
 
+    def _end_workspaces(self):
+        return [b.end_workspace for b in self._buffers.values() if b.end_workspace is not None]
+
+    def check_finished(self):
+        """Raises when a wait within a layer's end gave up in any pass so far.  `run` and `consume_prompt` call it; behind `advance`, whose logits are NaN
+        then, it is the caller's to call (it waits for the stream)."""
+        if any(HK.depth_end_failed(ws) for ws in self._end_workspaces()):
+            raise RuntimeError("the end of a layer: a workgroup gave up waiting, and what the passes since have made is not valid.  The failure word is "
+                               "sticky: clear_failure() re-arms the decoder")
+
+    def clear_failure(self):
+        """Re-arms the decoder after check_finished has raised.  Sequences that were on their way start again."""
+        torch.cuda.synchronize()
+        for ws in self._end_workspaces():
+            ws.zero_()
+        torch.cuda.synchronize()
+
     def _logits(self, b, done, count, out, gather=None):
         h = b.h
         if gather is not None:

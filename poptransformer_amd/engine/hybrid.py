@@ -590,7 +590,8 @@ class HybridDecoder(DecodeLoop):
 
     def advance(self, entries):
         """entries [(slot, token ids, wanted places)]: the sequences' next tokens, as one batch, cut into passes where they
-        are many.  Returns the logits fp32 [sum of wanted, vocab] at the wanted places, in their order."""
+        are many.  Returns the logits fp32 [sum of wanted, vocab] at the wanted places, in their order, without waiting for them (nor calling
+        `check_finished`)."""
         spec, store = self.spec, self.store
         if len({e[0] for e in entries}) != len(entries):
             raise ValueError("advance: a sequence appears twice in one batch")
@@ -691,4 +692,5 @@ class HybridDecoder(DecodeLoop):
                     self.store.length[b] += ids.shape[1]
             self.step.fill_(n)
         self._stream.synchronize()
+        self.check_finished()
         return n

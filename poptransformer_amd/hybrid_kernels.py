@@ -552,6 +552,13 @@ def depth_end(x, rows, h, parts, gate, own, proj, norm, workspace):
     H.check(H.load().pta_depth_end(ctypes.byref(a), _stream()))
 
 
+def depth_end_failed(workspace):
+    """Whether a wait of a `depth_end` with this workspace gave up (waits for the stream)."""
+    flag = ctypes.c_int(0)
+    H.check(H.load().pta_depth_end_failed(_p(workspace), ctypes.byref(flag), _stream()))
+    return bool(flag.value)
+
+
 class ExpertWeight:
     """Linear weights of one shape, one per expert, one after the other: bf16 tiled (channels rounded up to 16, many to 128), fp32
     as they are.  main_to: further zero channels, as WideWeight's.  That of a single expert also serves `linear`."""

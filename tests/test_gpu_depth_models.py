@@ -280,6 +280,39 @@ def test_prompt_passes_leave_what_the_loop_leaves(dtype, name, batch):
         check()
 
 
+def test_a_wait_that_gave_up_is_reported_and_cleared():
+    """The word that a wait in a layer's end sets when it gives up, set by hand: `run` and `consume_prompt` raise, `advance` returns no numbers and its caller
+    can ask; cleared, the decoder computes what it did."""
+    cfg = DEPTH["small"]
+    dec = _decoder(cfg, random_depth(cfg, 9), "bfloat16", max_len=60, batch=2)
+    ids = np.zeros((2, 60), np.int32)
+    ids[:, :20] = np.random.default_rng(0).integers(2, cfg["vocab"], (2, 20))
+    dec.capture()
+    want, _ = dec.run(ids, 30)
+    own = dec.open()
+    logits = dec.advance([(own, [5], [0])]).cpu()
+    for rows in (2, 1):                                          # the loop's buffers; those of a single row
+        workspace = dec._buffers[rows].end_workspace
+        workspace.view(torch.int32)[2] = 1
+        torch.cuda.synchronize()
+        with pytest.raises(RuntimeError, match="clear_failure"):
+            dec.run(ids, 30)
+        dec.reset(ids)
+        with pytest.raises(RuntimeError, match="clear_failure"):
+            dec.consume_prompt(10, rows_per_pass=1)
+        dec.close(own)
+        own = dec.open()
+        assert bool(torch.isnan(dec.advance([(own, [5], [0])])).all()) == (rows == 1)
+        with pytest.raises(RuntimeError, match="clear_failure"):
+            dec.check_finished()
+        dec.clear_failure()
+        dec.check_finished()
+        got, _ = dec.run(ids, 30)
+        dec.close(own)
+        own = dec.open()
+        assert np.array_equal(got, want) and torch.equal(dec.advance([(own, [5], [0])]).cpu(), logits)
+
+
 # ------------------------------------------------------------------------------------------- trace runner
 @pytest.mark.parametrize("dtype", DTYPES)
 def test_trace_runner(tmp_path, dtype):
