@@ -497,7 +497,7 @@ __global__ __launch_bounds__(DE_THREADS) void depth_end_kernel(DE a) {
   }
   const int r = id - g.gates - g.projections;
   if (r >= M) return;
-  if (!given_up && (width & 3) == 0) {
+  if (!given_up && (width & 3) == 0 && (a.norm.h_ld & 3) == 0) {                // (whole pieces of a row, and of a row of h)
     de_row(a, r, ys + (size_t)r * width, launch, failed, reinterpret_cast<float*>(smem));
     return;
   }

@@ -4,8 +4,9 @@ import torch
 
 pytestmark = pytest.mark.gpu
 
-# rows, width, features of the token's own part, depths, parts (0: none), experts (0: no routing): one block and one tile, remainders of both, the most of each
-SHAPES = [(1, 72, 8, 1, 0, 0), (2, 2048, 256, 3, 3, 0), (1, 2056, 264, 9, 2, 5), (4, 4096, 256, 2, 3, 8), (3, 1000, 136, 4, 0, 4), (4, 8192, 1024, 2, 2, 0), (4, 136, 24, 3, 1, 0)]
+# rows, width, features of the token's own part, depths, parts (0: none), experts (0: no routing): one block and one tile, remainders of both, the most of each,
+# widths that are no multiple of eight, of four and of two
+SHAPES = [(2, 76, 16, 2, 2, 3), (1, 70, 8, 1, 0, 0), (3, 70, 24, 3, 2, 5), (2, 1001, 136, 2, 1, 0), (4, 8190, 1024, 3, 2, 4), (1, 72, 8, 1, 0, 0), (2, 2048, 256, 3, 3, 0), (1, 2056, 264, 9, 2, 5), (4, 4096, 256, 2, 3, 8), (3, 1000, 136, 4, 0, 4), (4, 8192, 1024, 2, 2, 0), (4, 136, 24, 3, 1, 0)]
 
 
 @pytest.mark.parametrize("rows, width, side, depths, n_parts, experts", SHAPES)
@@ -88,6 +89,29 @@ def test_as_the_four_calls(rows, width, side, depths, n_parts, experts):
         check(bounds)
         torch.cuda.synchronize()
     assert not torch.isnan(h).any()
+
+
+@pytest.mark.parametrize("width, h_ld", [(12, 13), (64, 71), (1000, 1002), (70, 70)])
+def test_rows_of_h_that_are_not_whole_pieces(width, h_ld):
+    """h may have any number of columns from the width to seven more."""
+    from poptransformer_amd import hybrid_kernels as HK
+    g = torch.Generator(device="cuda").manual_seed(5)
+
+    def f32(*shape):
+        return torch.randn(shape, generator=g, device="cuda")
+    side, rows, bf16 = 24, 3, torch.bfloat16
+    gate, proj = HK.WideWeight(f32(side, width), bf16), HK.WideWeight(f32(width, side), bf16)
+    x, rounded, own = f32(3, 4, width), torch.zeros(rows, HK.pad8(width), dtype=bf16, device="cuda"), f32(rows, side).bfloat16()
+    ws, results = HK.depth_end_workspace(rows, width, side, bf16, "cuda"), []
+    kw = dict(rows=rows, eps=1e-5, norm_weight=f32(width), weights=f32(2), y_weight=f32(width), next=2)
+    for ld in (HK.pad8(width), h_ld):
+        history, h = x.clone(), torch.full((rows + 1, ld), 7.0, dtype=bf16, device="cuda")
+        HK.depth_end(history[1], rows, rounded, {}, gate, own, proj, (history, 2, dict(kw, h=h)), ws)
+        assert (h[:rows, width:] == 0).all() and (h[rows] == 7).all()
+        results.append((history, h[:rows, :width].float()))
+    (ha, a), (hb, b) = results
+    # (sums of whole pieces and of single columns in another order: fp32, then to one or the other neighbour of bf16)
+    assert torch.allclose(ha, hb, rtol=1e-5, atol=1e-5) and ((a - b).abs() <= 2.0 ** -7 * a.abs() + 1e-4).all()
 
 
 def test_what_is_refused():
