@@ -316,11 +316,18 @@ class RowNorm:
 
     def __init__(self, gamma, beta, eps, out=None, grid=None, shift=None):
         prev, mixes, mixed = shift if shift is not None else (None, (), ())
-        for t, what in [(gamma, "gamma"), (beta, "beta"), (out, "out"), (prev, "previous rows")] + [(t, "mixing vector") for t in mixes] + [(t, "mixed rows") for t in mixed]:
-            if t is not None:
-                _need(t, torch.float16, what)
+        if shift is not None and (len(mixes) != len(mixed) or not 1 <= len(mixes) <= 3):
+            raise ValueError("a token shift has one to three mixing vectors, and an output each")
+        _need(gamma, torch.float16, "gamma", 1)
+        if beta is not None:
+            _need(beta, torch.float16, "beta", 1)
+        for t in (*mixes, *mixed):
+            _need(t, torch.float16, "mixing vector / output")
+        if grid is not None:
+            _need(grid[0], _i32, "fp8_scale")
         self.cols = gamma.numel()
-        self.rows = [t for t in (out, prev, *mixed) if t is not None]
+        self.rows = [(t, what) for t, what in ((out, "out"), (prev, "previous rows")) if t is not None]
+        self.mixed = mixed
         V = ctypes.c_void_p * 3
         self.args = _lib.RowNorm(_lib.NORM_RMS if beta is None else _lib.NORM_LAYER, _p(gamma), _p(beta), eps, _p(out), _p(grid[0]) if grid else None,
                                  _fmt(grid[1]) if grid else 0, _p(prev), V(*[_p(t) for t in mixes]), V(*[_p(t) for t in mixed]))
@@ -333,7 +340,11 @@ def linear_then_norm(x, w, out, then, x_scale=None, bias=None, residual=None, ac
     M = x.shape[0]
     if w.K != x.shape[1]:
         raise ValueError(f"matmul: contracting dimensions differ ({x.shape[1]} vs {w.K})")
-    if then.cols != w.N or any(t.numel() < M * w.N for t in then.rows):
+    for t, what in [(out, "result"), *then.rows]:
+        _need(t, torch.float16, what, 2)
+        if tuple(t.shape) != (M, w.N):
+            raise ValueError(f"linear_then_norm: {what} {tuple(t.shape)} of a product [{M}, {w.N}]")
+    if then.cols != w.N or any(t.numel() < M * w.N for t in then.mixed):
         raise ValueError(f"linear_then_norm: a norm of {then.cols} columns behind [{M}, {w.N}], or too few rows for its results")
     desc = _desc(w, None, _lib.ACT_NONE, None)
     check(_lib.load().pta_linear_then_norm(_p(x), _p(x_scale), ctypes.byref(desc), None, _p(out), M, _fusion(bias, residual, act, None, mul, post_scale, workspace),

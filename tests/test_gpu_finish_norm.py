@@ -72,3 +72,25 @@ def test_what_is_refused():
         K.linear_then_norm(x, w, out, K.RowNorm(gamma, None, 1e-5))
     with pytest.raises(ValueError):
         K.linear_then_norm(x, w, out, K.RowNorm(gamma, gamma, 1e-5, out=torch.empty_like(out), grid=(torch.zeros(1, dtype=torch.int32, device="cuda"), "F143")))
+
+
+def test_tensors_that_the_norms_own_entry_points_refuse():
+    """The result that is normed, the previous rows and the mixing vectors: as layer_norm_ce_mix and rmsnorm look at them."""
+    from poptransformer_amd import kernels as K
+    g = torch.Generator(device="cuda").manual_seed(3)
+    x, w = torch.randn((20, 256), generator=g, device="cuda").half(), weight("f16", 64, 256, g)
+
+    def rows(*shape, dtype=torch.float16):
+        return torch.zeros(shape, dtype=dtype, device="cuda")
+    gamma = rows(64)
+    for out in (rows(20, 64, dtype=torch.float32), rows(20, 128)[:, ::2], rows(10, 128), rows(21, 64)):
+        with pytest.raises(ValueError):
+            K.linear_then_norm(x, w, out, K.RowNorm(gamma, None, 1e-5, out=rows(20, 64)))
+    for prev, mixes, mixed in ((rows(40, 32), [gamma], [rows(20, 64)]), (rows(20, 64), [gamma, gamma], [rows(20, 64)]), (rows(20, 64), [], []),
+                               (rows(20, 64), [gamma], [rows(20, 63)]), (rows(20, 64), [gamma.float()], [rows(20, 64)])):
+        with pytest.raises(ValueError):
+            K.linear_then_norm(x, w, rows(20, 64), K.RowNorm(gamma, gamma, 1e-5, shift=(prev, mixes, mixed)))
+    with pytest.raises(ValueError):
+        K.RowNorm(gamma, None, 1e-5, out=rows(20, 64), grid=(torch.zeros(1, dtype=torch.int64, device="cuda"), "F143"))
+    with pytest.raises(ValueError):
+        K.RowNorm(gamma.reshape(8, 8), None, 1e-5, out=rows(20, 64))
