@@ -130,6 +130,15 @@ struct GemmMat {
   WideOut wide;        // of the formats whose epilogue works in fp32 (Fmt::kWide)
 };
 
+// The fp32 activations of the wide formats, of every kernel the same.
+__device__ __forceinline__ float sigmoid_wide(float v) { return 1.0f / (1.0f + expf(-v)); }
+__device__ __forceinline__ float swiglu_f32(float g, float u) { return u * g / (1.0f + expf(-g)); }
+__device__ __forceinline__ float clamped_glu_f32(float g, float u, float limit, float slope) {
+  g = fminf(g, limit);
+  u = fminf(fmaxf(u, -limit), limit);
+  return g / (1.0f + expf(-slope * g)) * (u + 1.0f);
+}
+
 // The fp32 epilogue of the wide formats (Y is a bf16 or fp32 buffer behind the f16* of GemmMat).
 __device__ __forceinline__ float wide_value(const WideOut& w, int n, float v) {
   if (w.bias) v += w.bias[n];
@@ -137,7 +146,7 @@ __device__ __forceinline__ float wide_value(const WideOut& w, int n, float v) {
   switch (w.act) {
     case PTA_ACT_GELU_TANH: return 0.5f * v * (1.0f + tanhf(0.7978845608028654f * (v + 0.044715f * v * v * v)));
     case PTA_ACT_RELU_SQUARE: return v > 0.f ? v * v : 0.f;
-    case PTA_ACT_SIGMOID: return 1.0f / (1.0f + expf(-v));
+    case PTA_ACT_SIGMOID: return sigmoid_wide(v);
     default: return v;
   }
 }
@@ -145,10 +154,7 @@ __device__ __forceinline__ float wide_value(const WideOut& w, int n, float v) {
 __device__ __forceinline__ float wide_pair_value(const WideOut& w, int n, float g, float u) {
   if (w.bias) g += w.bias[n];
   if (w.bias2) u += w.bias2[n];
-  if (!w.clamped) return u * g / (1.0f + expf(-g));
-  g = fminf(g, w.limit);
-  u = fminf(fmaxf(u, -w.limit), w.limit);
-  return g / (1.0f + expf(-w.slope * g)) * (u + 1.0f);
+  return w.clamped ? clamped_glu_f32(g, u, w.limit, w.slope) : swiglu_f32(g, u);
 }
 
 __device__ __forceinline__ void wide_store(const WideOut& w, const GemmMat& mat, int m, int n, float v) {
@@ -2049,16 +2055,20 @@ __device__ __forceinline__ u32x4 eight_channels(T4 first, T4 second) {
   return u32x4{a0, a1, b0, b1};
 }
 
-// What is rounded to 16 bits: sigmoid and swish by the hardware's exponential and reciprocal (2 to 4 units of the 24-bit result).
-__device__ __forceinline__ float quick_sigmoid(float v) { return __builtin_amdgcn_rcpf(1.0f + __expf(-v)); }
-__device__ __forceinline__ float quick_swish(float v) { return v * quick_sigmoid(v); }
+// swish_f16 by the hardware's reciprocal, for the tiles: of all 65536 gates none comes out further from 64 bits than by the division (one, -0.7139, comes
+// out nearer; zeros lose their sign).
+__device__ __forceinline__ f16 tile_swish_f16(f16 x) {
+  const float v = (float)x;
+  return (f16)(v * __builtin_amdgcn_rcpf(1.0f + __expf(-v)));
+}
 
 // The ends of a tile that most products have, straight from the registers and without a loop; false: another one (panel_store).  What bounds
 // them is what they wait for: through LDS, row group by row group, each stretch of a residual, a gate or an old sum was a round trip to memory
-// of its own behind the one before, and swish by a division of eleven instructions kept a unit's vector ALU for 8 us a tile; here
-// all that a tile adds is requested together.  A launch of 2048 x 4096 without its products 10.3 -> 8.2 us (an empty one 2.6), 2048 x 8192 11.0 ->
-// 9.2; with them, weights from HBM: fp16, 2048 rows, 4096 x 8192 117 -> 114, 4096 x 4096 74 -> 72; bf16, 2048 rows, 11008 x 4096 with gate and
-// fp32 residual 215 -> 201, a pair of 4096 x 11008 341 -> 300, two of 4096 x 4096 with biases and sigmoids 137 -> 113.
+// of its own behind the one before; here all that a tile adds is requested together.  A launch of 2048 x 4096 without its products 10.3 -> 8.2 us
+// (an empty one 2.6), 2048 x 8192 11.0 -> 9.2; with them, weights from HBM: fp16, 2048 rows, 4096 x 8192 117 -> 114, 4096 x 4096 74 -> 72; bf16, 2048
+// rows, 11008 x 4096 with gate and fp32 residual 215 -> 201, a pair of 4096 x 11008 341 -> 310, two of 4096 x 4096 with biases and sigmoids in turn 151.
+// Not kept: sigmoid and swish of fp32 sums by the hardware's exponential and reciprocal (the pair 299, the two 143): their error is 4 to 60 units of the
+// 24-bit result where the exact exponential and a division make two, and results would depend on the kernel that the number of rows selects.
 template <class Fmt, int NST, int RG, bool PAIR>
 __device__ __forceinline__ bool straight_store(const GemmMat& mat, const GemmEpilogue& epi, float* part, const f32x4 (&acc)[RG][NST], int blk0, int row0, int nsl,
                                                typename Fmt::Scale s0, typename Fmt::Scale s1, int M, const int32_t* order) {
@@ -2091,7 +2101,7 @@ __device__ __forceinline__ bool straight_store(const GemmMat& mat, const GemmEpi
         for (int st = 0; st < 2; ++st)
 #pragma unroll
           for (int e = 0; e < 4; ++e)
-            v[st][e] = (f16)Fmt::finish(acc[rg][2 + st][e], s1) * (f16)quick_swish((float)(f16)Fmt::finish(acc[rg][st][e], s0));
+            v[st][e] = (f16)Fmt::finish(acc[rg][2 + st][e], s1) * tile_swish_f16((f16)Fmt::finish(acc[rg][st][e], s0));
         const u32x4 out = eight_channels(v[0], v[1]);
         if (in && row0 + rg * 16 + r < M) *reinterpret_cast<u32x4*>(y + (size_t)rg * 16 * N) = out;
       }
@@ -2163,12 +2173,8 @@ __device__ __forceinline__ bool straight_store(const GemmMat& mat, const GemmEpi
         }
       };
       const float limit = w.limit, slope = w.slope;
-      if (w.clamped) all([=](float a, float b) {
-        a = fminf(a, limit);
-        b = fminf(fmaxf(b, -limit), limit);
-        return a * quick_sigmoid(slope * a) * (b + 1.0f);
-      });
-      else all([](float a, float b) { return b * quick_swish(a); });
+      if (w.clamped) all([=](float a, float b) { return clamped_glu_f32(a, b, limit, slope); });
+      else all([](float a, float b) { return swiglu_f32(a, b); });
     } else {
       if (w.cap > 0.f || (w.act != PTA_ACT_NONE && (w.act != PTA_ACT_SIGMOID || w.out_f32))) return false;
       if (!w.out_f32 && (w.mul || w.accumulate)) return false;
@@ -2203,7 +2209,7 @@ __device__ __forceinline__ bool straight_store(const GemmMat& mat, const GemmEpi
                 *reinterpret_cast<u32x4*>(reinterpret_cast<bf16*>(mat.Y) + (size_t)m[rg] * w.ld + n0 + p * 32 + c8) = out;
             }
         };
-        if (w.act == PTA_ACT_SIGMOID) all([](float v) { return quick_sigmoid(v); });
+        if (w.act == PTA_ACT_SIGMOID) all([](float v) { return sigmoid_wide(v); });
         else all([](float v) { return v; });
       } else {
         // (some row groups at a time, as many as the registers hold: what they are multiplied by and added to is requested together)

@@ -531,3 +531,46 @@ def test_tiles_of_other_sizes(kind, form, M, Kd, N):
     last = 2.0 ** -8 if kind == "bf16" else 2.5 * 2.0 ** -11
     bound = 1.1 * dg * (upv.abs() + du) + du * silu.abs() + last * (silu * upv).abs() + 2.0 ** -20 * (1 + upv.abs())
     assert ((outs[0].double() - silu * upv).abs() <= bound).all()
+
+
+def test_no_gate_is_further_from_64_bits_than_by_the_operator():
+    """Every finite fp16 gate through the end of a tile: rows that pick one feature, so that sums are the weights' own values, beside 1 from the other weight."""
+    from poptransformer_amd import kernels as K
+    gates = torch.arange(-32768, 32768, dtype=torch.int32, device="cuda").to(torch.int16).view(torch.float16)
+    gates = gates[torch.isfinite(gates)].contiguous()
+    x = torch.zeros((136, 32), dtype=torch.float16, device="cuda")
+    x[:, 5] = 1
+    g, u = torch.zeros((2, len(gates), 32), dtype=torch.float16, device="cuda")
+    g[:, 5], u[:, 5] = gates, 1
+    out = torch.full((136, len(gates)), float("nan"), dtype=torch.float16, device="cuda")
+    K.linear(x, [K.F16Weight(g), K.F16Weight(u)], [out, out], swiglu=True)
+    assert K.linear_kernel() == "gemm_block_kernel" and torch.equal(out, out[:1].expand_as(out))
+    exact = torch.nn.functional.silu(gates.double())
+    by_operator = K.swiglu(gates, torch.ones_like(gates))
+    assert ((out[0].double() - exact).abs() <= (by_operator.double() - exact).abs()).all()
+
+
+@pytest.mark.parametrize("end", ["sigmoid", "swiglu", "clamped"])
+def test_activations_do_not_depend_on_how_many_rows_there_are(end):
+    """The same sums, exact by rows that pick one feature, through the kernels of few and of many rows: gates of all fp32 fractions from -60 to 60."""
+    from poptransformer_amd import _hybrid_lib as H
+    from poptransformer_amd import hybrid_kernels as HK
+    N = 262144
+    x = torch.zeros((264, 64), dtype=torch.bfloat16, device="cuda")
+    x[:, 9] = 1
+    w = torch.zeros((2, N, 64), device="cuda")
+    w[1, :, 9] = torch.linspace(-3, 3, N, device="cuda").bfloat16().float()
+    made = [HK.WideWeight(t, torch.bfloat16) for t in w]
+    b1, b2 = torch.linspace(-60, 60, N, device="cuda") * 1.0003, torch.linspace(-1, 1, N, device="cuda")
+    kw = {"sigmoid": dict(bias=b1, act=H.ACT_SIGMOID), "swiglu": dict(up=made[1], pair=H.PAIR_SWIGLU, bias=b1, bias2=b2),
+          "clamped": dict(up=made[1], pair=H.PAIR_CLAMPED, limit=7.0, slope=1.7, bias=b1, bias2=b2)}[end]
+    results = {}
+    for rows in (4, 16, 264):
+        out = torch.full((rows, N), float("nan"), dtype=torch.bfloat16, device="cuda")
+        HK.linear(x, made[0], out, rows, ld=N, **kw)
+        results[HK.linear_kernel()] = out[:1]
+        assert torch.equal(out, out[:1].expand_as(out))
+    assert "gemm_block_kernel" in results and len(results) > 1
+    for out in results.values():
+        differ = (out != results["gemm_block_kernel"]).sum().item()
+        assert differ == 0, differ
