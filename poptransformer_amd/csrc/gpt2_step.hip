@@ -218,7 +218,7 @@ __device__ __forceinline__ void g2_product(const G2Args& a, const G2Product& q, 
       const f16 mean16 = (f16)mean;
       const float about = MB == 1 ? mean : (float)mean16;                        // (as the norm of a single row, and of several)
       const float var = (MB == 1 ? sq - about * about : fmaxf(sq - about * about, 0.0f)) + a.m.eps;
-      const f16 r16 = (f16)__builtin_amdgcn_rsqf(var);
+      const f16 r16 = (f16)(1.0f / sqrtf(var));
 #pragma unroll
       for (int i = 0; i < OWN; ++i) {
         const int c = first + i * SPAN;

@@ -197,3 +197,43 @@ def test_a_wait_that_gave_up_is_reported_and_cleared(clear):
         got, step = one.run(ids, 12)
         assert step == 12
         _close(one.logits, per_op.logits)
+
+
+@pytest.mark.parametrize("B", [1, 2, 3, 8])
+def test_norms_are_those_of_the_operators(B):
+    """A key projection that hands the normed row on: the ring then holds the norms' results, bit for bit those of layer_norm_ce.  Rows of small multiples of
+    1/16 with mean 0, whose sums are the same in any order; their squares add up to numbers whose reciprocal root lies so near the middle of two fp16
+    numbers that the hardware's own (v_rsq_f32) falls on the other side of it."""
+    from poptransformer_amd import kernels as K
+    from poptransformer_amd.engine import fused, loader
+    squares = [17680, 21316, 114192, 147636, 295638, 296560, 302818, 312250, 505720, 521874, 621112, 626752, 643156, 653108, 672664, 693112, 798424, 883610, 899668,
+               963054, 1027398, 1058372, 1111148, 1136136, 1216374, 1292714, 1302582, 1328482, 1423866, 1461878, 1468644, 1508476, 1604728, 1695658, 1767344, 1771834]
+    L, d = 72, 64
+    cfg = _cfg(1, layers=1, vocab=2 + 2 * len(squares), positions=L)
+    sd, rng = OM.make_gpt2_state_dict(cfg, seed=3), np.random.default_rng(8)
+    table = np.zeros((cfg["vocab_size"], d))
+    for token in range(2, len(table)):
+        rest, half = squares[(token - 2) % len(squares)] // 2, []
+        while rest:
+            half.append(min(int(np.sqrt(rest)), 255))
+            rest -= half[-1] ** 2
+        row = np.zeros(d)
+        row[:2 * len(half)] = half + [-v for v in half]
+        table[token] = rng.permutation(row) / 16
+    a, n = "transformer.h.0.attn.c_attn.", "transformer.h.0.ln_1."
+    for key, value in {"transformer.wte.weight": table, "transformer.wpe.weight": np.zeros((L, d)), a + "weight": np.concatenate([np.zeros((d, d)), np.eye(d), np.eye(d)]),
+                       a + "bias": np.zeros(3 * d), n + "weight": np.ones(d), n + "bias": np.zeros(d)}.items():
+        sd[key] = value.astype(np.float16)
+    dec = fused.FusedDecoder(loader.gpt2_spec(cfg, L, B, 0, 1), loader.gpt2_weights(sd, cfg))
+    ids = np.stack([rng.permutation(np.arange(2, 2 + L)) for _ in range(B)]).astype(np.int32)
+    dec.reset(ids)
+    for _ in range(L):
+        dec.step_fn()
+    torch.cuda.synchronize()
+    assert dec.chained is not None and not dec.chained.failed()
+    x = torch.from_numpy(sd["transformer.wte.weight"][ids]).cuda()
+    gamma, beta = torch.ones(d, dtype=torch.float16, device="cuda"), torch.zeros(d, dtype=torch.float16, device="cuda")
+    want = torch.stack([K.layer_norm_ce(x[:, t].contiguous(), gamma, beta, cfg["layer_norm_epsilon"]) for t in range(L)], 1)
+    for got in dec.rings[0].reshape(2, B, L, d):                                  # keys, values
+        differ = (got != want).any(2).sum().item()
+        assert differ == 0, differ
