@@ -321,6 +321,11 @@ class FusedDecoder(DecodeLoop, LayerOps):
             return None
         if any(len(b.qkv) != 1 or len(b.mlp_in) != 1 for b in w.blocks) or len(w.blocks) != s.n_layer:
             return None
+        # A head's cache rows are one workgroup's there, where the operators cut them among several: beyond some 4500 to 6500 positions those are the faster ones.
+        # us a token, one launch and operators, contexts of 1024, 4096, 8000 - GPT-2 small, batch 1: 236 372, 404 458, 618 512; 4: 293 422, 476 492, 709 580;
+        # 8: 356 482, 566 616, 847 805; width 256, batch 8: 272 391, 445 459, 669 508; 8 layers of 1280: 211 311, 324 360, 471 387
+        if s.max_len > 4096:
+            return None
         d, ffn = s.d_model, w.blocks[0].mlp_out.K
 
         def plain(t, *shape):

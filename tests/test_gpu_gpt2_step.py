@@ -237,3 +237,10 @@ def test_norms_are_those_of_the_operators(B):
     for got in dec.rings[0].reshape(2, B, L, d):                                  # keys, values
         differ = (got != want).any(2).sum().item()
         assert differ == 0, differ
+
+
+def test_caches_of_several_thousand_positions_stay_per_operator():
+    from poptransformer_amd.engine import fused, loader
+    cfg = _cfg(1, layers=1, positions=5000)
+    w = loader.gpt2_weights(OM.make_gpt2_state_dict(cfg, seed=3), cfg)
+    assert [fused.FusedDecoder(loader.gpt2_spec(cfg, n, 1, 0, 1), w).chained is not None for n in (4096, 4097, 5000)] == [True, False, False]
