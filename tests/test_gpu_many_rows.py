@@ -533,21 +533,23 @@ def test_tiles_of_other_sizes(kind, form, M, Kd, N):
     assert ((outs[0].double() - silu * upv).abs() <= bound).all()
 
 
-def test_no_gate_is_further_from_64_bits_than_by_the_operator():
-    """Every finite fp16 gate through the end of a tile: rows that pick one feature, so that sums are the weights' own values, beside 1 from the other weight."""
+def test_every_gate_comes_out_as_by_the_operator():
+    """Every fp16 gate but NaN through the end of a tile, bit for bit: rows that pick one feature, so that sums are the weights' own values, beside 1 from the
+    other weight."""
     from poptransformer_amd import kernels as K
     gates = torch.arange(-32768, 32768, dtype=torch.int32, device="cuda").to(torch.int16).view(torch.float16)
-    gates = gates[torch.isfinite(gates)].contiguous()
+    gates = gates[~torch.isnan(gates) & (gates.view(torch.int16) != -32768)]      # (a sum has no negative zero)
+    gates = torch.cat([gates, gates.new_ones(-len(gates) % 8)])
     x = torch.zeros((136, 32), dtype=torch.float16, device="cuda")
     x[:, 5] = 1
     g, u = torch.zeros((2, len(gates), 32), dtype=torch.float16, device="cuda")
     g[:, 5], u[:, 5] = gates, 1
-    out = torch.full((136, len(gates)), float("nan"), dtype=torch.float16, device="cuda")
+    out = torch.full((136, len(gates)), 7.0, dtype=torch.float16, device="cuda")
     K.linear(x, [K.F16Weight(g), K.F16Weight(u)], [out, out], swiglu=True)
-    assert K.linear_kernel() == "gemm_block_kernel" and torch.equal(out, out[:1].expand_as(out))
-    exact = torch.nn.functional.silu(gates.double())
-    by_operator = K.swiglu(gates, torch.ones_like(gates))
-    assert ((out[0].double() - exact).abs() <= (by_operator.double() - exact).abs()).all()
+    assert K.linear_kernel() == "gemm_block_kernel"
+    want = K.swiglu(gates, torch.ones_like(gates))
+    differ = ((out.view(torch.int16) != want.view(torch.int16)) & ~(torch.isnan(out) & torch.isnan(want))).any(0)
+    assert not differ.any(), (gates[differ], out[0, differ], want[differ])
 
 
 @pytest.mark.parametrize("end", ["sigmoid", "swiglu", "clamped"])
