@@ -117,20 +117,24 @@ class LayerOps:
     """The per-layer operators over `rows` activation rows: the row buffers and the calls that the decode
     iteration (rows = batch) and the prompt passes (rows = batch * positions) share."""
 
-    def __init__(self, spec: DecoderSpec, weights: ModelWeights, device, rows):
+    def __init__(self, spec: DecoderSpec, weights: ModelWeights, device, rows, memory=None):
+        """memory: where the row buffers lie (prompt.RowMemory), or None: in tensors of their own."""
         self.spec, self.w, self.dev, self._rows = spec, weights, device, rows
         s, f16 = spec, torch.float16
 
-        def buf(*shape, dtype=f16):
+        def own(*shape, dtype=f16):
             return torch.zeros(shape, dtype=dtype, device=device)
 
-        self._buf = buf
+        def own_scratch(make, n):
+            return make(n)
+        self._buf = buf = own if memory is None else memory.buffer
+        self._scratch = scratch = own_scratch if memory is None else memory.scratch
         d, ffn = s.d_model, weights.blocks[0].mlp_out.K
         self.x, self.h, self.ctx = buf(rows, d), buf(rows, d), buf(rows, d)
         self.qkv = buf(rows, sum(lw.N for lw in weights.blocks[0].qkv))
         self.q_rot = buf(rows, s.n_head, s.head_dim)
         self.act = buf(rows, ffn)
-        self.attn_ws = K.decode_attention_workspace(rows, s.n_head, s.head_dim, s.max_len, device)
+        self.attn_ws = scratch(lambda n: K.decode_attention_workspace(n, s.n_head, s.head_dim, s.max_len, device), rows)
         # The norm inside the GEMM: every workgroup normalises the rows it stages.  Up to 4 rows that is cheaper than
         # a launch of its own since the rows' sums over a wave are made by data-parallel moves (Llama 2 at the 7B
         # width, batch 1, one launch per operator: 1.687 -> 1.593 ms per step; with shuffles it cost 5 us per
@@ -142,7 +146,10 @@ class LayerOps:
         self._gate, self._up = buf(rows, ffn), buf(rows, ffn)
         self._on_grid = {}      # buffer address -> the FP8 grid (format, exponent) its values are on
         # scratch that lets a Linear of more than 16 rows with few output channels (attention output, MLP down) split K
-        self._lin_ws = K.linear_workspace(rows, d, device) if rows > 16 else None
+        self._lin_ws = self._linear_workspace(d, ffn) if rows > 16 else None
+
+    def _linear_workspace(self, d, ffn):
+        return K.linear_workspace(self._rows, d, self.dev)
 
     def _norm(self, x, gb, out):
         if self.spec.norm == "rms":
@@ -245,17 +252,16 @@ class LayerOps:
         """Output buffers of the projections and the (pointer, row stride) views of q, k, v."""
         s = self.spec
         B, Hq, Hkv, D = self._rows, s.n_head, s.n_kv_head, s.head_dim
-        f16 = torch.float16
         if len(blk.qkv) == 1:           # GPT-2: one row holds q | k | v
             row = (Hq + 2 * Hkv) * D
             self._qkv_bufs = [self.qkv]
             self._qkv_views = (self.qkv, self.qkv[:, Hq * D:], self.qkv[:, (Hq + Hkv) * D:], row, row, row)
         elif len(blk.qkv) == 3:         # Llama 2: separate q, k, v
-            self._qkv_bufs = [torch.zeros((B, lw.N), dtype=f16, device=self.dev) for lw in blk.qkv]
+            self._qkv_bufs = [self._buf(B, lw.N) for lw in blk.qkv]
             q, k, v = self._qkv_bufs
             self._qkv_views = (q, k, v, Hq * D, Hkv * D, Hkv * D)
         else:                           # ChatGLM2: query, and key_value holding k | v
-            self._qkv_bufs = [torch.zeros((B, lw.N), dtype=f16, device=self.dev) for lw in blk.qkv]
+            self._qkv_bufs = [self._buf(B, lw.N) for lw in blk.qkv]
             q, kv = self._qkv_bufs
             self._qkv_views = (q, kv, kv[:, Hkv * D:], Hq * D, 2 * Hkv * D, 2 * Hkv * D)
 
@@ -445,7 +451,7 @@ class FusedDecoder(DecodeLoop, LayerOps):
         Each weight matrix is then read once per pass instead of once per position.  The KV rings and the loop
         state end up as `n` iterations of the loop leave them; the logits of these positions are not computed
         (the loop would discard their tokens).  Call after `reset`.  Returns n."""
-        from .prompt import PromptPass
+        from .prompt import PromptPasses
         s = self.spec
         n = self.checked_prompt_count(n)
         if n == 0:
@@ -457,14 +463,12 @@ class FusedDecoder(DecodeLoop, LayerOps):
         if R < 1 or R * s.batch > 2048:
             raise ValueError(f"consume_prompt: rows_per_pass * batch must lie in [1, 2048], got {R} * {s.batch}")
         if not hasattr(self, "_prompt_passes"):
-            self._prompt_passes = {}
+            self._prompt_passes = PromptPasses(self)
         with torch.cuda.stream(self._stream):
             p0 = 0
             while p0 < n:
                 rc = min(R, n - p0)
-                if rc not in self._prompt_passes:
-                    self._prompt_passes[rc] = PromptPass(self, rc)
-                self._prompt_passes[rc].run(p0)
+                self._prompt_passes.of(rc).run(p0)
                 p0 += rc
             # the state n iterations leave behind (pta_step_update n times): positions 0..n open, no stop
             self.mask[:, :n + 1] = 0

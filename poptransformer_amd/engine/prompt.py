@@ -13,6 +13,8 @@ causal attention of row r over positions 0..p0+r.  The final norm, the head and 
 are skipped: the loop would discard their result.  What it leaves in the KV rings is what R iterations
 of the loop leave there, up to the rounding of a different summation order in the GEMMs.
 """
+from collections import OrderedDict
+
 import torch
 
 from .. import _lib
@@ -20,18 +22,83 @@ from .. import kernels as K
 from .fused import LayerOps
 
 
-class PromptPass(LayerOps):
-    """Buffers for B*rows rows and one pass over the layers; shares weights and KV rings with the decoder `dec`."""
+class RowMemory:
+    """The row buffers of all passes of up to `rows` rows: each pass takes the first rows of every buffer, in the same order.  Passes follow each other on one
+    stream, and none looks at what another has left."""
 
-    def __init__(self, dec, rows):
-        super().__init__(dec.spec, dec.w, dec.dev, dec.spec.batch * int(rows))
-        self.dec, self.rows = dec, int(rows)
+    def __init__(self, rows, device):
+        self.rows, self.device, self.made = rows, device, []
+
+    def taken(self):
+        """The buffers from the first one on, for one pass."""
+        return RowBuffers(self)
+
+
+class RowBuffers:
+    def __init__(self, memory):
+        self.memory, self.next = memory, 0
+
+    def _next(self, make):
+        if self.next == len(self.memory.made):
+            self.memory.made.append(make(self.memory.rows))
+        self.next += 1
+        return self.memory.made[self.next - 1]
+
+    def buffer(self, rows, *shape, dtype=torch.float16):
+        t = self._next(lambda n: torch.zeros((n, *shape), dtype=dtype, device=self.memory.device))
+        if t.shape[1:] != shape or t.dtype != dtype or rows > len(t):
+            raise RuntimeError(f"prompt pass: buffer [{rows}, {shape}] {dtype} where others have {tuple(t.shape)} {t.dtype}")
+        return t[:rows]
+
+    def scratch(self, make, rows):
+        """make(rows): the bytes that so many rows need."""
+        return self._next(make)
+
+
+class PromptPasses:
+    """The passes of a decoder by their number of positions, those used last.  Row buffers are shared, in sizes of powers of two, so that all of them together
+    are less than twice the largest (at the 7B width, 2048 rows with a cache of 2048: 2 GB, which each length of prompts would hold for itself else); recorded
+    passes take what else they need from one pool."""
+
+    most = 256                       # passes that are kept
+
+    def __init__(self, dec):
+        self.dec, self.memory, self.passes, self.pool = dec, {}, OrderedDict(), None
+
+    def of(self, rows):
+        if rows not in self.passes:
+            n = self.dec.spec.batch * rows
+            size = max(64, 1 << (n - 1).bit_length())
+            if size not in self.memory:
+                self.memory[size] = RowMemory(size, self.dec.dev)
+            while len(self.passes) >= self.most:
+                torch.cuda.current_stream().synchronize()      # (a replay may be on its way)
+                self.passes.popitem(last=False)
+            if self.pool is None:
+                self.pool = torch.cuda.graph_pool_handle()
+            self.passes[rows] = PromptPass(self.dec, rows, self.memory[size].taken(), self.pool)
+        self.passes.move_to_end(rows)
+        return self.passes[rows]
+
+
+class PromptPass(LayerOps):
+    """One pass over the layers of B*rows rows; shares weights and KV rings with the decoder `dec`, row buffers with its other passes."""
+
+    def __init__(self, dec, rows, memory, pool):
+        super().__init__(dec.spec, dec.w, dec.dev, dec.spec.batch * int(rows), memory)
+        self.dec, self.rows, self.pool = dec, int(rows), pool
         s, i32 = self.spec, torch.int32
         self.first = torch.zeros((), dtype=i32, device=self.dev)       # position of row 0 of every sequence
         self._offsets = torch.arange(self.rows, dtype=i32, device=self.dev)
         self.graph = None
-        # scratch for the K split of the projections with few output channels (attention output, MLP down)
-        self._lin_ws = K.linear_workspace(self._rows, max(s.d_model, self.w.blocks[0].mlp_out.K), self.dev)
+        if self._lin_ws is None:
+            self._lin_ws = self._linear_workspace(s.d_model, self.w.blocks[0].mlp_out.K)
+
+    def _linear_workspace(self, d, ffn):
+        """Scratch for the K split of the projections with few output channels (attention output, MLP down): what this pass's rows need of the shared one, so
+        that a product is cut alike whatever passes there were."""
+        shared = self._scratch(lambda n: K.linear_workspace(n, max(d, ffn), self.dev), self._rows)
+        return shared[:K.linear_workspace_bytes(self._rows, max(d, ffn))]
 
     def run(self, p0):
         """Positions p0 .. p0+rows-1 of every sequence (row b*rows + r is sequence b at p0 + r).  The pass
@@ -50,7 +117,7 @@ class PromptPass(LayerOps):
             stream = torch.cuda.current_stream()
             stream.synchronize()
             self.graph = torch.cuda.CUDAGraph()
-            with torch.cuda.graph(self.graph, stream=stream):
+            with torch.cuda.graph(self.graph, pool=self.pool, stream=stream):
                 self._layers()
             self.graph.replay()
 

@@ -69,9 +69,13 @@ def _fusion(bias=None, residual=None, act=_lib.ACT_NONE, norm=None, mul=None, po
     return ctypes.byref(e)
 
 
+def linear_workspace_bytes(M, N):
+    return _lib.load().pta_linear_workspace_bytes(M, N)
+
+
 def linear_workspace(M, N, device):
     """Scratch that lets a single-weight `linear` of more than 16 rows split K across workgroups."""
-    return torch.empty(_lib.load().pta_linear_workspace_bytes(M, N), dtype=torch.uint8, device=device)
+    return torch.empty(linear_workspace_bytes(M, N), dtype=torch.uint8, device=device)
 
 
 def linear_kernel():

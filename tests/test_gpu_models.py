@@ -304,6 +304,58 @@ def test_prompt_in_passes_equals_the_loop(family, B, plen, rows_per_pass):
     _equal_up_to_a_near_tie(dec.container.cpu().numpy(), ref_container, trace)
 
 
+@pytest.mark.parametrize("family,B", [("llama2", 1), ("llama2", 3), ("gpt2", 2), ("chatglm2", 1)])
+def test_prompts_of_many_lengths_share_their_row_buffers(family, B, monkeypatch):
+    """Lengths in turn, each eagerly, recorded and replayed: the caches are those of a decoder that knows one length only, and memory does not grow with the
+    number of lengths - also where passes are given up for others."""
+    from poptransformer_amd.engine import fused, loader, prompt
+    L = 200
+    if family == "llama2":
+        weights, spec = loader.llama2_weights(OM.make_llama2_state_dict(LLAMA_TINY, seed=1, int4=True), LLAMA_TINY), loader.llama2_spec(LLAMA_TINY, L, B, 0, 2)
+    elif family == "gpt2":
+        cfg = dict(GPT2_TINY, n_positions=L)
+        weights, spec = loader.gpt2_weights(OM.make_gpt2_state_dict(cfg, seed=2), cfg), loader.gpt2_spec(cfg, L, B, 0, 2)
+    else:
+        weights, spec = loader.chatglm2_weights(OM.make_chatglm2_state_dict(GLM2_TINY, seed=4), GLM2_TINY, "fp16"), loader.chatglm2_spec(GLM2_TINY, L, B, 0, 2)
+    dec = fused.FusedDecoder(spec, weights)
+    rng = np.random.default_rng(4)
+    ids = rng.integers(3, spec.vocab, size=(B, L)).astype(np.int32)
+    lengths = [129, 64, 20, 100, 199, 5, 101, 128, 17, 99, 1, 16]
+    want = {}
+    for n in lengths:
+        alone = fused.FusedDecoder(spec, weights)
+        alone.reset(ids)
+        alone.consume_prompt(n)
+        want[n] = [r[:, :n].clone() for r in alone.rings]
+        del alone
+
+    def check(n):
+        for ring in dec.rings:
+            ring.zero_()
+        dec.reset(ids)
+        assert dec.consume_prompt(n) == n
+        for got, ref in zip(dec.rings, want[n]):
+            assert torch.equal(got[:, :n], ref), n
+    for _ in range(3):
+        for n in lengths:
+            check(n)
+    torch.cuda.synchronize()
+    before = torch.cuda.memory_allocated()
+    for n in range(30, 190):
+        for _ in range(2):
+            dec.reset(ids)
+            dec.consume_prompt(n)
+    assert torch.cuda.memory_allocated() - before < 160 * 64 * 1024                   # (a few numbers and a recording's own each)
+    monkeypatch.setattr(prompt.PromptPasses, "most", 2)
+    before = torch.cuda.memory_allocated()
+    dec.reset(ids)
+    dec.consume_prompt(190)
+    for order in (lengths, [100, 100, 100, 64, 100, 64, 64, 100, 20], lengths):
+        for n in order:
+            check(n)
+    assert len(dec._prompt_passes.passes) <= 2 and torch.cuda.memory_allocated() <= before
+
+
 def test_prompt_passes_stop_before_an_end_token_and_check_their_arguments():
     from poptransformer_amd.engine import fused, loader
     B, L, pad, eos = 2, 48, 0, 2
