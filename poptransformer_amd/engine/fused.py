@@ -460,7 +460,7 @@ class FusedDecoder(DecodeLoop, LayerOps):
         # fewer products, and read the weights half as often.  2048 against 1024 rows: ChatGLM2 FP8 8 x 255 27.1 -> 24.1 ms, six layers
         # of Llama2 INT4 2 x 552 3.90 -> 3.46, of 2048 channels 3 x 417 to 8 x 225 1.2 to 1.4 times, GPT-2 small 6 x 203 2.43 -> 1.85
         R = max(1, min(n, 2048 // s.batch)) if rows_per_pass is None else int(rows_per_pass)
-        if R < 1 or R * s.batch > 2048:
+        if R < 1 or R * s.batch > PromptPasses.most_rows:
             raise ValueError(f"consume_prompt: rows_per_pass * batch must lie in [1, 2048], got {R} * {s.batch}")
         if not hasattr(self, "_prompt_passes"):
             self._prompt_passes = PromptPasses(self)

@@ -45,10 +45,10 @@ class RowBuffers:
         return self.memory.made[self.next - 1]
 
     def buffer(self, rows, *shape, dtype=torch.float16):
-        t = self._next(lambda n: torch.zeros((n, *shape), dtype=dtype, device=self.memory.device))
+        t = self._next(lambda n: torch.empty((n, *shape), dtype=dtype, device=self.memory.device))
         if t.shape[1:] != shape or t.dtype != dtype or rows > len(t):
             raise RuntimeError(f"prompt pass: buffer [{rows}, {shape}] {dtype} where others have {tuple(t.shape)} {t.dtype}")
-        return t[:rows]
+        return t[:rows].zero_()
 
     def scratch(self, make, rows):
         """make(rows): the bytes that so many rows need."""
@@ -56,27 +56,32 @@ class RowBuffers:
 
 
 class PromptPasses:
-    """The passes of a decoder by their number of positions, those used last.  Row buffers are shared, in sizes of powers of two, so that all of them together
-    are less than twice the largest (at the 7B width, 2048 rows with a cache of 2048: 2 GB, which each length of prompts would hold for itself else); recorded
-    passes take what else they need from one pool."""
+    """The passes of a decoder by their number of positions, those used last.  They share row buffers (at the 7B width, 2048 rows with a cache of 2048: 2 GB,
+    which each length of prompts would hold for itself else): a pass takes the smallest set that has its rows.  The first set is as large as its pass needs, a
+    larger one that is needed later at least half as large again, so that all of them together stay below four times the largest pass's.  Recorded passes take
+    what else they need from one pool."""
 
-    most = 256                       # passes that are kept
+    most_rows, most = 2048, 256      # of a pass; passes that are kept
 
     def __init__(self, dec):
-        self.dec, self.memory, self.passes, self.pool = dec, {}, OrderedDict(), None
+        self.dec, self.memory, self.passes, self.pool = dec, [], OrderedDict(), None
+
+    def _memory(self, rows):
+        fit = [m for m in self.memory if m.rows >= rows]
+        if not fit:
+            largest = max((m.rows for m in self.memory), default=0)
+            fit.append(RowMemory(max(rows, min(self.most_rows, largest * 3 // 2)), self.dec.dev))
+            self.memory += fit
+        return min(fit, key=lambda m: m.rows)
 
     def of(self, rows):
         if rows not in self.passes:
-            n = self.dec.spec.batch * rows
-            size = max(64, 1 << (n - 1).bit_length())
-            if size not in self.memory:
-                self.memory[size] = RowMemory(size, self.dec.dev)
             while len(self.passes) >= self.most:
                 torch.cuda.current_stream().synchronize()      # (a replay may be on its way)
                 self.passes.popitem(last=False)
             if self.pool is None:
                 self.pool = torch.cuda.graph_pool_handle()
-            self.passes[rows] = PromptPass(self.dec, rows, self.memory[size].taken(), self.pool)
+            self.passes[rows] = PromptPass(self.dec, rows, self._memory(self.dec.spec.batch * rows).taken(), self.pool)
         self.passes.move_to_end(rows)
         return self.passes[rows]
 
