@@ -125,6 +125,8 @@ typedef struct pta_row_norm {
 } pta_row_norm;
 /* the name of the kernel that the calling thread's last product took, "" before the first (a product of several launches: the last one's) */
 const char* pta_linear_kernel(void);
+/* the tiles (rows x channels) of the calling thread's last product by gemm_block_kernel, behind a space those of its last channels where they are others */
+const char* pta_linear_tiles(void);
 
 enum { PTA_NORM_NONE = 0, PTA_NORM_RMS = 1, PTA_NORM_LAYER = 2 };
 enum { PTA_ACT_NONE = 0, PTA_ACT_GELU_TANH = 1, PTA_ACT_RELU_SQUARE = 2, PTA_ACT_SIGMOID = 3 };

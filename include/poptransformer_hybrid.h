@@ -67,6 +67,8 @@ typedef struct pta_wide_linear_args {
 size_t pta_wide_linear_workspace_bytes(int M, int N);
 /* the name of the kernel that the calling thread's last bf16 product (or listed product of experts) took, "" before the first */
 const char* pta_wide_linear_kernel(void);
+/* as pta_linear_tiles */
+const char* pta_wide_linear_tiles(void);
 int pta_wide_linear(const pta_wide_linear_args* host_args, pta_stream_t stream);
 /* up to four single weights over inputs of the same shape, each with its own input and result: one launch where
  * there are few rows, or many rows and whole tiles of channels */

@@ -100,6 +100,7 @@ SIGNATURES = {
     "pta_bf16_tile": (_I, [_P, _P, _I, _I, _P]),
     "pta_wide_linear_workspace_bytes": (c_size_t, [_I, _I]),
     "pta_wide_linear_kernel": (c_char_p, []),
+    "pta_wide_linear_tiles": (c_char_p, []),
     "pta_wide_linear": (_I, [POINTER(WideLinearArgs), _P]),
     "pta_wide_linear_group": (_I, [POINTER(WideLinearArgs), _I, _P]),
     "pta_shift_norm": (_I, [POINTER(ShiftNormArgs), _P]),

@@ -344,6 +344,7 @@ static inline int device_compute_units();
 // The kernel that the calling thread's last product took (its last launch's, where it was several; without the finish of a K split): for
 // tests that are meant for one of them.
 inline thread_local const char* gemm_kernel_taken = "";
+inline thread_local const char* gemm_tiles_taken = "";           // of gemm_block_kernel: rows x channels of its tiles, then of the rest's
 constexpr int GEMM_MAX_KSPLIT = 4;
 constexpr int GEMM_MAX_ROWS = 4096;
 // From so many features on the rows of a workgroup (up to 256, and 48 rows past the last one) take more bytes than the 32-bit offsets of
@@ -2895,6 +2896,8 @@ static int dispatch_gemm_block(const GemmArgs& a, hipStream_t s, const char* nam
       default: return launch_gemm_block<Fmt, 2, PAIR>(b, 2 * group0, group1 < 0 ? narrow : 2 * group1, s, name);
     }
   };
+  static const char* const tiles[4][4] = {{"128x128"}, {"128x256"}, {"192x256"}, {"256x256", "256x256 128x128", "256x256 128x256", "256x256 192x256"}};
+  gemm_tiles_taken = tiles[rg / 2 - 1][rest / 2];
   int rc = launch(rg, 0, rest ? whole : -1);
   if (!rc && rest) rc = launch(rest, whole, -1);
   if (rc) return rc;

@@ -157,6 +157,7 @@ extern "C" int pta_linear_then_norm(const pta_half* X, const int32_t* x_scale, c
 }
 
 extern "C" const char* pta_linear_kernel(void) { return gemm_kernel_taken; }
+extern "C" const char* pta_linear_tiles(void) { return gemm_tiles_taken; }
 
 extern "C" size_t pta_linear_workspace_bytes(int M, int N) {
   if (M <= 0 || N <= 0) return 0;

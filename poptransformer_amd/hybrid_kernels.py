@@ -72,6 +72,11 @@ def linear_kernel():
     return H.load().pta_wide_linear_kernel().decode()
 
 
+def linear_tiles():
+    """The tiles of this thread's last bf16 product by gemm_block_kernel (pta_linear_tiles)."""
+    return H.load().pta_wide_linear_tiles().decode()
+
+
 def _linear_args(x, w, out, rows, ld=None, tail=None, cap=0.0, up=None, pair=H.PAIR_NONE, limit=0.0, slope=0.0, workspace=None, bias=None,
                  bias2=None, act=H.ACT_NONE, mul=None, accumulate=False):
     _need(x, w.dtype, "x", rows * w.K)

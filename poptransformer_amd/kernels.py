@@ -83,6 +83,11 @@ def linear_kernel():
     return _lib.load().pta_linear_kernel().decode()
 
 
+def linear_tiles():
+    """The tiles of this thread's last product by gemm_block_kernel (pta_linear_tiles)."""
+    return _lib.load().pta_linear_tiles().decode()
+
+
 # ------------------------------------------------------------------ INT4 -----------------
 def int4_to_half(packed, scale, axis=1):
     """ops.int4_to_half (reference: poptransformer/ops/customized.py:115-125)."""

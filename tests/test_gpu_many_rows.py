@@ -488,14 +488,16 @@ def test_ends_of_wide_results(M, Kd, N, end):
         assert torch.equal(out[:, N:].double(), before[:, N:])                              # columns past the last channel are left alone
 
 
-# gemm_block_kernel's tiles of 192 rows and of 128 x 128, alone and behind whole rounds of 256 rows: rows one past a tile, channels short of a block and of a tile
-TILES = [("one", 1537, 200, 5000), ("one", 385, 72, 5003), ("one", 1921, 1032, 8195), ("pair", 257, 200, 11000), ("pair", 385, 520, 1500),
-         ("pair", 1537, 1032, 5000), ("pair", 1921, 2056, 6152), ("three", 1153, 200, 2051), ("three", 577, 136, 1030), ("three", 1921, 2056, 4100)]
+# gemm_block_kernel's tiles, alone and behind whole rounds of 256 rows: rows one past a tile, channels short of a block and of a tile
+TILES = [("one", 1537, 200, 5000, "192x256"), ("one", 385, 72, 5003, "128x128"), ("one", 641, 200, 4100, "128x128"), ("pair", 385, 2056, 1500, "128x128"), ("one", 1921, 1032, 8195, "256x256 128x128"), ("one", 1921, 2056, 12300, "256x256 192x256"),
+         ("pair", 257, 200, 11000, "256x256"), ("pair", 385, 520, 1500, "128x128"), ("pair", 385, 72, 8195, "192x256"), ("pair", 129, 72, 8195, "128x256"),
+         ("pair", 1537, 1032, 5000, "256x256 128x128"), ("pair", 1537, 72, 11000, "256x256 128x256"), ("pair", 1921, 2056, 6152, "256x256 192x256"),
+         ("three", 1153, 200, 2051, "192x256"), ("three", 577, 136, 1030, "128x128"), ("three", 961, 72, 11000, "256x256 128x256"), ("three", 1921, 2056, 4100, "256x256 192x256")]
 
 
 @pytest.mark.parametrize("kind", ["f16", "f8", "bf16"])
-@pytest.mark.parametrize("form, M, Kd, N", TILES)
-def test_tiles_of_other_sizes(kind, form, M, Kd, N):
+@pytest.mark.parametrize("form, M, Kd, N, tiles", TILES)
+def test_tiles_of_other_sizes(kind, form, M, Kd, N, tiles):
     from poptransformer_amd import hybrid_kernels as HK
     from poptransformer_amd import kernels as K
     if kind == "bf16" and form == "three":
@@ -512,13 +514,17 @@ def test_tiles_of_other_sizes(kind, form, M, Kd, N):
             HK.linear(x, tws[0], out, M, ld=ld, up=tws[1], pair=H.PAIR_SWIGLU)
         else:
             HK.linear(x, tws[0], out, M, ld=ld)
+        if (M, Kd, N) in ((385, 72, 5003), (385, 520, 1500)):                                              # (few tiles and short K: bf16 has another kernel for them)
+            assert HK.linear_kernel() == "gemm_rows_kernel"
+        else:
+            assert (HK.linear_kernel(), HK.linear_tiles()) == ("gemm_block_kernel", tiles)
         outs = [out[:, :N]]
     else:
         x = (x * 0.02 if kind == "f8" and form == "pair" else x).half()                     # (as in test_pair: the product stays far below 65504)
         tws, plains = zip(*(weight_of(kind, p) for p in parts))
         outs = [torch.full((M, N), float("nan"), dtype=torch.float16, device="cuda") for _ in range(3 if form == "three" else 1)]
         K.linear(x, list(tws), outs * 2 if form == "pair" else outs, swiglu=form == "pair")
-        assert K.linear_kernel() == "gemm_block_kernel"
+        assert (K.linear_kernel(), K.linear_tiles()) == ("gemm_block_kernel", tiles)
     if form != "pair":
         for out, plain in zip(outs, plains):
             close(out, x.double() @ plain.T, x.double().abs() @ plain.abs().T, Kd, 24 if kind == "bf16" else 11)
