@@ -6,7 +6,7 @@ transformer blocks (RMSNorm, INT4 q/k/v/o and SwiGLU projections, rotary embeddi
 attention over the cache, residuals), final norm, fp16 lm_head, greedy selection and the loop
 bookkeeping.  The default run follows the headline configuration: batch 1, a 128-token prompt, then
 256 timed new tokens (contexts 128..383), KV cache length 2048.  The prompt's 128 loop iterations are
-always run untimed first (in passes of up to 1024 rows; ``--prompt-loop``: one iteration per position, as
+always run untimed first (in passes of up to 2048 rows; ``--prompt-loop``: one iteration per position, as
 the reference's loop does), then ``--warmup`` further untimed iterations, then ``--steps`` timed ones: the
 timed iterations generate new tokens whatever the flags are.
 
@@ -298,7 +298,7 @@ def other_model_workload(workload, B, steps, warmup, prompt_loop=False):
         "steps": steps, "warmup": warmup, "ms_per_step": dt / steps * 1e3, "higher_is_better": True,
         "scaling": "weak", "vs_baseline": None, "dtype": dtype, "data": "synthetic",
         "config": {"workload": f"{name}, batch {B}, prompt {prompt} consumed "
-                               f"{'in passes of up to 1024 rows' if done else 'token by token'} (untimed), timed context "
+                               f"{'in passes of up to 2048 rows' if done else 'token by token'} (untimed), timed context "
                                f"{first}..{first + steps - 1}", "batch": B, "executor": "operators"},
         "step_algorithmic_bytes": mean_bytes,
         "step_roofline_frac": mean_bytes / (dt / steps) / (HBM_PEAK_GBS * 1e9),
@@ -642,7 +642,7 @@ def main():
                     help="operators executor: run the norms inside the projections that consume them (default: the decoder's choice)")
     ap.add_argument("--prompt-loop", action="store_true",
                     help="decode workload: consume the (untimed) prompt one loop iteration per position, as the reference's "
-                         "loop does, instead of in passes of up to 1024 rows (FusedDecoder.consume_prompt)")
+                         "loop does, instead of in passes of up to 2048 rows (FusedDecoder.consume_prompt)")
     ap.add_argument("--no-batch16", action="store_true",
                     help="default run only: skip the second, batch-16 measurement that is reported beside the headline")
     ap.add_argument("--no-extras", action="store_true",
@@ -707,7 +707,7 @@ def main():
         return d
 
     def timed_decode(d, batch):
-        """The prompt's 128 loop iterations untimed (contexts 0..127; in passes of up to 1024 rows unless
+        """The prompt's 128 loop iterations untimed (contexts 0..127; in passes of up to 2048 rows unless
         --prompt-loop), then --warmup further iterations, then --steps timed ones: whatever --warmup is, the timed
         iterations start at context 128 + warmup and generate new tokens.  Wall clock around the timed iterations,
         and events around the same launches on the stream they are launched on."""

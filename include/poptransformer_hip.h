@@ -563,7 +563,7 @@ typedef struct pta_gpt2_model {
 } pta_gpt2_model;
 
 /* Bytes of the workspace of pta_gpt2_step; 0 for unsupported shapes (supported: batch up to 8, heads of 64, hidden up to 2048, ffn
- * up to 8192 and a multiple of 8, n_positions >= max_len; with 8 rows less, where LDS does not hold them).  The caller zeroes it once after allocating it (256-byte aligned). */
+ * up to 8192 and a multiple of 8, n_positions >= max_len; batches from 5 on less, where LDS does not hold eight rows of the widest).  The caller zeroes it once after allocating it (256-byte aligned). */
 size_t pta_gpt2_step_workspace_bytes(const pta_gpt2_model* model);
 
 /* Enqueues one loop iteration.  Launches with one workspace must follow each other in stream order.  Every wait is bounded: if one gives up,

@@ -14,16 +14,18 @@
 // stored and read at device scope; one whose upper half is not this iteration's has not arrived.  Nothing is counted, cleared or
 // fenced: a slot's words are written once an iteration, and the last workgroup moves the number on when all others are done.
 //
-// The workgroups are few (24 to 48 a product) and of 16 waves: a compute unit has one at a time, so about six products' workgroups are
+// The workgroups are few (24 to 48 a product at a width of 768; where the registers hold fewer channels of one more of them, at 2048 up to 128; the head 390
+// to 790) and of 16 waves: a compute unit has one at a time, so about six products' workgroups are
 // there at once, each with its weights on their way, and the machine starts some 100 workgroups a microsecond at most (a link of the
 // chain with nothing to multiply: 48 workgroups 1.25 us, 96 1.7, 256 3.2; in one launch that stays 0.93).
 //
-// GPT-2 small, us a token, per operator and here: batch 1, context 16 284 -> 178, 400 322 -> 193, 900 336 -> 221; batch 2 304 -> 204, 4 318 ->
-// 232, 8 368 -> 293 (context 900 480 -> 339); width 256 242 -> 143; 8 layers of width 1280 252 -> 169.  A link takes 2.0 (attention) to 3.0
-// us: 1.0 to 1.6 until the last producer's words have come, 0.4 the norm, 0.4 the products, 0.4 to 0.5 the sums and the end; the head 20.
+// GPT-2 small, us a token, per operator and here: batch 1, context 16 314 -> 184, 400 324 -> 198, 900 340 -> 226; batch 2 336 -> 209, 4 362 ->
+// 239, 8 395 -> 298 (context 900 467 -> 345); width 256 267 -> 150; 8 layers of width 1280 276 -> 173.  A link takes 2.0 (attention) to 3.0
+// us: 1.0 to 1.6 until the last producer's words have come, 0.4 to 0.6 the norm, 0.4 the products, 0.4 to 0.5 the sums and the end; the head 20.
 // Measured and not kept: eight copies of every word, each for an eighth of the readers (no gain: the lines are not what is
 // contended); two workgroups a compute unit by half the registers (176 -> 213: twice the waiting ones); the norm applied to the
-// operands of the matrix instructions (every wave of a unit repeats it: +1.3 us a link).
+// operands of the matrix instructions (every wave of a unit repeats it: +1.3 us a link); v_rsq_f32 for the norms' reciprocal root (184 -> 179, but it
+// rounds some variances to the other fp16 neighbour than 1 / sqrtf, which the operators take).
 #include "common.h"
 #include "formats.h"
 

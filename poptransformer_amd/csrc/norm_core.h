@@ -49,8 +49,8 @@ struct NormArgs {
 // row.request(i, c), row.value(i), row.keep(c, value): a thread's i-th piece, columns 8 c to 8 c + 7 of the workgroup's row.  VECS: pieces of a thread, as few as the row
 // needs.  All requests, the weights' and the cast's exponent's go before the first value is used, and without a branch round them (where paths meet
 // the compiler waits for what is in flight; a thread without a piece reads the row's last one): one round trip to memory before the sums.
-// Few rows are bounded by this chain: 32 rows of 4096 behind a split product 6.1 -> 5.7 us with the branches gone; a token of 28 layers of eight rows of
-// 4096 with the cast to the FP8 grid 0.9 % less, of 32 layers of 32 rows with the shift 1.4 %.
+// Few rows are bounded by this chain: 32 rows of 4096 behind a split product 6.1 -> 5.7 us with the branches gone; a token of 32 layers of 32 rows with the
+// shift 1.4 % less, of 28 layers of eight rows with the cast to the FP8 grid nothing that runs on several machines show (0 to 0.7 %, they differ by up to 2).
 template <int MODE, bool MIX, int VECS, class Row>
 __device__ __forceinline__ void norm_row(const NormArgs& a, const NormMix& mix, size_t r, Row& row) {
   const size_t base = r * a.cols;
