@@ -2844,8 +2844,9 @@ static int launch_gemm_block_listed(const GemmArgs& a, size_t x_rows, int max_ti
 // bytes of LDS a product (a step of 64 features, MFMAs alone 1.2, 0.9, 0.6, 0.3 us), so it wins by its rounds only.
 // us, with two tiles (256 and 128 by 256) and with four, weights from HBM: fp16, 1960 rows, 2048 x 2048 33.4 -> 25.0, 2048 x 4608 50.6 -> 45.0,
 // 5632 x 2048 73.2 -> 58.2; 300 rows, 4096 x 4096 53.1 -> 38.2; 1656 rows, 11008 x 2048 117 -> 90; pair of 5632 x 5632, 791 rows 126 -> 109;
-// bf16 pair of 11008 x 1024, 1100 rows 111 -> 76; F143, 2040 rows, 4096 x 4608 83.6 -> 77.9, 1601 rows, 5632 x 5632 118 -> 104.  Of 215 launches
-// of 140 to 2000 rows that changed their tile, the slowest ratio was 0.98 (bf16, 1837 rows, 3072 x 11008: 136 -> 139), the middle one 1.1.
+// bf16 pair of 11008 x 1024, 1100 rows 115 -> 81; F143, 2040 rows, 4096 x 4608 83.6 -> 77.9, 1601 rows, 5632 x 5632 118 -> 104.  Of 215 launches
+// of 140 to 2000 rows that changed their tile, the slowest ratio was 0.98 (bf16, 1837 rows, 3072 x 11008: 136 -> 139), the middle one 1.1; of 160
+// of 45 to 2000 rows by any channels and features two were below 0.98 (0.95: bf16, 692 rows, 2456 x 2200, scratch for three slices; 0.97: fp16, 229 rows, 5408 x 824).
 // Not kept: 192 rows with K in slices (F143, 1583 rows, 11008 x 2304 94 -> 146), 192 rows for the rest at 4 us (0.97 to 1.04; hence 8), as many
 // tiles of 192 as of 256 rows (three fp16 weights, 372 rows, 4288 x 7744 92 -> 99).
 template <class Fmt, bool PAIR>
