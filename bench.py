@@ -317,7 +317,7 @@ GPT2_SMALL = dict(vocab_size=50257, n_embd=768, n_head=12, n_layer=12, n_positio
 
 def gpt2_small_workload(cpu=True):
     """GPT-2 small fp16 greedy decode, batch 1, prompt 16, 32 new tokens, KV length 128 (the plumbing configuration):
-    the decode loop on the GPU (one launch per operator, HIP graph) and - the configuration's CPU reference path -
+    the decode loop on the GPU (an iteration as one launch, replayed from a HIP graph) and - the configuration's CPU reference path -
     the numpy oracle of the same graph on the host cores, with the generated tokens compared."""
     import torch
     from poptransformer_amd.engine import fused, loader, synthetic
@@ -341,7 +341,7 @@ def gpt2_small_workload(cpu=True):
     wbytes = sum(int(np.prod(v.shape)) * 2 for k, v in sd.items() if "wpe" not in k)
     out = {"value": B * new / dt, "unit": "tokens/s", "ms_per_step": dt / new * 1e3, "steps": new,
            "workload": f"GPT-2 small fp16 greedy decode, batch 1, prompt {prompt} (untimed, token by token), {new} new tokens, "
-                       f"KV cache of {L}", "executor": "operators",
+                       f"KV cache of {L}", "executor": "operators" if dec.chained is None else "one launch",
            "step_algorithmic_bytes": float(wbytes), "step_roofline_frac": wbytes / (dt / new) / (HBM_PEAK_GBS * 1e9)}
     note(f"gpt2 small: {dt / new * 1e3:.3f} ms per token on the GPU")
     if cpu:
