@@ -78,8 +78,7 @@ struct FmtF16 : F16Product {
     return bitcast<f16x8>(raw[j]);
   }
   static __device__ __forceinline__ float finish(float acc, Scale) { return acc; }
-  // of gemm_block_kernel: features of a stage; a lane's bytes of an operand, where those of half m of 64 features lie, and the operand
-  static constexpr int kStage = 32;
+  // of gemm_block_kernel: a lane's bytes of an operand, where those of half m of a stage's 64 features lie, and the operand
   typedef f16x8 Piece;
   static constexpr int piece_at(int m) { return m * 1024; }
   static __device__ __forceinline__ f16x8 operand(Piece p) { return p; }
@@ -157,8 +156,7 @@ struct FmtF8 : F16Product {
 // would be infinite from 2^121 on, and its product with a sum of zero a NaN.
 struct FmtF143Block : FmtF8<0> {
   static __device__ __forceinline__ float finish(float acc, Scale s) { return acc * 128.0f * s.mul; }
-  static constexpr int kStage = 64;                          // (a vector holds 64 features of a channel)
-  typedef u32x2 Piece;
+  typedef u32x2 Piece;                                       // (a vector holds 64 features of a channel)
   static constexpr int piece_at(int m) { return m * 8; }
   static __device__ __forceinline__ uint32_t pair(uint32_t bytes, uint32_t select) {
     typedef short i16x2 __attribute__((ext_vector_type(2)));
@@ -181,7 +179,6 @@ struct FmtBF16 {
   static __device__ __forceinline__ Scale load_scale(const void*, const int32_t*, int, int) { return Scale{}; }
   static __device__ __forceinline__ f16x8 a_operand(const u32x4 (&raw)[4], int j, Scale) { return bitcast<f16x8>(raw[j]); }
   static __device__ __forceinline__ float finish(float acc, Scale) { return acc; }
-  static constexpr int kStage = 32;
   typedef f16x8 Piece;
   static constexpr int piece_at(int m) { return m * 1024; }
   static __device__ __forceinline__ f16x8 operand(Piece p) { return p; }

@@ -2565,23 +2565,27 @@ __global__ __launch_bounds__(PANEL_WAVES * 64) __attribute__((amdgpu_waves_per_e
 // ------------------------------------------------------------------------------------------
 // Variant for hundreds of rows of formats with more than one vector per tile (16-bit and FP8 weights): both operands
 // through LDS.  A workgroup of 8 waves owns 256, 192 or 128 rows and 256 channels (a pair: 128 gate and 128 up channels), or 128 rows and
-// 128 channels; loads that write LDS directly bring stages of Fmt::kStage features of both.
+// 128 channels; loads that write LDS directly bring stages of 64 features of both.
 // At 256 x 256 a 64-feature step is 64 KiB for 8.4 MFLOP, a quarter of the bytes per product that gemm_rows_kernel's
 // workgroups (256 x 128, weights through registers) take.
-// What bounds it: the matrix unit at the clock that the power leaves (1.7 GHz in long launches), and the loads.  A step of 64
-// features takes 1.1 us without them on zeros, 1.27 on random numbers, 1.5 from the caches and 1.6 to 1.75 with weights
-// from HBM (1.2 PFLOP/s; 128 rows: 0.85 to 0.95).  FP8: two stages of 64 features 1.75, three 1.6; 16-bit: two of 64 or five of 32 alike.
-// One load per block of MFMAs: a compute unit holds a wave that asks for more at once.
+// What bounds it: the loads.  A compute unit has about 32 KiB of them on their way, 128 bytes a line, so what counts is lines and how long each takes:
+// 110 GB/s from L2, 37 weights from memory, 54 to 60 both as they come - 1.2, 0.77 and 0.53 us for a step's 64 KiB (256 x 256), 48 (128 x 256) and 32 (128 x 128),
+// against 1.1, 0.64 and 0.35 of the products alone at the clock that the power leaves.  Hence stages of 64 features, whole lines of the rows (with 32,
+// half lines: as many requests for half the bytes), tiles of a die that share rows and weights both (BLOCK_BAND), and requests all the time (APART; one load
+// per block of MFMAs: a wave that asks for more at once is held).  bf16, weights from memory, with stages of 32 and now: 2048 rows, 8192 x 8192 203 -> 193 us (256 x
+// 256), 1920 rows, 8192 x 6144 175 -> 148 (192 x 256), 2048 rows, 11008 x 4096 183 -> 150 (128 x 256), 5632 x 2048 63 -> 51 (128 x 128).
+// Not kept: the order of a stage's loads turned by the workgroup, so that each line is asked for early by another one (the scalar arithmetic between the products
+// costs 5 %); wave priorities round the products or for half of the waves (0 to 3 % slower); the next operand converted among this one's products (2 to 6 % slower).
 // Channels need not divide: blocks past a matrix's last one lie past its descriptor and read as zeros.
 // ------------------------------------------------------------------------------------------
 constexpr int BLOCK_WAVES = 8;
+constexpr int BLOCK_BAND = 4;               // channel groups that a die's workgroups share the rows of (one: 2 to 5 % slower at 128 rows a tile and 2048 rows)
 // The tile of a wave's RG row groups x 4 channel blocks: 2 x 4 waves of 8, 6 or 4 groups (256, 192 or 128 rows by 256 channels), or 4 x 2 of 2 (128 x 128)
 constexpr int block_row_parts(int rg) { return rg == 2 ? 4 : 2; }
 constexpr int block_rows(int rg) { return block_row_parts(rg) * rg * 16; }
 constexpr int block_cb(int rg) { return 8 / block_row_parts(rg) * 4; }         // channel blocks of a workgroup
-// us of a step of 64 features (measured, all compute units at work; the smaller tiles of weights that are decoded read their operands more often),
-// and of a tile's begin and end
-constexpr double block_step_us(int rg, bool decoded) { return rg == 8 ? 1.6 : rg == 6 ? (decoded ? 1.3 : 1.25) : rg == 4 ? 0.92 : decoded ? 0.74 : 0.6; }
+// us of a step of 64 features (measured, all compute units at work), and of a tile's begin and end
+constexpr double block_step_us(int rg) { return rg == 8 ? 1.45 : rg == 6 ? 1.1 : rg == 4 ? 0.84 : 0.55; }
 constexpr double block_ends_us(int rg) { return rg == 8 ? 9.0 : rg == 6 ? 7.5 : rg == 4 ? 6.0 : 5.0; }
 
 // v, of which the compiler no longer knows where it is from
@@ -2595,39 +2599,53 @@ __device__ __forceinline__ u32x4 as_computed(u32x4 v) {
   return v;
 }
 
-// row loads (of 1 KiB) per wave and stage
+// Bytes of a stage (64 features) of the rows and of the weights, and how many stages of each LDS holds
+constexpr int block_x_bytes(int rg) { return block_rows(rg) * 128; }
 template <class Fmt>
-constexpr int block_row_loads(int rg) { return (block_rows(rg) * Fmt::kStage * 2 + BLOCK_WAVES * 1024 - 1) / (BLOCK_WAVES * 1024); }
+constexpr int block_w_bytes(int rg) { return block_cb(rg) * Fmt::kVec * 512; }
+// whether the weights are asked for in a step's first half (to the place that the stage before has left) and only the rows in its second
 template <class Fmt>
-constexpr int block_stage_bytes(int rg) { return block_row_loads<Fmt>(rg) * BLOCK_WAVES * 1024 + block_cb(rg) * Fmt::kVec * 8 * Fmt::kStage; }
+constexpr bool block_apart(int rg) { return Fmt::kVec == 4 || rg != 8; }
 template <class Fmt>
-constexpr int block_stages(int rg) {
-  const int most = rg == 2 ? 8 : 5, fit = 160 * 1024 / block_stage_bytes<Fmt>(rg);      // (a small tile's stages go by in half the time)
-  return fit < most ? fit : most;
+constexpr int block_x_stages(int rg) {
+  const int both = 160 * 1024 / (block_x_bytes(rg) + block_w_bytes<Fmt>(rg));
+  return both < 5 ? both : 5;
+}
+template <class Fmt>
+constexpr int block_w_stages(int rg) {            // one more where it fits
+  const int x = block_x_stages<Fmt>(rg);
+  return block_apart<Fmt>(rg) && x < 5 && x * block_x_bytes(rg) + (x + 1) * block_w_bytes<Fmt>(rg) <= 160 * 1024 ? x + 1 : x;
+}
+template <class Fmt>
+constexpr int block_lds_bytes(int rg) { return block_x_stages<Fmt>(rg) * block_x_bytes(rg) + block_w_stages<Fmt>(rg) * block_w_bytes<Fmt>(rg); }
+
+// waits until at most N of this wave's loads from memory are on their way, and (LDS) for all of its LDS requests
+template <int N, bool LDS = false>
+__device__ __forceinline__ void wait_loads() {
+  static_assert(N < 64, "the counter of requests");
+  __builtin_amdgcn_s_waitcnt((LDS ? 0x0070 : 0x0f70) | (N & 15) | (N >> 4) << 14);
 }
 
 template <class Fmt, int RG, bool PAIR, class Rows = AllRows>
 __global__ __launch_bounds__(BLOCK_WAVES * 64) __attribute__((amdgpu_waves_per_eu(2, 2))) void gemm_block_kernel(GemmArgs a, int group0, int groups, int row_blocks, Rows rows) {
   constexpr int KV = Fmt::kVec, NST = 4;
-  constexpr int SF = Fmt::kStage;                 // features of a stage: 32 or 64
-  constexpr int WVEC = KV * 8 * SF;               // bytes of a channel block's features of a stage
+  constexpr int WVEC = KV * 512;                  // bytes of a channel block's features of a stage
   constexpr int ROWS = block_rows(RG), WR = block_row_parts(RG), WC = BLOCK_WAVES / WR;
   constexpr int CB = block_cb(RG), BPW = CB / BLOCK_WAVES;      // channel blocks of the workgroup, and how many a wave brings
-  constexpr int XL = block_row_loads<Fmt>(RG);    // row loads per wave and stage
-  constexpr int XB = XL * BLOCK_WAVES * 1024;     // bytes of a stage's rows (rounded up to whole loads)
-  constexpr int STAGE = XB + CB * WVEC;
-  constexpr int NS = block_stages<Fmt>(RG);
-  constexpr int PPR = SF / 8;                     // 16-byte pieces of a row
-  constexpr int RPL = 64 / PPR;                   // rows of a load
-  constexpr int WL = WVEC / 1024;                 // loads per channel block
-  constexpr int LOADS = XL + BPW * WL;
-  constexpr int WAIT = (NS - 2) * LOADS;          // loads that may be on their way when a stage must have landed
-  static_assert((SF == 32 || SF == 64) && WVEC % 1024 == 0 && NS >= 2 && WAIT < 16 && STAGE == block_stage_bytes<Fmt>(RG), "stages");
+  constexpr int XB = block_x_bytes(RG), WB = block_w_bytes<Fmt>(RG), NX = block_x_stages<Fmt>(RG), NW = block_w_stages<Fmt>(RG);
+  constexpr int XL = XB / (BLOCK_WAVES * 1024);   // loads per wave and stage: rows (eight of them each)
+  constexpr int WPB = WVEC / 1024, WL = BPW * WPB;              // and weights, of a channel block and in all
+  constexpr bool APART = block_apart<Fmt>(RG);
+  // loads that may be on their way when the next stage must have landed: those asked for behind its weights, and behind its rows
+  constexpr int BEHIND_W = (NW - 2) * (XL + WL), BEHIND_X = APART ? (NX - 2) * XL + (NX - 1) * WL : BEHIND_W;
+  constexpr int WAIT = BEHIND_W < BEHIND_X ? BEHIND_W : BEHIND_X;
+  constexpr int W_BEGIN = APART ? NW - 1 : NW;    // stages of weights that are asked for at the begin
+  static_assert(XB % (BLOCK_WAVES * 1024) == 0 && WVEC % 1024 == 0 && NX >= 2 && (APART ? NW >= 3 : NW == NX) && block_lds_bytes<Fmt>(RG) <= 160 * 1024, "stages");
   extern __shared__ __align__(16) unsigned char smem[];
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int wr = wave / WC, wc = wave % WC;
   const int K = a.K;
-  // workgroup id -> tile as in gemm_panel_kernel: contiguous stretches of the tile list per die, the row block fastest
+  // workgroup id -> tile: contiguous stretches of the tile list per die, in bands of BLOCK_BAND channel groups, within a band the group fastest
   int per = (int)gridDim.x / 8;
   if constexpr (Rows::kListed) {                  // (the launch has room for the most tiles there can be)
     row_blocks = *rows.n_tiles;
@@ -2636,8 +2654,10 @@ __global__ __launch_bounds__(BLOCK_WAVES * 64) __attribute__((amdgpu_waves_per_e
   }
   const int tile = ((int)blockIdx.x % 8) * per + (int)blockIdx.x / 8;
   if (tile >= groups * row_blocks) return;
-  const int row_block = tile % row_blocks;
-  int group = group0 + tile / row_blocks;
+  const int band = tile / (BLOCK_BAND * row_blocks), in_band = tile - band * (BLOCK_BAND * row_blocks);
+  const int band_groups = groups - band * BLOCK_BAND < BLOCK_BAND ? groups - band * BLOCK_BAND : BLOCK_BAND;
+  const int row_block = in_band / band_groups;
+  int group = group0 + band * BLOCK_BAND + in_band - row_block * band_groups;
   int M = a.M;
   const int32_t* order = nullptr;
   size_t weight_at = 0;
@@ -2662,8 +2682,6 @@ __global__ __launch_bounds__(BLOCK_WAVES * 64) __attribute__((amdgpu_waves_per_e
   const int all = (K + 63) / 64, per_slice = ((a.KT + nsl - 1) / nsl) * 2;
   const int first = (int)blockIdx.y * per_slice;
   const int last = first + per_slice < all ? first + per_slice : all;
-  const int steps = last > first ? last - first : 0;
-
   // this wave brings blocks BPW * wave and on of the workgroup's (of a pair: first the gate's, then the up blocks)
   const GemmMat& wm = a.mat[PAIR ? wave >> 2 : mi];
   const int wb = blk0 + BPW * (PAIR ? wave & 3 : wave);
@@ -2677,64 +2695,60 @@ __global__ __launch_bounds__(BLOCK_WAVES * 64) __attribute__((amdgpu_waves_per_e
   const __amdgpu_buffer_rsrc_t xres = __builtin_amdgcn_make_buffer_rsrc(
       const_cast<f16*>(X + (size_t)row0 * K), 0, Rows::kListed ? 0x7fffffff : (int)((size_t)rows_here * K * 2), 0x00020000);
 
-  // A row's 16-byte pieces are exchanged: piece c of row r at c ^ swap(r), so that the sixteen rows of an operand read
-  // cover 256 bytes of banks once, and every eight of them 128.
-  auto swap = [](int r) { return SF == 64 ? ((r >> 1) & 7) ^ ((r & 1) << 2) : ((r >> 2) & 3) ^ (r & 2); };
-  const int lane_row = lane / PPR;
-  const int piece = (lane % PPR) ^ swap(RPL == 8 ? (wave & 1) * 8 + lane_row : lane_row);      // (the same in all loads of a lane)
-  const int x0 = (wave * RPL + lane_row) * (K * 2) + piece * 16;  // byte offset of its first row (past the last row: past the descriptor)
+  // A row's 128 bytes of a stage are eight pieces of 16, exchanged: piece c of row r at c ^ swap(r), so that no sixteen lanes of an operand read that
+  // the LDS serves at once (0-3, 12-15, 20-23, 24-27, ...) meet in a bank.
+  auto swap = [](int r) { return ((r >> 1) & 7) ^ ((r & 1) << 2); };
+  const int lane_row = lane >> 3;
+  const int piece = (lane & 7) ^ swap((wave & 1) * 8 + lane_row);               // (the same in all loads of a lane)
+  const int x0 = (wave * 8 + lane_row) * (K * 2) + piece * 16;    // byte offset of its first row (past the last row: past the descriptor)
   int listed[XL];
   if constexpr (Rows::kListed) {
 #pragma unroll
     for (int j = 0; j < XL; ++j) {
-      const int r = (j * BLOCK_WAVES + wave) * RPL + lane_row;
+      const int r = (j * BLOCK_WAVES + wave) * 8 + lane_row;
       listed[j] = r < M ? order[r] / rows.x_div * (K * 2) + piece * 16 : -1;
     }
   }
   // load q of stage s (of the K axis) into LDS at byte `at`; past the slice's end: zeros, from nowhere
-  const int end = last * (64 / SF);
-  auto bring = [&](int s, int at, int q) {
-    const bool in = s < end;
-    if (q < XL) {
-      int off = Rows::kListed ? listed[q] : x0 + q * (BLOCK_WAVES * RPL * 2) * K;
-      if (XL * BLOCK_WAVES * RPL > ROWS && (q * BLOCK_WAVES + wave) * RPL >= ROWS) off = -1;      // (rows that the tile does not have)
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(xres, (__attribute__((address_space(3))) void*)(smem + at + (q * BLOCK_WAVES + wave) * 1024), 16,
-                                               in && s * SF + piece * 8 < K ? off : -1, s * (SF * 2), 0, 0);
-    } else {
-      const int b = (q - XL) / WL, v = (q - XL) % WL;
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(wres, (__attribute__((address_space(3))) void*)(smem + at + XB + (BPW * wave + b) * WVEC + v * 1024), 16,
-                                               in ? (int)(b * blk_bytes) + lane * 16 : -1, s * WVEC + v * 1024, 0, 0);
-    }
+  auto bring_x = [&](int s, int at, int q) {
+    const int off = Rows::kListed ? listed[q] : x0 + q * (BLOCK_WAVES * 16) * K;
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(xres, (__attribute__((address_space(3))) void*)(smem + at + (q * BLOCK_WAVES + wave) * 1024), 16,
+                                             s < last && s * 64 + piece * 8 < K ? off : -1, s * 128, 0, 0);
+  };
+  auto bring_w = [&](int s, int at, int q) {
+    const int b = q / WPB, v = q % WPB;
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(wres, (__attribute__((address_space(3))) void*)(smem + at + (BPW * wave + b) * WVEC + v * 1024), 16,
+                                             s < last ? (int)(b * blk_bytes) + lane * 16 : -1, s * WVEC + v * 1024, 0, 0);
   };
 
   f32x4 acc[RG][NST];
-#pragma unroll
-  for (int rg = 0; rg < RG; ++rg)
-#pragma unroll
-    for (int st = 0; st < NST; ++st) acc[rg][st] = f32x4{0.f, 0.f, 0.f, 0.f};
 
-  // operands of 32 features: half m of the stage at byte `at` (stages of 32 features are their half)
+  // operands of 32 features: half m of the stage at byte `at`
   typedef typename Fmt::Piece Piece;              // a lane's bytes of a weight operand
-  const int a_at = XB + (PAIR ? wc * 2 : wc * 4) * WVEC + lane * 16;
+  const int a_at = (PAIR ? wc * 2 : wc * 4) * WVEC + lane * 16;
   auto a_piece = [&](int at, int m, int st) {
     const int blk = PAIR ? st % 2 + (st / 2) * (CB / 2) : st;
-    return *reinterpret_cast<const Piece*>(smem + at + a_at + blk * WVEC + (SF == 64 ? Fmt::piece_at(m) : 0));
+    return *reinterpret_cast<const Piece*>(smem + at + a_at + blk * WVEC + Fmt::piece_at(m));
   };
-  const int b_row = (wr * (RG * 16) + (lane & 15)) * (SF * 2);
-  const int b0 = b_row + ((lane >> 4) ^ swap(lane & 15)) * 16, b1 = SF == 64 ? b_row + ((4 + (lane >> 4)) ^ swap(lane & 15)) * 16 : b0;
-  auto b_operand = [&](int at, int m, int rg) { return *reinterpret_cast<const f16x8*>(smem + at + (m ? b1 : b0) + rg * (SF * 32)); };
+  const int b_row = (wr * (RG * 16) + (lane & 15)) * 128;
+  const int b0 = b_row + ((lane >> 4) ^ swap(lane & 15)) * 16, b1 = b_row + ((4 + (lane >> 4)) ^ swap(lane & 15)) * 16;
+  auto b_operand = [&](int at, int m, int rg) { return *reinterpret_cast<const f16x8*>(smem + at + (m ? b1 : b0) + rg * 2048); };
 
   // One pipeline over all steps: a step is two halves of 32 features, a half four blocks of RG MFMAs with one weight operand
-  // each.  The row operands of the next half are requested while this one's are multiplied (two sets of registers), the
+  // each.  The row operands of the next half are requested in this one's first two blocks (two sets of registers; over all four 1 % slower), the
   // weight operand four blocks ahead.  The barrier stands where everything of a stage has been requested: behind it
-  // the stage takes what is NS stages on.  (The last half requests operands of one that does not exist and
-  // drops them: a condition here would stand between the MFMAs.)
-  f16x8 xf[2][RG];
-  Piece ahead[NST];
+  // the stage takes what is some stages on, its weights (APART) half a step later, so that requests go out all the time.  (The last
+  // half requests operands of a stage that does not exist and drops them: a condition here would stand between the MFMAs.)
+  constexpr int W0 = NX * XB;                     // where the weights' stages begin
 #pragma unroll
-  for (int n = 0; n < NS; ++n)
+  for (int n = 0; n < NX || n < W_BEGIN; ++n) {
 #pragma unroll
-    for (int q = 0; q < LOADS; ++q) bring(first * (64 / SF) + n, n * STAGE, q);
+    for (int q = 0; q < XL; ++q)
+      if (n < NX) bring_x(first + n, n * XB, q);
+#pragma unroll
+    for (int q = 0; q < WL; ++q)
+      if (n < W_BEGIN) bring_w(first + n, W0 + n * WB, q);
+  }
   // (the wide epilogue's many arguments, read while the first stages are on their way: bf16, 1024 x 8192, 1000 rows 29.5 -> 28.1 us; 2048 x 8192 46.9 -> 45.4; the
   // fp16 one's few gain nothing)
   GemmMat wide;
@@ -2743,43 +2757,52 @@ __global__ __launch_bounds__(BLOCK_WAVES * 64) __attribute__((amdgpu_waves_per_e
     wide = a.mat[PAIR ? 0 : mi];
     read_end<Fmt, PAIR>(wide, none);
   }
-  __builtin_amdgcn_s_waitcnt(0x0f70);             // vmcnt(0)
+  wait_loads<(NX - 1) * XL + (W_BEGIN - 1) * WL>();             // the first stage has landed
   __syncthreads();
+  f16x8 xf[2][RG];
+  Piece ahead[NST];
+#pragma unroll
+  for (int rg = 0; rg < RG; ++rg)
+#pragma unroll
+    for (int st = 0; st < NST; ++st) acc[rg][st] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
   for (int rg = 0; rg < RG; ++rg) xf[0][rg] = b_operand(0, 0, rg);
 #pragma unroll
-  for (int st = 0; st < NST; ++st) ahead[st] = a_piece(0, 0, st);
+  for (int st = 0; st < NST; ++st) ahead[st] = a_piece(W0, 0, st);
   // (the compiler would otherwise make one load of these and of the same ones at the end of a step, at the step's begin)
 #pragma unroll
   for (int rg = 0; rg < RG; ++rg) xf[0][rg] = bitcast<f16x8>(as_computed(bitcast<u32x4>(xf[0][rg])));
-  int at = 0, stage = first * (64 / SF) + NS;     // the stage whose operands are multiplied; the one to be asked for next
-  for (int i = 0; i < steps; ++i) {
+  __builtin_amdgcn_s_waitcnt(0xc07f);             // lgkmcnt(0): where the loop begins, nothing is on its way that its end does not know of
+  int xat = 0, wat = W0, wfree = W0 + (NW - 1) * WB;            // the stage whose operands are multiplied; the place of the weights before it
+  for (int i = first; i < last; ++i) {
+    const int xnext = xat + XB == W0 ? 0 : xat + XB, wnext = wat + WB == W0 + NW * WB ? W0 : wat + WB;
 #pragma unroll
     for (int m = 0; m < 2; ++m) {
-      const bool turn = SF == 32 || m == 1;       // this half's stage has been requested as a whole
-      const int nx = turn ? (at + STAGE == NS * STAGE ? 0 : at + STAGE) : at;
-      if (turn) {
-        __builtin_amdgcn_s_waitcnt(0x0070 | WAIT);      // the next stage has landed, and this wave's requests from this one
+      if (m == 1) {
+        wait_loads<WAIT, true>();                 // the next stage has landed, and this wave's requests from this one
         __builtin_amdgcn_s_barrier();
         __builtin_amdgcn_sched_barrier(0);
       }
 #pragma unroll
       for (int st = 0; st < NST; ++st) {
-        if (turn) {
+        const int from = APART && m == 0 ? XL : 0, n = APART ? (m == 0 ? WL : XL) : m == 0 ? 0 : XL + WL;      // requests of this half: rows, then weights
 #pragma unroll
-          for (int q = st * LOADS / NST; q < (st + 1) * LOADS / NST; ++q) bring(stage, at, q);
+        for (int q = from + st * n / NST; q < from + (st + 1) * n / NST; ++q) {
+          if (q < XL) bring_x(i + NX, xat, q);
+          else bring_w(i + (APART ? NW - 1 : NW), APART ? wfree : wat, q - XL);
         }
         const f16x8 av = Fmt::operand(ahead[st]);
-        ahead[st] = a_piece(nx, 1 - m, st);
+        ahead[st] = a_piece(m ? wnext : wat, 1 - m, st);
 #pragma unroll
-        for (int r = st * RG / NST; r < (st + 1) * RG / NST; ++r) xf[1 - m][r] = b_operand(nx, 1 - m, r);
+        for (int r = st * RG / 2; r < (st + 1) * RG / 2 && r < RG; ++r) xf[1 - m][r] = b_operand(m ? xnext : xat, 1 - m, r);
 #pragma unroll
         for (int rg = 0; rg < RG; ++rg) acc[rg][st] = Fmt::mma(av, xf[m][rg], acc[rg][st]);
         __builtin_amdgcn_sched_barrier(0);        // (the requests stay where they are)
       }
-      if (turn) ++stage;
-      at = nx;
     }
+    xat = xnext;
+    wfree = wat;
+    wat = wnext;
   }
   __builtin_amdgcn_s_waitcnt(0x0070);
   __syncthreads();                                // (what follows reuses the stages)
@@ -2791,7 +2814,7 @@ __global__ __launch_bounds__(BLOCK_WAVES * 64) __attribute__((amdgpu_waves_per_e
 template <class Fmt, int RG, bool PAIR, class Rows>
 static int reserve_gemm_block(const char* name) {
   static bool ready = false;
-  constexpr int smem = block_stages<Fmt>(RG) * block_stage_bytes<Fmt>(RG);
+  constexpr int smem = block_lds_bytes<Fmt>(RG);
   static_assert(smem <= 160 * 1024 && smem >= BLOCK_WAVES * 16 * 68 * 4, "LDS");
   if (!ready) {
     PTA_REQUIRE(hipFuncSetAttribute((const void*)gemm_block_kernel<Fmt, RG, PAIR, Rows>, hipFuncAttributeMaxDynamicSharedMemorySize, smem) == hipSuccess,
@@ -2817,7 +2840,7 @@ static int launch_gemm_block(const GemmArgs& a, int group0, int group1, hipStrea
   const int nsl = a.ksplit > 1 ? a.ksplit : 1;
   const int per = (groups * row_blocks + 7) / 8;
   gemm_kernel_taken = "gemm_block_kernel";
-  hipLaunchKernelGGL((gemm_block_kernel<Fmt, RG, PAIR>), dim3(per * 8, nsl), dim3(BLOCK_WAVES * 64), block_stages<Fmt>(RG) * block_stage_bytes<Fmt>(RG), s, a,
+  hipLaunchKernelGGL((gemm_block_kernel<Fmt, RG, PAIR>), dim3(per * 8, nsl), dim3(BLOCK_WAVES * 64), block_lds_bytes<Fmt>(RG), s, a,
                      group0, groups, row_blocks, AllRows{});
   if (nsl > 1) launch_splitk_finish<Fmt>(a, s);
   return PTA_OK;
@@ -2833,7 +2856,7 @@ static int launch_gemm_block_listed(const GemmArgs& a, size_t x_rows, int max_ti
   const int groups = block_groups(a, PAIR);
   gemm_kernel_taken = "gemm_block_kernel";
   hipLaunchKernelGGL((gemm_block_kernel<Fmt, RG, PAIR, ListedRows>), dim3((groups * max_tiles + 7) / 8 * 8), dim3(BLOCK_WAVES * 64),
-                     block_stages<Fmt>(RG) * block_stage_bytes<Fmt>(RG), s, a, 0, groups, max_tiles, rows);
+                     block_lds_bytes<Fmt>(RG), s, a, 0, groups, max_tiles, rows);
   return PTA_OK;
 }
 
@@ -2856,7 +2879,7 @@ static int dispatch_gemm_block(const GemmArgs& a, hipStream_t s, const char* nam
   auto blocks = [&](int rg) { return (a.M + block_rows(rg) - 1) / block_rows(rg); };
   auto cost = [&](int rg, int tiles, int nsl) {
     const double finish = nsl > 1 ? 5.0 + (double)a.M * a.mat[0].N * (4.0 * nsl + 6.0) / 4.5e6 : 0.0;
-    return ((tiles * nsl + cus - 1) / cus) * (block_step_us(rg, Fmt::kVec == 2) * steps / nsl + block_ends_us(rg)) + finish;
+    return ((tiles * nsl + cus - 1) / cus) * (block_step_us(rg) * steps / nsl + block_ends_us(rg)) + finish;
   };
   const int whole = (groups * blocks(8) / cus) * cus / blocks(8);               // channel groups within whole rounds
   double best = cost(8, groups * blocks(8), 1);
