@@ -81,6 +81,8 @@ struct FmtF16 : F16Product {
   // of gemm_block_kernel: a lane's bytes of an operand, where those of half m of a stage's 64 features lie, and the operand
   typedef f16x8 Piece;
   static constexpr int piece_at(int m) { return m * 1024; }
+  static constexpr bool kCodes = false;
+  template <bool>
   static __device__ __forceinline__ f16x8 operand(Piece p) { return p; }
 };
 
@@ -150,12 +152,20 @@ struct FmtF8 : F16Product {
   static __device__ __forceinline__ float finish(float acc, Scale s) { return acc * s.mul; }
 };
 
-// F143 weights for gemm_block_kernel.  Moved to fp16 bits 13..7 with their sign in bit 15 the seven magnitude bits are the
-// fp16 number decode(byte) * 2^-7, subnormals among them, which the matrix unit takes at their value: three instructions for two
-// weights where f143_pair, whose result is the number itself, has five.  The sum takes the 2^7 before the scale: one exponent for both
-// would be infinite from 2^121 on, and its product with a sum of zero a NaN.
+// flag bytes of a tiled FP8 weight: one per tile, nonzero when the tile holds 0x7F, 0xFF or 0x80
+__host__ __device__ inline size_t f8_tile_flags_offset(int N, int K) {
+  return (size_t)((N + 15) / 16) * (size_t)((K + 127) / 128) * 2048;
+}
+
+// F143 weights for gemm_block_kernel.  The hardware's conversion knows the bytes as OCP e4m3 numbers, twice the F143 ones of all codes but 0x7F and 0xFF (and 0x80,
+// which both take as a zero here): one instruction for two weights.  What bounds a launch is the vector unit beside the matrix unit, which multiplies
+// two waves' operands a SIMD: with three instructions for two weights, as for blocks of channels with one of those codes, 2048 rows, 8192 x 8192
+// 197 -> 182 us, 13696 x 4096 199 -> 170.
+// Those three: moved to fp16 bits 13..7 with their sign in bit 15 the seven magnitude bits are the
+// fp16 number decode(byte) * 2^-7, subnormals among them, which the matrix unit takes at their value; the sums take the 2^7 at the end.
 struct FmtF143Block : FmtF8<0> {
-  static __device__ __forceinline__ float finish(float acc, Scale s) { return acc * 128.0f * s.mul; }
+  static constexpr bool kCodes = true;
+  static constexpr float kSlowSum = 128.0f;
   typedef u32x2 Piece;                                       // (a vector holds 64 features of a channel)
   static constexpr int piece_at(int m) { return m * 8; }
   static __device__ __forceinline__ uint32_t pair(uint32_t bytes, uint32_t select) {
@@ -163,9 +173,35 @@ struct FmtF143Block : FmtF8<0> {
     const i16x2 t = bitcast<i16x2>(__builtin_amdgcn_perm(0, bytes, select)) >> (short)1;      // sign in bits 15 and 14
     return bitcast<uint32_t>(t) & 0xBF80BF80u;
   }
+  template <bool FAST>
   static __device__ __forceinline__ f16x8 operand(Piece p) {
+    if constexpr (FAST) {
+      typedef f16x2 Four[4];
+      const Four r = {__builtin_amdgcn_cvt_scalef32_pk_f16_fp8(p[0], 0.5f, false), __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(p[0], 0.5f, true),
+                      __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(p[1], 0.5f, false), __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(p[1], 0.5f, true)};
+      return f16x8{r[0][0], r[0][1], r[1][0], r[1][1], r[2][0], r[2][1], r[3][0], r[3][1]};
+    }
     const u32x4 r = {pair(p[0], 0x010C000Cu), pair(p[0], 0x030C020Cu), pair(p[1], 0x010C000Cu), pair(p[1], 0x030C020Cu)};
     return bitcast<f16x8>(r);
+  }
+  // Not zero in some lane: a tile of blocks [blk, blk + count) of the matrix holds one of the codes (or one of a neighbour that shares a word of flags with
+  // them).  The flags end with a whole 16 bytes.
+  static __device__ __forceinline__ uint32_t codes(const GemmMat& m, int blk, int count, int K, int KT, int lane) {
+    const int there = (m.N + 15) / 16 - blk;
+    count = there < count ? there : count;
+    if (count <= 0) return 0;
+    const size_t at = f8_tile_flags_offset(m.N, K) + (size_t)blk * KT;
+    const uint32_t* words = reinterpret_cast<const uint32_t*>(reinterpret_cast<const unsigned char*>(m.tiled) + (at & ~(size_t)3));
+    const int n = ((int)(at & 3) + count * KT + 3) / 4;
+    uint32_t any = 0;
+    for (int i = lane; i < n; i += 256) {                    // (four words a lane at a time: 1024 tiles)
+      uint32_t w[4];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) w[j] = words[i + j * 64 < n ? i + j * 64 : i];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) any |= w[j];
+    }
+    return any;
   }
 };
 
@@ -181,6 +217,8 @@ struct FmtBF16 {
   static __device__ __forceinline__ float finish(float acc, Scale) { return acc; }
   typedef f16x8 Piece;
   static constexpr int piece_at(int m) { return m * 1024; }
+  static constexpr bool kCodes = false;
+  template <bool>
   static __device__ __forceinline__ f16x8 operand(Piece p) { return p; }
   static __device__ __forceinline__ f32x4 mma(f16x8 a, f16x8 b, f32x4 c) {
     return __builtin_amdgcn_mfma_f32_16x16x32_bf16(bitcast<bf16x8>(a), bitcast<bf16x8>(b), c, 0, 0, 0);

@@ -2749,6 +2749,11 @@ __global__ __launch_bounds__(BLOCK_WAVES * 64) __attribute__((amdgpu_waves_per_e
     for (int q = 0; q < WL; ++q)
       if (n < W_BEGIN) bring_w(first + n, W0 + n * WB, q);
   }
+  uint32_t codes = 0;                             // (a lane's share) whether this wave's weights hold codes that the fast conversion does not know
+  if constexpr (Fmt::kCodes) {
+    if constexpr (PAIR) codes = Fmt::codes(a.mat[0], blk0 + wc * 2, 2, K, a.KT, lane) | Fmt::codes(a.mat[1], blk0 + wc * 2, 2, K, a.KT, lane);
+    else codes = Fmt::codes(a.mat[mi], blk0 + wc * 4, 4, K, a.KT, lane);
+  }
   // (the wide epilogue's many arguments, read while the first stages are on their way: bf16, 1024 x 8192, 1000 rows 29.5 -> 28.1 us; 2048 x 8192 46.9 -> 45.4; the
   // fp16 one's few gain nothing)
   GemmMat wide;
@@ -2759,50 +2764,68 @@ __global__ __launch_bounds__(BLOCK_WAVES * 64) __attribute__((amdgpu_waves_per_e
   }
   wait_loads<(NX - 1) * XL + (W_BEGIN - 1) * WL>();             // the first stage has landed
   __syncthreads();
-  f16x8 xf[2][RG];
-  Piece ahead[NST];
+  auto products = [&](auto fast) {
+    constexpr bool FAST = decltype(fast)::value;
+    f16x8 xf[2][RG];
+    Piece ahead[NST];
 #pragma unroll
-  for (int rg = 0; rg < RG; ++rg)
+    for (int rg = 0; rg < RG; ++rg)
 #pragma unroll
-    for (int st = 0; st < NST; ++st) acc[rg][st] = f32x4{0.f, 0.f, 0.f, 0.f};
+      for (int st = 0; st < NST; ++st) acc[rg][st] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-  for (int rg = 0; rg < RG; ++rg) xf[0][rg] = b_operand(0, 0, rg);
+    for (int rg = 0; rg < RG; ++rg) xf[0][rg] = b_operand(0, 0, rg);
 #pragma unroll
-  for (int st = 0; st < NST; ++st) ahead[st] = a_piece(W0, 0, st);
-  // (the compiler would otherwise make one load of these and of the same ones at the end of a step, at the step's begin)
+    for (int st = 0; st < NST; ++st) ahead[st] = a_piece(W0, 0, st);
+    // (the compiler would otherwise make one load of these and of the same ones at the end of a step, at the step's begin)
 #pragma unroll
-  for (int rg = 0; rg < RG; ++rg) xf[0][rg] = bitcast<f16x8>(as_computed(bitcast<u32x4>(xf[0][rg])));
-  __builtin_amdgcn_s_waitcnt(0xc07f);             // lgkmcnt(0): where the loop begins, nothing is on its way that its end does not know of
-  int xat = 0, wat = W0, wfree = W0 + (NW - 1) * WB;            // the stage whose operands are multiplied; the place of the weights before it
-  for (int i = first; i < last; ++i) {
-    const int xnext = xat + XB == W0 ? 0 : xat + XB, wnext = wat + WB == W0 + NW * WB ? W0 : wat + WB;
+    for (int rg = 0; rg < RG; ++rg) xf[0][rg] = bitcast<f16x8>(as_computed(bitcast<u32x4>(xf[0][rg])));
+    __builtin_amdgcn_s_waitcnt(0xc07f);             // lgkmcnt(0): where the loop begins, nothing is on its way that its end does not know of
+    int xat = 0, wat = W0, wfree = W0 + (NW - 1) * WB;            // the stage whose operands are multiplied; the place of the weights before it
+    for (int i = first; i < last; ++i) {
+      const int xnext = xat + XB == W0 ? 0 : xat + XB, wnext = wat + WB == W0 + NW * WB ? W0 : wat + WB;
 #pragma unroll
-    for (int m = 0; m < 2; ++m) {
-      if (m == 1) {
-        wait_loads<WAIT, true>();                 // the next stage has landed, and this wave's requests from this one
-        __builtin_amdgcn_s_barrier();
-        __builtin_amdgcn_sched_barrier(0);
-      }
-#pragma unroll
-      for (int st = 0; st < NST; ++st) {
-        const int from = APART && m == 0 ? XL : 0, n = APART ? (m == 0 ? WL : XL) : m == 0 ? 0 : XL + WL;      // requests of this half: rows, then weights
-#pragma unroll
-        for (int q = from + st * n / NST; q < from + (st + 1) * n / NST; ++q) {
-          if (q < XL) bring_x(i + NX, xat, q);
-          else bring_w(i + (APART ? NW - 1 : NW), APART ? wfree : wat, q - XL);
+      for (int m = 0; m < 2; ++m) {
+        if (m == 1) {
+          wait_loads<WAIT, true>();                 // the next stage has landed, and this wave's requests from this one
+          __builtin_amdgcn_s_barrier();
+          __builtin_amdgcn_sched_barrier(0);
         }
-        const f16x8 av = Fmt::operand(ahead[st]);
-        ahead[st] = a_piece(m ? wnext : wat, 1 - m, st);
 #pragma unroll
-        for (int r = st * RG / 2; r < (st + 1) * RG / 2 && r < RG; ++r) xf[1 - m][r] = b_operand(m ? xnext : xat, 1 - m, r);
+        for (int st = 0; st < NST; ++st) {
+          const int from = APART && m == 0 ? XL : 0, n = APART ? (m == 0 ? WL : XL) : m == 0 ? 0 : XL + WL;      // requests of this half: rows, then weights
 #pragma unroll
-        for (int rg = 0; rg < RG; ++rg) acc[rg][st] = Fmt::mma(av, xf[m][rg], acc[rg][st]);
-        __builtin_amdgcn_sched_barrier(0);        // (the requests stay where they are)
+          for (int q = from + st * n / NST; q < from + (st + 1) * n / NST; ++q) {
+            if (q < XL) bring_x(i + NX, xat, q);
+            else bring_w(i + (APART ? NW - 1 : NW), APART ? wfree : wat, q - XL);
+          }
+          const f16x8 av = Fmt::template operand<FAST>(ahead[st]);
+          ahead[st] = a_piece(m ? wnext : wat, 1 - m, st);
+#pragma unroll
+          for (int r = st * RG / 2; r < (st + 1) * RG / 2 && r < RG; ++r) xf[1 - m][r] = b_operand(m ? xnext : xat, 1 - m, r);
+#pragma unroll
+          for (int rg = 0; rg < RG; ++rg) acc[rg][st] = Fmt::mma(av, xf[m][rg], acc[rg][st]);
+          __builtin_amdgcn_sched_barrier(0);        // (the requests stay where they are)
+        }
       }
+      xat = xnext;
+      wfree = wat;
+      wat = wnext;
     }
-    xat = xnext;
-    wfree = wat;
-    wat = wnext;
+  };
+  if constexpr (Fmt::kCodes) {
+    if (__any(codes != 0)) {
+      products(std::false_type{});
+#pragma unroll
+      for (int rg = 0; rg < RG; ++rg)
+#pragma unroll
+        for (int st = 0; st < NST; ++st)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) acc[rg][st][r] *= Fmt::kSlowSum;
+    } else {
+      products(std::true_type{});
+    }
+  } else {
+    products(std::true_type{});
   }
   __builtin_amdgcn_s_waitcnt(0x0070);
   __syncthreads();                                // (what follows reuses the stages)

@@ -24,11 +24,6 @@
 #include "gemm_core.h"
 #include "formats.h"
 
-// flag bytes of a tiled FP8 weight: one per tile, nonzero when the tile holds 0x7F, 0xFF or 0x80
-__host__ __device__ inline size_t f8_tile_flags_offset(int N, int K) {
-  return (size_t)((N + 15) / 16) * (size_t)((K + 127) / 128) * 2048;
-}
-
 // 8 fp16 values on the F143 grid (|v| <= 240 or NaN) -> their 8 F143 bytes (+-240 -> 0x7F / 0xFF), and whether any of
 // them is beyond 240 (NaN).  v * 2^-7 is exact (an F143 subnormal becomes an fp16 subnormal) and carries the byte's exponent and
 // mantissa in bits 13..7 of each half.

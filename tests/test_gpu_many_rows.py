@@ -539,6 +539,42 @@ def test_tiles_of_other_sizes(kind, form, M, Kd, N, tiles):
     assert ((outs[0].double() - silu * upv).abs() <= bound).all()
 
 
+@pytest.mark.parametrize("form, M, Kd, N", [("one", 1000, 328, 2100), ("one", 600, 13704, 2100), ("slices", 1500, 2056, 1040), ("pair", 900, 200, 1500)])
+def test_blocks_of_fp8_channels_with_the_largest_codes(form, M, Kd, N):
+    """A few blocks of channels that hold 0x7F or 0xFF (+-240, which the fast conversion does not know) in their first, a middle and their last tile: they are right,
+    and the channels of all others are bit for bit what they are beside weights without these codes."""
+    from poptransformer_amd import kernels as K
+    x, w = operands(M, Kd, 2 * N, 61)
+    x = (x * 0.02).half()
+    scale = torch.tensor([-1], dtype=torch.int32, device="cuda")
+    codes = K.half_to_fp8(w.half(), scale)
+    assert not ((codes.view(torch.uint8) & 0x7F) == 0x7F).any()
+    marked = codes.clone()
+    flat = marked.view(torch.uint8)
+    at = [(3, 0), (N // 2, Kd // 2), (N - 1, Kd - 1), (N + 40, Kd // 3)]
+    for i, (n, k) in enumerate(at):
+        flat[n, k] = 0x7F if i % 2 else 0xFF
+    outs = []
+    for c in (codes, marked):
+        ws = [K.F8Weight(c[i * N:(i + 1) * N].contiguous(), scale) for i in range(2 if form == "pair" else 1)]
+        out = torch.full((M, N), float("nan"), dtype=torch.float16, device="cuda")
+        K.linear(x, ws, [out] * len(ws), swiglu=form == "pair", workspace=K.linear_workspace(M, N, "cuda") if form == "slices" else None)
+        assert K.linear_kernel() == "gemm_block_kernel"
+        outs.append(out)
+    plain = K.fp8_to_half(marked, scale).double()
+    # a wave's channels, four blocks of a matrix (two of each of a pair's), go one way together, and a neighbour's flags may send more of them there: the same sums
+    assert torch.equal(outs[0][:, 128:N // 2 - 128], outs[1][:, 128:N // 2 - 128]) and torch.equal(outs[0][:, N // 2 + 128:N - 128], outs[1][:, N // 2 + 128:N - 128])
+    xd = x.double()
+    if form != "pair":
+        close(outs[1], xd @ plain[:N].T, xd.abs() @ plain[:N].abs().T, Kd, 11)
+        return
+    gate, upv = xd @ plain[:N].T, xd @ plain[N:].T
+    silu = torch.nn.functional.silu(gate)
+    dg, du = (2.0 ** -11 * t.abs() + (Kd + 2) * 2.0 ** -24 * (xd.abs() @ p.abs().T) for t, p in ((gate, plain[:N]), (upv, plain[N:])))
+    bound = 1.1 * dg * (upv.abs() + du) + du * silu.abs() + 2.5 * 2.0 ** -11 * (silu * upv).abs() + 2.0 ** -20 * (1 + upv.abs())      # as in test_pair
+    assert ((outs[1].double() - silu * upv).abs() <= bound).all()
+
+
 def test_every_gate_comes_out_as_by_the_operator():
     """Every fp16 gate but NaN through the end of a tile, bit for bit: rows that pick one feature, so that sums are the weights' own values, beside 1 from the
     other weight."""
