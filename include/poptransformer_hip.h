@@ -399,7 +399,12 @@ int pta_half_to_fp8_grid(const pta_half* x, pta_half* out, const int32_t* scale,
 /* ------------------------------------------------------------------------------------
  * Linear layers, general form (layers/linear.py:19-46 + precision_strategy.py:56-81)
  * ---------------------------------------------------------------------------------- */
-enum { PTA_W_INT4 = 0, PTA_W_F16 = 1, PTA_W_F143 = 2, PTA_W_F152 = 3 };
+enum { PTA_W_INT4 = 0, PTA_W_F16 = 1, PTA_W_F143 = 2, PTA_W_F152 = 3,
+       /* F143 weights that hold none of the codes 0x7F, 0xFF and 0x80: all flag bytes that pta_fp8_tile has left behind the
+          tiles (one a tile: ceil(N / 16) * ceil(K / 128) of them from 2048 times as many bytes on) are zero.  The caller says so;
+          a weight of this kind that holds 0x7F or 0xFF all the same makes results NaN.  Same results as PTA_W_F143, sooner; the
+          two may be mixed in a call. */
+       PTA_W_F143_PLAIN = 4 };
 
 typedef struct pta_weight {
   int kind;            /* PTA_W_*                                                              */

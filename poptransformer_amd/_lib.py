@@ -29,7 +29,7 @@ class Weight(ctypes.Structure):
                 ("x", c_void_p), ("act", c_int), ("mix", c_void_p)]
 
 
-W_INT4, W_F16, W_F143, W_F152 = 0, 1, 2, 3
+W_INT4, W_F16, W_F143, W_F152, W_F143_PLAIN = 0, 1, 2, 3, 4
 
 
 class DecodeLayer(ctypes.Structure):

@@ -9,6 +9,7 @@
 #include "gemm_f8n.h"
 
 int f8_decode_unscaled_launch(const uint8_t* in, f16* out, size_t n, int format, hipStream_t s);
+int run_linear_f143_plain(GemmArgs& a, int total_nb, int swiglu, hipStream_t s, const char* name);      // linear_f143_plain.hip
 
 template <class Fmt>
 static int run_linear(GemmArgs& a, int total_nb, int swiglu, hipStream_t s, const char* name) {
@@ -46,7 +47,10 @@ static int linear_impl(const void* X, const int32_t* x_scale, int x_bytes, int c
   PTA_REQUIRE(host_w && host_Y, "pta_linear: null pointer");
   PTA_REQUIRE(count >= 1 && count <= 4, "pta_linear: count must be in [1, 4], got %d", count);
   PTA_REQUIRE(!swiglu || count == 2, "pta_linear: a SwiGLU pair is exactly two weights (gate, up)");
-  const int kind = host_w[0].kind, K = host_w[0].K;
+  // (F143 weights with and without the codes that the conversion does not know: one kind but for which kernels multiply them)
+  auto kind_of = [&](int i) { return host_w[i].kind == PTA_W_F143_PLAIN ? (int)PTA_W_F143 : host_w[i].kind; };
+  const int kind = kind_of(0), K = host_w[0].K;
+  bool plain = true;
   int rc = check_gemv_common("pta_linear", X ? (const void*)X : (const void*)host_w[0].x, M, K);
   if (rc) return rc;
   for (int i = 0; i < count; ++i) PTA_REQUIRE(X || host_w[i].x, "pta_linear: entry %d has no input", i);
@@ -58,7 +62,8 @@ static int linear_impl(const void* X, const int32_t* x_scale, int x_bytes, int c
   int nb = 0;
   for (int i = 0; i < count; ++i) {
     const pta_weight& w = host_w[i];
-    PTA_REQUIRE(w.kind == kind && w.K == K, "pta_linear: weights of one call must share their kind and K");
+    PTA_REQUIRE(kind_of(i) == kind && w.K == K, "pta_linear: weights of one call must share their kind and K");
+    plain = plain && w.kind == PTA_W_F143_PLAIN;
     PTA_REQUIRE(w.tiled && host_Y[i] && w.N > 0, "pta_linear: entry %d is incomplete", i);
     PTA_REQUIRE(kind == PTA_W_F16 || w.scale, "pta_linear: entry %d needs its scale", i);
     PTA_REQUIRE(pta_aligned(w.tiled, 16), "pta_linear: tiled[%d] must be 16-byte aligned", i);
@@ -118,7 +123,7 @@ static int linear_impl(const void* X, const int32_t* x_scale, int x_bytes, int c
   switch (kind) {
     case PTA_W_INT4: return run_linear<FmtW4>(a, nb, swiglu, s, "pta_linear");
     case PTA_W_F16: return run_linear<FmtF16>(a, nb, swiglu, s, "pta_linear");
-    case PTA_W_F143: return run_linear<FmtF8<0>>(a, nb, swiglu, s, "pta_linear");
+    case PTA_W_F143: return plain ? run_linear_f143_plain(a, nb, swiglu, s, "pta_linear") : run_linear<FmtF8<0>>(a, nb, swiglu, s, "pta_linear");
     default: return run_linear<FmtF8<1>>(a, nb, swiglu, s, "pta_linear");
   }
 }

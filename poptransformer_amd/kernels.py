@@ -233,6 +233,10 @@ class F8Weight:
         lib = _lib.load()
         self.tiled = torch.zeros(lib.pta_fp8_tiled_bytes(self.N, self.K), dtype=torch.uint8, device=w.device)
         check(lib.pta_fp8_tile(_p(w), _p(self.tiled), self.N, self.K, 1 if kn else 0, _stream()))
+        # whether the hardware's conversion knows all of the codes: looked up once, here (a stream that records cannot be waited for)
+        tiles = -(-self.N // 16) * -(-self.K // 128)
+        self.plain = (self.format == _lib.F143 and not torch.cuda.is_current_stream_capturing()
+                      and not self.tiled[tiles * 2048:tiles * 2049].any().item())
 
     @property
     def nbytes(self):
@@ -283,8 +287,8 @@ def _desc(w, x=None, act=_lib.ACT_NONE, mix=None):
     if isinstance(w, F16Weight):
         return _lib.Weight(_lib.W_F16, w.tiled.data_ptr(), None, w.N, w.K, xp, act, mp)
     if isinstance(w, F8Weight):
-        return _lib.Weight(_lib.W_F143 if w.format == _lib.F143 else _lib.W_F152, w.tiled.data_ptr(), w.scale.data_ptr(),
-                           w.N, w.K, xp, act, mp)
+        kind = _lib.W_F143_PLAIN if w.plain else _lib.W_F143 if w.format == _lib.F143 else _lib.W_F152
+        return _lib.Weight(kind, w.tiled.data_ptr(), w.scale.data_ptr(), w.N, w.K, xp, act, mp)
     raise TypeError(f"not a tiled weight: {type(w)}")
 
 

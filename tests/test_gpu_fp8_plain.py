@@ -1,0 +1,65 @@
+"""F143 weights that hold none of the codes 0x7F, 0xFF and 0x80 go to kernels of their own (PTA_W_F143_PLAIN), whose conversion is the hardware's: the same numbers, and the
+same results as by the kernels for all codes."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def scale():
+    return torch.tensor([-1], dtype=torch.int32, device="cuda")
+
+
+@pytest.mark.parametrize("rows", [1, 8, 40, 300])
+def test_every_code(rows):
+    from poptransformer_amd import kernels as K
+    codes = torch.tensor([c for c in range(256) if c not in (0x7F, 0xFF, 0x80)], dtype=torch.uint8, device="cuda")
+    w8 = torch.zeros((len(codes), 32), dtype=torch.uint8, device="cuda")
+    w8[:, 7] = codes
+    w = K.F8Weight(w8, scale())
+    assert w.plain
+    x = torch.zeros((rows, 32), dtype=torch.float16, device="cuda")
+    x[:, 7] = 1
+    out = torch.full((rows, len(codes)), float("nan"), dtype=torch.float16, device="cuda")
+    K.linear(x, [w], [out])
+    assert torch.equal(out, K.fp8_to_half(codes, scale()).expand_as(out))
+
+
+@pytest.mark.parametrize("kind, Kd, N", [("one", 4096, 4100), ("one", 200, 136), ("one", 13704, 520), ("slices", 2048, 1024), ("pair", 4096, 4096), ("three", 1032, 2050)])
+@pytest.mark.parametrize("rows", [1, 4, 5, 8, 16, 17, 33, 64, 65, 128, 129, 500])
+def test_like_the_kernels_for_all_codes(kind, Kd, N, rows):
+    from poptransformer_amd import kernels as K
+    g = torch.Generator(device="cuda").manual_seed(rows)
+    n = {"pair": 2, "three": 3}.get(kind, 1)
+    x = (torch.randn((rows, Kd), generator=g, device="cuda") * 0.2).half()
+    ws = [K.F8Weight(K.half_to_fp8((torch.randn((N, Kd), generator=g, device="cuda") * 0.02).half(), scale()), scale()) for _ in range(n)]
+    results = []
+    for plain in (True, False):
+        for w in ws:
+            assert w.plain or plain is False
+            w.plain = plain
+        outs = [torch.full((rows, N), float("nan"), dtype=torch.float16, device="cuda") for _ in range(3 if kind == "three" else 1)]
+        K.linear(x, ws, outs * 2 if kind == "pair" else outs, swiglu=kind == "pair", workspace=K.linear_workspace(rows, N, "cuda") if kind == "slices" else None)
+        results.append((K.linear_kernel(), outs))
+    assert results[0][0] == results[1][0]
+    for a, b in zip(results[0][1], results[1][1]):
+        assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("rows", [2, 8, 64, 260])
+def test_codes_beyond_the_conversion(rows):
+    """Such a weight is not called plain, also beside one that is."""
+    from poptransformer_amd import kernels as K
+    g = torch.Generator(device="cuda").manual_seed(5)
+    Kd, N = 1024, 512
+    x = (torch.randn((rows, Kd), generator=g, device="cuda") * 0.05).half()
+    codes = [K.half_to_fp8((torch.randn((N, Kd), generator=g, device="cuda") * 0.02).half(), scale()) for _ in range(2)]
+    codes[1].view(torch.uint8)[N - 1, 3] = 0xFF
+    ws = [K.F8Weight(c, scale()) for c in codes]
+    assert [w.plain for w in ws] == [True, False] and not K.F8Weight(codes[0], scale(), "F152").plain
+    outs = [torch.full((rows, N), float("nan"), dtype=torch.float16, device="cuda") for _ in ws]
+    K.linear(x, ws, outs)
+    for c, out in zip(codes, outs):
+        p = K.fp8_to_half(c, scale()).double()
+        ref, mag = x.double() @ p.T, x.double().abs() @ p.abs().T
+        assert ((out.double() - ref).abs() <= 2.0 ** -11 * ref.abs() + (Kd + 2) * 2.0 ** -24 * mag + 2.0 ** -24).all()
