@@ -112,7 +112,7 @@ size_t pta_linear_workspace_bytes(int M, int N);
 
 /* The norm of a product's rows that pta_linear_then_norm does behind it. */
 typedef struct pta_row_norm {
-  int norm;                    /* PTA_NORM_RMS or PTA_NORM_LAYER                                              */
+  int norm;                    /* PTA_NORM_RMS or PTA_NORM_LAYER, | PTA_NORM_ANY_ORDER                        */
   const pta_half* weight;      /* [N]                                                                         */
   const pta_half* bias;        /* [N], PTA_NORM_LAYER only                                                    */
   float eps;
@@ -128,7 +128,10 @@ const char* pta_linear_kernel(void);
 /* the tiles (rows x channels) of the calling thread's last product by gemm_block_kernel, behind a space those of its last channels where they are others */
 const char* pta_linear_tiles(void);
 
-enum { PTA_NORM_NONE = 0, PTA_NORM_RMS = 1, PTA_NORM_LAYER = 2 };
+enum { PTA_NORM_NONE = 0, PTA_NORM_RMS = 1, PTA_NORM_LAYER = 2,
+       /* pta_row_norm only: the product may be cut otherwise than pta_linear cuts it (its fp32 sums in another order), for what is
+          the faster launch with a norm behind it */
+       PTA_NORM_ANY_ORDER = 256 };
 enum { PTA_ACT_NONE = 0, PTA_ACT_GELU_TANH = 1, PTA_ACT_RELU_SQUARE = 2, PTA_ACT_SIGMOID = 3 };
 
 /* Fused Int4ToHalf(axis=1) + MatMul (utils/param_handler/precision_strategy.py:56-60,74-75):
@@ -427,7 +430,7 @@ int pta_linear(const pta_half* X, const int32_t* x_scale, int count, const pta_w
                const pta_fusion* fuse, pta_stream_t stream);
 
 /* pta_linear of one weight, then pta_rmsnorm, pta_rmsnorm_fp8_grid, pta_layer_norm_ce or pta_layer_norm_ce_mix of Y's rows: bit-identical to the
- * two calls.  Where the product's K is split across workgroups (fuse->workspace), adding the slices and the norm are one launch. */
+ * two calls (but with PTA_NORM_ANY_ORDER).  Where the product's K is split across workgroups (fuse->workspace), adding the slices and the norm are one launch. */
 int pta_linear_then_norm(const pta_half* X, const int32_t* x_scale, const pta_weight* host_w, const pta_half* bias, pta_half* Y, int M,
                          const pta_fusion* fuse, const pta_row_norm* host_norm, pta_stream_t stream);
 

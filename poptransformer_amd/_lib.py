@@ -21,7 +21,7 @@ F143, F152 = 0, 1
 FP8_FORMATS = {"F143": F143, "F152": F152}
 
 
-NORM_NONE, NORM_RMS, NORM_LAYER = 0, 1, 2
+NORM_NONE, NORM_RMS, NORM_LAYER, NORM_ANY_ORDER = 0, 1, 2, 256
 
 
 class Weight(ctypes.Structure):

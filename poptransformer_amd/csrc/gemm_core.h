@@ -275,6 +275,7 @@ struct FinishNorm {
   NormMix mix;
   int mode;            // of norm_row
   bool shifted;        // with the mix
+  bool any_order;      // the product's sums may be taken in another order than without a norm
   bool done;
 };
 
@@ -1397,15 +1398,22 @@ static void launch_finish_norm(const GemmArgs& a, const FinishNorm& t, hipStream
   else hipLaunchKernelGGL((splitk_finish_norm_kernel<Fmt, 2, false, VECS>), dim3(a.M), dim3(NORM_THREADS), 0, s, a, t.norm, t.mix);
 }
 
-template <class Fmt>
-static bool launch_splitk_finish_norm(const GemmArgs& a, hipStream_t s) {
+static inline bool finish_norm_fits(const GemmArgs& a) {
   const GemmMat& mat = a.mat[0];
-  FinishNorm* t = a.then;
+  const FinishNorm* t = a.then;
   const void* whole[] = {mat.Y, mat.bias, a.epi.bias, a.epi.mul, a.epi.residual};
   for (const void* p : whole)
     if (p && !pta_aligned(p, 16)) return false;
   // (no activation: a row's sixteen of each kind are more instructions than the rest of the kernel)
-  if (t->norm.cols != mat.N || a.epi.out_fp8_scale || mat.act != PTA_ACT_NONE || a.epi.act != PTA_ACT_NONE || t->mode == 1 || a.ksplit > GEMM_MAX_KSPLIT) return false;
+  if (t->norm.cols != mat.N || a.epi.out_fp8_scale || mat.act != PTA_ACT_NONE || a.epi.act != PTA_ACT_NONE || t->mode == 1) return false;
+  return true;
+}
+
+template <class Fmt>
+static bool launch_splitk_finish_norm(const GemmArgs& a, hipStream_t s) {
+  const GemmMat& mat = a.mat[0];
+  FinishNorm* t = a.then;
+  if (!finish_norm_fits(a) || a.ksplit > GEMM_MAX_KSPLIT) return false;
   // (as few pieces of a thread as the row needs: what a row is made of stays in registers)
   if (mat.N <= 8 * NORM_THREADS) launch_finish_norm<Fmt, 1>(a, *t, s);
   else if (mat.N <= 16 * NORM_THREADS) launch_finish_norm<Fmt, 2>(a, *t, s);
@@ -2994,22 +3002,33 @@ struct OwnPlan { int mt, nb, slices, rounds; double us; };
 // own, of a row group, of a channel block - its products, and its weights, which the row blocks share; of the second launch of a
 // split) are fitted to measured launches: they order the choices.  64 rows, INT4, 11008 x 4096, blocks x slices: 1 x 1 23.5, 2 x 2
 // 19.2, 4 x 4 20.5 us; 4096 x 11008: 1 block 29.3, 2 21.9, 3 14.5, 4 16.4; 4096 x 4096: 1 x 1 11.1, 1 x 2 16.3, 2 x 2 11.9, 4 x 4 13.4.
+// A launch with a norm behind it takes a second kernel however K is cut (splitk_finish_norm_kernel in the norm kernel's place), so that
+// slices cost it little more than their sums' bytes, and a workgroup of fewer features reads fewer bytes of X.  Up to 128 rows and a block
+// a compute unit, by a grid of 3600 plans (12 shapes of 768 to 5120 channels, 9 to 128 rows, weights from HBM), launch and norm, us, with the plan of launches
+// without a norm and with this: F143, 13696 x 4096, 64 rows 26.4 -> 23.4, 16 rows 18.4 -> 17.3, 16384 x 4096, 16 rows 23.3 ->
+// 19.6; INT4, 8192 x 2048, 32 rows 10.8 -> 9.6, 4096 x 4096, 64 rows 13.9 -> 12.9, 3072 x 768, 32 rows 8.6 -> 7.2, 96 rows 9.9 -> 8.6; fp16, 11008 x 4096, 32 rows
+// 29.0 -> 24.7, 2048 x 2048, 32 rows 9.1 -> 8.4.  9 to 16 rows only with 80 feature tiles and more (INT4 from 13 rows on): 4096 x 4096, 16 rows, F143
+// 9.8 and 10.7, INT4 8.8 and 9.8; 11008 x 4096, 9 rows, INT4 12.9 and 13.5.  5120 x 5120 keeps the dearer estimate: 17 rows, INT4 12.0 and 13.4.
 template <class Fmt, bool PAIR>
 static OwnPlan plan_gemm_own(const GemmArgs& a) {
   constexpr double PRODUCTS = Fmt::kVec == 1 ? 0.48 : Fmt::kVec == 2 ? 0.6 : 0.7, WEIGHTS = Fmt::kVec == 1 ? 0.0 : Fmt::kVec == 2 ? 0.36 : 0.9;
   const int cus = device_compute_units();
   const int row_blocks = (a.M + 63) / 64;
-  const bool split = !PAIR && a.count == 1 && a.part && a.M > 16;
+  // (up to 128 rows and a block of channels a compute unit)
+  const bool normed = a.then && a.then->any_order && a.M <= 128 && a.mat[0].N <= 16 * cus && finish_norm_fits(a);
+  const bool split = !PAIR && a.count == 1 && a.part && (a.M > 16 || (normed && a.M > (Fmt::kVec == 1 ? 12 : 8) && a.KT >= 80));
   OwnPlan best{((a.M + 15) / 16 + row_blocks - 1) / row_blocks, 1, 1, 0, 0.0};
+  const double rows = normed ? a.M / 16.0 / row_blocks : best.mt;      // groups of them that a workgroup reads
   for (int nb = 1; nb <= own_cap<Fmt, PAIR>(best.mt); ++nb) {
     const int groups = own_groups(a, nb, PAIR) * row_blocks;
-    for (int sl = 1; sl <= (split ? GEMM_MAX_KSPLIT : 1); ++sl) {
+    // (four blocks by four slices, more than 64 rows: 2 x 2 is the faster by 2 to 5 %)
+    for (int sl = 1; sl <= (!split ? 1 : normed && row_blocks > 1 ? 3 : GEMM_MAX_KSPLIT); ++sl) {
       if (sl > 1 && (a.KT < sl * OWN_WAVES || a.part_bytes < (size_t)sl * a.M * a.mat[0].N * sizeof(float))) break;
       const int rounds = (groups * sl + cus - 1) / cus, tiles = ((a.KT + sl - 1) / sl + OWN_WAVES - 1) / OWN_WAVES;
-      double us = 3.2 + rounds * tiles * (0.5 + 0.29 * best.mt + (PRODUCTS + WEIGHTS / row_blocks) * nb * (PAIR ? 2 : 1));
+      double us = 3.2 + rounds * tiles * (0.5 + 0.29 * rows + (PRODUCTS + WEIGHTS / row_blocks) * nb * (PAIR ? 2 : 1));
       if (sl > 1) {
         const double size = (double)a.M * a.mat[0].N / 262144;
-        us += 2.7 * sl - 0.9 + (size > 1 ? 0.5 * sl * (size - 1) : 0.0);
+        us += normed ? sl * (0.35 + 0.5 * size) + (Fmt::kVec > 1 ? 1.0 : 0.8) : 2.7 * sl - 0.9 + (size > 1 ? 0.5 * sl * (size - 1) : 0.0);
       }
       if (best.rounds == 0 || us < best.us) best.nb = nb, best.slices = sl, best.rounds = rounds, best.us = us;
     }

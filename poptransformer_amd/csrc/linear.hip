@@ -140,19 +140,20 @@ extern "C" int pta_linear_then_norm(const pta_half* X, const int32_t* x_scale, c
   PTA_REQUIRE(host_w && Y && host_norm, "%s: null pointer", name);
   const pta_row_norm& n = *host_norm;
   const bool shifted = n.prev != nullptr;
-  PTA_REQUIRE(n.norm == PTA_NORM_RMS || n.norm == PTA_NORM_LAYER, "%s: unknown norm %d", name, n.norm);
-  PTA_REQUIRE(!shifted || n.norm == PTA_NORM_LAYER, "%s: a token shift follows a LayerNorm", name);
-  PTA_REQUIRE(!n.grid_scale || n.norm == PTA_NORM_RMS, "%s: the FP8 grid follows an RMSNorm", name);
+  const int norm = n.norm & ~PTA_NORM_ANY_ORDER;
+  PTA_REQUIRE(norm == PTA_NORM_RMS || norm == PTA_NORM_LAYER, "%s: unknown norm %d", name, n.norm);
+  PTA_REQUIRE(!shifted || norm == PTA_NORM_LAYER, "%s: a token shift follows a LayerNorm", name);
+  PTA_REQUIRE(!n.grid_scale || norm == PTA_NORM_RMS, "%s: the FP8 grid follows an RMSNorm", name);
   PTA_REQUIRE(!(fuse && fuse->out_fp8_scale), "%s: the rows to be normed are left as they are", name);
   const int cols = host_w->N;
   int rc = check_norm(name, Y, n.weight, shifted ? n.prev : n.y, M, cols);
   if (rc) return rc;
-  if (n.norm == PTA_NORM_LAYER) rc = check_layer_norm(name, n.bias, cols);
+  if (norm == PTA_NORM_LAYER) rc = check_layer_norm(name, n.bias, cols);
   if (!rc && n.grid_scale) rc = check_grid(name, n.grid_scale, n.grid_format);
   if (!rc && shifted) rc = check_norm_mix(name, n.y, n.mix, n.mixed);
   if (rc) return rc;
   FinishNorm then{NormArgs{(const f16*)n.weight, (const f16*)n.bias, (f16*)n.y, cols, n.eps, n.grid_scale, n.grid_format}, NormMix{},
-                  n.norm == PTA_NORM_RMS ? 0 : M == 1 ? 1 : 2, shifted, false};
+                  norm == PTA_NORM_RMS ? 0 : M == 1 ? 1 : 2, shifted, (n.norm & PTA_NORM_ANY_ORDER) != 0, false};
   if (shifted) then.mix = NormMix{(f16*)n.prev, {(const f16*)n.mix[0], (const f16*)n.mix[1], (const f16*)n.mix[2]}, {(f16*)n.mixed[0], (f16*)n.mixed[1], (f16*)n.mixed[2]}};
   rc = linear_impl(X, x_scale, 0, 1, host_w, &bias, &Y, M, 0, fuse, stream, &then);
   if (rc || then.done) return rc;

@@ -145,8 +145,8 @@ class LayerOps:
         self._fp8_buf = {k: buf(rows, k) for k in {d, ffn}}
         self._gate, self._up = buf(rows, ffn), buf(rows, ffn)
         self._on_grid = {}      # buffer address -> the FP8 grid (format, exponent) its values are on
-        # scratch that lets a Linear of more than 16 rows with few output channels (attention output, MLP down) split K
-        self._lin_ws = self._linear_workspace(d, ffn) if rows > 16 else None
+        # scratch that lets a Linear of more than 16 rows (8 where a norm follows) with few output channels (attention output, MLP down) split K
+        self._lin_ws = self._linear_workspace(d, ffn) if rows > 8 else None
 
     def _linear_workspace(self, d, ffn):
         return K.linear_workspace(self._rows, d, self.dev)
@@ -181,7 +181,7 @@ class LayerOps:
         self._on_grid.pop(self.x.data_ptr(), None)
         grid = self._common_grid(consumers) if self.spec.norm == "rms" else None
         out = self.h if grid is None else self._fp8_buf[self.x.shape[1]]
-        K.linear_then_norm(xin, lw.w, self.x, K.RowNorm(gb[0], gb[1] if self.spec.norm == "ln" else None, self.spec.eps, out=out, grid=grid), x_scale=xs,
+        K.linear_then_norm(xin, lw.w, self.x, K.RowNorm(gb[0], gb[1] if self.spec.norm == "ln" else None, self.spec.eps, out=out, grid=grid, any_order=True), x_scale=xs,
                            bias=lw.bias, residual=self.x, workspace=self._lin_ws)
         if grid is not None:
             self._on_grid[out.data_ptr()] = self._grid_id(consumers[0])

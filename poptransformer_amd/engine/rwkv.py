@@ -100,9 +100,9 @@ class RWKVDecoder(DecodeLoop):
         self.st_max = [buf(B, d, dtype=f32) for _ in range(s.n_layer)]
         self.graph = None
         self._stream = torch.cuda.Stream()
-        # more than 16 rows: scratch that lets the two single-weight Linears of a layer (4096 channels: too few
+        # more than 8 rows: scratch that lets the two single-weight Linears of a layer (4096 channels: too few
         # channel blocks to fill the machine) split K across workgroups
-        self._lin_ws = K.linear_workspace(B, d, device) if B > 16 else None
+        self._lin_ws = K.linear_workspace(B, d, device) if B > 8 else None
 
     @staticmethod
     def _group(xs, lws, outs, acts):
@@ -147,19 +147,19 @@ class RWKVDecoder(DecodeLoop):
                 self._shifted(x, blk.ln2, [blk.ffn_key, blk.ffn_receptance], blk.ffn_mix, self.st_ffn[i], [self.fk, self.fr],
                               [_lib.ACT_RELU_SQUARE, _lib.ACT_SIGMOID])
             else:
-                K.linear_then_norm(self.y, blk.att_output.w, x, K.RowNorm(blk.ln2[0], blk.ln2[1], s.eps, shift=(self.st_ffn[i], blk.ffn_mix, self.mix[:2])),
+                K.linear_then_norm(self.y, blk.att_output.w, x, K.RowNorm(blk.ln2[0], blk.ln2[1], s.eps, shift=(self.st_ffn[i], blk.ffn_mix, self.mix[:2]), any_order=True),
                                    residual=x, workspace=self._lin_ws)
                 self._group(self.mix[:2], [blk.ffn_key, blk.ffn_receptance], [self.fk, self.fr],
                             [_lib.ACT_RELU_SQUARE, _lib.ACT_SIGMOID])
             halve = s.rescale_every > 0 and (i + 1) % s.rescale_every == 0
             end = dict(mul=self.fr, residual=x, post_scale=0.5 if halve else 0.0, workspace=self._lin_ws)
             if i + 1 == s.n_layer:
-                K.linear_then_norm(self.fk, blk.ffn_value.w, x, K.RowNorm(w.ln_out[0], w.ln_out[1], s.eps, out=self.h), **end)
+                K.linear_then_norm(self.fk, blk.ffn_value.w, x, K.RowNorm(w.ln_out[0], w.ln_out[1], s.eps, out=self.h, any_order=True), **end)
             elif self.fuse_shift or w.blocks[i + 1].pre_ln is not None:
                 K.linear(self.fk, [blk.ffn_value.w], [x], **end)
             else:
                 ln, mixes = w.blocks[i + 1].ln1, w.blocks[i + 1].att_mix
-                K.linear_then_norm(self.fk, blk.ffn_value.w, x, K.RowNorm(ln[0], ln[1], s.eps, shift=(self.st_att[i + 1], mixes, self.mix)), **end)
+                K.linear_then_norm(self.fk, blk.ffn_value.w, x, K.RowNorm(ln[0], ln[1], s.eps, shift=(self.st_att[i + 1], mixes, self.mix), any_order=True), **end)
         K.linear(self.h, [w.head.w], [self.logits])
         self.select(self.logits, self.next_ids)
         K.step_update(self.container, None, self.stop_mask, self.step, self.next_ids, None, self.keep_going,

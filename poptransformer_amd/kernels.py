@@ -325,9 +325,10 @@ def linear(x, weights, outs, biases=None, x_scale=None, swiglu=False, bias=None,
 
 class RowNorm:
     """The norm that `linear_then_norm` does behind a product: `rmsnorm`, `rmsnorm_fp8_grid` (grid = (exponent, format)), `layer_norm_ce` (beta) or
-    `layer_norm_ce_mix` (shift = (previous rows, mixing vectors, results)), into `out`."""
+    `layer_norm_ce_mix` (shift = (previous rows, mixing vectors, results)), into `out`.  any_order: the product's sums may be taken in another order than
+    `linear` takes them, for what is faster with a norm behind it."""
 
-    def __init__(self, gamma, beta, eps, out=None, grid=None, shift=None):
+    def __init__(self, gamma, beta, eps, out=None, grid=None, shift=None, any_order=False):
         prev, mixes, mixed = shift if shift is not None else (None, (), ())
         if shift is not None and (len(mixes) != len(mixed) or not 1 <= len(mixes) <= 3):
             raise ValueError("a token shift has one to three mixing vectors, and an output each")
@@ -342,7 +343,7 @@ class RowNorm:
         self.rows = [(t, what) for t, what in ((out, "out"), (prev, "previous rows")) if t is not None]
         self.mixed = mixed
         V = ctypes.c_void_p * 3
-        self.args = _lib.RowNorm(_lib.NORM_RMS if beta is None else _lib.NORM_LAYER, _p(gamma), _p(beta), eps, _p(out), _p(grid[0]) if grid else None,
+        self.args = _lib.RowNorm((_lib.NORM_RMS if beta is None else _lib.NORM_LAYER) | (_lib.NORM_ANY_ORDER if any_order else 0), _p(gamma), _p(beta), eps, _p(out), _p(grid[0]) if grid else None,
                                  _fmt(grid[1]) if grid else 0, _p(prev), V(*[_p(t) for t in mixes]), V(*[_p(t) for t in mixed]))
         self._keep = (gamma, beta, out, grid, shift)
 

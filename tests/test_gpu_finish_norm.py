@@ -94,3 +94,30 @@ def test_tensors_that_the_norms_own_entry_points_refuse():
         K.RowNorm(gamma, None, 1e-5, out=rows(20, 64), grid=(torch.zeros(1, dtype=torch.int64, device="cuda"), "F143"))
     with pytest.raises(ValueError):
         K.RowNorm(gamma.reshape(8, 8), None, 1e-5, out=rows(20, 64))
+
+
+# rows, features, channels: the edges of what may be cut otherwise (blocks x slices of its plan), odd channels and feature tiles
+@pytest.mark.parametrize("kind, M, Kd, N", [("int4", 13, 11008, 4096), ("int4", 12, 11008, 4096), ("int4", 64, 4096, 4096), ("int4", 128, 3072, 768), ("int4", 129, 3072, 768), ("F143", 9, 13696, 4096),
+                                            ("F143", 64, 13696, 4096), ("F143", 17, 8192, 2056), ("F143", 40, 4096, 4104), ("f16", 24, 11008, 4096), ("f16", 80, 5632, 2048), ("f16", 31, 2824, 1016),
+                                            ("F152", 33, 4096, 1024), ("int4", 16, 1024, 64)])
+@pytest.mark.parametrize("room", [4, 3, 1, 0])
+def test_sums_in_any_order(kind, M, Kd, N, room):
+    """With any_order the product may be cut otherwise, by the scratch that there is: within the bound of fp32 sums, and the norm is that of the rows it leaves."""
+    from poptransformer_amd import kernels as K
+    g = torch.Generator(device="cuda").manual_seed(71)
+    x = torch.randn((M, Kd), generator=g, device="cuda").half() * 0.1
+    w = weight(kind, N, Kd, g)
+    gamma, res = torch.randn(N, generator=g, device="cuda").half(), torch.randn((M, N), generator=g, device="cuda").half()
+    got, out, one, plain = (torch.full((M, N), float("nan"), dtype=torch.float16, device="cuda") for _ in range(4))
+    workspace = K.linear_workspace(M, N, "cuda")[:room * M * N * 4] if room else None
+    K.linear_then_norm(x, w, got, K.RowNorm(gamma, None, 1e-5, out=out, any_order=True), residual=res, workspace=workspace)
+    K.linear(x, [w], [plain], residual=res)
+    K.rmsnorm(got, gamma, 1e-5, one)
+    assert torch.equal(out, one)
+    # either one's sums of fp32 products are within K 2^-24 of the sum of magnitudes, and rounded twice to fp16 (the product, and with the residual)
+    unit = torch.eye(Kd, dtype=torch.float16, device="cuda")
+    dense = torch.cat([K.linear(unit[i:i + 256], [w], [torch.empty((min(256, Kd - i), N), dtype=torch.float16, device="cuda")])[0] for i in range(0, Kd, 256)]).double()
+    mag = x.double().abs() @ dense.abs()
+    ref = x.double() @ dense
+    for y in (got, plain):
+        assert ((y.double() - (ref + res.double())).abs() <= 2.0 ** -10 * (ref.abs() + res.double().abs()) + (Kd + 2) * 2.0 ** -24 * mag + 2.0 ** -23).all()
