@@ -2081,7 +2081,7 @@ __device__ __forceinline__ f16 tile_swish_f16(f16 x) {
 template <class Fmt, int NST, int RG, bool PAIR>
 __device__ __forceinline__ bool straight_store(const GemmMat& mat, const GemmEpilogue& epi, const f32x4 (&acc)[RG][NST], int blk0, int row0, int nsl,
                                                typename Fmt::Scale s0, typename Fmt::Scale s1, int M, const int32_t* order) {
-  static_assert(NST == 4 && RG % 2 == 0, "tile");
+  static_assert(NST == 4 && (RG % 2 == 0 || !Fmt::kWide), "tile");
   const int lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4;
   const int N = mat.N, n0 = blk0 * 16;
   // A slice's sums wait for nothing, and go out as whole lines from LDS faster than a quarter of a line a lane group from here: bf16, with straight stores and
@@ -2387,11 +2387,11 @@ __global__ __launch_bounds__(PANEL_WAVES * 64) __attribute__((amdgpu_waves_per_e
   constexpr int ROWS = RG * 16;
   constexpr int XPART = ROWS * 128;               // halves of one feature tile of the workgroup's rows
   constexpr int XSTAGE = KH * XPART;              // one stage: a tile per part
-  constexpr int QN = KH * RG / 2;                 // row loads (4 rows each) per wave and stage
+  constexpr int LOADS = KH * RG * 4, QN = (LOADS + PANEL_WAVES - 1) / PANEL_WAVES;      // row loads (4 rows each) per stage, and per wave
   constexpr int SW = NST * 16 + 4;                // floats per row of a wave's epilogue strip
   static_assert(!PAIR || NST % 2 == 0, "gate and up blocks in equal numbers");
   static_assert(KH == 1 || KH == 2 || KH == 4, "parts of K");
-  static_assert((KH * RG) % 2 == 0 && RG <= 8, "row loads per wave");
+  static_assert(RG <= 8, "registers");
   static_assert(KH == 1 || (KH - 1) * CW * RG * NST * 1024 <= 2 * XSTAGE * 2, "the parts' sums meet in the row buffers");
   extern __shared__ __align__(16) unsigned char smem[];
   f16* xbuf = reinterpret_cast<f16*>(smem);                                              // [2][KH][ROWS][128], pieces exchanged (see fetch_x)
@@ -2458,6 +2458,7 @@ __global__ __launch_bounds__(PANEL_WAVES * 64) __attribute__((amdgpu_waves_per_e
 #pragma unroll
     for (int j = 0; j < QN; ++j) {
       const int q = j * PANEL_WAVES + wave;
+      if (LOADS % PANEL_WAVES != 0 && q >= LOADS) break;
       const int part = q / (4 * RG), rb = q % (4 * RG);
       const int row = rb * 4 + (lane >> 4);
       const int piece = (lane & 15) ^ (row & 15);
@@ -2985,6 +2986,92 @@ static int launch_gemm_panel(const GemmArgs& a, int unit0, int unit1, hipStream_
   return PTA_OK;
 }
 
+// Formats with a form of gemm_block_kernel
+template <class Fmt> struct BlockFormat { static constexpr bool ok = false; };
+// Formats whose launches of more than 128 rows gemm_panel_kernel takes (those without a form of gemm_block_kernel)
+template <class Fmt> struct PanelFormat { static constexpr bool ok = Fmt::kVec <= 2 && !BlockFormat<Fmt>::ok; };
+
+// A launch of gemm_panel_kernel: row groups of a tile, parts of K inside a workgroup, slices of workgroups; and those of the channel groups beyond
+// the first `whole` (0: all alike).
+struct PanelPlan { int rg, kh, slices, whole, rest_rg, rest_kh; double us; };
+// the tiles there are (F152 not with 128 rows: their decoding's registers spill)
+constexpr int PANEL_TILES[][2] = {{8, 1}, {7, 1}, {6, 1}, {5, 1}, {8, 2}, {7, 2}, {6, 2}, {5, 2}, {4, 2}, {5, 4}, {4, 4}, {3, 4}};
+
+// How a launch is cut: the tile, and the slices of K (one matrix, a workspace at hand), that come out shortest, or tiles of one kind for the whole rounds and
+// another kind for the rest.  What bounds most launches is that a wave goes through its part of K alone, tile by tile: the step of 128 features of 8 waves
+// takes what its products and its decoding take one after the other, whether the other compute units have work or not.  So fewer rows a tile and more parts
+// of K make a launch of few tiles shorter, and one of several rounds where these come out even.  us of a step and of a tile's begin and end (INT4, weights from
+// HBM): 5 to 8 row groups 1.76 to 2.37 and 6.5, two parts 1.72 (4 groups) to 2.77 and 5.5, four 2.0 (3) to 2.8 and 2.7; up to a quarter more where all
+// compute units work; F152 6.4 a step more.  For 130 shapes (1024 to 11008 channels, 130 to 2000 rows), each measured with all of them, the plan's is within 2 % of the best
+// in all but one (4.5 %).  us with 128 rows and one or two parts only, and now: INT4, three of 4096 x 4096, 160 rows 49 -> 28, 1000 rows 90 -> 85; 8192 x 6144, 256 rows 93 -> 42;
+// pair of 2048 x 5632, 400 rows 28.8 -> 22.3; 4096 x 4096 with scratch, 500 rows 37 -> 23, 1000 rows 50 -> 36; pair of 4096 x 11008, 320 rows 83 -> 64; F152, 8192 x 6144, 160 rows 480 -> 134.
+template <class Fmt, bool PAIR>
+static PanelPlan plan_gemm_panel(const GemmArgs& a, int total_nb) {
+  constexpr bool F152 = OwnStreams<Fmt>::long_decode;
+  constexpr double NORM = 7.0;       // the norm launch whose place the adding of slices takes: who gives scratch has one behind the product (11008 x 4096, 1000 rows, both: 93 us, whole 94)
+  const int cus = device_compute_units(), all = PAIR ? total_nb / 2 : total_nb / 4;
+  auto time = [&](int rg, int kh, int slices, int units) {
+    const double step = (F152 ? 6.4 : 0.0) + (kh == 1 ? 0.7 + 0.21 * rg : kh == 2 ? 0.68 + 0.26 * rg : 0.83 + 0.39 * rg), ends = kh == 1 ? 6.5 : kh == 2 ? 5.5 : 2.7;
+    // (each die its share of a slice's tiles: 84 tiles in three slices are 33 for the 32 compute units of most, and twice as long, 53 us against 35)
+    const int cw = PANEL_WAVES / kh, tiles = ((units + cw - 1) / cw * ((a.M + rg * 16 - 1) / (rg * 16)) + 7) / 8 * 8 * slices;
+    const double last = (double)(tiles % cus) / cus, load = 0.03 * rg;
+    const double one = ends + ((a.KT + slices - 1) / slices + kh - 1) / kh * step;
+    return one * (tiles / cus * (1.0 + load) + (last > 0.0 ? 1.0 + load * last * last : 0.0)) + (slices > 1 ? 3.0 + (double)a.M * a.mat[0].N * (4.0 * slices + 6.0) / 5.5e6 - NORM : 0.0);
+  };
+  PanelPlan best{F152 ? 7 : 8, 1, 1, 0, 0, 0, 1e30};
+  for (const auto& t : PANEL_TILES) {
+    if (F152 && t[0] == 8) continue;
+    for (int slices = 1; slices <= (!PAIR && a.count == 1 && a.part ? GEMM_MAX_KSPLIT : 1); ++slices) {
+      if (t[1] * slices > 1 && a.KT < t[1] * slices * 4) break;
+      if (slices > 1 && a.part_bytes < (size_t)slices * a.M * a.mat[0].N * sizeof(float)) break;
+      const double us = time(t[0], t[1], slices, all);
+      if (us < best.us) best = PanelPlan{t[0], t[1], slices, 0, 0, 0, us};
+    }
+    if (t[1] > 1) continue;
+    const int groups = (all + PANEL_WAVES - 1) / PANEL_WAVES, row_blocks = (a.M + t[0] * 16 - 1) / (t[0] * 16), whole = groups * row_blocks / cus * cus / row_blocks;
+    if (whole == 0 || whole >= groups) continue;
+    const double first = time(t[0], 1, 1, whole * PANEL_WAVES);
+    for (const auto& r : PANEL_TILES) {
+      if ((F152 && r[0] == 8) || (r[1] > 1 && a.KT < r[1] * 4)) continue;
+      const double us = first + time(r[0], r[1], 1, all - whole * PANEL_WAVES) + 1.0;
+      if (us < best.us) best = PanelPlan{t[0], 1, 1, whole, r[0], r[1], us};
+    }
+  }
+  return best;
+}
+
+template <class Fmt, bool PAIR>
+static int launch_gemm_panel_plan(const GemmArgs& a, const PanelPlan& p, int total_nb, hipStream_t s, const char* name) {
+  const int units = PAIR ? total_nb / 2 : total_nb / 4;
+  GemmArgs b = a;
+  b.ksplit = p.slices;
+  auto launch = [&](int rg, int kh, int unit0, int unit1) {
+    switch (rg * 10 + kh) {
+      case 71: return launch_gemm_panel<Fmt, 4, 7, 1, PAIR>(b, unit0, unit1, s, name);
+      case 61: return launch_gemm_panel<Fmt, 4, 6, 1, PAIR>(b, unit0, unit1, s, name);
+      case 51: return launch_gemm_panel<Fmt, 4, 5, 1, PAIR>(b, unit0, unit1, s, name);
+      case 72: return launch_gemm_panel<Fmt, 4, 7, 2, PAIR>(b, unit0, unit1, s, name);
+      case 62: return launch_gemm_panel<Fmt, 4, 6, 2, PAIR>(b, unit0, unit1, s, name);
+      case 52: return launch_gemm_panel<Fmt, 4, 5, 2, PAIR>(b, unit0, unit1, s, name);
+      case 42: return launch_gemm_panel<Fmt, 4, 4, 2, PAIR>(b, unit0, unit1, s, name);
+      case 54: return launch_gemm_panel<Fmt, 4, 5, 4, PAIR>(b, unit0, unit1, s, name);
+      case 44: return launch_gemm_panel<Fmt, 4, 4, 4, PAIR>(b, unit0, unit1, s, name);
+      case 34: return launch_gemm_panel<Fmt, 4, 3, 4, PAIR>(b, unit0, unit1, s, name);
+      default: break;
+    }
+    if constexpr (!OwnStreams<Fmt>::long_decode) {
+      if (rg == 8) return kh == 1 ? launch_gemm_panel<Fmt, 4, 8, 1, PAIR>(b, unit0, unit1, s, name) : launch_gemm_panel<Fmt, 4, 8, 2, PAIR>(b, unit0, unit1, s, name);
+    }
+    pta_set_error("%s: no tile of %d rows and %d parts", name, rg * 16, kh);
+    return (int)PTA_EINVAL;
+  };
+  int rc = launch(p.rg, p.kh, 0, p.whole ? p.whole * PANEL_WAVES : units);
+  if (!rc && p.whole) rc = launch(p.rest_rg, p.rest_kh, p.whole * PANEL_WAVES, units);
+  if (rc) return rc;
+  PTA_CHECK_LAUNCH(name);
+  return PTA_OK;
+}
+
 template <class Fmt, int MT, bool PAIR>
 static int launch_gemm_own_for(const GemmArgs& a, int nb, hipStream_t s, const char* name) {
   constexpr int CAP = own_cap<Fmt, PAIR>(MT);
@@ -3122,8 +3209,6 @@ static int rows_in_turn(const GemmArgs& a, int chunk, int total_nb, hipStream_t 
   return PTA_OK;
 }
 
-template <class Fmt> struct BlockFormat { static constexpr bool ok = false; };
-
 // More than 128 rows, 16-bit weights: whether one round of gemm_rows_kernel's workgroups (128 rows, and half the channels of
 // gemm_block_kernel's) is the faster launch.  gemm_block_kernel's time follows the rows that its blocks hold, gemm_rows_kernel's does not,
 // and with few tiles half the chip has none; a single weight's K can be split instead, a pair's cannot.  Ratios gemm_block_kernel to
@@ -3167,10 +3252,15 @@ static int dispatch_many_rows(const GemmArgs& a, int total_nb, hipStream_t s, co
   // 26.8 against 21.3; pair 768 x 11008, three, 17.7 against 13.7; bf16 256 x 11008, 65 rows, two, 1.14 times; 512 x 4096, 1000 rows, four,
   // 1.14 times; 1024 x 6144, 768 rows, five, 1.10.  And 16-bit weights of long K, two rounds: 8192 x 8192, 65 to 128 rows, 1.08 to 1.18 times,
   // 11008 x 8192 1.2 to 1.34 (4096 x 8192 0.83 to 0.97).
+  PanelPlan panel;
+  const bool paneled = PanelFormat<Fmt>::ok && a.M > 128 && panel_fits(a, 4, PAIR);
+  if (paneled) panel = plan_gemm_panel<Fmt, PAIR>(a, total_nb);
   if (a.epi.norm == PTA_NORM_NONE) {
     const OwnPlan plan = plan_gemm_own<Fmt, PAIR>(a);
     const int most = a.M <= 128 ? ((Fmt::kWide && a.KT <= 2) || (Fmt::kVec > 2 && a.KT >= 56) ? 1 : Fmt::kVec == 1 && a.KT >= 12 ? 3 : 2) : a.KT >= 8 || PAIR ? 4 : 3;
-    if (plan.rounds == 1 || (plan.rounds <= most && (a.M <= 128 || plan.us <= (Fmt::kVec == 1 ? 22.0 : 11.0))))
+    // (a round after the first begins with nothing on its way: 3.6 us more than the plan says; 768 rows of three 1024 x 1024 21.5 against gemm_panel_kernel's 20.8,
+    // 1200 rows 27.8 against 21.3, the pair of 1024 x 2816, 640 rows 25.1 against 20.4; two rounds, and short K, stay)
+    if (plan.rounds == 1 || (plan.rounds <= most && (a.M <= 128 || plan.us <= (Fmt::kVec == 1 ? 22.0 : 11.0)) && !(paneled && a.KT >= 8 && plan.rounds > 2 && plan.us + 3.6 * (plan.rounds - 1) > 1.2 * panel.us)))
       return launch_gemm_own_plan<Fmt, PAIR>(a, plan, s, name);
   }
   const int cus = device_compute_units();
@@ -3189,35 +3279,8 @@ static int dispatch_many_rows(const GemmArgs& a, int total_nb, hipStream_t s, co
     if (a.M > 128 && a.epi.norm == PTA_NORM_NONE && !(tiles && rows_before_blocks<Fmt, PAIR>(a, total_nb, cus)))
       return dispatch_gemm_block<typename BlockFormat<Fmt>::type, PAIR>(a, s, name);
   }
-  if constexpr (Fmt::kVec <= 2 && !BlockFormat<Fmt>::ok) {
-    if (a.M > 128 && panel_fits(a, 4, PAIR)) {
-      const int units = PAIR ? total_nb / 2 : total_nb / 4;
-      const int row_blocks = (a.M + 127) / 128;
-      // few workgroup tiles (4096 channels: 8 per row block): K in halves inside the workgroup, tiles of half the channels
-      const int groups = (units + 7) / 8, tiles_all = groups * row_blocks;
-      const bool halves = tiles_all * 2 <= cus && a.KT >= 16;
-      const int wgs = ((units + (halves ? 3 : 7)) / (halves ? 4 : 8)) * row_blocks;
-      GemmArgs b = a;
-      int nsl = wgs > 0 ? cus / wgs : 1;
-      nsl = nsl > GEMM_MAX_KSPLIT ? GEMM_MAX_KSPLIT : nsl;
-      while (nsl > 1 && a.KT < nsl * 16) --nsl;
-      if (!PAIR && a.count == 1 && a.part && nsl > 1 && a.part_bytes >= (size_t)nsl * a.M * a.mat[0].N * sizeof(float)) b.ksplit = nsl;
-      // More tiles than compute units and a last round that fills at most half of them (344 tiles are 1.34 rounds
-      // of 256 and would take 2): the channel groups of the whole rounds in one launch, the rest with K in halves -
-      // twice the workgroups, each half as long.
-      const int whole = (tiles_all / cus) * cus / row_blocks;             // channel groups within the whole rounds
-      const int rest = (groups - whole) * row_blocks;
-      int rc;
-      if (!halves && whole > 0 && rest > 0 && rest * 2 <= cus && a.KT >= 16 && b.ksplit <= 1) {
-        rc = launch_gemm_panel<Fmt, 4, 8, 1, PAIR>(b, 0, whole * 8, s, name);
-        if (!rc) rc = launch_gemm_panel<Fmt, 4, 8, 2, PAIR>(b, whole * 8, units, s, name);
-      } else {
-        rc = halves ? launch_gemm_panel<Fmt, 4, 8, 2, PAIR>(b, 0, units, s, name) : launch_gemm_panel<Fmt, 4, 8, 1, PAIR>(b, 0, units, s, name);
-      }
-      if (rc) return rc;
-      PTA_CHECK_LAUNCH(name);
-      return PTA_OK;
-    }
+  if constexpr (PanelFormat<Fmt>::ok) {
+    if (paneled) return launch_gemm_panel_plan<Fmt, PAIR>(a, panel, total_nb, s, name);
   }
   if (tiles) {
     // fragments in registers, weights through LDS: 256 rows per workgroup where that still fills the machine,

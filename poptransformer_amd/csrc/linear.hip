@@ -10,6 +10,7 @@
 
 int f8_decode_unscaled_launch(const uint8_t* in, f16* out, size_t n, int format, hipStream_t s);
 int run_linear_f143_plain(GemmArgs& a, int total_nb, int swiglu, hipStream_t s, const char* name);      // linear_f143_plain.hip
+int run_linear_f152(GemmArgs& a, int total_nb, int swiglu, hipStream_t s, const char* name);            // linear_f152.hip
 
 template <class Fmt>
 static int run_linear(GemmArgs& a, int total_nb, int swiglu, hipStream_t s, const char* name) {
@@ -124,7 +125,7 @@ static int linear_impl(const void* X, const int32_t* x_scale, int x_bytes, int c
     case PTA_W_INT4: return run_linear<FmtW4>(a, nb, swiglu, s, "pta_linear");
     case PTA_W_F16: return run_linear<FmtF16>(a, nb, swiglu, s, "pta_linear");
     case PTA_W_F143: return plain ? run_linear_f143_plain(a, nb, swiglu, s, "pta_linear") : run_linear<FmtF8<0>>(a, nb, swiglu, s, "pta_linear");
-    default: return run_linear<FmtF8<1>>(a, nb, swiglu, s, "pta_linear");
+    default: return run_linear_f152(a, nb, swiglu, s, "pta_linear");
   }
 }
 
