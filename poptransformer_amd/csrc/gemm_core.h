@@ -2374,6 +2374,8 @@ __device__ __forceinline__ void panel_store(const GemmMat& mat, const GemmEpilog
 // PAIR: a wave owns NST / 2 gate blocks and the same blocks of the up weight.
 // ------------------------------------------------------------------------------------------
 constexpr int PANEL_WAVES = 8;
+// units of `blocks` channel blocks of a matrix, the last one's perhaps fewer
+constexpr int panel_units(int N, int blocks) { return ((N + 15) / 16 + blocks - 1) / blocks; }
 
 // RG: row groups of 16 per workgroup (every wave multiplies all of them); KH: parts of K inside the workgroup - the
 // waves are 8 / KH channel units x KH parts, part kh takes the feature tiles kh, kh + KH, ... of the workgroup's
@@ -2414,31 +2416,34 @@ __global__ __launch_bounds__(PANEL_WAVES * 64) __attribute__((amdgpu_waves_per_e
   // last unit only help with the rows
   const int wu = unit0 + group * CW + cw;
   const bool active = wu < units;
-  const int gb = (active ? wu : 0) * (PAIR ? NST / 2 : NST);      // first block (of the launch; of the pair's matrices)
-  int mi = 0;
+  constexpr int NBW = PAIR ? NST / 2 : NST;                        // consecutive blocks of a unit
+  int mi = 0, unit = active ? wu : 0;
   if (!PAIR) {
 #pragma unroll
-    for (int i = 1; i < 4; ++i)
-      if (i < a.count && gb >= a.mat[i].nb_begin) mi = i;
+    for (int i = 0; i < 3; ++i) {
+      const int there = panel_units(a.mat[i].N, NBW);
+      if (mi == i && i + 1 < a.count && unit >= there) unit -= there, mi = i + 1;
+    }
   }
-  const int blk0 = PAIR ? gb : gb - a.mat[mi].nb_begin;           // first block within its matrix
+  const int blk0 = unit * NBW;                                    // first block within its matrix
+  const int have = (a.mat[mi].N + 15) / 16 - blk0;                // blocks from there on (at least one)
   // Loads through buffer descriptors: the descriptor and the tile's offset travel in scalar registers and one
   // 32-bit offset per lane serves all streams, another all rows (with 64-bit addresses per lane the loop keeps a
   // pointer per stream and row in vector registers, which this kernel does not have).  Rows past M lie past
   // the end of the rows' descriptor and read as zero.
-  constexpr int NBW = PAIR ? NST / 2 : NST;                        // consecutive blocks behind one descriptor
   const uint32_t blk_bytes = (uint32_t)a.KT * (KV * 1024);
   const unsigned char* w0 = reinterpret_cast<const unsigned char*>(a.mat[PAIR ? 0 : mi].tiled) + (size_t)blk0 * blk_bytes;
   const unsigned char* w1 = reinterpret_cast<const unsigned char*>(a.mat[PAIR ? 1 : mi].tiled) + (size_t)blk0 * blk_bytes;
-  const __amdgpu_buffer_rsrc_t wr0 = __builtin_amdgcn_make_buffer_rsrc(const_cast<unsigned char*>(w0), 0, (int)(NBW * blk_bytes), 0x00020000);
-  const __amdgpu_buffer_rsrc_t wr1 = __builtin_amdgcn_make_buffer_rsrc(const_cast<unsigned char*>(w1), 0, (int)(NBW * blk_bytes), 0x00020000);
+  const __amdgpu_buffer_rsrc_t wr0 = __builtin_amdgcn_make_buffer_rsrc(const_cast<unsigned char*>(w0), 0, (int)((have < NBW ? have : NBW) * blk_bytes), 0x00020000);
+  const __amdgpu_buffer_rsrc_t wr1 = __builtin_amdgcn_make_buffer_rsrc(const_cast<unsigned char*>(w1), 0, (int)((have < NBW ? have : NBW) * blk_bytes), 0x00020000);
   const int wlane = lane * 16;
   const int row0 = row_block * ROWS;
   const int rows_here = M - row0 < ROWS ? M - row0 : ROWS;
   const __amdgpu_buffer_rsrc_t xr0 = __builtin_amdgcn_make_buffer_rsrc(
       const_cast<f16*>(a.X + (size_t)row0 * K), 0, (int)((size_t)rows_here * K * 2), 0x00020000);
 
-  // this wave's weight tiles of step i (past the end of the range: zeros - the rows of that tile are zeros too)
+  // this wave's weight tiles of step i (past the end of the range: zeros - the rows of that tile are zeros too; past the matrix's last block: that one again,
+  // whose sums go nowhere)
   auto fetch_w = [&](int i, u32x4 (&wv)[NST][KV]) {
     const int kt = kt_first + i * KH + kh;
 #pragma unroll
@@ -2446,7 +2451,7 @@ __global__ __launch_bounds__(PANEL_WAVES * 64) __attribute__((amdgpu_waves_per_e
 #pragma unroll
       for (int v = 0; v < KV; ++v)
         wv[st][v] = kt < kt_end ? __builtin_amdgcn_raw_buffer_load_b128(PAIR && st >= NST / 2 ? wr1 : wr0, wlane,
-                                      (int)((PAIR ? st % (NST / 2) : st) * blk_bytes + (uint32_t)(kt * KV + v) * 1024), 0)
+                                      (int)((st % NBW < have ? st % NBW : have - 1) * blk_bytes + (uint32_t)(kt * KV + v) * 1024), 0)
                                 : u32x4{0, 0, 0, 0};
   };
   // The rows go from memory into LDS without passing through registers: load q = 8 j + w (w: the wave) of a stage
@@ -2962,6 +2967,23 @@ static inline bool panel_fits(const GemmArgs& a, int nst, bool pair) {
   return true;
 }
 
+// gemm_panel_kernel's launches: panel_fits, and channels that do not divide into its units, up to 24576 a matrix (a head has more, but is asked for few
+// rows; those of more than 128 go 64 rows at a time, as these did: INT4, 1964 rows, 6336 x 1296 383 -> 50 us, 662 rows, three of 2304 x 1264 85 -> 22).
+static inline bool panel_takes(const GemmArgs& a, bool pair) {
+  if (panel_fits(a, 4, pair)) return true;
+  if (a.epi.norm != PTA_NORM_NONE || a.KT < 2) return false;
+  for (int i = 0; i < (pair ? 1 : a.count); ++i)
+    if (a.mat[i].N > 24576 || (!pair && a.mat[i].X && a.mat[i].X != a.X)) return false;
+  return true;
+}
+
+static inline int panel_units(const GemmArgs& a, bool pair) {
+  if (pair) return panel_units(a.mat[0].N, 2);
+  int n = 0;
+  for (int i = 0; i < a.count; ++i) n += panel_units(a.mat[i].N, 4);
+  return n;
+}
+
 // units [unit0, unit1) of the launch's matrices (a unit: NST channel blocks, or NST / 2 gate and up blocks)
 template <class Fmt, int NST, int RG, int KH, bool PAIR>
 static int launch_gemm_panel(const GemmArgs& a, int unit0, int unit1, hipStream_t s, const char* name) {
@@ -3006,10 +3028,10 @@ constexpr int PANEL_TILES[][2] = {{8, 1}, {7, 1}, {6, 1}, {5, 1}, {8, 2}, {7, 2}
 // in all but one (4.5 %).  us with 128 rows and one or two parts only, and now: INT4, three of 4096 x 4096, 160 rows 49 -> 28, 1000 rows 90 -> 85; 8192 x 6144, 256 rows 93 -> 42;
 // pair of 2048 x 5632, 400 rows 28.8 -> 22.3; 4096 x 4096 with scratch, 500 rows 37 -> 23, 1000 rows 50 -> 36; pair of 4096 x 11008, 320 rows 83 -> 64; F152, 8192 x 6144, 160 rows 480 -> 134.
 template <class Fmt, bool PAIR>
-static PanelPlan plan_gemm_panel(const GemmArgs& a, int total_nb) {
+static PanelPlan plan_gemm_panel(const GemmArgs& a) {
   constexpr bool F152 = OwnStreams<Fmt>::long_decode;
   constexpr double NORM = 7.0;       // the norm launch whose place the adding of slices takes: who gives scratch has one behind the product (11008 x 4096, 1000 rows, both: 93 us, whole 94)
-  const int cus = device_compute_units(), all = PAIR ? total_nb / 2 : total_nb / 4;
+  const int cus = device_compute_units(), all = panel_units(a, PAIR);
   auto time = [&](int rg, int kh, int slices, int units) {
     const double step = (F152 ? 6.4 : 0.0) + (kh == 1 ? 0.7 + 0.21 * rg : kh == 2 ? 0.68 + 0.26 * rg : 0.83 + 0.39 * rg), ends = kh == 1 ? 6.5 : kh == 2 ? 5.5 : 2.7;
     // (each die its share of a slice's tiles: 84 tiles in three slices are 33 for the 32 compute units of most, and twice as long, 53 us against 35)
@@ -3041,8 +3063,8 @@ static PanelPlan plan_gemm_panel(const GemmArgs& a, int total_nb) {
 }
 
 template <class Fmt, bool PAIR>
-static int launch_gemm_panel_plan(const GemmArgs& a, const PanelPlan& p, int total_nb, hipStream_t s, const char* name) {
-  const int units = PAIR ? total_nb / 2 : total_nb / 4;
+static int launch_gemm_panel_plan(const GemmArgs& a, const PanelPlan& p, hipStream_t s, const char* name) {
+  const int units = panel_units(a, PAIR);
   GemmArgs b = a;
   b.ksplit = p.slices;
   auto launch = [&](int rg, int kh, int unit0, int unit1) {
@@ -3253,8 +3275,8 @@ static int dispatch_many_rows(const GemmArgs& a, int total_nb, hipStream_t s, co
   // 1.14 times; 1024 x 6144, 768 rows, five, 1.10.  And 16-bit weights of long K, two rounds: 8192 x 8192, 65 to 128 rows, 1.08 to 1.18 times,
   // 11008 x 8192 1.2 to 1.34 (4096 x 8192 0.83 to 0.97).
   PanelPlan panel;
-  const bool paneled = PanelFormat<Fmt>::ok && a.M > 128 && panel_fits(a, 4, PAIR);
-  if (paneled) panel = plan_gemm_panel<Fmt, PAIR>(a, total_nb);
+  const bool paneled = PanelFormat<Fmt>::ok && a.M > 128 && panel_takes(a, PAIR);
+  if (paneled) panel = plan_gemm_panel<Fmt, PAIR>(a);
   if (a.epi.norm == PTA_NORM_NONE) {
     const OwnPlan plan = plan_gemm_own<Fmt, PAIR>(a);
     const int most = a.M <= 128 ? ((Fmt::kWide && a.KT <= 2) || (Fmt::kVec > 2 && a.KT >= 56) ? 1 : Fmt::kVec == 1 && a.KT >= 12 ? 3 : 2) : a.KT >= 8 || PAIR ? 4 : 3;
@@ -3280,7 +3302,7 @@ static int dispatch_many_rows(const GemmArgs& a, int total_nb, hipStream_t s, co
       return dispatch_gemm_block<typename BlockFormat<Fmt>::type, PAIR>(a, s, name);
   }
   if constexpr (PanelFormat<Fmt>::ok) {
-    if (paneled) return launch_gemm_panel_plan<Fmt, PAIR>(a, panel, total_nb, s, name);
+    if (paneled) return launch_gemm_panel_plan<Fmt, PAIR>(a, panel, s, name);
   }
   if (tiles) {
     // fragments in registers, weights through LDS: 256 rows per workgroup where that still fills the machine,

@@ -1,5 +1,5 @@
 """Products of more than 128 rows by INT4 and F152 weights (gemm_panel_kernel) against float64: every tile of 48 to 128 rows with one, two and four parts of K,
-slices of workgroups, and tiles of two kinds in one product."""
+slices of workgroups, and tiles of two kinds in one product; channels of any number."""
 import pytest
 import torch
 
@@ -19,8 +19,8 @@ def weight(kind, N, Kd, g):
 
 
 # features, channels, form; rows: one past 128, tiles that rows fill and that they do not, one round and several
-SHAPES = {"int4": [(4096, 6144, "one"), (2056, 4096, "scratch"), (11008, 1024, "scratch"), (1032, 5632, "pair"), (520, 2048, "three"), (4104, 11008, "pair"), (8192, 6144, "one")],
-          "F152": [(4096, 2048, "one"), (2056, 4096, "pair"), (8200, 1024, "scratch")]}
+SHAPES = {"int4": [(4096, 6144, "one"), (2056, 4096, "scratch"), (11008, 1024, "scratch"), (1032, 5632, "pair"), (520, 2048, "three"), (4104, 11008, "pair"), (8192, 6144, "one"), (4096, 1000, "one"), (1032, 50, "three"), (2048, 1303, "scratch"), (4104, 1297, "pair"), (2048, 2088, "three")],
+          "F152": [(4096, 2048, "one"), (2056, 4096, "pair"), (8200, 1024, "scratch"), (1032, 1111, "pair")]}
 
 
 @pytest.mark.parametrize("M", [129, 145, 200, 333, 470, 640, 900, 1201])
