@@ -3158,6 +3158,20 @@ static int launch_gemm_own_plan(const GemmArgs& a, const OwnPlan& p, hipStream_t
   return PTA_OK;
 }
 
+// 33 to 128 rows by INT4 weights, several rounds of gemm_own_kernel: gemm_panel_kernel, if its plan is that much shorter (both plans' us a little long, the
+// latter's begin with nothing on its way).  K of more than 2048.  us, gemm_own_kernel and it, weights from HBM: three of 4096 x 4096, 65 rows 24.0 and 20.6, 128
+// rows 28.1 and 24.9; pair of 4096 x 11008, 48 rows 25.4 and 22.5, 64 rows 29.3 and 25.8, 128 rows 42.3 and 36.3 (96 rows 35.7 and 36.0, plans 42.7 and 34.9);
+// 4096 x 11008, 65 rows 21.3 and 20.2.
+template <class Fmt, bool PAIR>
+static bool panel_before_own(const GemmArgs& a, const OwnPlan& own, PanelPlan& panel) {
+  if constexpr (PanelFormat<Fmt>::ok && Fmt::kVec == 1) {
+    if (a.M <= 32 || a.KT <= 16 || own.rounds < 2 || !panel_takes(a, PAIR)) return false;
+    panel = plan_gemm_panel<Fmt, PAIR>(a);
+    return panel.us < 0.8 * own.us;
+  }
+  return false;
+}
+
 // whether the launch fits gemm_tile_kernel with `per_wg` channel blocks per workgroup: every matrix
 // a whole number of workgroups, enough feature tiles for the K groups
 static inline bool tile_fits(const GemmArgs& a, int per_wg, int kq, bool pair) {
@@ -3282,8 +3296,12 @@ static int dispatch_many_rows(const GemmArgs& a, int total_nb, hipStream_t s, co
     const int most = a.M <= 128 ? ((Fmt::kWide && a.KT <= 2) || (Fmt::kVec > 2 && a.KT >= 56) ? 1 : Fmt::kVec == 1 && a.KT >= 12 ? 3 : 2) : a.KT >= 8 || PAIR ? 4 : 3;
     // (a round after the first begins with nothing on its way: 3.6 us more than the plan says; 768 rows of three 1024 x 1024 21.5 against gemm_panel_kernel's 20.8,
     // 1200 rows 27.8 against 21.3, the pair of 1024 x 2816, 640 rows 25.1 against 20.4; two rounds, and short K, stay)
-    if (plan.rounds == 1 || (plan.rounds <= most && (a.M <= 128 || plan.us <= (Fmt::kVec == 1 ? 22.0 : 11.0)) && !(paneled && a.KT >= 8 && plan.rounds > 2 && plan.us + 3.6 * (plan.rounds - 1) > 1.2 * panel.us)))
-      return launch_gemm_own_plan<Fmt, PAIR>(a, plan, s, name);
+    bool own = plan.rounds == 1 || (plan.rounds <= most && (a.M <= 128 || plan.us <= (Fmt::kVec == 1 ? 22.0 : 11.0)));
+    if (own && a.M > 128) own = !(paneled && a.KT >= 8 && plan.rounds > 2 && plan.us + 3.6 * (plan.rounds - 1) > 1.2 * panel.us);
+    if constexpr (PanelFormat<Fmt>::ok) {
+      if (own && a.M <= 128 && panel_before_own<Fmt, PAIR>(a, plan, panel)) return launch_gemm_panel_plan<Fmt, PAIR>(a, panel, s, name);
+    }
+    if (own) return launch_gemm_own_plan<Fmt, PAIR>(a, plan, s, name);
   }
   const int cus = device_compute_units();
   const int per_wg = PAIR ? 4 : 8;
@@ -3426,6 +3444,10 @@ static int dispatch_gemv(const GemmArgs& a, int total_nb, hipStream_t s, const c
           PTA_CHECK_LAUNCH(name);
           return PTA_OK;
         }
+      }
+      if constexpr (PanelFormat<Fmt>::ok) {
+        PanelPlan panel;
+        if (own && panel_before_own<Fmt, PAIR>(a, plan, panel)) return launch_gemm_panel_plan<Fmt, PAIR>(a, panel, s, name);
       }
       if (own) return launch_gemm_own_plan<Fmt, PAIR>(a, plan, s, name);
       int rc = 1;

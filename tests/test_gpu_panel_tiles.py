@@ -1,4 +1,4 @@
-"""Products of more than 128 rows by INT4 and F152 weights (gemm_panel_kernel) against float64: every tile of 48 to 128 rows with one, two and four parts of K,
+"""Products of 33 rows and more by INT4 and F152 weights (gemm_panel_kernel) against float64: every tile of 48 to 128 rows with one, two and four parts of K,
 slices of workgroups, and tiles of two kinds in one product; channels of any number."""
 import pytest
 import torch
@@ -23,7 +23,7 @@ SHAPES = {"int4": [(4096, 6144, "one"), (2056, 4096, "scratch"), (11008, 1024, "
           "F152": [(4096, 2048, "one"), (2056, 4096, "pair"), (8200, 1024, "scratch"), (1032, 1111, "pair")]}
 
 
-@pytest.mark.parametrize("M", [129, 145, 200, 333, 470, 640, 900, 1201])
+@pytest.mark.parametrize("M", [33, 65, 128, 129, 145, 200, 333, 470, 640, 900, 1201])
 @pytest.mark.parametrize("kind, Kd, N, form", [(k, *s) for k, shapes in SHAPES.items() for s in shapes])
 def test_every_tile(kind, Kd, N, form, M):
     from poptransformer_amd import kernels as K
