@@ -2365,10 +2365,10 @@ __device__ __forceinline__ void panel_store(const GemmMat& mat, const GemmEpilog
 // ------------------------------------------------------------------------------------------
 // Variant for hundreds of rows: the roles turned round.  The tiled weight format IS the A operand order, so a
 // wave fetches the tiles of its own NST channel blocks straight into registers (1 KiB per instruction, no LDS)
-// and decodes them there; the 128 activation rows of the workgroup go through LDS once per 128-feature tile
+// and decodes them there; the RG * 16 activation rows of the workgroup (48 to 128) go through LDS once per 128-feature tile
 // (whole-row loads, double-buffered, one barrier per tile) and every wave reads all of them as B operands.
-// A wave's tile is 128 rows x NST * 16 channels: one B operand read from LDS feeds NST MFMAs and one decoded
-// A operand feeds 8, which is what keeps both LDS (128 bytes per clock and compute unit) and the vector ALU
+// A wave's tile is RG * 16 rows x NST * 16 channels: one B operand read from LDS feeds NST MFMAs and one decoded
+// A operand feeds RG (8 in a launch that fills the chip), which is what keeps both LDS (128 bytes per clock and compute unit) and the vector ALU
 // behind the matrix unit.  (With the weights through LDS and the rows in registers - gemm_rows_kernel - every
 // wave reads every decoded weight: 1 KiB of LDS per 2 MFMAs, more than the LDS delivers.)
 // PAIR: a wave owns NST / 2 gate blocks and the same blocks of the up weight.
@@ -2379,9 +2379,9 @@ constexpr int panel_units(int N, int blocks) { return ((N + 15) / 16 + blocks - 
 
 // RG: row groups of 16 per workgroup (every wave multiplies all of them); KH: parts of K inside the workgroup - the
 // waves are 8 / KH channel units x KH parts, part kh takes the feature tiles kh, kh + KH, ... of the workgroup's
-// range and the parts' sums meet in LDS at the end.  KH > 1 is for launches with few channels: it halves or
+// range and the parts' sums meet in LDS at the end.  KH > 1 is for launches of few tiles: it halves or
 // quarters the channels of a workgroup tile, so more workgroups, without the fp32 round trip through memory that
-// slices of workgroups (ksplit) cost.
+// slices of workgroups (ksplit) cost, and fewer steps for each wave.  plan_gemm_panel chooses.
 template <class Fmt, int NST, int RG, int KH, bool PAIR>
 __global__ __launch_bounds__(PANEL_WAVES * 64) __attribute__((amdgpu_waves_per_eu(2, 2))) void gemm_panel_kernel(GemmArgs a, int groups, int row_blocks, int unit0, int units) {
   constexpr int KV = Fmt::kVec;
@@ -2598,8 +2598,11 @@ constexpr int BLOCK_BAND = 4;               // channel groups that a die's workg
 constexpr int block_row_parts(int rg) { return rg == 2 ? 4 : 2; }
 constexpr int block_rows(int rg) { return block_row_parts(rg) * rg * 16; }
 constexpr int block_cb(int rg) { return 8 / block_row_parts(rg) * 4; }         // channel blocks of a workgroup
-// us of a step of 64 features (measured, all compute units at work), and of a tile's begin and end
-constexpr double block_step_us(int rg) { return rg == 8 ? 1.45 : rg == 6 ? 1.1 : rg == 4 ? 0.84 : 0.55; }
+// us of a step of 64 features (measured, all compute units at work), and of a tile's begin and end.  16-bit weights take 0.88 to 0.92 of theirs, as F143 ones do: these
+// figures are those of stages of 32 features, and stay because slices of K, and with them the order of a product's sums, follow from them.
+constexpr double block_step_us(int rg, bool f143) {
+  return f143 ? (rg == 8 ? 1.45 : rg == 6 ? 1.1 : rg == 4 ? 0.84 : 0.55) : rg == 8 ? 1.6 : rg == 6 ? 1.25 : rg == 4 ? 0.92 : 0.6;
+}
 constexpr double block_ends_us(int rg) { return rg == 8 ? 9.0 : rg == 6 ? 7.5 : rg == 4 ? 6.0 : 5.0; }
 
 // v, of which the compiler no longer knows where it is from
@@ -2916,7 +2919,7 @@ static int dispatch_gemm_block(const GemmArgs& a, hipStream_t s, const char* nam
   auto blocks = [&](int rg) { return (a.M + block_rows(rg) - 1) / block_rows(rg); };
   auto cost = [&](int rg, int tiles, int nsl) {
     const double finish = nsl > 1 ? 5.0 + (double)a.M * a.mat[0].N * (4.0 * nsl + 6.0) / 4.5e6 : 0.0;
-    return ((tiles * nsl + cus - 1) / cus) * (block_step_us(rg) * steps / nsl + block_ends_us(rg)) + finish;
+    return ((tiles * nsl + cus - 1) / cus) * (block_step_us(rg, Fmt::kVec == 2) * steps / nsl + block_ends_us(rg)) + finish;
   };
   const int whole = (groups * blocks(8) / cus) * cus / blocks(8);               // channel groups within whole rounds
   double best = cost(8, groups * blocks(8), 1);
@@ -3030,7 +3033,9 @@ constexpr int PANEL_TILES[][2] = {{8, 1}, {7, 1}, {6, 1}, {5, 1}, {8, 2}, {7, 2}
 template <class Fmt, bool PAIR>
 static PanelPlan plan_gemm_panel(const GemmArgs& a) {
   constexpr bool F152 = OwnStreams<Fmt>::long_decode;
-  constexpr double NORM = 7.0;       // the norm launch whose place the adding of slices takes: who gives scratch has one behind the product (11008 x 4096, 1000 rows, both: 93 us, whole 94)
+  // The norm launch whose place the adding of slices takes: who gives scratch has one behind the product (11008 x 4096: 1000 rows, the two together 93 us in slices and
+  // 94 whole; 2000 rows 162 and 146 without the norm)
+  constexpr double NORM = 4.3;
   const int cus = device_compute_units(), all = panel_units(a, PAIR);
   auto time = [&](int rg, int kh, int slices, int units) {
     const double step = (F152 ? 6.4 : 0.0) + (kh == 1 ? 0.7 + 0.21 * rg : kh == 2 ? 0.68 + 0.26 * rg : 0.83 + 0.39 * rg), ends = kh == 1 ? 6.5 : kh == 2 ? 5.5 : 2.7;
