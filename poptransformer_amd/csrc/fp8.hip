@@ -106,7 +106,10 @@ __global__ __launch_bounds__(256) void f8_tile_kernel(const uint8_t* __restrict_
 __global__ __launch_bounds__(64) void f8_tile_flags_kernel(const u32x4* __restrict__ tiled, uint8_t* __restrict__ flags,
                                                            size_t tiles) {
   const size_t tile = blockIdx.x;
-  if (tile >= tiles) return;
+  if (tile >= tiles) {                            // (the flags end with a whole 16 bytes, which are read a word at a time)
+    if (threadIdx.x == 0) flags[tile] = 0;
+    return;
+  }
   bool special = false;
 #pragma unroll
   for (int v = 0; v < 2; ++v) {
@@ -138,7 +141,8 @@ extern "C" int pta_fp8_tile(const uint8_t* w, void* tiled, int N, int K, int w_i
   const size_t total = tile_bytes / 16;
   hipLaunchKernelGGL(f8_tile_kernel, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, (hipStream_t)stream, w,
                      (u32x4*)tiled, N, K, KT, w_is_kn, total);
-  hipLaunchKernelGGL(f8_tile_flags_kernel, dim3((unsigned)(tile_bytes / 2048)), dim3(64), 0, (hipStream_t)stream,
+  const size_t flag_bytes = pta_fp8_tiled_bytes(N, K) - tile_bytes;
+  hipLaunchKernelGGL(f8_tile_flags_kernel, dim3((unsigned)flag_bytes), dim3(64), 0, (hipStream_t)stream,
                      (const u32x4*)tiled, (uint8_t*)tiled + tile_bytes, tile_bytes / 2048);
   PTA_CHECK_LAUNCH("pta_fp8_tile");
   return PTA_OK;

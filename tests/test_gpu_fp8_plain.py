@@ -63,3 +63,17 @@ def test_codes_beyond_the_conversion(rows):
         p = K.fp8_to_half(c, scale()).double()
         ref, mag = x.double() @ p.T, x.double().abs() @ p.abs().T
         assert ((out.double() - ref).abs() <= 2.0 ** -11 * ref.abs() + (Kd + 2) * 2.0 ** -24 * mag + 2.0 ** -24).all()
+
+
+# one tile, a number of tiles that is no multiple of sixteen, one that is
+@pytest.mark.parametrize("N, Kd", [(16, 128), (40, 200), (264, 4104), (256, 1024)])
+def test_every_byte_of_a_tiled_weight_is_written(N, Kd):
+    """What a tiled weight holds is no matter of what its buffer held: kernels read the flags behind the tiles in whole words."""
+    from poptransformer_amd import _lib
+    lib, stream = _lib.load(), torch.cuda.current_stream().cuda_stream
+    codes = torch.randint(1, 120, (N, Kd), dtype=torch.int32, device="cuda").to(torch.uint8)
+    buffers = [torch.full((lib.pta_fp8_tiled_bytes(N, Kd),), fill, dtype=torch.uint8, device="cuda") for fill in (0, 0xFF)]
+    for b in buffers:
+        assert lib.pta_fp8_tile(codes.data_ptr(), b.data_ptr(), N, Kd, 0, stream) == 0
+    assert torch.equal(*buffers)
+    assert not buffers[1][-(-N // 16) * -(-Kd // 128) * 2048:].any()
