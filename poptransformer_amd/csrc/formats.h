@@ -157,15 +157,28 @@ __host__ __device__ inline size_t f8_tile_flags_offset(int N, int K) {
   return (size_t)((N + 15) / 16) * (size_t)((K + 127) / 128) * 2048;
 }
 
-// F143 weights for gemm_block_kernel.  The hardware's conversion knows the bytes as OCP e4m3 numbers, twice the F143 ones of all codes but 0x7F and 0xFF (and 0x80,
-// which both take as a zero here): one instruction for two weights.  What bounds a launch is the vector unit beside the matrix unit, which multiplies
-// two waves' operands a SIMD: with three instructions for two weights, as for blocks of channels with one of those codes, 2048 rows, 8192 x 8192
-// 197 -> 182 us, 13696 x 4096 199 -> 170.
-// Those three: moved to fp16 bits 13..7 with their sign in bit 15 the seven magnitude bits are the
-// fp16 number decode(byte) * 2^-7, subnormals among them, which the matrix unit takes at their value; the sums take the 2^7 at the end.
+// The hardware's conversion of eight F143 bytes to decode(byte) * 2^EXP.  It knows them as OCP e4m3 numbers, twice the F143 ones of all codes but 0x7F and 0xFF
+// (NaN there) and 0x80 (a zero here as there): one instruction for two weights.
+template <int EXP>
+__device__ __forceinline__ f16x8 f143_convert8(u32x2 p) {
+  constexpr float k = EXP == 0 ? 0.5f : 0.5f / 128.0f;
+  static_assert(EXP == 0 || EXP == -7, "the two that are used");
+  typedef f16x2 Four[4];
+  const Four r = {__builtin_amdgcn_cvt_scalef32_pk_f16_fp8(p[0], k, false), __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(p[0], k, true),
+                  __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(p[1], k, false), __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(p[1], k, true)};
+  return f16x8{r[0][0], r[0][1], r[1][0], r[1][1], r[2][0], r[2][1], r[3][0], r[3][1]};
+}
+
+// F143 weights for gemm_block_kernel: operands are decode(byte) * 2^-7, fp16 subnormals among them, which the matrix unit takes at their value, and the sum takes
+// the 2^7 before the scale (one exponent for both would be infinite from 2^121 on, and its product with a sum of zero a NaN).
+// By the hardware's conversion, or, for blocks of channels that hold a code which that does not know, by three instructions for two weights: the seven magnitude bits
+// moved to fp16 bits 13..7 with their sign in bit 15 are that number.  The same operands either way, so that a channel's sums do not follow the codes of those
+// beside it.  (Operands of the numbers themselves are a fourth instruction there, 85 -> 101 us for 300 rows, 8192 x 4096.)
+// What bounds a launch is the vector unit beside the matrix unit, which multiplies two waves' operands a SIMD: with three instructions and with one, 2048 rows,
+// 8192 x 8192 230 and 194, 13696 x 4096 205 and 178 us.
 struct FmtF143Block : FmtF8<0> {
+  static __device__ __forceinline__ float finish(float acc, Scale s) { return acc * 128.0f * s.mul; }
   static constexpr bool kCodes = true;
-  static constexpr float kSlowSum = 128.0f;
   typedef u32x2 Piece;                                       // (a vector holds 64 features of a channel)
   static constexpr int piece_at(int m) { return m * 8; }
   static __device__ __forceinline__ uint32_t pair(uint32_t bytes, uint32_t select) {
@@ -175,12 +188,7 @@ struct FmtF143Block : FmtF8<0> {
   }
   template <bool FAST>
   static __device__ __forceinline__ f16x8 operand(Piece p) {
-    if constexpr (FAST) {
-      typedef f16x2 Four[4];
-      const Four r = {__builtin_amdgcn_cvt_scalef32_pk_f16_fp8(p[0], 0.5f, false), __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(p[0], 0.5f, true),
-                      __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(p[1], 0.5f, false), __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(p[1], 0.5f, true)};
-      return f16x8{r[0][0], r[0][1], r[1][0], r[1][1], r[2][0], r[2][1], r[3][0], r[3][1]};
-    }
+    if constexpr (FAST) return f143_convert8<-7>(p);
     const u32x4 r = {pair(p[0], 0x010C000Cu), pair(p[0], 0x030C020Cu), pair(p[1], 0x010C000Cu), pair(p[1], 0x030C020Cu)};
     return bitcast<f16x8>(r);
   }
@@ -206,18 +214,17 @@ struct FmtF143Block : FmtF8<0> {
 };
 
 
-// F143 weights of which none is 0x7F or 0xFF (PTA_W_F143_PLAIN): every kernel converts as FmtF143Block's faster way does, and no kernel looks at flags.
+// F143 weights of which none is 0x7F, 0xFF or 0x80 (PTA_W_F143_PLAIN): every kernel converts by the hardware, and no kernel looks at flags.
 // Beside f143_decode8's twenty instructions for eight weights, weights from memory, us: pairs of 4096 x 13696, 8 rows 23.5 -> 21.8, 64 rows 37.3 -> 34.9,
 // 128 rows 54.6 -> 49.8; 4096 x 11008, 1 row 11.1 -> 10.4, 8 rows 11.6 -> 10.5, 100 rows 30.1 -> 27.9.  The same numbers.
 struct FmtF143Plain : FmtF8<0> {
-  static constexpr bool kCodes = false;
   static __device__ __forceinline__ f16x8 a_operand(const u32x4 (&raw)[2], int j, Scale) {
-    return FmtF143Block::template operand<true>(u32x2{raw[j >> 1][(j & 1) * 2], raw[j >> 1][(j & 1) * 2 + 1]});
+    return f143_convert8<0>(u32x2{raw[j >> 1][(j & 1) * 2], raw[j >> 1][(j & 1) * 2 + 1]});
   }
-  typedef u32x2 Piece;
-  static constexpr int piece_at(int m) { return m * 8; }
-  template <bool>
-  static __device__ __forceinline__ f16x8 operand(Piece p) { return FmtF143Block::template operand<true>(p); }
+};
+// and for gemm_block_kernel
+struct FmtF143PlainBlock : FmtF143Block {
+  static constexpr bool kCodes = false;
 };
 
 
@@ -245,4 +252,4 @@ template <> struct OwnStreams<FmtF8<1>> { static constexpr int cap = 3; static c
 template <> struct BlockFormat<FmtF16> { static constexpr bool ok = true; typedef FmtF16 type; };
 template <> struct BlockFormat<FmtBF16> { static constexpr bool ok = true; typedef FmtBF16 type; };
 template <> struct BlockFormat<FmtF8<0>> { static constexpr bool ok = true; typedef FmtF143Block type; };
-template <> struct BlockFormat<FmtF143Plain> { static constexpr bool ok = true; typedef FmtF143Plain type; };
+template <> struct BlockFormat<FmtF143Plain> { static constexpr bool ok = true; typedef FmtF143PlainBlock type; };

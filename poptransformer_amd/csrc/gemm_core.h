@@ -2832,12 +2832,6 @@ __global__ __launch_bounds__(BLOCK_WAVES * 64) __attribute__((amdgpu_waves_per_e
   if constexpr (Fmt::kCodes) {
     if (__any(codes != 0)) {
       products(std::false_type{});
-#pragma unroll
-      for (int rg = 0; rg < RG; ++rg)
-#pragma unroll
-        for (int st = 0; st < NST; ++st)
-#pragma unroll
-          for (int r = 0; r < 4; ++r) acc[rg][st][r] *= Fmt::kSlowSum;
     } else {
       products(std::true_type{});
     }

@@ -77,3 +77,25 @@ def test_every_byte_of_a_tiled_weight_is_written(N, Kd):
         assert lib.pta_fp8_tile(codes.data_ptr(), b.data_ptr(), N, Kd, 0, stream) == 0
     assert torch.equal(*buffers)
     assert not buffers[1][-(-N // 16) * -(-Kd // 128) * 2048:].any()
+
+
+@pytest.mark.parametrize("form, M, Kd, N", [("one", 600, 4096, 2048), ("slices", 1500, 13704, 1032), ("pair", 600, 4104, 2048)])
+def test_channels_beside_the_largest_codes(form, M, Kd, N):
+    """A wave of gemm_block_kernel converts all of its channels one way: those beside a code that the hardware's conversion does not know are bit for bit what they
+    are without it, and so is a plain weight in a pair with one that holds such a code.  Weights that are subnormal numbers, which the matrix unit would add with
+    fewer bits if they were multiplied as such."""
+    from poptransformer_amd import kernels as K
+    g = torch.Generator(device="cuda").manual_seed(9)
+    n = 2 if form == "pair" else 1
+    x = (torch.randn((M, Kd), generator=g, device="cuda") * torch.exp2(torch.randint(-6, 4, (M, Kd), generator=g, device="cuda").float())).half()
+    codes = (torch.randint(1, 8, (n, N, Kd), generator=g, device="cuda") | torch.randint(0, 2, (n, N, Kd), generator=g, device="cuda") << 7).to(torch.uint8)
+    marked = codes.clone()
+    marked[-1, ::32, 5] = 0x7F
+    outs = []
+    for c in (codes, marked):
+        out = torch.full((M, N), float("nan"), dtype=torch.float16, device="cuda")
+        K.linear(x, [K.F8Weight(w.contiguous(), scale()) for w in c], [out] * n, swiglu=form == "pair", workspace=K.linear_workspace(M, N, "cuda") if form == "slices" else None)
+        assert K.linear_kernel() == "gemm_block_kernel"
+        outs.append(out)
+    beside = torch.arange(N, device="cuda") % 32 != 0
+    assert torch.equal(outs[0][:, beside], outs[1][:, beside])

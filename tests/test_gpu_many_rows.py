@@ -562,7 +562,7 @@ def test_blocks_of_fp8_channels_with_the_largest_codes(form, M, Kd, N):
         assert K.linear_kernel() == "gemm_block_kernel"
         outs.append(out)
     plain = K.fp8_to_half(marked, scale).double()
-    # a wave's channels, four blocks of a matrix (two of each of a pair's), go one way together, and a neighbour's flags may send more of them there: the same sums
+    # (a wave's channels, four blocks of a matrix or two of each of a pair's, are converted one way together)
     assert torch.equal(outs[0][:, 128:N // 2 - 128], outs[1][:, 128:N // 2 - 128]) and torch.equal(outs[0][:, N // 2 + 128:N - 128], outs[1][:, N // 2 + 128:N - 128])
     xd = x.double()
     if form != "pair":
