@@ -175,7 +175,7 @@ __device__ __forceinline__ f16x8 f143_convert8(u32x2 p) {
 // moved to fp16 bits 13..7 with their sign in bit 15 are that number.  The same operands either way, so that a channel's sums do not follow the codes of those
 // beside it.  (Operands of the numbers themselves are a fourth instruction there, 85 -> 101 us for 300 rows, 8192 x 4096.)
 // What bounds a launch is the vector unit beside the matrix unit, which multiplies two waves' operands a SIMD: with three instructions and with one, 2048 rows,
-// 8192 x 8192 230 and 194, 13696 x 4096 205 and 178 us.
+// 8192 x 8192 216 and 194, 13696 x 4096 205 and 178 us.
 struct FmtF143Block : FmtF8<0> {
   static __device__ __forceinline__ float finish(float acc, Scale s) { return acc * 128.0f * s.mul; }
   static constexpr bool kCodes = true;

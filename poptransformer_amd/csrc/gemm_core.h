@@ -2752,8 +2752,8 @@ __global__ __launch_bounds__(BLOCK_WAVES * 64) __attribute__((amdgpu_waves_per_e
   auto b_operand = [&](int at, int m, int rg) { return *reinterpret_cast<const f16x8*>(smem + at + (m ? b1 : b0) + rg * 2048); };
 
   // One pipeline over all steps: a step is two halves of 32 features, a half four blocks of RG MFMAs with one weight operand
-  // each.  The row operands of the next half are requested in this one's first two blocks (two sets of registers; over all four 1 % slower), the
-  // weight operand four blocks ahead.  The barrier stands where everything of a stage has been requested: behind it
+  // each.  The row operands of the next half are requested in this one's first blocks (two sets of registers), the weight operand four blocks
+  // ahead.  The barrier stands where everything of a stage has been requested: behind it
   // the stage takes what is some stages on, its weights (APART) half a step later, so that requests go out all the time.  (The last
   // half requests operands of a stage that does not exist and drops them: a condition here would stand between the MFMAs.)
   constexpr int W0 = NX * XB;                     // where the weights' stages begin
@@ -2783,6 +2783,9 @@ __global__ __launch_bounds__(BLOCK_WAVES * 64) __attribute__((amdgpu_waves_per_e
   __syncthreads();
   auto products = [&](auto fast) {
     constexpr bool FAST = decltype(fast)::value;
+    // blocks of a half that its reads of row operands are spread over: two (four 1 % slower), but the vector unit's conversion beside reads of 256 rows takes all
+    // four (F143, 2048 rows, 8192 x 8192 with codes in every block 229 -> 216 us, pair of 4096 x 13696 387 -> 363)
+    constexpr int OVER = !FAST && RG == 8 ? 4 : 2;
     f16x8 xf[2][RG];
     Piece ahead[NST];
 #pragma unroll
@@ -2818,7 +2821,7 @@ __global__ __launch_bounds__(BLOCK_WAVES * 64) __attribute__((amdgpu_waves_per_e
           const f16x8 av = Fmt::template operand<FAST>(ahead[st]);
           ahead[st] = a_piece(m ? wnext : wat, 1 - m, st);
 #pragma unroll
-          for (int r = st * RG / 2; r < (st + 1) * RG / 2 && r < RG; ++r) xf[1 - m][r] = b_operand(m ? xnext : xat, 1 - m, r);
+          for (int r = st * RG / OVER; r < (st + 1) * RG / OVER && r < RG; ++r) xf[1 - m][r] = b_operand(m ? xnext : xat, 1 - m, r);
 #pragma unroll
           for (int rg = 0; rg < RG; ++rg) acc[rg][st] = Fmt::mma(av, xf[m][rg], acc[rg][st]);
           __builtin_amdgcn_sched_barrier(0);        // (the requests stay where they are)

@@ -79,8 +79,8 @@ def test_every_byte_of_a_tiled_weight_is_written(N, Kd):
     assert not buffers[1][-(-N // 16) * -(-Kd // 128) * 2048:].any()
 
 
-@pytest.mark.parametrize("form, M, Kd, N", [("one", 600, 4096, 2048), ("slices", 1500, 13704, 1032), ("pair", 600, 4104, 2048)])
-def test_channels_beside_the_largest_codes(form, M, Kd, N):
+@pytest.mark.parametrize("form, M, Kd, N, tiles", [("one", 600, 4096, 2048, "128x128"), ("slices", 1500, 13704, 1032, None), ("pair", 600, 4104, 2048, None), ("one", 2040, 1032, 8192, "256x256")])
+def test_channels_beside_the_largest_codes(form, M, Kd, N, tiles):
     """A wave of gemm_block_kernel converts all of its channels one way: those beside a code that the hardware's conversion does not know are bit for bit what they
     are without it, and so is a plain weight in a pair with one that holds such a code.  Weights that are subnormal numbers, which the matrix unit would add with
     fewer bits if they were multiplied as such."""
@@ -95,7 +95,7 @@ def test_channels_beside_the_largest_codes(form, M, Kd, N):
     for c in (codes, marked):
         out = torch.full((M, N), float("nan"), dtype=torch.float16, device="cuda")
         K.linear(x, [K.F8Weight(w.contiguous(), scale()) for w in c], [out] * n, swiglu=form == "pair", workspace=K.linear_workspace(M, N, "cuda") if form == "slices" else None)
-        assert K.linear_kernel() == "gemm_block_kernel"
+        assert K.linear_kernel() == "gemm_block_kernel" and tiles in (None, K.linear_tiles())
         outs.append(out)
     beside = torch.arange(N, device="cuda") % 32 != 0
     assert torch.equal(outs[0][:, beside], outs[1][:, beside])
