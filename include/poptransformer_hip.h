@@ -125,8 +125,11 @@ typedef struct pta_row_norm {
 } pta_row_norm;
 /* the name of the kernel that the calling thread's last product took, "" before the first (a product of several launches: the last one's) */
 const char* pta_linear_kernel(void);
-/* the tiles (rows x channels) of the calling thread's last product by gemm_block_kernel, behind a space those of its last channels where they are others */
+/* the tiles (rows x channels) of the calling thread's last product by gemm_block_kernel or gemm_panel_kernel, behind a space those of its last channels where they
+ * are others; the text is the thread's, until its next call */
 const char* pta_linear_tiles(void);
+/* the slices of K across workgroups of the calling thread's last product (1: not split) */
+int pta_linear_slices(void);
 
 enum { PTA_NORM_NONE = 0, PTA_NORM_RMS = 1, PTA_NORM_LAYER = 2,
        /* pta_row_norm only: the product may be cut otherwise than pta_linear cuts it (its fp32 sums in another order), for what is

@@ -121,6 +121,7 @@ SIGNATURES = {
     "pta_linear_workspace_bytes": (c_size_t, [c_int, c_int]),
     "pta_linear_kernel": (c_char_p, []),
     "pta_linear_tiles": (c_char_p, []),
+    "pta_linear_slices": (c_int, []),
     "pta_argmax": (c_int, [c_void_p, c_void_p, c_void_p, c_int, c_int, c_void_p]),
     "pta_topk": (c_int, [c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_void_p]),
     "pta_take_column": (c_int, [c_void_p, c_void_p, c_void_p, c_int, c_int, c_void_p]),

@@ -345,7 +345,18 @@ static inline int device_compute_units();
 // The kernel that the calling thread's last product took (its last launch's, where it was several; without the finish of a K split): for
 // tests that are meant for one of them.
 inline thread_local const char* gemm_kernel_taken = "";
-inline thread_local const char* gemm_tiles_taken = "";           // of gemm_block_kernel: rows x channels of its tiles, then of the rest's
+// Its tiles, of gemm_block_kernel and gemm_panel_kernel: rows x channels (a pair's: of both weights), and those of the last channels where they are others; and the
+// slices of K.
+struct TilesTaken { int rows, channels, rest_rows, rest_channels; };
+inline thread_local TilesTaken gemm_tiles_taken{};
+inline thread_local int gemm_slices_taken = 1;
+static inline const char* gemm_tiles_name() {
+  static thread_local char name[48];
+  const TilesTaken& t = gemm_tiles_taken;
+  const int n = t.rows ? snprintf(name, sizeof name, "%dx%d", t.rows, t.channels) : (name[0] = 0);
+  if (t.rest_rows) snprintf(name + n, sizeof name - n, " %dx%d", t.rest_rows, t.rest_channels);
+  return name;
+}
 constexpr int GEMM_MAX_KSPLIT = 4;
 constexpr int GEMM_MAX_ROWS = 4096;
 // From so many features on the rows of a workgroup (up to 256, and 48 rows past the last one) take more bytes than the 32-bit offsets of
@@ -1423,6 +1434,7 @@ static bool launch_splitk_finish_norm(const GemmArgs& a, hipStream_t s) {
 
 template <class Fmt>
 static void launch_splitk_finish(const GemmArgs& a, hipStream_t s) {
+  gemm_slices_taken = a.ksplit;
   const size_t total = (size_t)a.M * a.mat[0].N;
   if constexpr (!Fmt::kWide) {
     if (a.then && launch_splitk_finish_norm<Fmt>(a, s)) return;
@@ -2947,8 +2959,7 @@ static int dispatch_gemm_block(const GemmArgs& a, hipStream_t s, const char* nam
       default: return launch_gemm_block<Fmt, 2, PAIR>(b, 2 * group0, group1 < 0 ? narrow : 2 * group1, s, name);
     }
   };
-  static const char* const tiles[4][4] = {{"128x128"}, {"128x256"}, {"192x256"}, {"256x256", "256x256 128x128", "256x256 128x256", "256x256 192x256"}};
-  gemm_tiles_taken = tiles[rg / 2 - 1][rest / 2];
+  gemm_tiles_taken = {block_rows(rg), block_cb(rg) * 16, rest ? block_rows(rest) : 0, rest ? block_cb(rest) * 16 : 0};
   int rc = launch(rg, 0, rest ? whole : -1);
   if (!rc && rest) rc = launch(rest, whole, -1);
   if (rc) return rc;
@@ -3089,6 +3100,7 @@ static int launch_gemm_panel_plan(const GemmArgs& a, const PanelPlan& p, hipStre
     pta_set_error("%s: no tile of %d rows and %d parts", name, rg * 16, kh);
     return (int)PTA_EINVAL;
   };
+  gemm_tiles_taken = {p.rg * 16, PANEL_WAVES / p.kh * 64, p.whole ? p.rest_rg * 16 : 0, p.whole ? PANEL_WAVES / p.rest_kh * 64 : 0};
   int rc = launch(p.rg, p.kh, 0, p.whole ? p.whole * PANEL_WAVES : units);
   if (!rc && p.whole) rc = launch(p.rest_rg, p.rest_kh, p.whole * PANEL_WAVES, units);
   if (rc) return rc;

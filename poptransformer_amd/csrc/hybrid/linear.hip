@@ -133,7 +133,7 @@ static void launch_f32(const pta_wide_linear_args& a, const GemmMat& mat, hipStr
 }
 
 extern "C" const char* pta_wide_linear_kernel(void) { return gemm_kernel_taken; }
-extern "C" const char* pta_wide_linear_tiles(void) { return gemm_tiles_taken; }
+extern "C" const char* pta_wide_linear_tiles(void) { return gemm_tiles_name(); }
 
 extern "C" size_t pta_wide_linear_workspace_bytes(int M, int N) {
   if (M <= 0 || N <= 0) return 0;

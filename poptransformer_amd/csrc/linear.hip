@@ -56,6 +56,7 @@ static int linear_impl(const void* X, const int32_t* x_scale, int x_bytes, int c
   if (rc) return rc;
   for (int i = 0; i < count; ++i) PTA_REQUIRE(X || host_w[i].x, "pta_linear: entry %d has no input", i);
   PTA_REQUIRE(kind >= PTA_W_INT4 && kind <= PTA_W_F152, "pta_linear: unknown weight kind %d", kind);
+  gemm_slices_taken = 1;
   GemmArgs a{};
   a.then = then;
   a.count = count; a.X = (const f16*)X; a.x_scale = x_scale; a.M = M; a.K = K; a.KT = (K + 127) / 128;
@@ -164,7 +165,8 @@ extern "C" int pta_linear_then_norm(const pta_half* X, const int32_t* x_scale, c
 }
 
 extern "C" const char* pta_linear_kernel(void) { return gemm_kernel_taken; }
-extern "C" const char* pta_linear_tiles(void) { return gemm_tiles_taken; }
+extern "C" const char* pta_linear_tiles(void) { return gemm_tiles_name(); }
+extern "C" int pta_linear_slices(void) { return gemm_slices_taken; }
 
 extern "C" size_t pta_linear_workspace_bytes(int M, int N) {
   if (M <= 0 || N <= 0) return 0;

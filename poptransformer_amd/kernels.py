@@ -84,8 +84,13 @@ def linear_kernel():
 
 
 def linear_tiles():
-    """The tiles of this thread's last product by gemm_block_kernel (pta_linear_tiles)."""
+    """The tiles of this thread's last product by gemm_block_kernel or gemm_panel_kernel (pta_linear_tiles)."""
     return _lib.load().pta_linear_tiles().decode()
+
+
+def linear_slices():
+    """How many slices of K across workgroups this thread's last product was cut into (1: not split)."""
+    return _lib.load().pta_linear_slices()
 
 
 # ------------------------------------------------------------------ INT4 -----------------

@@ -1,5 +1,6 @@
-"""Products of 33 rows and more by INT4 and F152 weights (gemm_panel_kernel) against float64: every tile of 48 to 128 rows with one, two and four parts of K,
-slices of workgroups, and tiles of two kinds in one product; channels of any number."""
+"""Products of 33 rows and more by INT4 and F152 weights (gemm_panel_kernel) against float64: every tile of 48 to 128 rows with one, two and four parts of K, for a pair
+and for others, and tiles of two kinds in one product; channels and features of any number.  Which tile a launch takes is its plan's choice, so each is asked for by sizes
+and looked at."""
 import pytest
 import torch
 
@@ -18,20 +19,27 @@ def weight(kind, N, Kd, g):
     return K.F8Weight(codes, scale, "F152"), K.fp8_to_half(codes, scale, "F152").double()
 
 
-# features, channels, form; rows: one past 128, tiles that rows fill and that they do not, one round and several
-SHAPES = {"int4": [(4096, 6144, "one"), (2056, 4096, "scratch"), (11008, 1024, "scratch"), (1032, 5632, "pair"), (520, 2048, "three"), (4104, 11008, "pair"), (8192, 6144, "one"), (4096, 1000, "one"), (1032, 50, "three"), (2048, 1303, "scratch"), (4104, 1297, "pair"), (2048, 2088, "three")],
-          "F152": [(4096, 2048, "one"), (2056, 4096, "pair"), (8200, 1024, "scratch"), (1032, 1111, "pair")]}
+# tile (rows x channels of a workgroup: 512 channels are one part of K, 256 two, 128 four), form, rows, features, channels
+TILES = {"int4": [("128x512", "three", 452, 712, 8848), ("128x512", "pair", 674, 720, 9332), ("112x512", "three", 433, 680, 8712), ("112x512", "pair", 780, 680, 7778), ("96x512", "three", 561, 680, 5504), ("96x512", "pair", 575, 680, 8456),
+                  ("80x512", "three", 133, 704, 5831), ("80x512", "pair", 201, 696, 8237), ("128x256", "three", 228, 984, 7352), ("128x256", "pair", 351, 904, 8712), ("112x256", "three", 201, 912, 7320), ("112x256", "pair", 394, 936, 6978),
+                  ("96x256", "three", 161, 960, 7336), ("96x256", "pair", 321, 912, 6904), ("80x256", "three", 138, 920, 7424), ("80x256", "pair", 197, 984, 8212), ("64x256", "three", 145, 912, 3680), ("64x256", "pair", 135, 904, 5912),
+                  ("80x128", "three", 66, 2280, 5480), ("80x128", "pair", 68, 2144, 8649), ("64x128", "three", 99, 2064, 3591), ("64x128", "pair", 99, 2136, 5810), ("48x128", "three", 67, 2112, 2737), ("48x128", "pair", 76, 2080, 4304),
+                  ("96x512 64x256", "pair", 833, 920, 9264), ("80x512 80x256", "three", 514, 912, 8770), ("112x512 80x256", "one", 1864, 1024, 9824), ("64x256", "one", 1024, 1024, 4096), ("48x128", "pair", 48, 4104, 11008)],
+         "F152": [("112x512", "three", 328, 696, 7440), ("112x512", "pair", 967, 680, 4896), ("96x512", "three", 167, 728, 9272), ("96x512", "pair", 562, 760, 6188), ("80x512", "three", 131, 696, 2808), ("80x512", "pair", 141, 688, 2782),
+                  ("112x256", "three", 328, 936, 3960), ("112x256", "pair", 322, 912, 6016), ("96x256", "three", 176, 904, 7234), ("96x256", "pair", 324, 928, 5608), ("80x256", "three", 129, 944, 5088), ("80x256", "pair", 134, 1016, 7524),
+                  ("64x256", "three", 134, 1064, 1352), ("64x256", "pair", 130, 1128, 1454), ("80x128", "three", 130, 1944, 3600), ("80x128", "pair", 194, 1952, 4187), ("64x128", "one", 146, 1944, 8640), ("64x128", "pair", 155, 1984, 4279),
+                  ("48x128", "three", 129, 2000, 1413), ("48x128", "pair", 130, 1968, 1456), ("80x512 64x256", "three", 600, 904, 7458), ("80x512 64x256", "pair", 1346, 920, 5223), ("112x512", "one", 1963, 904, 5952)]}
 
 
-@pytest.mark.parametrize("M", [33, 65, 128, 129, 145, 200, 333, 470, 640, 900, 1201])
-@pytest.mark.parametrize("kind, Kd, N, form", [(k, *s) for k, shapes in SHAPES.items() for s in shapes])
-def test_every_tile(kind, Kd, N, form, M):
+@pytest.mark.parametrize("kind, tiles, form, M, Kd, N", [(k, *t) for k, all_tiles in TILES.items() for t in all_tiles])
+def test_every_tile(kind, tiles, form, M, Kd, N):
     from poptransformer_amd import kernels as K
     g = torch.Generator(device="cuda").manual_seed(M)
     x = torch.randn((M, Kd), generator=g, device="cuda").half() * 0.1
     ws, dense = zip(*[weight(kind, N, Kd, g) for _ in range({"pair": 2, "three": 3}.get(form, 1))])
     outs = [torch.full((M, N), float("nan"), dtype=torch.float16, device="cuda") for _ in range(3 if form == "three" else 1)]
-    K.linear(x, list(ws), outs * 2 if form == "pair" else outs, swiglu=form == "pair", workspace=K.linear_workspace(M, N, "cuda") if form == "scratch" else None)
+    K.linear(x, list(ws), outs * 2 if form == "pair" else outs, swiglu=form == "pair")
+    assert (K.linear_kernel(), K.linear_tiles(), K.linear_slices()) == ("gemm_panel_kernel", tiles, 1)
     xd, refs = x.double(), []
     for p in dense:
         ref = xd @ p.T
