@@ -3041,9 +3041,10 @@ constexpr int PANEL_TILES[][2] = {{8, 1}, {7, 1}, {6, 1}, {5, 1}, {8, 2}, {7, 2}
 template <class Fmt, bool PAIR>
 static PanelPlan plan_gemm_panel(const GemmArgs& a) {
   constexpr bool F152 = OwnStreams<Fmt>::long_decode;
-  // The norm launch whose place the adding of slices takes: who gives scratch has one behind the product (11008 x 4096: 1000 rows, the two together 93 us in slices and
-  // 94 whole; 2000 rows 162 and 146 without the norm)
+  // A norm's launch, in whose place the slices are added.  Without a norm behind the product as much again, but no more than 4 % of the time, which these estimates do not
+  // tell apart: a product that this leaves in slices has its sums in the order that they have before a norm (11008 x 4096, 1000 rows: 95 us, 92 whole).
   constexpr double NORM = 4.3;
+  const bool normed = a.then && a.then->any_order && finish_norm_fits(a);
   const int cus = device_compute_units(), all = panel_units(a, PAIR);
   auto time = [&](int rg, int kh, int slices, int units) {
     const double step = (F152 ? 6.4 : 0.0) + (kh == 1 ? 0.7 + 0.21 * rg : kh == 2 ? 0.68 + 0.26 * rg : 0.83 + 0.39 * rg), ends = kh == 1 ? 6.5 : kh == 2 ? 5.5 : 2.7;
@@ -3051,16 +3052,20 @@ static PanelPlan plan_gemm_panel(const GemmArgs& a) {
     const int cw = PANEL_WAVES / kh, tiles = ((units + cw - 1) / cw * ((a.M + rg * 16 - 1) / (rg * 16)) + 7) / 8 * 8 * slices;
     const double last = (double)(tiles % cus) / cus, load = 0.03 * rg;
     const double one = ends + ((a.KT + slices - 1) / slices + kh - 1) / kh * step;
-    return one * (tiles / cus * (1.0 + load) + (last > 0.0 ? 1.0 + load * last * last : 0.0)) + (slices > 1 ? 3.0 + (double)a.M * a.mat[0].N * (4.0 * slices + 6.0) / 5.5e6 - NORM : 0.0);
+    return one * (tiles / cus * (1.0 + load) + (last > 0.0 ? 1.0 + load * last * last : 0.0)) + (slices > 1 ? 3.0 + (double)a.M * a.mat[0].N * (4.0 * slices + 6.0) / 5.5e6 - (normed ? NORM : 0.0) : 0.0);
   };
   PanelPlan best{F152 ? 7 : 8, 1, 1, 0, 0, 0, 1e30};
+  double least = best.us;
+  auto choose = [&](const PanelPlan& p) {
+    const double us = p.slices > 1 && !normed ? p.us - (0.04 * p.us < NORM ? 0.04 * p.us : NORM) : p.us;
+    if (us < least) least = us, best = p;
+  };
   for (const auto& t : PANEL_TILES) {
     if (F152 && t[0] == 8) continue;
     for (int slices = 1; slices <= (!PAIR && a.count == 1 && a.part ? GEMM_MAX_KSPLIT : 1); ++slices) {
       if (t[1] * slices > 1 && a.KT < t[1] * slices * 4) break;
       if (slices > 1 && a.part_bytes < (size_t)slices * a.M * a.mat[0].N * sizeof(float)) break;
-      const double us = time(t[0], t[1], slices, all);
-      if (us < best.us) best = PanelPlan{t[0], t[1], slices, 0, 0, 0, us};
+      choose(PanelPlan{t[0], t[1], slices, 0, 0, 0, time(t[0], t[1], slices, all)});
     }
     if (t[1] > 1) continue;
     const int groups = (all + PANEL_WAVES - 1) / PANEL_WAVES, row_blocks = (a.M + t[0] * 16 - 1) / (t[0] * 16), whole = groups * row_blocks / cus * cus / row_blocks;
@@ -3068,8 +3073,7 @@ static PanelPlan plan_gemm_panel(const GemmArgs& a) {
     const double first = time(t[0], 1, 1, whole * PANEL_WAVES);
     for (const auto& r : PANEL_TILES) {
       if ((F152 && r[0] == 8) || (r[1] > 1 && a.KT < r[1] * 4)) continue;
-      const double us = first + time(r[0], r[1], 1, all - whole * PANEL_WAVES) + 1.0;
-      if (us < best.us) best = PanelPlan{t[0], 1, 1, whole, r[0], r[1], us};
+      choose(PanelPlan{t[0], 1, 1, whole, r[0], r[1], first + time(r[0], r[1], 1, all - whole * PANEL_WAVES) + 1.0});
     }
   }
   return best;

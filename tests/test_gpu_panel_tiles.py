@@ -1,6 +1,6 @@
 """Products of 33 rows and more by INT4 and F152 weights (gemm_panel_kernel) against float64: every tile of 48 to 128 rows with one, two and four parts of K, for a pair
-and for others, and tiles of two kinds in one product; channels and features of any number.  Which tile a launch takes is its plan's choice, so each is asked for by sizes
-and looked at."""
+and for others, and tiles of two kinds in one product; slices of K across workgroups; channels and features of any number.  Which tile and how many slices a launch takes
+is its plan's choice, so each is asked for by sizes and looked at."""
 import pytest
 import torch
 
@@ -53,3 +53,32 @@ def test_every_tile(kind, tiles, form, M, Kd, N):
     else:
         for out, (ref, bound) in zip(outs, refs):
             assert ((out.double() - ref).abs() <= bound).all()
+
+
+# rows, features, channels; tile and slices of a product with scratch, and of one with a norm behind it whose sums may be taken in any order
+@pytest.mark.parametrize("kind, M, Kd, N, alone, normed", [
+    ("int4", 266, 7272, 7000, ("80x512", 4), ("80x512", 4)), ("int4", 144, 4624, 5656, ("80x256", 4), ("80x256", 4)), ("int4", 577, 8240, 816, ("64x128", 3), ("64x128", 3)),
+    ("int4", 1000, 11008, 4096, ("128x512", 4), ("128x512", 4)), ("int4", 602, 4104, 4616, ("64x256", 1), ("80x512", 3)), ("int4", 133, 3136, 5712, ("48x128", 1), ("64x256", 3)),
+    ("int4", 323, 4088, 2696, ("48x128", 1), ("80x128", 2)),
+    ("F152", 133, 1432, 4112, ("80x512", 3), ("80x512", 3)), ("F152", 134, 2960, 4208, ("64x256", 3), ("64x256", 3)), ("F152", 133, 4048, 4224, ("48x128", 2), ("48x128", 2)),
+    ("F152", 512, 1416, 6896, ("64x256", 1), ("112x512", 3)), ("F152", 268, 3184, 7192, ("80x128", 1), ("96x256", 2))])
+def test_slices(kind, M, Kd, N, alone, normed):
+    """Adding the slices is a launch more, but where a norm's launch makes room for it: more slices there, and only if the call allows other sums than the two calls'."""
+    from poptransformer_amd import kernels as K
+    g = torch.Generator(device="cuda").manual_seed(M)
+    x = torch.randn((M, Kd), generator=g, device="cuda").half() * 0.1
+    (w, dense), gamma = weight(kind, N, Kd, g), torch.randn(N, generator=g, device="cuda").half()
+    workspace = K.linear_workspace(M, N, "cuda")
+    ref = x.double() @ dense.T
+    bound = 2.0 ** -11 * ref.abs() + (Kd + 2) * 2.0 ** -24 * (x.double().abs() @ dense.abs().T) + 2.0 ** -24
+    first, one = (torch.full((M, N), float("nan"), dtype=torch.float16, device="cuda") for _ in range(2))
+    K.linear(x, [w], [first], workspace=workspace)
+    assert (K.linear_kernel(), K.linear_tiles(), K.linear_slices()) == ("gemm_panel_kernel", *alone)
+    assert ((first.double() - ref).abs() <= bound).all()
+    for any_order, plan in ((False, alone), (True, normed)):
+        y, out = (torch.full((M, N), float("nan"), dtype=torch.float16, device="cuda") for _ in range(2))
+        K.linear_then_norm(x, w, y, K.RowNorm(gamma, None, 1e-5, out=out, any_order=any_order), workspace=workspace)
+        assert (K.linear_tiles(), K.linear_slices()) == plan
+        assert torch.equal(y, first) if plan == alone else ((y.double() - ref).abs() <= bound).all()
+        K.rmsnorm(y, gamma, 1e-5, one)
+        assert torch.equal(out, one)
