@@ -3141,25 +3141,45 @@ static OwnPlan plan_gemm_own(const GemmArgs& a) {
   constexpr double PRODUCTS = Fmt::kVec == 1 ? 0.48 : Fmt::kVec == 2 ? 0.6 : 0.7, WEIGHTS = Fmt::kVec == 1 ? 0.0 : Fmt::kVec == 2 ? 0.36 : 0.9;
   const int cus = device_compute_units();
   const int row_blocks = (a.M + 63) / 64;
-  // (up to 128 rows and a block of channels a compute unit)
-  const bool normed = a.then && a.then->any_order && a.M <= 128 && a.mat[0].N <= 16 * cus && finish_norm_fits(a);
-  const bool split = !PAIR && a.count == 1 && a.part && (a.M > 16 || (normed && a.M > (Fmt::kVec == 1 ? 12 : 8) && a.KT >= 80));
-  OwnPlan best{((a.M + 15) / 16 + row_blocks - 1) / row_blocks, 1, 1, 0, 0.0};
-  const double rows = normed ? a.M / 16.0 / row_blocks : best.mt;      // groups of them that a workgroup reads
-  for (int nb = 1; nb <= own_cap<Fmt, PAIR>(best.mt); ++nb) {
-    const int groups = own_groups(a, nb, PAIR) * row_blocks;
-    // (four blocks by four slices, more than 64 rows: 2 x 2 is the faster by 2 to 5 %)
-    for (int sl = 1; sl <= (!split ? 1 : normed && row_blocks > 1 ? 3 : GEMM_MAX_KSPLIT); ++sl) {
-      if (sl > 1 && (a.KT < sl * OWN_WAVES || a.part_bytes < (size_t)sl * a.M * a.mat[0].N * sizeof(float))) break;
-      const int rounds = (groups * sl + cus - 1) / cus, tiles = ((a.KT + sl - 1) / sl + OWN_WAVES - 1) / OWN_WAVES;
-      double us = 3.2 + rounds * tiles * (0.5 + 0.29 * rows + (PRODUCTS + WEIGHTS / row_blocks) * nb * (PAIR ? 2 : 1));
-      if (sl > 1) {
-        const double size = (double)a.M * a.mat[0].N / 262144;
-        us += normed ? sl * (0.35 + 0.5 * size) + (Fmt::kVec > 1 ? 1.0 : 0.8) : 2.7 * sl - 0.9 + (size > 1 ? 0.5 * sl * (size - 1) : 0.0);
-      }
-      if (best.rounds == 0 || us < best.us) best.nb = nb, best.slices = sl, best.rounds = rounds, best.us = us;
+  const int mt = ((a.M + 15) / 16 + row_blocks - 1) / row_blocks;
+  const bool slices = !PAIR && a.count == 1 && a.part;
+  auto time = [&](int nb, int sl, bool normed, int& rounds) {
+    const double rows = normed ? a.M / 16.0 / row_blocks : mt;         // groups of them that a workgroup reads
+    const int tiles = ((a.KT + sl - 1) / sl + OWN_WAVES - 1) / OWN_WAVES;
+    rounds = (own_groups(a, nb, PAIR) * row_blocks * sl + cus - 1) / cus;
+    double us = 3.2 + rounds * tiles * (0.5 + 0.29 * rows + (PRODUCTS + WEIGHTS / row_blocks) * nb * (PAIR ? 2 : 1));
+    if (sl > 1) {
+      const double size = (double)a.M * a.mat[0].N / 262144;
+      us += normed ? sl * (0.35 + 0.5 * size) + (Fmt::kVec > 1 ? 1.0 : 0.8) : 2.7 * sl - 0.9 + (size > 1 ? 0.5 * sl * (size - 1) : 0.0);
     }
-  }
+    return us;
+  };
+  auto room = [&](int sl) { return sl == 1 || (a.KT >= sl * OWN_WAVES && a.part_bytes >= (size_t)sl * a.M * a.mat[0].N * sizeof(float)); };
+  OwnPlan best{mt, 1, 1, 0, 0.0};
+  for (int nb = 1; nb <= own_cap<Fmt, PAIR>(mt); ++nb)
+    for (int sl = 1; sl <= (slices && a.M > 16 ? GEMM_MAX_KSPLIT : 1) && room(sl); ++sl) {
+      int rounds;
+      const double us = time(nb, sl, false, rounds);
+      if (best.rounds == 0 || us < best.us) best = OwnPlan{mt, nb, sl, rounds, us};
+    }
+  // (up to 128 rows and a block of channels a compute unit)
+  if (!slices || !a.then || !a.then->any_order || a.M > 128 || a.mat[0].N > 16 * cus || !finish_norm_fits(a)) return best;
+  // with a norm behind it: that plan, or one that is shorter by the other estimate
+  best.us = time(best.nb, best.slices, true, best.rounds);
+  if (a.M <= (Fmt::kVec == 1 ? 12 : 8) || (a.M <= 16 && a.KT < 80)) return best;
+  const bool sliced = best.slices > 1;
+  // Not taken, though their estimates are shorter: beyond 64 rows four blocks, and four slices (INT4, 6144 x 4096, 80 rows, 4 x 2 16.0 against 2 x 1 15.4; 11008 x 2048, 112
+  // rows, 4 x 3 18.2 against 2 x 2 16.9; F143, 16384 x 2048, 112 rows, 2 x 2 26.1 against 4 x 4 22.4, which is the plan without a norm); of fewer feature tiles, four blocks
+  // and more in place of fewer with slices (INT4, 8192 x 4096, 40 rows, 4 x 4 14.6 against 2 x 2 14.0, 11008 x 4096, 20 rows 14.3 against 13.9, F143 8192 x 4096, 40 rows 17.1
+  // against 16.5; 13696 x 4096 17.6 against 19.0), and of INT4 for up to 16 rows (11008 x 4096, 13 rows, 4 x 4 13.6 against 13.1); of 16-bit weights three blocks in their
+  // place (6144 x 3072, 56 rows, 3 x 3 18.4 against 2 x 2 17.9).
+  const int most = row_blocks > 1 || ((sliced || (Fmt::kVec == 1 && a.M <= 16)) && a.KT < (Fmt::kVec == 1 ? 96 : 80)) ? Fmt::kVec > 2 && sliced ? 2 : 3 : own_cap<Fmt, PAIR>(mt);
+  for (int nb = 1; nb <= own_cap<Fmt, PAIR>(mt) && nb <= most; ++nb)
+    for (int sl = 1; sl <= (row_blocks > 1 ? 3 : GEMM_MAX_KSPLIT) && room(sl); ++sl) {
+      int rounds;
+      const double us = time(nb, sl, true, rounds);
+      if (us < best.us) best = OwnPlan{mt, nb, sl, rounds, us};
+    }
   return best;
 }
 

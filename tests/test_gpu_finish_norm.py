@@ -96,28 +96,61 @@ def test_tensors_that_the_norms_own_entry_points_refuse():
         K.RowNorm(gamma.reshape(8, 8), None, 1e-5, out=rows(20, 64))
 
 
-# rows, features, channels: the edges of what may be cut otherwise (blocks x slices of its plan), odd channels and feature tiles
-@pytest.mark.parametrize("kind, M, Kd, N", [("int4", 13, 11008, 4096), ("int4", 12, 11008, 4096), ("int4", 64, 4096, 4096), ("int4", 128, 3072, 768), ("int4", 129, 3072, 768), ("F143", 9, 13696, 4096),
-                                            ("F143", 64, 13696, 4096), ("F143", 17, 8192, 2056), ("F143", 40, 4096, 4104), ("f16", 24, 11008, 4096), ("f16", 80, 5632, 2048), ("f16", 31, 2824, 1016),
-                                            ("F152", 33, 4096, 1024), ("int4", 16, 1024, 64)])
-@pytest.mark.parametrize("room", [4, 3, 1, 0])
-def test_sums_in_any_order(kind, M, Kd, N, room):
-    """With any_order the product may be cut otherwise, by the scratch that there is: within the bound of fp32 sums, and the norm is that of the rows it leaves."""
+# rows, features, channels; the slices of K without and with any_order: the fewest and the most rows, more or fewer slices with it and the same, blocks of channels and feature
+# tiles that do not divide
+ANY_ORDER = [("int4", 12, 11008, 2048, 1, 1), ("int4", 13, 11008, 2048, 1, 4), ("int4", 16, 1024, 64, 1, 1), ("int4", 20, 11008, 4096, 2, 2), ("int4", 64, 4104, 4096, 1, 2), ("int4", 100, 16392, 2048, 4, 4),
+             ("int4", 128, 3072, 768, 1, 3), ("int4", 129, 3072, 768, 1, 1), ("F143", 8, 13704, 4096, 1, 1), ("F143", 9, 13704, 4096, 1, 2), ("F143", 16, 11008, 1032, 1, 3), ("F143", 17, 8192, 2056, 3, 4),
+             ("F143", 40, 4096, 4104, 2, 2), ("F143", 64, 13696, 4096, 2, 4), ("f16", 12, 16392, 2040, 1, 4), ("f16", 24, 11008, 4096, 1, 2), ("f16", 31, 2824, 1016, 1, 2), ("f16", 60, 6144, 3080, 2, 2),
+             ("f16", 80, 5632, 2048, 1, 2), ("F152", 33, 4096, 1024, 2, 4)]
+
+
+@pytest.mark.parametrize("kind, M, Kd, N, alone, any_order", ANY_ORDER)
+@pytest.mark.parametrize("form", ["rms", "grid", "layer", "shift"])
+def test_sums_in_any_order(kind, M, Kd, N, alone, any_order, form):
+    """With any_order the product is cut otherwise where that is faster, and by the scratch that there is: within the bound of fp32 sums, and the norm is that of the rows it
+    leaves."""
     from poptransformer_amd import kernels as K
     g = torch.Generator(device="cuda").manual_seed(71)
-    x = torch.randn((M, Kd), generator=g, device="cuda").half() * 0.1
-    w = weight(kind, N, Kd, g)
-    gamma, res = torch.randn(N, generator=g, device="cuda").half(), torch.randn((M, N), generator=g, device="cuda").half()
-    got, out, one, plain = (torch.full((M, N), float("nan"), dtype=torch.float16, device="cuda") for _ in range(4))
-    workspace = K.linear_workspace(M, N, "cuda")[:room * M * N * 4] if room else None
-    K.linear_then_norm(x, w, got, K.RowNorm(gamma, None, 1e-5, out=out, any_order=True), residual=res, workspace=workspace)
-    K.linear(x, [w], [plain], residual=res)
-    K.rmsnorm(got, gamma, 1e-5, one)
-    assert torch.equal(out, one)
-    # either one's sums of fp32 products are within K 2^-24 of the sum of magnitudes, and rounded twice to fp16 (the product, and with the residual)
+    x, w = torch.randn((M, Kd), generator=g, device="cuda").half() * 0.1, weight(kind, N, Kd, g)
+
+    def rows(*shape):
+        return torch.randn(shape, generator=g, device="cuda").half()
+    gamma, beta, bias, mul, res, prev = rows(N), rows(N), rows(N), rows(M, N), rows(M, N), rows(M, N)
+    mixes, exponent = [rows(N) for _ in range(3)], torch.tensor([-2], dtype=torch.int32, device="cuda")
+    ends = {"rms": dict(residual=res), "grid": dict(bias=bias, residual=res), "layer": dict(bias=bias), "shift": dict(mul=mul, residual=res, post_scale=0.5)}[form]
     unit = torch.eye(Kd, dtype=torch.float16, device="cuda")
     dense = torch.cat([K.linear(unit[i:i + 256], [w], [torch.empty((min(256, Kd - i), N), dtype=torch.float16, device="cuda")])[0] for i in range(0, Kd, 256)]).double()
-    mag = x.double().abs() @ dense.abs()
     ref = x.double() @ dense
-    for y in (got, plain):
-        assert ((y.double() - (ref + res.double())).abs() <= 2.0 ** -10 * (ref.abs() + res.double().abs()) + (Kd + 2) * 2.0 ** -24 * mag + 2.0 ** -23).all()
+    # fp32 sums of exact products within K 2^-24 of the sum of magnitudes, and fp16 roundings of the product and of each value on the way to the end: every one within
+    # 2^-11 of what it rounds, which the factors behind it carry on
+    err = 2.0 ** -11 * ref.abs() + (Kd + 2) * 2.0 ** -24 * (x.double().abs() @ dense.abs()) + 2.0 ** -24
+    for name, t in ends.items():
+        if name == "post_scale":
+            ref, err = ref * t, err * t
+        elif name == "mul":
+            ref, err = ref * t.double(), err * t.double().abs()
+        else:
+            ref = ref + t.double()
+        err = err + 2.0 ** -11 * (ref.abs() + err) + 2.0 ** -24
+    for room in (0, 1, 2, 3, 4):
+        got, out, one = (torch.full((M, N), float("nan"), dtype=torch.float16, device="cuda") for _ in range(3))
+        mixed, plain, was, before = [torch.empty_like(got) for _ in range(3)], [torch.empty_like(got) for _ in range(3)], prev.clone(), prev.clone()
+        then = {"rms": dict(out=out), "grid": dict(out=out, grid=(exponent, "F143")), "layer": dict(out=out), "shift": dict(shift=(was, mixes[:2], mixed[:2]), out=out)}[form]
+        workspace = K.linear_workspace(M, N, "cuda")[:room * M * N * 4] if room else None
+        norm_beta = beta if form in ("layer", "shift") else None
+        K.linear_then_norm(x, w, got, K.RowNorm(gamma, norm_beta, 1e-5, any_order=True, **then), workspace=workspace, **ends)
+        slices = K.linear_slices()
+        assert slices == any_order if room == 4 else slices <= max(room, 1)
+        assert ((got.double() - ref).abs() <= err).all()
+        if form == "rms":
+            K.rmsnorm(got, gamma, 1e-5, one)
+        elif form == "grid":
+            K.rmsnorm_fp8_grid(got, gamma, 1e-5, exponent, "F143", out=one)
+        elif form == "layer":
+            K.layer_norm_ce(got, gamma, beta, 1e-5, one)
+        else:
+            K.layer_norm_ce_mix(got, gamma, beta, 1e-5, before, mixes[:2], plain[:2], out=one)
+            assert torch.equal(was, before) and all(torch.equal(a, b) for a, b in zip(mixed[:2], plain[:2]))
+        assert torch.equal(out, one)
+    K.linear_then_norm(x, w, got, K.RowNorm(gamma, norm_beta, 1e-5, **dict(then, **({"shift": (prev.clone(), mixes[:2], mixed[:2])} if form == "shift" else {}))), workspace=workspace, **ends)
+    assert K.linear_slices() == alone
