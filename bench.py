@@ -182,6 +182,7 @@ def gemm_measure(M, steps, warmup, weights=None):
     the weight copies (so that several M share them)."""
     import torch
     from poptransformer_amd import kernels as K
+    from poptransformer_amd.engine.loop import recording
     Kd, N, copies = 4096, 11008, 48
     gen = torch.Generator(device="cuda").manual_seed(7)
     x = torch.randn(M, Kd, device="cuda", dtype=torch.float16, generator=gen)
@@ -200,7 +201,7 @@ def gemm_measure(M, steps, warmup, weights=None):
             K.w4a16_gemm(x, w, out=out)
         stream.synchronize()
         g = torch.cuda.CUDAGraph()
-        with torch.cuda.graph(g, stream=stream):
+        with recording(g, stream=stream):
             for w in ws:
                 K.w4a16_gemm(x, w, out=out)
         rounds_w = max(1, warmup // copies)
@@ -669,6 +670,7 @@ def main():
     import torch
     from poptransformer_amd import kernels as K
     from poptransformer_amd.engine import fused, loader, synthetic
+    from poptransformer_amd.engine.loop import recording
 
     if not torch.cuda.is_available():
         print("no GPU visible", file=sys.stderr)
@@ -766,7 +768,7 @@ def main():
             e0, e1 = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
             g = torch.cuda.CUDAGraph()
             stream.synchronize()
-            with torch.cuda.graph(g, stream=stream):
+            with recording(g, stream=stream):
                 for blk in weights.blocks:
                     K.w4a16_gemm_swiglu(dec.h, blk.mlp_in[0].w, blk.mlp_in[1].w, dec.act)
             g.replay()

@@ -4,8 +4,34 @@ iterations only read the prompt, the recording of one iteration into a HIP graph
 An executor provides `spec` (batch, max_len, pad_id, eos_id, early_stop), `reset(input_ids)`, `step_fn()` (one iteration
 from device state only) and the device tensors `container`, `step`, `keep_going`; optionally `consume_prompt(n)`.
 """
+import contextlib
+import gc
+import threading
+
 import numpy as np
 import torch
+
+_recordings, _recordings_lock, _collects = 0, threading.Lock(), False
+
+
+@contextlib.contextmanager
+def recording(graph, **where):
+    """torch.cuda.graph, and no garbage collection before it ends: a decoder and its prompt passes refer to each other, so one that is no longer used goes with a
+    collection, and its graphs and streams are not to be destroyed while a stream records (the process ends)."""
+    global _recordings, _collects
+    with _recordings_lock:
+        if _recordings == 0:
+            _collects = gc.isenabled()
+            gc.disable()
+        _recordings += 1
+    try:
+        with torch.cuda.graph(graph, **where):
+            yield
+    finally:
+        with _recordings_lock:
+            _recordings -= 1
+            if _recordings == 0 and _collects:
+                gc.enable()
 
 
 class DecodeLoop:
@@ -52,7 +78,7 @@ class DecodeLoop:
             self.step_fn()
             torch.cuda.synchronize()
             self.graph = torch.cuda.CUDAGraph()
-            with torch.cuda.graph(self.graph, stream=self._stream):
+            with recording(self.graph, stream=self._stream):
                 self.step_fn()
         torch.cuda.synchronize()
         return self.graph

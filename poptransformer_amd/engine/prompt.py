@@ -20,6 +20,7 @@ import torch
 from .. import _lib
 from .. import kernels as K
 from .fused import LayerOps
+from .loop import recording
 
 
 class RowMemory:
@@ -122,7 +123,7 @@ class PromptPass(LayerOps):
             stream = torch.cuda.current_stream()
             stream.synchronize()
             self.graph = torch.cuda.CUDAGraph()
-            with torch.cuda.graph(self.graph, pool=self.pool, stream=stream):
+            with recording(self.graph, pool=self.pool, stream=stream):
                 self._layers()
             self.graph.replay()
 
