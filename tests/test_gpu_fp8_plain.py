@@ -99,3 +99,35 @@ def test_channels_beside_the_largest_codes(form, M, Kd, N, tiles):
         outs.append(out)
     beside = torch.arange(N, device="cuda") % 32 != 0
     assert torch.equal(outs[0][:, beside], outs[1][:, beside])
+
+
+def test_a_weight_does_not_wait_for_its_codes():
+    """Building one leaves the device at work; a product that is recorded without one before it has the answer as well, or the kernels for all codes, and the same result."""
+    from poptransformer_amd import kernels as K
+    from poptransformer_amd.engine.loop import recording
+    g = torch.Generator(device="cuda").manual_seed(2)
+    codes = K.half_to_fp8((torch.randn((520, 1032), generator=g, device="cuda") * 0.02).half(), scale())
+    marked = codes.clone()
+    marked.view(torch.uint8)[519, 1031] = 0x7F
+    x = (torch.randn((3, 1032), generator=g, device="cuda") * 0.2).half()
+    outs = [torch.empty((3, 520), dtype=torch.float16, device="cuda") for _ in range(6)]
+    K.F8Weight(codes, scale()).plain
+    torch.cuda.synchronize()
+    torch.cuda._sleep(50_000_000)                 # (some 20 ms, of which building takes a hundredth)
+    ws, behind = [K.F8Weight(c, scale()) for c in (codes, marked, codes)], torch.cuda.Event()
+    behind.record()
+    assert not behind.query()
+    host, done = ws[2]._asked
+    ws[2]._asked = torch.full((1,), 2, dtype=torch.uint8), done       # (one whose answer is not there)
+    graph, stream = torch.cuda.CUDAGraph(), torch.cuda.Stream()
+    stream.wait_stream(torch.cuda.current_stream())
+    with recording(graph, stream=stream):
+        for w, out in zip(ws, outs):
+            K.linear(x, [w], [out])
+    assert [(w._plain, w._asked is None) for w in ws] == [(True, True), (False, True), (False, False)]
+    graph.replay()
+    ws[2]._asked = host, done
+    assert [w.plain for w in ws] == [True, False, True]
+    for w, out in zip(ws, outs[3:]):
+        K.linear(x, [w], [out])
+    assert all(torch.equal(a, b) for a, b in zip(outs, outs[3:])) and torch.equal(outs[0], outs[2]) and not torch.equal(outs[0], outs[1])
