@@ -3326,16 +3326,19 @@ static int dispatch_many_rows(const GemmArgs& a, int total_nb, hipStream_t s, co
   // 26.8 against 21.3; pair 768 x 11008, three, 17.7 against 13.7; bf16 256 x 11008, 65 rows, two, 1.14 times; 512 x 4096, 1000 rows, four,
   // 1.14 times; 1024 x 6144, 768 rows, five, 1.10.  And 16-bit weights of long K, two rounds: 8192 x 8192, 65 to 128 rows, 1.08 to 1.18 times,
   // 11008 x 8192 1.2 to 1.34 (4096 x 8192 0.83 to 0.97).
-  PanelPlan panel;
+  PanelPlan panel{};                              // (made where it is first asked for)
   const bool paneled = PanelFormat<Fmt>::ok && a.M > 128 && panel_takes(a, PAIR);
-  if (paneled) panel = plan_gemm_panel<Fmt, PAIR>(a);
+  auto panel_plan = [&]() -> const PanelPlan& {
+    if (panel.rg == 0) panel = plan_gemm_panel<Fmt, PAIR>(a);
+    return panel;
+  };
   if (a.epi.norm == PTA_NORM_NONE) {
     const OwnPlan plan = plan_gemm_own<Fmt, PAIR>(a);
     const int most = a.M <= 128 ? ((Fmt::kWide && a.KT <= 2) || (Fmt::kVec > 2 && a.KT >= 56) ? 1 : Fmt::kVec == 1 && a.KT >= 12 ? 3 : 2) : a.KT >= 8 || PAIR ? 4 : 3;
     // (a round after the first begins with nothing on its way: 3.6 us more than the plan says; 768 rows of three 1024 x 1024 21.5 against gemm_panel_kernel's 20.8,
     // 1200 rows 27.8 against 21.3, the pair of 1024 x 2816, 640 rows 25.1 against 20.4; two rounds, and short K, stay)
     bool own = plan.rounds == 1 || (plan.rounds <= most && (a.M <= 128 || plan.us <= (Fmt::kVec == 1 ? 22.0 : 11.0)));
-    if (own && a.M > 128) own = !(paneled && a.KT >= 8 && plan.rounds > 2 && plan.us + 3.6 * (plan.rounds - 1) > 1.2 * panel.us);
+    if (own && a.M > 128) own = !(paneled && a.KT >= 8 && plan.rounds > 2 && plan.us + 3.6 * (plan.rounds - 1) > 1.2 * panel_plan().us);
     if constexpr (PanelFormat<Fmt>::ok) {
       if (own && a.M <= 128 && panel_before_own<Fmt, PAIR>(a, plan, panel)) return launch_gemm_panel_plan<Fmt, PAIR>(a, panel, s, name);
     }
@@ -3358,7 +3361,7 @@ static int dispatch_many_rows(const GemmArgs& a, int total_nb, hipStream_t s, co
       return dispatch_gemm_block<typename BlockFormat<Fmt>::type, PAIR>(a, s, name);
   }
   if constexpr (PanelFormat<Fmt>::ok) {
-    if (paneled) return launch_gemm_panel_plan<Fmt, PAIR>(a, panel, s, name);
+    if (paneled) return launch_gemm_panel_plan<Fmt, PAIR>(a, panel_plan(), s, name);
   }
   if (tiles) {
     // fragments in registers, weights through LDS: 256 rows per workgroup where that still fills the machine,
