@@ -81,7 +81,8 @@ int pta_w4_tile(const int8_t* packed, void* tiled, int N, int K, pta_stream_t st
  * workspace (optional): scratch of pta_linear_workspace_bytes(M, N) bytes, 16-byte aligned.  With it, a
  * single-weight launch of more than 16 rows whose channel count alone cannot fill the machine also
  * splits K across workgroups (fp32 partial sums in the workspace, summed by a second kernel that
- * applies the epilogue).  Calls sharing one workspace must not overlap.
+ * applies the epilogue); pta_linear_then_norm with PTA_NORM_ANY_ORDER one of more than 8 rows.  Calls
+ * sharing one workspace must not overlap.
  * Last of all, with out_fp8_scale: Y = pta_half_to_fp8_grid(Y) - the cast of the next FP8 Linear
  * (precision_strategy.py:62-66) done where its input is produced; it also applies to the SwiGLU pair. */
 typedef struct pta_fusion {
@@ -133,7 +134,7 @@ int pta_linear_slices(void);
 
 enum { PTA_NORM_NONE = 0, PTA_NORM_RMS = 1, PTA_NORM_LAYER = 2,
        /* pta_row_norm only: the product may be cut otherwise than pta_linear cuts it (its fp32 sums in another order), for what is
-          the faster launch with a norm behind it */
+          the faster launch with a norm behind it; its K is split from 9 rows on (INT4 from 13), where pta_linear's is from 17 */
        PTA_NORM_ANY_ORDER = 256 };
 enum { PTA_ACT_NONE = 0, PTA_ACT_GELU_TANH = 1, PTA_ACT_RELU_SQUARE = 2, PTA_ACT_SIGMOID = 3 };
 

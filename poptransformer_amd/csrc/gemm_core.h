@@ -2978,8 +2978,10 @@ static inline bool panel_fits(const GemmArgs& a, int nst, bool pair) {
   return true;
 }
 
-// gemm_panel_kernel's launches: panel_fits, and channels that do not divide into its units, up to 24576 a matrix (a head has more, but is asked for few
-// rows; those of more than 128 go 64 rows at a time, as these did: INT4, 1964 rows, 6336 x 1296 383 -> 50 us, 662 rows, three of 2304 x 1264 85 -> 22).
+// gemm_panel_kernel's launches: panel_fits, and channels that do not divide into its units, up to 24576 a matrix (64 rows in turn before: INT4, 1964 rows, 6336 x 1296
+// 383 -> 50 us, 662 rows, three of 2304 x 1264 85 -> 22).  More channels than that still go 64 rows in turn, which is the slower: INT4, 32008 channels, 1032 features, 200
+// rows 67 and 23 here, 4096 features, 1000 rows 466 and 202; F152, 32040 channels, 520 features, 136 rows 80 and 48.  That path is what they have had; the line is no
+// line of speed.
 static inline bool panel_takes(const GemmArgs& a, bool pair) {
   if (panel_fits(a, 4, pair)) return true;
   if (a.epi.norm != PTA_NORM_NONE || a.KT < 2) return false;
@@ -3197,9 +3199,10 @@ static int launch_gemm_own_plan(const GemmArgs& a, const OwnPlan& p, hipStream_t
 }
 
 // 33 to 128 rows by INT4 weights, several rounds of gemm_own_kernel: gemm_panel_kernel, if its plan is that much shorter (both plans' us a little long, the
-// latter's begin with nothing on its way).  K of more than 2048.  us, gemm_own_kernel and it, weights from HBM: three of 4096 x 4096, 65 rows 24.0 and 20.6, 128
+// latter's begin with nothing on its way).  us, gemm_own_kernel and it, weights from HBM: three of 4096 x 4096, 65 rows 24.0 and 20.6, 128
 // rows 28.1 and 24.9; pair of 4096 x 11008, 48 rows 25.4 and 22.5, 64 rows 29.3 and 25.8, 128 rows 42.3 and 36.3 (96 rows 35.7 and 36.0, plans 42.7 and 34.9);
-// 4096 x 11008, 65 rows 21.3 and 20.2.
+// 4096 x 11008, 65 rows 21.3 and 20.2.  K of up to 2048 stays with gemm_own_kernel, which it has had; where the plans differ as much this would be the faster there too (pair
+// of 2048 x 5632, 65 rows 16.9 and 12.8, 128 rows 19.6 and 15.2; 2048 x 12288, 65 rows 16.4 and 13.1; pair of 1792 x 10608, 114 rows 28.2 and 19.9).
 template <class Fmt, bool PAIR>
 static bool panel_before_own(const GemmArgs& a, const OwnPlan& own, PanelPlan& panel) {
   if constexpr (PanelFormat<Fmt>::ok && Fmt::kVec == 1) {

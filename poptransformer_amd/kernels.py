@@ -75,7 +75,7 @@ def linear_workspace_bytes(M, N):
 
 
 def linear_workspace(M, N, device):
-    """Scratch that lets a single-weight `linear` of more than 16 rows split K across workgroups."""
+    """Scratch that lets a single-weight `linear` of more than 16 rows split K across workgroups, and a `linear_then_norm` in any order of more than 8."""
     return torch.empty(linear_workspace_bytes(M, N), dtype=torch.uint8, device=device)
 
 
@@ -371,7 +371,7 @@ def linear(x, weights, outs, biases=None, x_scale=None, swiglu=False, bias=None,
 class RowNorm:
     """The norm that `linear_then_norm` does behind a product: `rmsnorm`, `rmsnorm_fp8_grid` (grid = (exponent, format)), `layer_norm_ce` (beta) or
     `layer_norm_ce_mix` (shift = (previous rows, mixing vectors, results)), into `out`.  any_order: the product's sums may be taken in another order than
-    `linear` takes them, for what is faster with a norm behind it."""
+    `linear` takes them, for what is faster with a norm behind it (and the workspace is used from 9 rows on)."""
 
     def __init__(self, gamma, beta, eps, out=None, grid=None, shift=None, any_order=False):
         prev, mixes, mixed = shift if shift is not None else (None, (), ())
