@@ -283,6 +283,9 @@ class F8Weight:
     def plain(self, value):
         self._plain, self._asked = value, None
 
+    def __getstate__(self):                       # (copies and pickles hold the answer, not the question)
+        return dict(self.__dict__, _plain=self.plain, _asked=None)
+
     @property
     def nbytes(self):
         return self.N * self.K

@@ -131,3 +131,18 @@ def test_a_weight_does_not_wait_for_its_codes():
     for w, out in zip(ws, outs[3:]):
         K.linear(x, [w], [out])
     assert all(torch.equal(a, b) for a, b in zip(outs, outs[3:])) and torch.equal(outs[0], outs[2]) and not torch.equal(outs[0], outs[1])
+
+
+def test_copies_know_their_codes():
+    """A weight may be copied before a product has asked for the answer."""
+    import copy
+    from poptransformer_amd import kernels as K
+    codes = torch.randint(1, 120, (2, 40, 200), dtype=torch.int32, device="cuda").to(torch.uint8)
+    codes[1, 39, 199] = 0xFF
+    x = torch.randn((3, 200), device="cuda").half()
+    for c, plain in zip(codes, (True, False)):
+        copies, out = [f(K.F8Weight(c.contiguous(), scale())) for f in (lambda w: w, copy.copy, copy.deepcopy)], []
+        assert all(w.plain is plain for w in copies)
+        for w in copies:
+            out.append(K.linear(x, [w], [torch.empty((3, 40), dtype=torch.float16, device="cuda")])[0])
+        assert torch.equal(out[0], out[1]) and torch.equal(out[0], out[2])
