@@ -272,9 +272,10 @@ class F8Weight:
         asked = self._asked
         if asked is not None:
             host, done = asked
-            if not torch.cuda.is_current_stream_capturing():
-                done.synchronize()
             there = host.item()
+            if there == 2 and not torch.cuda.is_current_stream_capturing():      # (not if it is there: a wait ends what another thread may be recording)
+                done.synchronize()
+                there = host.item()
             if there != 2:
                 self._plain, self._asked = there == 0, None
         return self._plain

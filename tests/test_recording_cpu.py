@@ -1,4 +1,5 @@
-"""No garbage collection runs while an executor records: a decoder that is no longer used is part of a cycle, and what it recorded must not be destroyed then."""
+"""What stays out of the way of a recording: garbage collections (a decoder that is no longer used is part of a cycle, and what it recorded must not be destroyed then), and waits
+that nothing needs."""
 import contextlib
 import gc
 import threading
@@ -68,3 +69,15 @@ def test_with_two_threads_it_waits_for_the_last(recorded):
     leave.set()
     t.join(10)
     assert gc.isenabled()
+
+
+@pytest.mark.parametrize("answer, plain", [(0, True), (1, False)])
+def test_an_answer_that_is_there_is_not_waited_for(monkeypatch, answer, plain):
+    """A wait for an event ends what another thread may be recording: F8Weight.plain waits only as long as its byte holds 2."""
+    from poptransformer_amd import kernels as K
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: False)
+    for there in (True, False):
+        host, waits = torch.full((1,), answer if there else 2, dtype=torch.uint8), []
+        w = K.F8Weight.__new__(K.F8Weight)
+        w._plain, w._asked = False, (host, types.SimpleNamespace(synchronize=lambda: (waits.append(1), host.fill_(answer))))
+        assert w.plain is plain and w.plain is plain and len(waits) == (not there)
