@@ -3150,6 +3150,7 @@ static OwnPlan plan_gemm_own(const GemmArgs& a) {
     const int tiles = ((a.KT + sl - 1) / sl + OWN_WAVES - 1) / OWN_WAVES;
     rounds = (own_groups(a, nb, PAIR) * row_blocks * sl + cus - 1) / cus;
     double us = 3.2 + rounds * tiles * (0.5 + 0.29 * rows + (PRODUCTS + WEIGHTS / row_blocks) * nb * (PAIR ? 2 : 1));
+    if (normed && OwnStreams<Fmt>::long_decode) us = 3.2 + rounds * tiles * (0.13 * rows + 1.8 * nb);
     if (sl > 1) {
       const double size = (double)a.M * a.mat[0].N / 262144;
       us += normed ? sl * (0.35 + 0.5 * size) + (Fmt::kVec > 1 ? 1.0 : 0.8) : 2.7 * sl - 0.9 + (size > 1 ? 0.5 * sl * (size - 1) : 0.0);
@@ -3166,10 +3167,13 @@ static OwnPlan plan_gemm_own(const GemmArgs& a) {
     }
   // (up to 128 rows and a block of channels a compute unit)
   if (!slices || !a.then || !a.then->any_order || a.M > 128 || a.mat[0].N > 16 * cus || !finish_norm_fits(a)) return best;
-  // with a norm behind it: that plan, or one that is shorter by the other estimate
-  best.us = time(best.nb, best.slices, true, best.rounds);
+  // with a norm behind it: that plan, or one that is shorter by the other estimate.  F152's is one of its own, of blocks: their decoding bounds a workgroup, not its rows'
+  // bytes (548 launches, rms 1 us; with the others' constants 8904 x 1584, 24 rows, 16.5 -> 19.8 us, 5632 x 3072, 17 rows, 16.0 -> 21.4), half a us shorter and of no fewer slices
+  // (11008 x 2048, 100 rows, 1 x 1 33.5 against 2 x 2 31.3).
+  best.us = time(best.nb, best.slices, true, best.rounds) - (OwnStreams<Fmt>::long_decode ? 0.5 : 0.0);
   if (a.M <= (Fmt::kVec == 1 ? 12 : 8) || (a.M <= 16 && a.KT < 80)) return best;
   const bool sliced = best.slices > 1;
+  const int fewest = OwnStreams<Fmt>::long_decode ? best.slices : 1;
   // Not taken, though their estimates are shorter: beyond 64 rows four blocks, and four slices (INT4, 6144 x 4096, 80 rows, 4 x 2 16.0 against 2 x 1 15.4; 11008 x 2048, 112
   // rows, 4 x 3 18.2 against 2 x 2 16.9; F143, 16384 x 2048, 112 rows, 2 x 2 26.1 against 4 x 4 22.4, which is the plan without a norm); of fewer feature tiles, four blocks
   // and more in place of fewer with slices (INT4, 8192 x 4096, 40 rows, 4 x 4 14.6 against 2 x 2 14.0, 11008 x 4096, 20 rows 14.3 against 13.9, F143 8192 x 4096, 40 rows 17.1
@@ -3177,7 +3181,7 @@ static OwnPlan plan_gemm_own(const GemmArgs& a) {
   // place (6144 x 3072, 56 rows, 3 x 3 18.4 against 2 x 2 17.9).
   const int most = row_blocks > 1 || ((sliced || (Fmt::kVec == 1 && a.M <= 16)) && a.KT < (Fmt::kVec == 1 ? 96 : 80)) ? Fmt::kVec > 2 && sliced ? 2 : 3 : own_cap<Fmt, PAIR>(mt);
   for (int nb = 1; nb <= own_cap<Fmt, PAIR>(mt) && nb <= most; ++nb)
-    for (int sl = 1; sl <= (row_blocks > 1 ? 3 : GEMM_MAX_KSPLIT) && room(sl); ++sl) {
+    for (int sl = fewest; sl <= (row_blocks > 1 ? 3 : GEMM_MAX_KSPLIT) && room(sl); ++sl) {
       int rounds;
       const double us = time(nb, sl, true, rounds);
       if (us < best.us) best = OwnPlan{mt, nb, sl, rounds, us};
