@@ -3145,12 +3145,16 @@ static OwnPlan plan_gemm_own(const GemmArgs& a) {
   const int row_blocks = (a.M + 63) / 64;
   const int mt = ((a.M + 15) / 16 + row_blocks - 1) / row_blocks;
   const bool slices = !PAIR && a.count == 1 && a.part;
+  // (of a die, which has its share of each slice's groups: 84 blocks in three slices are 33 workgroups for the 32 compute units of most; 6144 x 1336, 33 rows, F143 14.4 us
+  // against 11.0 in two slices)
+  auto die_rounds = [&](int nb, int sl) { return ((own_groups(a, nb, PAIR) + 7) / 8 * 8 * row_blocks * sl + cus - 1) / cus; };
   auto time = [&](int nb, int sl, bool normed, int& rounds) {
     const double rows = normed ? a.M / 16.0 / row_blocks : mt;         // groups of them that a workgroup reads
     const int tiles = ((a.KT + sl - 1) / sl + OWN_WAVES - 1) / OWN_WAVES;
     rounds = (own_groups(a, nb, PAIR) * row_blocks * sl + cus - 1) / cus;
-    double us = 3.2 + rounds * tiles * (0.5 + 0.29 * rows + (PRODUCTS + WEIGHTS / row_blocks) * nb * (PAIR ? 2 : 1));
-    if (normed && OwnStreams<Fmt>::long_decode) us = 3.2 + rounds * tiles * (0.13 * rows + 1.8 * nb);
+    const int turns = normed ? die_rounds(nb, sl) : rounds;
+    double us = 3.2 + turns * tiles * (0.5 + 0.29 * rows + (PRODUCTS + WEIGHTS / row_blocks) * nb * (PAIR ? 2 : 1));
+    if (normed && OwnStreams<Fmt>::long_decode) us = 3.2 + turns * tiles * (0.13 * rows + 1.8 * nb);
     if (sl > 1) {
       const double size = (double)a.M * a.mat[0].N / 262144;
       us += normed ? sl * (0.35 + 0.5 * size) + (Fmt::kVec > 1 ? 1.0 : 0.8) : 2.7 * sl - 0.9 + (size > 1 ? 0.5 * sl * (size - 1) : 0.0);
@@ -3182,6 +3186,7 @@ static OwnPlan plan_gemm_own(const GemmArgs& a) {
   const int most = row_blocks > 1 || ((sliced || (Fmt::kVec == 1 && a.M <= 16)) && a.KT < (Fmt::kVec == 1 ? 96 : 80)) ? Fmt::kVec > 2 && sliced ? 2 : 3 : own_cap<Fmt, PAIR>(mt);
   for (int nb = 1; nb <= own_cap<Fmt, PAIR>(mt) && nb <= most; ++nb)
     for (int sl = fewest; sl <= (row_blocks > 1 ? 3 : GEMM_MAX_KSPLIT) && room(sl); ++sl) {
+      if (die_rounds(nb, sl) > 1) break;          // (a second round begins with nothing on its way)
       int rounds;
       const double us = time(nb, sl, true, rounds);
       if (us < best.us) best = OwnPlan{mt, nb, sl, rounds, us};

@@ -101,7 +101,9 @@ def test_tensors_that_the_norms_own_entry_points_refuse():
 ANY_ORDER = [("int4", 12, 11008, 2048, 1, 1), ("int4", 13, 11008, 2048, 1, 4), ("int4", 16, 1024, 64, 1, 1), ("int4", 20, 11008, 4096, 2, 2), ("int4", 64, 4104, 4096, 1, 2), ("int4", 100, 16392, 2048, 4, 4),
              ("int4", 128, 3072, 768, 1, 3), ("int4", 129, 3072, 768, 1, 1), ("F143", 8, 13704, 4096, 1, 1), ("F143", 9, 13704, 4096, 1, 2), ("F143", 16, 11008, 1032, 1, 3), ("F143", 17, 8192, 2056, 3, 4),
              ("F143", 40, 4096, 4104, 2, 2), ("F143", 64, 13696, 4096, 2, 4), ("f16", 12, 16392, 2040, 1, 4), ("f16", 24, 11008, 4096, 1, 2), ("f16", 31, 2824, 1016, 1, 2), ("f16", 60, 6144, 3080, 2, 2),
-             ("f16", 80, 5632, 2048, 1, 2), ("F152", 33, 4096, 1024, 2, 4), ("F152", 24, 8904, 1584, 2, 2), ("F152", 17, 5632, 3072, 1, 1)]
+             ("f16", 80, 5632, 2048, 1, 2), ("F152", 33, 4096, 1024, 2, 4), ("F152", 24, 8904, 1584, 2, 2), ("F152", 17, 5632, 3072, 1, 1),
+             # a slice's groups by eights: 84 blocks in three slices are two rounds
+             ("F143", 33, 6144, 1336, 2, 2), ("f16", 33, 6144, 1336, 3, 2), ("f16", 128, 8904, 3584, 1, 1)]
 
 
 @pytest.mark.parametrize("kind, M, Kd, N, alone, any_order", ANY_ORDER)
